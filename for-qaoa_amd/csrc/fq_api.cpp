@@ -227,6 +227,7 @@ struct TimingRec {
     int kind;
     hipEvent_t e0, e1;
     double bytes;
+    int count;   // passes in it
 };
 
 struct fq_state {
@@ -234,6 +235,9 @@ struct fq_state {
     size_t elem = 16, bytes = 0;
     void *sv = nullptr;
     hipStream_t own = nullptr, stream = nullptr;
+    // chunked runs (run_chunks): two streams forked from and joined to `stream`
+    hipStream_t side[2] = {nullptr, nullptr};
+    hipEvent_t forked = nullptr, joined[2] = {nullptr, nullptr};
     int qmap[FQ_MAXN];
     double init_amp = 0;
     // product of the RX factors of tile passes that left theirs to a later
@@ -291,7 +295,7 @@ static int timing_collect(fq_state *st)
             break;
         }
         st->t_ms[r.kind] += ms;
-        st->t_cnt[r.kind] += 1;
+        st->t_cnt[r.kind] += r.count;
         st->t_bytes[r.kind] += r.bytes;
         st->pool.push_back(r.e0);
         st->pool.push_back(r.e1);
@@ -301,9 +305,9 @@ static int timing_collect(fq_state *st)
     return rc;
 }
 
-// Wrap one launch with events when timing is on.
+// Wrap one launch (or the launches of `count` passes) with events when timing is on.
 template <typename F>
-static int timed(fq_state *st, int kind, double bytes, F &&launch)
+static int timed(fq_state *st, int kind, double bytes, F &&launch, int count = 1)
 {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (st->timing) {
@@ -333,7 +337,7 @@ static int timed(fq_state *st, int kind, double bytes, F &&launch)
         return set_err(FQ_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
     }
     if (st->timing)
-        st->pending.push_back({kind, e0, e1, bytes});
+        st->pending.push_back({kind, e0, e1, bytes, count});
     return FQ_OK;
 }
 
@@ -892,6 +896,14 @@ extern "C" int fq_state_destroy(fq_state *st)
         budget_give(st->bytes);
     hipFree(st->aux);
     hipFree(st->d_grad);
+    for (int i = 0; i < 2; ++i) {
+        if (st->side[i])
+            hipStreamDestroy(st->side[i]);
+        if (st->joined[i])
+            hipEventDestroy(st->joined[i]);
+    }
+    if (st->forked)
+        hipEventDestroy(st->forked);
     if (st->own) {
         own_stream(st->own, false);
         hipStreamDestroy(st->own);
@@ -1147,6 +1159,166 @@ static int pass_args(int N, int dtype, const std::vector<int> &tile, const std::
     return FQ_OK;
 }
 
+// The factor of a tile pass: sigma^(#gates) of each RX set (rx_tform: *t the
+// butterfly coefficient) times what earlier passes left pending.  It goes
+// into the cost phase, or is applied before the stores (apply), or stays
+// pending for a later pass of the same fq_run (cost or not defer: it does not).
+struct PassFactor {
+    double t = 0, pre_t = 0, re = 1.0, im = 0.0;
+    bool apply = false;
+};
+
+static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const double *pre_beta, bool cost, bool defer)
+{
+    PassFactor f;
+    double sr = st->pending_re, si = st->pending_im;
+    auto absorb = [&](double b, double *t) {
+        double gr, gi;
+        rx_tform(b, st->dtype, st->in_run, t, &gr, &gi);
+        for (size_t k = 0; k < ngates; ++k) {
+            const double nr = sr * gr - si * gi;
+            si = sr * gi + si * gr;
+            sr = nr;
+        }
+    };
+    absorb(beta, &f.t);
+    if (pre_beta)
+        absorb(*pre_beta, &f.pre_t);
+    const bool keep = !cost && defer;
+    if (!keep) {
+        f.re = sr;
+        f.im = si;
+        f.apply = !cost;
+    }
+    st->pending_re = keep ? sr : 1.0;
+    st->pending_im = keep ? si : 0.0;
+    return f;
+}
+
+// A tile pass on the compile-time kernel (fq_mix.hip), ready to launch over
+// all its tiles or a range of them.
+struct MixPass {
+    MixArgs a;
+    int K = 0, kind = 0, mir = 0;
+    bool lane = false;  // RX on one more thread bit by lane operations
+    double bytes = 0;   // read and written by the whole pass
+};
+
+// Arguments as tile_pass; queues the phase table of a cost pass.  The mirror pass may be a boundary pass too: the phase of a
+// mirror element is that of the N-qubit index it stands for (Cut(b) = Cut(~b)).
+static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
+                       fq_graph *g, double gamma, bool cost, bool first, int z2, const double *pre_beta, bool defer,
+                       MixPass &mp)
+{
+    const int N = st->N, Q = (int)tile.size(), A = mix_a_log(st->dtype, Q), nthr = Q - A;
+    const Geom geom = make_geom(N, tile, A);
+    MixArgs &a = mp.a;
+    memset(&a, 0, sizeof(a));
+    a.N = N;
+    a.Q = Q;
+    a.nh = geom.nh;
+    if (make_runs(geom.hpos, geom.nh, a.hruns) > FQ_MAX_RUNS)
+        return set_err(FQ_ERR_ARG, "internal: tile geometry needs more than %d bit runs", FQ_MAX_RUNS);
+    uint32_t gm = 0;
+    for (int p : gates) {
+        const auto it = std::find(tile.begin(), tile.end(), p);
+        if (it == tile.end())
+            return set_err(FQ_ERR_ARG, "internal: gate %d not in tile", p);
+        gm |= 1u << (it - tile.begin());
+    }
+    // exchanges: as many as it takes from the top thread bit down to the
+    // lowest gated one, one fewer if only the bit below them is left and RX on
+    // it can run on lanes
+    int K = 0, low = nthr;
+    for (int i = nthr - 1; i >= 0; --i)
+        if ((gm >> i) & 1u)
+            low = i;
+    K = (nthr - low + A - 1) / A;
+    if (K > 1 && low == nthr - (K - 1) * A - 1 && mix_lane_bit(Q, A, K - 1)) {
+        --K;
+        mp.lane = true;
+    }
+    for (int i = 0; i < Q; ++i)
+        a.tpos[i] = geom.tpos[i];
+    auto start = [&](int l) { return l == 0 ? nthr : std::max(0, nthr - A * (K - l + 1)); };
+    uint32_t left = mp.lane ? gm & ~(1u << low) : gm;
+    for (int l = 0; l <= K; ++l) {
+        const uint32_t m = (left >> start(l)) & ((1u << A) - 1u);
+        a.gates_w |= m << (A * l);
+        left &= ~(m << start(l));
+    }
+    for (int r = 0; r < A; ++r) {
+        a.rpos0_w |= (uint32_t)geom.tpos[nthr + r] << (6 * r);
+        a.rposk_w |= (uint32_t)geom.tpos[start(K) + r] << (6 * r);
+    }
+    a.order = getenv("FQ_TILE_ORDER") ? tile_order() : 3;   // (k_mix)
+    a.ntiles = 1ull << geom.nh;
+    if (z2 != Z2_OFF) {
+        // the lower half is the tiles whose top index bit (qubit N-1) is 0; a
+        // mirror pass pairs tile tau with ~tau instead
+        const bool ok = geom.nh >= 1 && (z2 == Z2_LOWER ? geom.hpos[geom.nh - 1] == N - 1
+                                                        : tile.back() == N - 1 && (!cost || first || pre_beta));
+        if (!ok)
+            return set_err(FQ_ERR_ARG, "internal: tile does not fit the half-state pass");
+        a.ntiles = 1ull << (geom.nh - 1);
+        if (z2 >= Z2_MIRROR)
+            for (int i = 0; i + 1 < Q; ++i)
+                a.mirror_pm += 1ull << tile[i];
+    }
+    const PassFactor f = pass_factor(st, gates.size(), beta, pre_beta, cost, defer);
+    a.t = f.t;
+    a.pre_t = f.pre_t;
+    a.tf = (float)f.t;   // exact for complex64 (rx_tform rounds t to FP32)
+    a.pre_tf = (float)f.pre_t;
+    a.scale_re = f.re;
+    a.scale_im = f.im;
+    a.apply_scale = f.apply;
+    if (cost) {
+        // phase table of the layout the cost phase runs in: layout 0, or for a
+        // boundary pass the last one (thread bits = the tile bits outside it)
+        Geom cgeom = geom;
+        if (pre_beta && K > 0) {
+            std::vector<int> t2;
+            for (int i = 0; i < Q; ++i)
+                if (i < start(K) || i >= start(K) + A)
+                    t2.push_back(tile[i]);
+            for (int r = 0; r < A; ++r)
+                t2.push_back(tile[start(K) + r]);
+            cgeom = make_geom(N, t2, A);
+        }
+        TileArgs ca;
+        geom_to_args(cgeom, ca);
+        ca.ntiles_run = a.ntiles;
+        if (int rc = get_plan(g, cgeom, &ca.plan, st->stream))
+            return rc;
+        set_cost(ca, gamma, st->init_amp);
+        if (int rc = prepare_phases(st, ca, A))
+            return rc;
+        a.has_rr = ca.has_rr;
+        a.init_amp = st->init_amp;
+    }
+    a.ntab = a.ntiles;
+    mp.K = K;
+    mp.kind = pre_beta ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
+    mp.mir = z2 == Z2_MIRROR ? 1 : z2 == Z2_EXPAND ? 2 : 0;
+    // a half-state pass reads and writes half the state; the expanding one
+    // writes the whole state
+    mp.bytes = (double)st->bytes * (z2 == Z2_OFF ? (first ? 1.0 : 2.0) : z2 == Z2_EXPAND ? 1.5 : first ? 0.5 : 1.0);
+    return FQ_OK;
+}
+
+static int mix_pass(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
+                    fq_graph *g, double gamma, bool cost, bool first, int kind, int z2, const double *pre_beta,
+                    bool defer)
+{
+    MixPass mp;
+    if (int rc = mix_prepare(st, tile, gates, beta, g, gamma, cost, first, z2, pre_beta, defer, mp))
+        return rc;
+    return timed(st, kind, mp.bytes, [&] {
+        return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, mp.a, st->d_phase, st->stream);
+    });
+}
+
 // One tile pass with RX on gate positions (and optionally the cost phase).
 // pre_beta (with cost, not first, not a mirror pass): RX(*pre_beta) on the
 // same positions before the cost phase -- the pass that ends one layer and
@@ -1161,8 +1333,12 @@ static int tile_pass(fq_state *st, const std::vector<int> &tile, const std::vect
                      double beta, fq_graph *g, double gamma, bool cost, bool first, int kind,
                      int z2 = Z2_OFF, const double *pre_beta = nullptr, bool defer = false)
 {
-    if (pre_beta && (!cost || first || z2 >= Z2_MIRROR))
+    if (pre_beta && (!cost || first))
         return set_err(FQ_ERR_ARG, "internal: a layer-boundary pass needs the cost phase of a later layer");
+    if (mix_a_log(st->dtype, (int)tile.size()) > 0)
+        return mix_pass(st, tile, gates, beta, g, gamma, cost, first, kind, z2, pre_beta, defer);
+    if (pre_beta && z2 >= Z2_MIRROR)
+        return set_err(FQ_ERR_ARG, "internal: no mirror boundary pass at this tile width");
     TileArgs a;
     Geom geom;
     if (int rc = pass_args(st->N, st->dtype, tile, gates, cost, z2, a, geom, 0, first))
@@ -1552,12 +1728,15 @@ static bool layer_pipe()
 struct LayerPlan {
     std::vector<FusedPass> ps;
     int end1;
+    int open0 = 0;   // pipelined: the pass that opens layer 0 (0 or end1)
+    bool split = false;  // exec_plan's split of the qubits (layers end on passes 0 and 2)
+    int chunk = 0;   // log2 amplitudes of a chunk (exec_plan; 0: passes run over the whole state)
 };
 
 static LayerPlan layer_plan(int N, int dtype, bool z2)
 {
     const int Qmax = z2 ? std::min(pass_tile_q(dtype), N - 1) : pass_tile_q(dtype);
-    LayerPlan lp{cover_passes(N, Qmax, dtype), -1};
+    LayerPlan lp{cover_passes(N, Qmax, dtype), -1, 0, false, 0};
     const int m = (int)lp.ps.size();
     if (layer_pipe() && m >= (z2 ? 3 : 2)) {
         lp.end1 = z2 ? 1 : m - 1;
@@ -1567,74 +1746,210 @@ static LayerPlan layer_plan(int N, int dtype, bool z2)
     return lp;
 }
 
-// The tile passes of layer p of P (pass 0 the low contiguous tile; z2:
-// half-state passes, the last one the mirror pass).  In layer order, layer p
-// runs passes 0..m-1 with its cost phase in pass 0.  Pipelined: the cost
-// phase is diagonal, so it can run in any pass; the pass that ends layer p
-// applies RX(beta_p), the phase of gamma_{p+1} and RX(beta_{p+1}) on its
-// qubits, which opens layer p+1.  Layers end alternately on end1 and pass 0,
-// so every layer after the first runs m-1 passes: 1 + P(m-1) passes in all
-// instead of Pm.  Every RX of a layer still follows its cost phase and
-// precedes the next one, and RX gates on distinct qubits commute.  Layer p
-// expects layers 0..p-1 to have run with the same plan.  expand: the last
-// layer's mirror pass also writes the upper half of the full state.
-static int run_layer(fq_state *st, fq_graph *g, const LayerPlan &lp, int p, int P, const double *gammas,
-                     const double *betas, bool z2, bool expand)
+// Chunked runs: log2 bytes of a chunk (0: off); FQ_CHUNK (environment, read
+// per call).  128 MiB by default, half of the memory-side cache, since two
+// chunks are in flight (run_layers).  Measured on MI355X per layer, N=30
+// complex128 fused: no chunks 14.59 ms; one stream with chunks of 64, 128, 256
+// and 512 MiB 15.9, 15.2, 14.2 and 15.2 ms; two streams with 64, 128 and
+// 256 MiB 13.3, 12.8 and 14.5 ms.
+static int chunk_log()
+{
+    const char *e = getenv("FQ_CHUNK");
+    return e ? atoi(e) : 27;
+}
+
+// The plan fq_run uses for P layers: layer_plan's, except that a plan of three
+// passes splits the qubits otherwise: pass 1 takes the 9 qubits right above
+// pass 0's and pass 2 the top ones, and layers end alternately on passes 0 and
+// 2, also on the half state (whose pass 2 is the mirror pass), so that pass 2 has
+// few gates, all in reach of one exchange.  Where the stored state is larger
+// than the memory-side cache (256 MiB), the launches between two uses of pass 2
+// (pass 1, the boundary pass 0, pass 1), which stay within the low `chunk`
+// qubits, run chunk by chunk, and a chunk crosses the HBM once for the three of
+// them: per layer at N=30 complex128 fused 14.47 -> 12.71 ms, N=32 complex64
+// 30.5 -> 27.8, half state N=30 complex64 3.88 -> 3.58.  9 qubits: per layer at N=30 complex128 fused 14.41, 12.72,
+// 12.80 and 13.07 ms with 7, 8, 9 and 10; N=32 complex64 30.6, 30.6, 27.9 and
+// 29.0; half state N=30 complex128 7.62, 6.79, 6.66 and 6.88.  Where the plan
+// of tuning knobs is asked for, layer_plan's passes run as they are.
+#define FQ_CACHE_LOG 28
+static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
+{
+    LayerPlan lp = layer_plan(N, dtype, z2);
+    for (const char *k : {"FQ_TILE_Q", "FQ_PASS_BLOCK", "FQ_CARRIER_GATES", "FQ_LAYER_PIPE"})
+        if (getenv(k))
+            return lp;
+    const int elem_log = dtype == FQ_C128 ? 4 : 3, Ns = z2 ? N - 1 : N;
+    if (lp.ps.size() != 3)
+        return lp;
+    const int Q = tile_max_q(dtype), rest = N - Q;
+    const int n1 = std::max(9, rest - (Q - carriers_for(dtype))), n2 = rest - n1;
+    if (n2 < 1)
+        return lp;
+    const int c1 = Q - n1, c2 = Q - n2;   // carried low qubits
+    FusedPass p0, p1, p2;
+    p0.tile = low_tile(Q);
+    p1.tile = low_tile(c1);
+    p2.tile = low_tile(c2);
+    for (int q = Q; q < N; ++q) {
+        FusedPass &p = q < Q + n1 ? p1 : p2;
+        p.tile.push_back(q);
+        p.gates.push_back(q);
+    }
+    // the carried qubits' RX goes to pass 1, which is no boundary pass; the
+    // one that a single exchange of pass 0 does not reach to pass 2
+    for (int q = 0; q < Q; ++q) {
+        const bool reach = q >= Q - 2 * mix_a_log(dtype, Q);
+        (q < c1 ? p1 : !reach && q < c2 ? p2 : p0).gates.push_back(q);
+    }
+    lp.ps = {p0, p1, p2};
+    lp.end1 = 2;
+    lp.split = true;
+    const int chunk = chunk_log() - elem_log;
+    if (Ns + elem_log > FQ_CACHE_LOG && chunk >= Q + n1 && chunk < Ns)
+        lp.chunk = chunk;
+    // the last layer must end on the mirror pass, which writes the full state
+    lp.open0 = z2 && P % 2 == 0 ? 2 : 0;
+    return lp;
+}
+
+// One pass of a run: pass index, kind, layer.
+enum { STEP_FIRST = 0, STEP_COST = 1, STEP_PLAIN = 2, STEP_BOUNDARY = 3 };
+struct Step {
+    int pass, kind, layer;
+};
+
+// The passes of layer p of P in launch order.  In layer order, layer p runs
+// passes 0..m-1 with its cost phase in pass 0.  Pipelined: the cost phase is
+// diagonal, so it can run in any pass; the pass that ends layer p applies
+// RX(beta_p), the phase of gamma_{p+1} and RX(beta_{p+1}) on its qubits, which
+// opens layer p+1.  Layers end alternately on two passes (end1 and pass 0), so
+// every layer after the first runs m-1 passes: 1 + P(m-1) passes in all
+// instead of Pm.  Every RX of a layer still follows its cost phase and precedes
+// the next one, and RX gates on distinct qubits commute.  Layer p expects
+// layers 0..p-1 to have run with the same plan.
+static void layer_steps(const LayerPlan &lp, int p, int P, std::vector<Step> &out)
+{
+    const int m = (int)lp.ps.size();
+    const bool last = p + 1 == P;
+    if (lp.end1 < 0) {
+        for (int i = 0; i < m; ++i)
+            out.push_back({i, i > 0 ? STEP_PLAIN : p == 0 ? STEP_FIRST : STEP_COST, p});
+        return;
+    }
+    const int open = p % 2 == 0 ? lp.open0 : lp.open0 == 0 ? lp.end1 : 0;
+    const int e = open == 0 ? lp.end1 : 0;   // the pass that ends layer p
+    if (p == 0)
+        out.push_back({open, STEP_FIRST, p});
+    // (a half-state plan that ends on pass 1 has the mirror pass among the
+    // middle ones, and it comes last in the last layer)
+    if (last && !lp.split)
+        out.push_back({e, STEP_PLAIN, p});
+    for (int i = 1; i < m; ++i)
+        if (i != lp.end1)
+            out.push_back({i, STEP_PLAIN, p});
+    if (last && lp.split)
+        out.push_back({e, STEP_PLAIN, p});
+    if (!last)
+        out.push_back({e, STEP_BOUNDARY, p});
+}
+
+// The passes of a group, chunk by chunk (2^nlog chunks), alternate chunks on
+// two streams of the state: while one chunk's first pass reads from the HBM,
+// the other's later passes run from the cache.  Every pass has its phase table
+// (at most one of them is a cost pass) before the streams fork.
+static int run_chunks(fq_state *st, std::vector<MixPass> &group, double bytes, int nlog)
+{
+    for (int i = 0; i < 2; ++i) {
+        if (!st->side[i])
+            FQ_HIP(hipStreamCreateWithFlags(&st->side[i], hipStreamNonBlocking));
+        if (!st->joined[i])
+            FQ_HIP(hipEventCreateWithFlags(&st->joined[i], hipEventDisableTiming));
+    }
+    if (!st->forked)
+        FQ_HIP(hipEventCreateWithFlags(&st->forked, hipEventDisableTiming));
+    return timed(st, FQ_K_FUSED, bytes, [&] {
+        hipError_t e = hipEventRecord(st->forked, st->stream);
+        for (int i = 0; i < 2 && e == hipSuccess; ++i)
+            e = hipStreamWaitEvent(st->side[i], st->forked, 0);
+        for (uint64_t c = 0; c < 1ull << nlog && e == hipSuccess; ++c)
+            for (const MixPass &mp : group) {
+                MixArgs a = mp.a;
+                a.ntiles >>= nlog;
+                a.tile0 = c * a.ntiles;
+                e = launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, a, st->d_phase, st->side[c & 1]);
+                if (e != hipSuccess)
+                    break;
+            }
+        // joined also after a failed launch: what was queued precedes the
+        // stream's later work
+        for (int i = 0; i < 2; ++i) {
+            hipError_t j = hipEventRecord(st->joined[i], st->side[i]);
+            if (j == hipSuccess)
+                j = hipStreamWaitEvent(st->stream, st->joined[i], 0);
+            e = e == hipSuccess ? j : e;
+        }
+        return e;
+    }, (int)group.size());
+}
+
+// Layers [p0, p1) of P.  expand: the last layer's mirror pass also writes the
+// upper half of the full state.
+static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, int p1, int P, const double *gammas,
+                      const double *betas, bool z2, bool expand)
 {
     const std::vector<FusedPass> &ps = lp.ps;
     const int m = (int)ps.size();
-    const bool last = p + 1 == P;
-    auto mode = [&](int i) {
-        if (!z2)
-            return (int)Z2_OFF;
-        return i + 1 < m ? (int)Z2_LOWER : last && expand ? (int)Z2_EXPAND : (int)Z2_MIRROR;
+    std::vector<Step> seq;
+    for (int p = p0; p < p1; ++p)
+        layer_steps(lp, p, P, seq);
+    // a pass that stays within one chunk
+    auto local = [&](const Step &s) {
+        return lp.chunk > 0 && *std::max_element(ps[s.pass].tile.begin(), ps[s.pass].tile.end()) < lp.chunk;
     };
-    // the passes of this layer in launch order: (pass, kind) with kind 0 the
-    // layer-0 launch-control pass, 1 a cost pass of layer order, 2 a plain
-    // pass, 3 the boundary pass that opens layer p+1
-    std::vector<std::pair<int, int>> seq;
-    if (lp.end1 < 0) {
-        for (int i = 0; i < m; ++i)
-            seq.push_back({i, i == 0 ? (p == 0 ? 0 : 1) : 2});
-    } else {
-        const int e = p % 2 == 0 ? lp.end1 : 0;   // the pass that ends layer p (the other one opened it)
-        if (p == 0)
-            seq.push_back({0, 0});
-        if (last)
-            seq.push_back({e, 2});
-        for (int i = 1; i < m; ++i)
-            if (i != lp.end1)
-                seq.push_back({i, 2});
-        if (!last)
-            seq.push_back({e, 3});
+    auto cost = [](const Step &s) { return s.kind != STEP_PLAIN; };
+    for (size_t k = 0; k < seq.size();) {
+        // passes of one group: a run of local ones with at most one cost
+        // phase among them (one phase table), else a single pass
+        size_t n = 1;
+        if (local(seq[k])) {
+            bool c = cost(seq[k]);
+            for (; k + n < seq.size() && local(seq[k + n]) && !(c && cost(seq[k + n])); ++n)
+                c = c || cost(seq[k + n]);
+        }
+        std::vector<MixPass> group(n > 1 ? n : 0);
+        double bytes = 0;
+        for (size_t i = 0; i < n; ++i) {
+            const Step &s = seq[k + i];
+            const FusedPass &fp = ps[s.pass];
+            const bool last = s.layer + 1 == P && k + i + 1 == seq.size();
+            const int mode = !z2 ? (int)Z2_OFF
+                             : s.pass + 1 < m ? (int)Z2_LOWER
+                                              : s.layer + 1 == P && s.kind == STEP_PLAIN && expand ? (int)Z2_EXPAND
+                                                                                                    : (int)Z2_MIRROR;
+            const bool bd = s.kind == STEP_BOUNDARY;
+            const int L = bd ? s.layer + 1 : s.layer;
+            const double gamma = cost(s) ? gammas[L] : 0.0;
+            const double *pre = bd ? &betas[s.layer] : nullptr;
+            // plain passes leave their RX factor to the next cost pass, except
+            // the run's very last pass, which leaves the state exact
+            int rc;
+            if (n == 1)
+                rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, FQ_K_FUSED,
+                               mode, pre, !last);
+            else
+                rc = mix_prepare(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, mode, pre,
+                                 !last, group[i]);
+            if (rc)
+                return rc;
+            if (n > 1)
+                bytes += group[i].bytes;
+        }
+        if (n > 1) {
+            if (int rc = run_chunks(st, group, bytes, (z2 ? st->N - 1 : st->N) - lp.chunk))
+                return rc;
+        }
+        k += n;
     }
-    for (size_t k = 0; k < seq.size(); ++k) {
-        const int i = seq[k].first, kind = seq[k].second;
-        // plain passes leave their RX factor to the next cost pass, except the
-        // run's very last pass, which leaves the state exact
-        const bool defer = !(last && k + 1 == seq.size());
-        int rc;
-        if (kind == 2)
-            rc = tile_pass(st, ps[i].tile, ps[i].gates, betas[p], g, 0.0, false, false, FQ_K_FUSED, mode(i),
-                           nullptr, defer);
-        else if (kind == 3)
-            rc = tile_pass(st, ps[i].tile, ps[i].gates, betas[p + 1], g, gammas[p + 1], true, false, FQ_K_FUSED,
-                           mode(i), &betas[p]);
-        else
-            rc = tile_pass(st, ps[i].tile, ps[i].gates, betas[p], g, gammas[p], true, kind == 0, FQ_K_FUSED,
-                           mode(i));
-        if (rc)
-            return rc;
-    }
-    return FQ_OK;
-}
-
-static int run_layers(fq_state *st, fq_graph *g, int P, const double *gammas, const double *betas, bool z2)
-{
-    const LayerPlan lp = layer_plan(st->N, st->dtype, z2);
-    for (int p = 0; p < P; ++p)
-        if (int rc = run_layer(st, g, lp, p, P, gammas, betas, z2, true))
-            return rc;
     return FQ_OK;
 }
 
@@ -1690,11 +2005,11 @@ extern "C" int fq_run(fq_state *st, fq_graph *g, int P, const double *gammas, co
         // half z_{N-1} = 0 and the other half is written once at the end.
         if (N < 3)
             return set_err(FQ_ERR_ARG, "the half-state schedule needs N >= 3");
-        return run_layers(st, g, P, gammas, betas, true);
+        return run_layers(st, g, exec_plan(N, st->dtype, true, P), 0, P, P, gammas, betas, true, true);
     }
     if (schedule != FQ_SCHED_FUSED)
         return set_err(FQ_ERR_ARG, "unknown schedule %d", schedule);
-    return run_layers(st, g, P, gammas, betas, false);
+    return run_layers(st, g, exec_plan(N, st->dtype, false, P), 0, P, P, gammas, betas, false, true);
 }
 
 extern "C" int fq_layer_passes(int N, int dtype, int schedule, int max_pass, int *npass, int *tile_q,
@@ -2763,8 +3078,8 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
                     v->pending_im = 0.0;
                 }
                 v->in_run = true;   // a slot runs fq_run's layers on a QAOA state
-                if (int rc = run_layer(v, h.g, sb->slot_plan, L, h.P, h.gammas.data(), h.betas.data(), sb->z2,
-                                       false))
+                if (int rc = run_layers(v, h.g, sb->slot_plan, L, L + 1, h.P, h.gammas.data(), h.betas.data(), sb->z2,
+                                        false))
                     return rc;
             }
         }

@@ -295,6 +295,25 @@ __device__ __forceinline__ uint64_t unpack_runs_uniform(uint64_t x, const BitRun
     return o;
 }
 
+// k-th tile of this work-group in a persistent pass of G = gridDim.x groups:
+//   order 0: k*G + b (the groups sweep the tiles together),
+//   order 1: the groups of one XCD (dispatched round-robin, b mod 8) take
+//            consecutive tiles of each sweep,
+//   order 2: one contiguous range of tiles per group,
+//   order 3: as 0 with one work-group per tile (no persistence).
+// Returns ntiles or more once the group has no tile left.
+__device__ __forceinline__ uint64_t tile_of(uint32_t order, uint64_t ntiles, uint64_t k)
+{
+    const uint64_t G = gridDim.x, b = blockIdx.x;
+    if (order == 1)
+        return k * G + (b & 7) * (G >> 3) + (b >> 3);
+    if (order == 2) {
+        const uint64_t per = (ntiles + G - 1) / G;
+        return k < per ? b * per + k : ntiles;
+    }
+    return k * G + b;
+}
+
 // Element offsets of a thread's 2^A_LOG registers: o[j] = sum of 2^pos[r]
 // over the set bits r < NB of j, from the packed positions pos_w (pos[r] in
 // bits 6r..6r+5), recomputed in scalar registers at each call (scalar_opaque).

@@ -85,6 +85,27 @@ struct TileArgs {
     PlanDev plan;
 };
 
+// One pass of the compile-time tile kernel (fq_mix.hip).
+enum { MIX_PLAIN = 0, MIX_FIRST = 1, MIX_COST = 2, MIX_BOUNDARY = 3 };
+struct MixArgs {
+    int N, Q, nh;
+    int has_rr;              // any register-register edge in the plan
+    BitRuns hruns;           // tile index -> high positions
+    uint8_t tpos[16];        // position of each tile bit (thread bits, then register bits)
+    uint32_t rpos0_w;        // positions of the register bits of layout 0, 6 bits each
+    uint32_t rposk_w;        // and of the last layout
+    uint32_t gates_w;        // gated register bits of layout l at bit A l
+    uint32_t order;          // tile order of the persistent loop
+    uint64_t tile0, ntiles;  // tiles [tile0, tile0 + ntiles) of this launch
+    uint64_t ntab;           // tiles of the whole pass (rows of its phase table)
+    uint64_t mirror_pm;      // mirror pass: sum of 2^p over the real tile positions
+    double t, pre_t;         // rx_tform coefficients of this layer and of the one before
+    float tf, pre_tf;
+    double scale_re, scale_im;  // factor of the pass: in the cost phase, or before the
+    int apply_scale;            // stores (apply_scale)
+    double init_amp;
+};
+
 // Tiles a launch processes (a Z2-reduced state runs the lower half only).
 __host__ __device__ inline uint64_t run_tiles(const TileArgs &a)
 {
@@ -132,6 +153,15 @@ hipError_t launch_tile(int dtype, int a_log, bool cost, bool first, bool gates, 
 // Layer-boundary pass: RX(pre) on the pass's qubits, cost phase, RX(rx).
 hipError_t launch_tile_pre(int dtype, int a_log, void *sv, const TileArgs &a, const double2 *ptab,
                            hipStream_t stream);
+// Tile passes of fq_mix.hip.  mix_a_log: register bits per thread of its
+// instance for tiles of 2^Q amplitudes (0: none).  k: exchanges one way (they
+// reach the tile bits from Q - (k + 1) A up), lane: RX also on the bit below
+// those, where mix_lane_bit says there is such an instance; kind MIX_*, mir:
+// 0, the half-state mirror pass (1; 2 writes the full state's upper half too).
+int mix_a_log(int dtype, int Q);
+bool mix_lane_bit(int Q, int A, int k);
+hipError_t launch_mix(int dtype, int k, bool lane, int kind, int mir, void *sv, const MixArgs &a, const double2 *ptab,
+                      hipStream_t stream);
 // Mirror pass of a Z2-reduced state: the top register bit of the virtual tile
 // selects the complementary tile (complemented element offsets) and RX on it
 // is the butterfly of the global spin flip.  expand: also write the upper

@@ -105,25 +105,6 @@ __device__ __forceinline__ int deposit(int x, unsigned mask, int q)
     return e;
 }
 
-// k-th tile of this work-group in a persistent pass of G = gridDim.x groups:
-//   order 0: k*G + b (the groups sweep the tiles together),
-//   order 1: the groups of one XCD (dispatched round-robin, b mod 8) take
-//            consecutive tiles of each sweep,
-//   order 2: one contiguous range of tiles per group,
-//   order 3: as 0 with one work-group per tile (no persistence).
-// Returns ntiles or more once the group has no tile left.
-__device__ __forceinline__ uint64_t tile_at(const TileArgs &a, uint64_t ntiles, uint64_t k)
-{
-    const uint64_t G = gridDim.x, b = blockIdx.x;
-    if (a.order == 1)
-        return k * G + (b & 7) * (G >> 3) + (b >> 3);
-    if (a.order == 2) {
-        const uint64_t per = (ntiles + G - 1) / G;
-        return k < per ? b * per + k : ntiles;
-    }
-    return k * G + b;
-}
-
 // Hides the value of an LDS base index from the compiler between a phase's
 // reads and its write-back, so the write-back recomputes its 2^A_LOG
 // addresses (one add each) instead of keeping them live in VGPRs through the
@@ -280,7 +261,7 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
     const double2 *rr_tab = COST ? thr_tab + ((size_t)(1 + A_LOG) << nthr) : nullptr;
 
     uint64_t kt = 0;
-    uint64_t tile = tile_at(a, ntiles, 0);
+    uint64_t tile = tile_of(a.order, ntiles, 0);
     // compile-time tile width: lane i of each wave holds factor i of the
     // tile's phase-table row, loaded one tile ahead with the amplitudes
     // (not in the complex64 read-write cost passes: the boundary pass
@@ -335,7 +316,7 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
         }
     }
     while (tile < ntiles) {
-        const uint64_t next = tile_at(a, ntiles, ++kt);
+        const uint64_t next = tile_of(a.order, ntiles, ++kt);
 
         // Cost phase: exp(i*gamma*s/2), s = 2*Cut - W, of register j is the
         // product of the thread's base factor, one factor per register bit

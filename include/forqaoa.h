@@ -225,14 +225,17 @@ int fq_slab_collect(fq_slab *sb, int *slots, double *expect, double *norm2, int 
 /* Amplitudes of one slot (logical = physical order).  Waits. */
 int fq_slab_copy_out(fq_slab *sb, int slot, void *host, size_t bytes);
 
-/* The tile passes one layer of FQ_SCHED_FUSED or FQ_SCHED_Z2 runs for N
- * qubits (no counterpart in the reference; host-only, no device needed):
+/* The tile passes that cover one layer of FQ_SCHED_FUSED or FQ_SCHED_Z2 for N
+ * qubits (no counterpart in the reference; host-only, no device needed; fq_run
+ * launches as many, but with three passes it may deal the qubits above pass 0
+ * out differently and run passes that stay within a part of the state part by
+ * part, environment FQ_CHUNK):
  * *npass passes of *tile_q positions each; pass p's tile positions (thread
  * bits first, the last ones register bits) in tiles[16*p .. 16*p+15] (-1
  * padded) and its RX targets as the bit mask gates[p].  In layer order pass
  * 0 applies every layer's cost phase; with pipelined layers it applies layer
- * 0's, and pass 0 and the last pass (FQ_SCHED_FUSED) or pass 1 (FQ_SCHED_Z2)
- * alternately end a layer and apply the next one's.  max_pass bounds the
+ * 0's, and pass 0 and another pass alternately end a layer and apply the next
+ * one's.  max_pass bounds the
  * output arrays. */
 int fq_layer_passes(int N, int dtype, int schedule, int max_pass, int *npass, int *tile_q, int *tiles,
                     uint64_t *gates);
