@@ -1073,23 +1073,29 @@ static void set_cost(TileArgs &a, double gamma, double init_amp)
             a.has_rr = 1;
 }
 
-// Phase factors for a cost-phase tile launch (grows the state's table; a
-// larger table needs the previous launches that read the old one to finish).
+// Grows the state's phase-table buffer (a larger one needs the previous
+// launches that read the old one to finish).
+static int reserve_phases(fq_state *st, size_t need)
+{
+    if (need <= st->phase_cap)
+        return FQ_OK;
+    FQ_HIP(hipStreamSynchronize(st->stream));
+    hipFree(st->d_phase);
+    st->d_phase = nullptr;
+    st->phase_cap = 0;
+    if (hipMalloc(&st->d_phase, need) != hipSuccess)
+        return set_err(FQ_ERR_OOM, "phase table allocation of %zu bytes failed", need);
+    st->phase_cap = need;
+    return FQ_OK;
+}
+
 // Phase table of one cost launch into d_phase; with cut, the table of cut
 // coefficients follows it in the same buffer (*cut points there).
 static int prepare_phases(fq_state *st, TileArgs &a, int a_log, double **cut = nullptr)
 {
     const size_t n = phase_table_entries(a, a_log);
-    const size_t need = n * sizeof(double2) + (cut ? n * sizeof(double) : 0);
-    if (need > st->phase_cap) {
-        FQ_HIP(hipStreamSynchronize(st->stream));
-        hipFree(st->d_phase);
-        st->d_phase = nullptr;
-        st->phase_cap = 0;
-        if (hipMalloc(&st->d_phase, need) != hipSuccess)
-            return set_err(FQ_ERR_OOM, "phase table allocation of %zu bytes failed", need);
-        st->phase_cap = need;
-    }
+    if (int rc = reserve_phases(st, n * sizeof(double2) + (cut ? n * sizeof(double) : 0)))
+        return rc;
     double *c = cut ? reinterpret_cast<double *>(st->d_phase + n) : nullptr;
     FQ_HIP(launch_phase_table(a, a_log, st->d_phase, c, st->stream));
     if (cut)
@@ -1195,16 +1201,25 @@ static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const do
     return f;
 }
 
+// Phase tables of one run made by one launch: up to this size together.  At
+// N=22 complex128 five of them are 1.3 MB; where a pass takes some hundred us
+// or more, its table's launch is under 2% of it.
+#define FQ_TABLES_BYTES ((size_t)8 << 20)
+
 // A tile pass on the compile-time kernel (fq_mix.hip), ready to launch over
 // all its tiles or a range of them.
 struct MixPass {
     MixArgs a;
     int K = 0, kind = 0, mir = 0;
     bool lane = false;  // RX on one more thread bit by lane operations
+    bool cost = false;
     double bytes = 0;   // read and written by the whole pass
+    TileArgs tab;       // cost pass: geometry, plan and angle of its phase table
+    size_t entries = 0; // and its size
+    const double2 *ptab = nullptr;  // where it is (mix_table, mix_tables)
 };
 
-// Arguments as tile_pass; queues the phase table of a cost pass.  The mirror pass may be a boundary pass too: the phase of a
+// Arguments as tile_pass.  The mirror pass may be a boundary pass too: the phase of a
 // mirror element is that of the N-qubit index it stands for (Cut(b) = Cut(~b)).
 static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
                        fq_graph *g, double gamma, bool cost, bool first, int z2, const double *pre_beta, bool defer,
@@ -1251,7 +1266,6 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
         a.rpos0_w |= (uint32_t)geom.tpos[nthr + r] << (6 * r);
         a.rposk_w |= (uint32_t)geom.tpos[start(K) + r] << (6 * r);
     }
-    a.order = getenv("FQ_TILE_ORDER") ? tile_order() : 3;   // (k_mix)
     a.ntiles = 1ull << geom.nh;
     if (z2 != Z2_OFF) {
         // the lower half is the tiles whose top index bit (qubit N-1) is 0; a
@@ -1286,17 +1300,17 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
                 t2.push_back(tile[start(K) + r]);
             cgeom = make_geom(N, t2, A);
         }
-        TileArgs ca;
+        TileArgs &ca = mp.tab;
         geom_to_args(cgeom, ca);
         ca.ntiles_run = a.ntiles;
         if (int rc = get_plan(g, cgeom, &ca.plan, st->stream))
             return rc;
         set_cost(ca, gamma, st->init_amp);
-        if (int rc = prepare_phases(st, ca, A))
-            return rc;
+        mp.entries = phase_table_entries(ca, A);
         a.has_rr = ca.has_rr;
         a.init_amp = st->init_amp;
     }
+    mp.cost = cost;
     a.ntab = a.ntiles;
     mp.K = K;
     mp.kind = pre_beta ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
@@ -1307,6 +1321,65 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
     return FQ_OK;
 }
 
+// The phase table of one pass, at the start of the state's buffer.
+static int mix_table(fq_state *st, MixPass &mp)
+{
+    if (!mp.cost)
+        return FQ_OK;
+    if (int rc = prepare_phases(st, mp.tab, mix_a_log(st->dtype, mp.a.Q)))
+        return rc;
+    mp.ptab = st->d_phase;
+    return FQ_OK;
+}
+
+// The phase tables of several passes in one launch where they are small and
+// of few geometries (*done); `done` false: each pass needs mix_table.
+static int mix_tables(fq_state *st, std::vector<MixPass> &mps, bool *done)
+{
+    *done = false;
+    TableJobs m;
+    size_t total = 0, most = 0;
+    int nj = 0, ng = 0;
+    for (const MixPass &mp : mps) {
+        if (!mp.cost)
+            continue;
+        if (nj == FQ_TABLE_JOBS)
+            return FQ_OK;
+        TableGeo g;
+        memset(&g, 0, sizeof(g));
+        g.Q = mp.tab.Q;
+        g.nthr = mp.tab.nthr;
+        g.nh = mp.tab.nh;
+        g.a_log = mp.tab.Q - mp.tab.nthr;
+        g.ntiles = mp.tab.ntiles_run;
+        g.plan = mp.tab.plan;
+        int k = 0;
+        while (k < ng && memcmp(&m.geo[k], &g, sizeof(g)) != 0)
+            ++k;
+        if (k == ng) {
+            if (ng == FQ_TABLE_GEOS)
+                return FQ_OK;
+            m.geo[ng++] = g;
+        }
+        m.job[nj++] = {mp.tab.gamma, (uint32_t)k, (uint32_t)total};
+        total += mp.entries;
+        most = std::max(most, mp.entries);
+        if (total * sizeof(double2) > FQ_TABLES_BYTES)
+            return FQ_OK;
+    }
+    if (nj < 2)
+        return FQ_OK;
+    if (int rc = reserve_phases(st, total * sizeof(double2)))
+        return rc;
+    FQ_HIP(launch_phase_tables(m, nj, most, st->d_phase, st->stream));
+    nj = 0;
+    for (MixPass &mp : mps)
+        if (mp.cost)
+            mp.ptab = st->d_phase + m.job[nj++].offset;
+    *done = true;
+    return FQ_OK;
+}
+
 static int mix_pass(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
                     fq_graph *g, double gamma, bool cost, bool first, int kind, int z2, const double *pre_beta,
                     bool defer)
@@ -1314,8 +1387,10 @@ static int mix_pass(fq_state *st, const std::vector<int> &tile, const std::vecto
     MixPass mp;
     if (int rc = mix_prepare(st, tile, gates, beta, g, gamma, cost, first, z2, pre_beta, defer, mp))
         return rc;
+    if (int rc = mix_table(st, mp))
+        return rc;
     return timed(st, kind, mp.bytes, [&] {
-        return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, mp.a, st->d_phase, st->stream);
+        return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, mp.a, mp.ptab, st->stream);
     });
 }
 
@@ -1469,7 +1544,8 @@ static bool carrier_gates()
 // of qubits per pass (N=30 complex128: strided passes 8.0 and 7.2 ms -> 6.8
 // and 7.0 ms; N=34 complex64: 65 and 98 ms -> 57 and 81 ms).  A pass that
 // would need more bit runs than the tile kernel takes gets larger blocks.
-static std::vector<FusedPass> cover_passes(int N, int Qmax, int dtype, int boundary = -1)
+// carriers: lowest qubits that every strided pass carries (0: carriers_for).
+static std::vector<FusedPass> cover_passes(int N, int Qmax, int dtype, int boundary = -1, int carriers = 0)
 {
     std::vector<FusedPass> ps;
     Qmax = std::min(Qmax, N);
@@ -1480,7 +1556,7 @@ static std::vector<FusedPass> cover_passes(int N, int Qmax, int dtype, int bound
     const int rest = N - Qmax;
     if (rest <= 0)
         return ps;
-    const int cmin = std::min(carriers_for(dtype), Qmax - 1);
+    const int cmin = std::min(carriers > 0 ? carriers : carriers_for(dtype), Qmax - 1);
     const int per_max = Qmax - cmin;
     const int npass = (rest + per_max - 1) / per_max;
     std::vector<int> want(npass);
@@ -1736,7 +1812,12 @@ struct LayerPlan {
 static LayerPlan layer_plan(int N, int dtype, bool z2)
 {
     const int Qmax = z2 ? std::min(pass_tile_q(dtype), N - 1) : pass_tile_q(dtype);
-    LayerPlan lp{cover_passes(N, Qmax, dtype), -1, 0, false, 0};
+    // one carrier fewer (64 B runs) where that covers the qubits in two passes:
+    // per layer at N=24 complex128 182 -> 149 us, N=25 complex64 198 -> 161 us
+    // (states of 256 MiB, which the memory-side cache holds)
+    const int fewer = carriers_for(dtype) - 1;
+    const bool two = !z2 && N - Qmax == Qmax - fewer;
+    LayerPlan lp{cover_passes(N, Qmax, dtype, -1, two ? fewer : 0), -1, 0, false, 0};
     const int m = (int)lp.ps.size();
     if (layer_pipe() && m >= (z2 ? 3 : 2)) {
         lp.end1 = z2 ? 1 : m - 1;
@@ -1779,6 +1860,32 @@ static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
         if (getenv(k))
             return lp;
     const int elem_log = dtype == FQ_C128 ? 4 : 3, Ns = z2 ? N - 1 : N;
+    if (lp.ps.size() == 2 && (!z2 || N < 24)) {
+        // Two passes of the narrowest tiles that cover N with 128 B runs: a
+        // full-width tile leaves most CUs of a small state idle (16 tiles at
+        // N=17) and takes a pass's whole latency for its 128 KiB.  Per layer,
+        // with one phase-table launch a run (mix_tables), full-width tiles and
+        // a launch per table before: N=14 complex128 17.6 -> 6.1 us, N=18 22.3
+        // -> 10.2, N=20 30.6 -> 16.7; half state N=20 complex64 31.1 -> 10.8
+        // (also one pass per layer instead of two).
+        const int Q = std::min(tile_max_q(dtype),
+                               std::max(dtype == FQ_C128 ? 9 : 10, (N + carriers_for(dtype) + 1) / 2));
+        if (Q >= N)
+            return lp;
+        FusedPass p0, p1;   // the carried qubits' RX stays in pass 0
+        p0.tile = low_tile(Q);
+        p0.gates = p0.tile;
+        p1.tile = low_tile(2 * Q - N);
+        for (int q = Q; q < N; ++q) {
+            p1.tile.push_back(q);
+            p1.gates.push_back(q);
+        }
+        lp.ps = {p0, p1};
+        lp.end1 = 1;
+        lp.split = true;
+        lp.open0 = z2 && P % 2 == 0 ? 1 : 0;
+        return lp;
+    }
     if (lp.ps.size() != 3)
         return lp;
     const int Q = tile_max_q(dtype), rest = N - Q;
@@ -1857,8 +1964,11 @@ static void layer_steps(const LayerPlan &lp, int p, int P, std::vector<Step> &ou
 // two streams of the state: while one chunk's first pass reads from the HBM,
 // the other's later passes run from the cache.  Every pass has its phase table
 // (at most one of them is a cost pass) before the streams fork.
-static int run_chunks(fq_state *st, std::vector<MixPass> &group, double bytes, int nlog)
+static int run_chunks(fq_state *st, const MixPass *group, size_t n, int nlog)
 {
+    double bytes = 0;
+    for (size_t i = 0; i < n; ++i)
+        bytes += group[i].bytes;
     for (int i = 0; i < 2; ++i) {
         if (!st->side[i])
             FQ_HIP(hipStreamCreateWithFlags(&st->side[i], hipStreamNonBlocking));
@@ -1872,11 +1982,12 @@ static int run_chunks(fq_state *st, std::vector<MixPass> &group, double bytes, i
         for (int i = 0; i < 2 && e == hipSuccess; ++i)
             e = hipStreamWaitEvent(st->side[i], st->forked, 0);
         for (uint64_t c = 0; c < 1ull << nlog && e == hipSuccess; ++c)
-            for (const MixPass &mp : group) {
+            for (size_t i = 0; i < n; ++i) {
+                const MixPass &mp = group[i];
                 MixArgs a = mp.a;
                 a.ntiles >>= nlog;
                 a.tile0 = c * a.ntiles;
-                e = launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, a, st->d_phase, st->side[c & 1]);
+                e = launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, a, mp.ptab, st->side[c & 1]);
                 if (e != hipSuccess)
                     break;
             }
@@ -1889,7 +2000,7 @@ static int run_chunks(fq_state *st, std::vector<MixPass> &group, double bytes, i
             e = e == hipSuccess ? j : e;
         }
         return e;
-    }, (int)group.size());
+    }, (int)n);
 }
 
 // Layers [p0, p1) of P.  expand: the last layer's mirror pass also writes the
@@ -1907,6 +2018,36 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
         return lp.chunk > 0 && *std::max_element(ps[s.pass].tile.begin(), ps[s.pass].tile.end()) < lp.chunk;
     };
     auto cost = [](const Step &s) { return s.kind != STEP_PLAIN; };
+    // every pass on the compile-time kernel (the pass widths of tuning knobs
+    // may have none): prepared first, and small phase tables made at once
+    const bool mix = mix_a_log(st->dtype, (int)ps[0].tile.size()) > 0;
+    std::vector<MixPass> mps(mix ? seq.size() : 0);
+    bool tables = false;
+    for (size_t k = 0; k < seq.size(); ++k) {
+        const Step &s = seq[k];
+        const FusedPass &fp = ps[s.pass];
+        const bool last = s.layer + 1 == P && k + 1 == seq.size();
+        const int mode = !z2 ? (int)Z2_OFF
+                         : s.pass + 1 < m ? (int)Z2_LOWER
+                                          : s.layer + 1 == P && s.kind == STEP_PLAIN && expand ? (int)Z2_EXPAND
+                                                                                                : (int)Z2_MIRROR;
+        const bool bd = s.kind == STEP_BOUNDARY;
+        const int L = bd ? s.layer + 1 : s.layer;
+        const double gamma = cost(s) ? gammas[L] : 0.0;
+        const double *pre = bd ? &betas[s.layer] : nullptr;
+        // plain passes leave their RX factor to the next cost pass, except
+        // the run's very last pass, which leaves the state exact
+        const int rc = mix ? mix_prepare(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, mode,
+                                         pre, !last, mps[k])
+                           : tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST,
+                                       FQ_K_FUSED, mode, pre, !last);
+        if (rc)
+            return rc;
+    }
+    if (!mix)
+        return FQ_OK;
+    if (int rc = mix_tables(st, mps, &tables))
+        return rc;
     for (size_t k = 0; k < seq.size();) {
         // passes of one group: a run of local ones with at most one cost
         // phase among them (one phase table), else a single pass
@@ -1916,38 +2057,19 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
             for (; k + n < seq.size() && local(seq[k + n]) && !(c && cost(seq[k + n])); ++n)
                 c = c || cost(seq[k + n]);
         }
-        std::vector<MixPass> group(n > 1 ? n : 0);
-        double bytes = 0;
-        for (size_t i = 0; i < n; ++i) {
-            const Step &s = seq[k + i];
-            const FusedPass &fp = ps[s.pass];
-            const bool last = s.layer + 1 == P && k + i + 1 == seq.size();
-            const int mode = !z2 ? (int)Z2_OFF
-                             : s.pass + 1 < m ? (int)Z2_LOWER
-                                              : s.layer + 1 == P && s.kind == STEP_PLAIN && expand ? (int)Z2_EXPAND
-                                                                                                    : (int)Z2_MIRROR;
-            const bool bd = s.kind == STEP_BOUNDARY;
-            const int L = bd ? s.layer + 1 : s.layer;
-            const double gamma = cost(s) ? gammas[L] : 0.0;
-            const double *pre = bd ? &betas[s.layer] : nullptr;
-            // plain passes leave their RX factor to the next cost pass, except
-            // the run's very last pass, which leaves the state exact
-            int rc;
-            if (n == 1)
-                rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, FQ_K_FUSED,
-                               mode, pre, !last);
-            else
-                rc = mix_prepare(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, mode, pre,
-                                 !last, group[i]);
-            if (rc)
-                return rc;
-            if (n > 1)
-                bytes += group[i].bytes;
+        int rc = FQ_OK;
+        for (size_t i = 0; i < n && !tables && rc == FQ_OK; ++i)
+            rc = mix_table(st, mps[k + i]);
+        if (rc == FQ_OK && n > 1) {
+            rc = run_chunks(st, &mps[k], n, (z2 ? st->N - 1 : st->N) - lp.chunk);
+        } else if (rc == FQ_OK) {
+            const MixPass &mp = mps[k];
+            rc = timed(st, FQ_K_FUSED, mp.bytes, [&] {
+                return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, mp.a, mp.ptab, st->stream);
+            });
         }
-        if (n > 1) {
-            if (int rc = run_chunks(st, group, bytes, (z2 ? st->N - 1 : st->N) - lp.chunk))
-                return rc;
-        }
+        if (rc)
+            return rc;
         k += n;
     }
     return FQ_OK;

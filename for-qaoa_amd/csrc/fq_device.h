@@ -164,19 +164,19 @@ __device__ __forceinline__ int deposit_runs(int x, unsigned mask)
 }
 
 // Exponent over gamma of entry gid of a cost launch's phase table (the
-// layout of k_phase_table): per tile the coefficients c_i(zH) (i < Q) and
+// layout of k_phase_table; Q, nthr, nh and a_log of its tiles): per tile the coefficients c_i(zH) (i < Q) and
 // K(zH) - W/2, then the per-thread and per-register entries and the 16
 // register-register entries.  Returns false past the end of the table.
-__device__ __forceinline__ bool phase_coef(const TileArgs &a, const PlanDev &p, int a_log, uint64_t gid,
-                                           double &coef)
+__device__ __forceinline__ bool phase_coef(int Q, uint64_t ntiles, int nthr, int nh, const PlanDev &p, int a_log,
+                                           uint64_t gid, double &coef)
 {
-    const uint64_t q1 = (uint64_t)a.Q + 1;
-    const uint64_t ntile_e = run_tiles(a) * q1;
-    const uint64_t nthr_e = (uint64_t)(1 + a_log) << a.nthr;
+    const uint64_t q1 = (uint64_t)Q + 1;
+    const uint64_t ntile_e = ntiles * q1;
+    const uint64_t nthr_e = (uint64_t)(1 + a_log) << nthr;
     if (gid < ntile_e) {
         const uint64_t tile = gid / q1;
         const int i = (int)(gid - tile * q1);
-        if (i < a.Q) {
+        if (i < Q) {
             double acc = 0.0;
             for (int e = p.csr_off[i]; e < p.csr_off[i + 1]; ++e)
                 acc += p.csr_w[e] * (double)((tile >> p.csr_h[e]) & 1ull);
@@ -185,7 +185,7 @@ __device__ __forceinline__ bool phase_coef(const TileArgs &a, const PlanDev &p, 
             double K = 0.0;
             for (int e = 0; e < p.n_hh; ++e)
                 K += p.hh_w[e] * (double)(((tile >> p.hh_u[e]) ^ (tile >> p.hh_v[e])) & 1ull);
-            for (int h = 0; h < a.nh; ++h)
+            for (int h = 0; h < nh; ++h)
                 K += p.omega[h] * (double)((tile >> h) & 1ull);
             coef = K - 0.5 * p.wtot;
         }

@@ -95,7 +95,6 @@ struct MixArgs {
     uint32_t rpos0_w;        // positions of the register bits of layout 0, 6 bits each
     uint32_t rposk_w;        // and of the last layout
     uint32_t gates_w;        // gated register bits of layout l at bit A l
-    uint32_t order;          // tile order of the persistent loop
     uint64_t tile0, ntiles;  // tiles [tile0, tile0 + ntiles) of this launch
     uint64_t ntab;           // tiles of the whole pass (rows of its phase table)
     uint64_t mirror_pm;      // mirror pass: sum of 2^p over the real tile positions
@@ -111,6 +110,25 @@ __host__ __device__ inline uint64_t run_tiles(const TileArgs &a)
 {
     return a.ntiles_run ? a.ntiles_run : (1ull << a.nh);
 }
+
+// The phase tables of the cost passes of one run (k_phase_tables): the distinct
+// geometries, and per pass its geometry, angle and place.
+#define FQ_TABLE_GEOS 3
+#define FQ_TABLE_JOBS 64
+struct TableGeo {
+    int Q, nthr, nh, a_log;
+    uint64_t ntiles;
+    PlanDev plan;
+};
+struct TableJob {
+    double gamma;
+    uint32_t geo;
+    uint32_t offset;         // entries
+};
+struct TableJobs {
+    TableGeo geo[FQ_TABLE_GEOS];
+    TableJob job[FQ_TABLE_JOBS];
+};
 
 // Per-slot parameters of a packed (slab) step, in device memory.
 struct SlotParams {
@@ -173,6 +191,8 @@ hipError_t launch_tile_mirror(int dtype, int a_log, bool expand, void *sv, const
 hipError_t launch_phase_table(const TileArgs &a, int a_log, double2 *tab, double *cut,
                               hipStream_t stream);
 size_t phase_table_entries(const TileArgs &a, int a_log);
+// njobs tables of at most `entries` entries each
+hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, hipStream_t stream);
 hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t stream);
 hipError_t launch_expect(int dtype, int a_log, const void *sv, const TileArgs &a, double *partials,
                          double *out2, hipStream_t stream);

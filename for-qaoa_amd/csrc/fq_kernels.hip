@@ -52,13 +52,29 @@ __global__ void __launch_bounds__(256) k_phase_table(const TileArgs a, int a_log
 {
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     double coef;
-    if (!phase_coef(a, a.plan, a_log, gid, coef))
+    if (!phase_coef(a.Q, run_tiles(a), a.nthr, a.nh, a.plan, a_log, gid, coef))
         return;
     double sn, cs;
     sincos(a.gamma * coef, &sn, &cs);
     tab[gid] = make_double2(cs, sn);
     if (cut)
         cut[gid] = coef;
+}
+
+// The phase tables of several cost passes in one launch (blockIdx.y: the
+// pass).  A small state's passes take 5 to 20 us each; a table launch before
+// each of them took another 4 to 6 us, most of it latency.
+__global__ void __launch_bounds__(256) k_phase_tables(const TableJobs m, double2 *__restrict__ tab)
+{
+    const TableJob &job = m.job[blockIdx.y];
+    const TableGeo &g = m.geo[job.geo];
+    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    double coef;
+    if (!phase_coef(g.Q, g.ntiles, g.nthr, g.nh, g.plan, g.a_log, gid, coef))
+        return;
+    double sn, cs;
+    sincos(job.gamma * coef, &sn, &cs);
+    tab[job.offset + gid] = make_double2(cs, sn);
 }
 
 __device__ __forceinline__ void zmul(double &x, double &y, double2 f)
@@ -1487,6 +1503,13 @@ hipError_t launch_phase_table(const TileArgs &a, int a_log, double2 *tab, double
     const size_t blocks = (n + 255) / 256;
     hipLaunchKernelGGL(k_phase_table, dim3((unsigned)blocks), dim3(256), 0, stream, a, a_log, tab,
                        cut);
+    return hipGetLastError();
+}
+
+hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_phase_tables, dim3((unsigned)((entries + 255) / 256), (unsigned)njobs), dim3(256), 0, stream, m,
+                       tab);
     return hipGetLastError();
 }
 

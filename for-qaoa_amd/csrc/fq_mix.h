@@ -1,4 +1,4 @@
-// fq_mix.hip -- gfx950 tile passes of the layer schedules, with the LDS
+// fq_mix.h -- gfx950 tile passes of the layer schedules, with the LDS
 // phases fixed at compile time.  fq_kernels.hip keeps the general tile pass
 // (any tile width, RX on any subset of the tile bits).
 //
@@ -18,6 +18,8 @@
 // pipelined to one) 50 -> 40 us per layer, N=24 (256 MiB, in the memory-side
 // cache) 216 -> 193 us, a plain pass over QAOA amplitudes 80 us (6.7 TB/s; 65 us
 // over zeros: the rate depends on how many bits toggle).
+#pragma once
+
 #include "fq_device.h"
 #include "fq_internal.h"
 
@@ -58,12 +60,60 @@ FQ_GEO(double, 13, 4, 2,
 FQ_GEO(double, 13, 4, 3,
        FQ_L(1, 2, 4, 8, 16, 34, 68, 136, 272, 548, 1121, 2216, 4452),
        FQ_L({0, 1, 2, 3, 4, 5, 6, 7, 8}, {4, 5, 6, 7, 10, 8, 9, 11, 12}, {0, 5, 6, 7, 8, 9, 10, 11, 12}, {0, 1, 2, 3, 4, 9, 10, 11, 12}))
+FQ_GEO(double, 12, 4, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 64, 128, 272, 548, 1092, 2192),
+       FQ_L({0, 1, 2, 3, 4, 5, 6, 7}, {0, 1, 2, 3, 8, 9, 10, 11}))
+FQ_GEO(double, 12, 4, 2,
+       FQ_L(1, 2, 4, 8, 16, 34, 68, 136, 272, 548, 1121, 2224),
+       FQ_L({0, 1, 2, 3, 4, 5, 6, 7}, {4, 5, 6, 7, 10, 8, 9, 11}, {0, 1, 2, 3, 8, 9, 10, 11}))
+FQ_GEO(double, 11, 4, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 68, 136, 272, 548, 1090),
+       FQ_L({0, 1, 2, 3, 4, 5, 6}, {0, 1, 2, 7, 8, 9, 10}))
+FQ_GEO(double, 11, 4, 2,
+       FQ_L(1, 2, 4, 8, 16, 33, 66, 136, 272, 552, 1092),
+       FQ_L({0, 1, 2, 3, 4, 5, 6}, {4, 5, 6, 7, 10, 8, 9}, {0, 1, 2, 7, 8, 9, 10}))
+FQ_GEO(double, 9, 3, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 72, 144, 288),
+       FQ_L({0, 1, 2, 3, 4, 5}, {0, 1, 2, 6, 7, 8}))
+FQ_GEO(double, 9, 3, 2,
+       FQ_L(1, 2, 4, 8, 16, 33, 68, 136, 290),
+       FQ_L({0, 1, 2, 3, 4, 5}, {3, 4, 5, 6, 8, 7}, {0, 1, 2, 6, 7, 8}))
+FQ_GEO(double, 10, 4, 1,
+       FQ_L(1, 2, 4, 8, 16, 34, 68, 136, 272, 546),
+       FQ_L({0, 1, 2, 3, 4, 5}, {0, 1, 6, 7, 8, 9}))
+FQ_GEO(double, 10, 4, 2,
+       FQ_L(1, 2, 4, 8, 16, 34, 68, 136, 272, 545),
+       FQ_L({0, 1, 2, 3, 4, 5}, {4, 5, 6, 7, 9, 8}, {0, 1, 6, 7, 8, 9}))
 FQ_GEO(float, 14, 5, 1,
        FQ_L(1, 2, 4, 8, 16, 32, 66, 136, 272, 544, 1104, 2242, 4484, 8912),
        FQ_L({0, 1, 2, 3, 4, 5, 6, 7, 8}, {0, 1, 2, 3, 9, 10, 11, 12, 13}))
 FQ_GEO(float, 14, 5, 2,
        FQ_L(1, 2, 4, 8, 16, 32, 66, 136, 272, 544, 1104, 2240, 4484, 8961),
        FQ_L({0, 1, 2, 3, 4, 5, 6, 7, 8}, {5, 6, 7, 8, 12, 13, 9, 10, 11}, {0, 1, 2, 3, 9, 10, 11, 12, 13}))
+FQ_GEO(float, 13, 5, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 66, 132, 264, 528, 1056, 2128, 4256),
+       FQ_L({0, 1, 2, 3, 4, 5, 6, 7}, {0, 1, 2, 8, 9, 10, 11, 12}))
+FQ_GEO(float, 13, 5, 2,
+       FQ_L(1, 2, 4, 8, 16, 32, 65, 132, 264, 528, 1056, 2128, 4290),
+       FQ_L({0, 1, 2, 3, 4, 5, 6, 7}, {5, 6, 7, 8, 9, 12, 10, 11}, {0, 1, 2, 8, 9, 10, 11, 12}))
+FQ_GEO(float, 12, 4, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 68, 136, 272, 544, 1092, 2176),
+       FQ_L({0, 1, 2, 3, 4, 5, 6, 7}, {0, 1, 2, 3, 8, 9, 10, 11}))
+FQ_GEO(float, 12, 4, 2,
+       FQ_L(1, 2, 4, 8, 16, 32, 68, 136, 272, 544, 1089, 2178),
+       FQ_L({0, 1, 2, 3, 4, 5, 6, 7}, {4, 5, 6, 7, 10, 11, 8, 9}, {0, 1, 2, 3, 8, 9, 10, 11}))
+FQ_GEO(float, 11, 4, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 65, 136, 272, 544, 1096),
+       FQ_L({0, 1, 2, 3, 4, 5, 6}, {0, 1, 2, 7, 8, 9, 10}))
+FQ_GEO(float, 11, 4, 2,
+       FQ_L(1, 2, 4, 8, 16, 32, 66, 132, 264, 528, 1089),
+       FQ_L({0, 1, 2, 3, 4, 5, 6}, {4, 5, 6, 7, 8, 10, 9}, {0, 1, 2, 7, 8, 9, 10}))
+FQ_GEO(float, 10, 4, 1,
+       FQ_L(1, 2, 4, 8, 16, 32, 68, 136, 272, 544),
+       FQ_L({0, 1, 2, 3, 4, 5}, {0, 1, 6, 7, 8, 9}))
+FQ_GEO(float, 10, 4, 2,
+       FQ_L(1, 2, 4, 8, 16, 32, 65, 132, 264, 528),
+       FQ_L({0, 1, 2, 3, 4, 5}, {4, 5, 6, 7, 8, 9}, {0, 1, 6, 7, 8, 9}))
 #undef FQ_GEO
 #undef FQ_L
 // no exchange: all gated bits are register bits
@@ -101,8 +151,6 @@ template <typename Lay, typename T, typename R, int A, int L0, int L1, bool YF>
 __device__ __forceinline__ void mix_exchange(T (&v)[1 << A], R *lds, int s0, int s1)
 {
     constexpr int N = 1 << A;
-    // addresses from opaque bases: recomputed here, not held across the tile loop
-    asm volatile("" : "+v"(s0), "+v"(s1));
 #pragma unroll
     for (int j = 0; j < N; ++j)
         lds[s0 + Lay::reg_slot(L0, j)] = YF ? v[j].y : v[j].x;
@@ -219,9 +267,9 @@ __device__ __forceinline__ void mix_phase(T (&v)[1 << A], const R (&fx)[A], cons
     }
 }
 
-// One work-group per tile by default (a.order 3): with two of them on a CU the
-// dispatcher's order keeps loads and butterflies apart better than a range of
-// tiles per group (N=30 complex128 13.64 -> 13.37 ms per layer).
+// One work-group per tile: with two of them on a CU the dispatcher's order keeps
+// loads and butterflies apart better than persistent groups with a range of
+// tiles each (N=30 complex128 13.64 -> 13.37 ms per layer).
 //
 // One tile pass.  KIND: MIX_PLAIN RX on the gated bits; MIX_FIRST the
 // launch-control write (no read) with the cost phase, then RX; MIX_COST the
@@ -271,113 +319,104 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
     const R rt = sizeof(R) == 4 ? (R)a.tf : (R)a.t;
     const R pt = sizeof(R) == 4 ? (R)a.pre_tf : (R)a.pre_t;
 
-    uint64_t kt = 0;
-    for (;;) {
-        const uint64_t it = tile_of(a.order, a.ntiles, kt++);
-        if (it >= a.ntiles)
-            break;
-        const uint64_t tile = a.tile0 + it;
-        const uint64_t base = unpack_runs_uniform(tile, a.hruns);
-        T v[N];
-        if (KIND != MIX_FIRST) {
-            uint64_t ro[N];
-            reg_offsets<N, NB>(a.rpos0_w, ro);
-            const T *p0 = sv + (base + toff);
-#pragma unroll
-            for (int j = 0; j < AH; ++j)
-                v[j] = p0[ro[j]];
-            if (MIR) {
-                const T *pm = sv + (unpack_runs_uniform(~tile & hmask, a.hruns) + a.mirror_pm - toff);
-#pragma unroll
-                for (int j = AH; j < N; ++j)
-                    v[j] = pm[-(int64_t)ro[j - AH]];
-            }
-        }
-        auto cost = [&]() {
-            // (the thread's own entries are read again for every tile, from
-            // the L2: 2^A amplitudes leave no registers to hold them)
-            const double2 *f_t = ptab + tile * q1;
-            int tb = t;
-            asm volatile("" : "+v"(tb));
-            const double2 f_thr = thr_tab[tb];
-            double x = f_thr.x, y = f_thr.y;
-            auto mul = [&](double2 f) {
-                const double nx = x * f.x - y * f.y;
-                y = x * f.y + y * f.x;
-                x = nx;
-            };
-            mul(f_t[Q]);
-#pragma unroll
-            for (int i = 0; i < NT; ++i) {
-                const double2 f = f_t[i];
-                const double nx = x * f.x - y * f.y;
-                const double ny = x * f.y + y * f.x;
-                const bool on = (tb >> i) & 1;
-                x = on ? nx : x;
-                y = on ? ny : y;
-            }
-            mul(KIND == MIX_FIRST ? make_double2(a.init_amp * a.scale_re, a.init_amp * a.scale_im)
-                                  : make_double2(a.scale_re, a.scale_im));
-            const R x0 = (R)x, y0 = (R)y;
-            R fx[A], fy[A];
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int r = 0; r < A; ++r) {
-                const double2 f = f_t[NT + r], g = thr_tab[((1 + r) << NT) + tb];
-                fx[r] = (R)(g.x * f.x - g.y * f.y);
-                fy[r] = (R)(g.x * f.y + g.y * f.x);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            mix_phase<T, R, A, A, KIND == MIX_FIRST>(v, fx, fy, x0, y0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (a.has_rr) {
-#pragma unroll
-                for (int j = 0; j < N; ++j) {
-                    const double2 f = rr_tab[j];
-                    cmul_by(v[j], (R)f.x, (R)f.y);
-                }
-            }
-        };
-        // the tile's first exchange writes slots that others may still read
-        // for the previous tile
-        if (K > 0)
-            lds_barrier();
-        if constexpr (KIND == MIX_FIRST || KIND == MIX_COST)
-            cost();
-        if constexpr (KIND == MIX_BOUNDARY) {
-            mix_up<Lay, T, R, A, K, 0, 0, LB>(v, lds, sb, a.gates_w, pt);
-            cost();
-            mix_down<Lay, T, R, A, K, K, K, LB>(v, lds, sb, a.gates_w, rt);
-        } else {
-            mix_up<Lay, T, R, A, K, 0, 0, LB>(v, lds, sb, a.gates_w, rt);
-            if constexpr (MIR && K > 0)
-                mix_exchange<Lay, T, R, A, K, 0, (K & 1) != 0>(v, lds, sb[K], sb[0]);
-        }
-        if (!COST && a.apply_scale) {
-#pragma unroll
-            for (int j = 0; j < N; ++j)
-                cmul_by(v[j], (R)a.scale_re, (R)a.scale_im);
-        }
+    const uint64_t tile = a.tile0 + blockIdx.x;
+    const uint64_t base = unpack_runs_uniform(tile, a.hruns);
+    // cost phase: the tile's row of the table, entry i in lane i (broadcast by
+    // readlane), and the thread's entry, loaded ahead of the amplitudes
+    double2 f_row = make_double2(1.0, 0.0), f_thr = make_double2(1.0, 0.0);
+    if (COST) {
+        f_row = ptab[tile * q1 + (t & 63) % (Q + 1)];
+        f_thr = thr_tab[t];
+    }
+    T v[N];
+    if (KIND != MIX_FIRST) {
         uint64_t ro[N];
-        reg_offsets<N, NB>(LS == 0 ? a.rpos0_w : a.rposk_w, ro);
-        T *const p0 = sv + (base + (LS == 0 ? toff : soff));
+        reg_offsets<N, NB>(a.rpos0_w, ro);
+        const T *p0 = sv + (base + toff);
 #pragma unroll
         for (int j = 0; j < AH; ++j)
-            p0[ro[j]] = v[j];
+            v[j] = p0[ro[j]];
         if (MIR) {
-            T *const pm = sv + (unpack_runs_uniform(~tile & hmask, a.hruns) + a.mirror_pm - toff);
+            const T *pm = sv + (unpack_runs_uniform(~tile & hmask, a.hruns) + a.mirror_pm - toff);
 #pragma unroll
             for (int j = AH; j < N; ++j)
-                pm[-(int64_t)ro[j - AH]] = v[j];
-            if (MIR == 2) {
-                const uint64_t half = 1ull << (a.N - 1);
+                v[j] = pm[-(int64_t)ro[j - AH]];
+        }
+    }
+    auto cost = [&]() {
+        double x = f_thr.x, y = f_thr.y;
+        auto mul = [&](double2 f) {
+            const double nx = x * f.x - y * f.y;
+            y = x * f.y + y * f.x;
+            x = nx;
+        };
+        mul(lane_bcast(f_row, Q));
 #pragma unroll
-                for (int j = 0; j < AH; ++j)
-                    p0[half + ro[j]] = v[j + AH];
+        for (int i = 0; i < NT; ++i) {
+            const double2 f = lane_bcast(f_row, i);
+            const double nx = x * f.x - y * f.y;
+            const double ny = x * f.y + y * f.x;
+            const bool on = (t >> i) & 1;
+            x = on ? nx : x;
+            y = on ? ny : y;
+        }
+        mul(KIND == MIX_FIRST ? make_double2(a.init_amp * a.scale_re, a.init_amp * a.scale_im)
+                              : make_double2(a.scale_re, a.scale_im));
+        const R x0 = (R)x, y0 = (R)y;
+        R fx[A], fy[A];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = AH; j < N; ++j)
-                    pm[half - ro[j - AH]] = v[j - AH];
+        for (int r = 0; r < A; ++r) {
+            const double2 f = lane_bcast(f_row, NT + r), g = thr_tab[((1 + r) << NT) + t];
+            fx[r] = (R)(g.x * f.x - g.y * f.y);
+            fy[r] = (R)(g.x * f.y + g.y * f.x);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        mix_phase<T, R, A, A, KIND == MIX_FIRST>(v, fx, fy, x0, y0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (a.has_rr) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const double2 f = rr_tab[j];
+                cmul_by(v[j], (R)f.x, (R)f.y);
             }
+        }
+    };
+    if constexpr (KIND == MIX_FIRST || KIND == MIX_COST)
+        cost();
+    if constexpr (KIND == MIX_BOUNDARY) {
+        mix_up<Lay, T, R, A, K, 0, 0, LB>(v, lds, sb, a.gates_w, pt);
+        cost();
+        mix_down<Lay, T, R, A, K, K, K, LB>(v, lds, sb, a.gates_w, rt);
+    } else {
+        mix_up<Lay, T, R, A, K, 0, 0, LB>(v, lds, sb, a.gates_w, rt);
+        if constexpr (MIR && K > 0)
+            mix_exchange<Lay, T, R, A, K, 0, (K & 1) != 0>(v, lds, sb[K], sb[0]);
+    }
+    if (!COST && a.apply_scale) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            cmul_by(v[j], (R)a.scale_re, (R)a.scale_im);
+    }
+    uint64_t ro[N];
+    reg_offsets<N, NB>(LS == 0 ? a.rpos0_w : a.rposk_w, ro);
+    T *const p0 = sv + (base + (LS == 0 ? toff : soff));
+#pragma unroll
+    for (int j = 0; j < AH; ++j)
+        p0[ro[j]] = v[j];
+    if (MIR) {
+        T *const pm = sv + (unpack_runs_uniform(~tile & hmask, a.hruns) + a.mirror_pm - toff);
+#pragma unroll
+        for (int j = AH; j < N; ++j)
+            pm[-(int64_t)ro[j - AH]] = v[j];
+        if (MIR == 2) {
+            const uint64_t half = 1ull << (a.N - 1);
+#pragma unroll
+            for (int j = 0; j < AH; ++j)
+                p0[half + ro[j]] = v[j + AH];
+#pragma unroll
+            for (int j = AH; j < N; ++j)
+                pm[half - ro[j - AH]] = v[j - AH];
         }
     }
 }
@@ -401,13 +440,8 @@ static hipError_t launch_mix_t(void *sv, const MixArgs &a, const double2 *ptab, 
         if (hipError_t e = allow_large_lds(fn))
             return e;
     }
-    const uint64_t resident = (uint64_t)occupancy_per_cu(fn, (int)threads, lds) * device_cu_count();
-    const uint64_t grid = a.ntiles < resident || a.order == 3 ? a.ntiles : resident;
-    MixArgs la = a;
-    if (la.order == 1 && grid % 8 != 0)
-        la.order = 0;
-    hipLaunchKernelGGL((k_mix<R, Q, A, K, KIND, MIR, LG>), dim3((unsigned)grid), dim3(threads), lds, stream,
-                       reinterpret_cast<T *>(sv), la, ptab);
+    hipLaunchKernelGGL((k_mix<R, Q, A, K, KIND, MIR, LG>), dim3((unsigned)a.ntiles), dim3(threads), lds, stream,
+                       reinterpret_cast<T *>(sv), a, ptab);
     return hipGetLastError();
 }
 
@@ -450,34 +484,6 @@ static hipError_t launch_mix_q(int k, bool lane, int kind, int mir, void *sv, co
             if constexpr (Q - A > 2 * A)
                 return launch_mix_l<R, Q, A, 3>(lane, kind, mir, sv, a, ptab, s);
             return hipErrorInvalidValue;
-        default: return hipErrorInvalidValue;
-    }
-}
-
-int mix_a_log(int dtype, int Q)
-{
-    if (dtype == 0)
-        return Q == 13 ? 4 : 0;
-    return Q == 14 ? 5 : 0;
-}
-
-bool mix_lane_bit(int Q, int A, int k)
-{
-    const int b = Q - A - k * A - 1;
-    return k > 0 && (b == 4 || b == 3 || b == 1 || b == 0);
-}
-
-hipError_t launch_mix(int dtype, int k, bool lane, int kind, int mir, void *sv, const MixArgs &a, const double2 *ptab,
-                      hipStream_t stream)
-{
-    if (dtype == 0) {
-        switch (a.Q) {
-            case 13: return launch_mix_q<double, 13, 4>(k, lane, kind, mir, sv, a, ptab, stream);
-            default: return hipErrorInvalidValue;
-        }
-    }
-    switch (a.Q) {
-        case 14: return launch_mix_q<float, 14, 5>(k, lane, kind, mir, sv, a, ptab, stream);
         default: return hipErrorInvalidValue;
     }
 }

@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256) k_slab_phase_table(const TileArgs a, int 
         return;
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     double coef;
-    if (!phase_coef(a, sp.plan, a_log, gid, coef))
+    if (!phase_coef(a.Q, run_tiles(a), a.nthr, a.nh, sp.plan, a_log, gid, coef))
         return;
     const double angle = sp.gamma * coef;
     double sn, cs;

@@ -105,3 +105,35 @@ def test_chunked_runs(chunk_env, N, dtype, schedule, P, oracle):
         err = float(np.linalg.norm(got - want) / np.linalg.norm(want))
         print(f"  relative L2 error vs oracle {err:.2e}", flush=True)
         assert err < {"c128": 1e-12, "c64": 1e-5}[dtype]
+
+
+@pytest.mark.parametrize("N,dtype,schedule,P", [
+    # the ends of each tile width of the two-pass plans (complex128 9..13,
+    # complex64 10..14 qubits), and two passes over 64 B runs
+    (14, "c128", "fused", 2), (15, "c128", "z2", 1), (15, "c128", "z2", 2), (16, "c128", "fused", 3),
+    (17, "c128", "fused", 2), (18, "c128", "z2", 3), (19, "c128", "fused", 2), (21, "c128", "fused", 3),
+    (22, "c128", "z2", 2), (23, "c128", "z2", 3), (24, "c128", "fused", 2),
+    (15, "c64", "fused", 2), (16, "c64", "z2", 2), (17, "c64", "fused", 3), (18, "c64", "z2", 1),
+    (20, "c64", "fused", 2), (21, "c64", "fused", 3), (22, "c64", "z2", 2), (23, "c64", "z2", 3),
+    (23, "c64", "fused", 2), (25, "c64", "fused", 3),
+    # more cost passes than one phase-table launch takes
+    (14, "c128", "fused", 66), (16, "c64", "z2", 65),
+])
+def test_two_pass_plans(N, dtype, schedule, P):
+    print(f"two passes N={N} {dtype} {schedule} P={P}", flush=True)
+    edges = G.gnp(N, 0.5, 4400 + N + P, ["uniform", "int16"][P % 2])
+    gm, bt = G.angles(P, 4500 + N + P)
+    sv, qmap, W = O.run_weighted(N, min(N, 8), edges, gm, bt)
+    want = O.to_logical(sv, qmap)
+    st, g = State(N, C=min(N, 8), dtype=dtype), Graph(N, edges)
+    st.run(g, gm, bt, schedule)
+    got = st.copy_out(logical=True).astype(np.complex128)
+    ex, _ = st.expect_cut(g)
+    st.destroy()
+    g.destroy()
+    err = float(np.linalg.norm(got - want) / np.linalg.norm(want))
+    rel = abs(ex - O.expect_cut(sv, W)) / abs(O.expect_cut(sv, W))
+    print(f"  relative L2 error vs oracle {err:.2e}, <C> {rel:.2e}", flush=True)
+    # (N + 2) roundings per layer and amplitude at most, in quadrature
+    tol = {"c128": 1e-12, "c64": 1e-5}[dtype]
+    assert err < tol and rel < tol
