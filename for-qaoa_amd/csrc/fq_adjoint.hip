@@ -15,6 +15,10 @@
 // uncompute pass; <lambda|S|phi> commutes with the diagonal U and is
 // accumulated in the pass that applies U^+.  FP64 accumulators, fixed-order
 // reductions.
+//
+// The pair pass here is the general one: states smaller than the tiles of
+// fq_pair.hip, states that its three passes do not cover, and plans of tuning
+// knobs.
 #include "fq_device.h"
 #include "fq_internal.h"
 

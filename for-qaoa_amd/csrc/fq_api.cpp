@@ -257,6 +257,8 @@ struct fq_state {
     void *aux = nullptr;         // adjoint state (lambda), allocated on first use
     double *d_grad = nullptr;    // adjoint per-pass sums
     size_t grad_cap = 0;
+    double *d_pair = nullptr;    // partial sums of the pair passes
+    size_t pair_cap = 0;
     bool timing = false;
     std::vector<TimingRec> pending;
     std::vector<hipEvent_t> pool;
@@ -896,6 +898,7 @@ extern "C" int fq_state_destroy(fq_state *st)
         budget_give(st->bytes);
     hipFree(st->aux);
     hipFree(st->d_grad);
+    hipFree(st->d_pair);
     for (int i = 0; i < 2; ++i) {
         if (st->side[i])
             hipStreamDestroy(st->side[i]);
@@ -1217,17 +1220,37 @@ struct MixPass {
     TileArgs tab;       // cost pass: geometry, plan and angle of its phase table
     size_t entries = 0; // and its size
     const double2 *ptab = nullptr;  // where it is (mix_table, mix_tables)
+    const double *ctab = nullptr;   // (pair passes) the table of exponents
 };
 
-// Arguments as tile_pass.  The mirror pass may be a boundary pass too: the phase of a
-// mirror element is that of the N-qubit index it stands for (Cut(b) = Cut(~b)).
-static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
-                       fq_graph *g, double gamma, bool cost, bool first, int z2, const double *pre_beta, bool defer,
-                       MixPass &mp)
+// First register bit of layout l of a tile pass with K exchanges (MixLay).
+static int layout_start(int nthr, int A, int K, int l)
 {
-    const int N = st->N, Q = (int)tile.size(), A = mix_a_log(st->dtype, Q), nthr = Q - A;
+    return l == 0 ? nthr : std::max(0, nthr - A * (K - l + 1));
+}
+
+// The tile as the last layout of K exchanges holds it: thread bits = the tile
+// bits outside its register bits, in increasing order.
+static Geom layout_geom(int N, const std::vector<int> &tile, int A, int K)
+{
+    const int Q = (int)tile.size(), start = layout_start(Q - A, A, K, K);
+    std::vector<int> t2;
+    for (int i = 0; i < Q; ++i)
+        if (i < start || i >= start + A)
+            t2.push_back(tile[i]);
+    for (int r = 0; r < A; ++r)
+        t2.push_back(tile[start + r]);
+    return make_geom(N, t2, A);
+}
+
+// Geometry of a pass on compile-time phases (2^A registers a thread) into a; K
+// exchanges, lane: RX on one more thread bit by lane operations (lane_bit: whether
+// there is an instance of that).
+static int pass_shape(int N, const std::vector<int> &tile, const std::vector<int> &gates, int A,
+                      bool (*lane_bit)(int, int, int), int z2, MixArgs &a, int &K, bool &lane)
+{
+    const int Q = (int)tile.size(), nthr = Q - A;
     const Geom geom = make_geom(N, tile, A);
-    MixArgs &a = mp.a;
     memset(&a, 0, sizeof(a));
     a.N = N;
     a.Q = Q;
@@ -1244,34 +1267,32 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
     // exchanges: as many as it takes from the top thread bit down to the
     // lowest gated one, one fewer if only the bit below them is left and RX on
     // it can run on lanes
-    int K = 0, low = nthr;
+    int low = nthr;
     for (int i = nthr - 1; i >= 0; --i)
         if ((gm >> i) & 1u)
             low = i;
     K = (nthr - low + A - 1) / A;
-    if (K > 1 && low == nthr - (K - 1) * A - 1 && mix_lane_bit(Q, A, K - 1)) {
+    lane = K > 1 && low == nthr - (K - 1) * A - 1 && lane_bit(Q, A, K - 1);
+    if (lane)
         --K;
-        mp.lane = true;
-    }
     for (int i = 0; i < Q; ++i)
         a.tpos[i] = geom.tpos[i];
-    auto start = [&](int l) { return l == 0 ? nthr : std::max(0, nthr - A * (K - l + 1)); };
-    uint32_t left = mp.lane ? gm & ~(1u << low) : gm;
+    uint32_t left = lane ? gm & ~(1u << low) : gm;
     for (int l = 0; l <= K; ++l) {
-        const uint32_t m = (left >> start(l)) & ((1u << A) - 1u);
+        const int start = layout_start(nthr, A, K, l);
+        const uint32_t m = (left >> start) & ((1u << A) - 1u);
         a.gates_w |= m << (A * l);
-        left &= ~(m << start(l));
+        left &= ~(m << start);
     }
     for (int r = 0; r < A; ++r) {
         a.rpos0_w |= (uint32_t)geom.tpos[nthr + r] << (6 * r);
-        a.rposk_w |= (uint32_t)geom.tpos[start(K) + r] << (6 * r);
+        a.rposk_w |= (uint32_t)geom.tpos[layout_start(nthr, A, K, K) + r] << (6 * r);
     }
     a.ntiles = 1ull << geom.nh;
     if (z2 != Z2_OFF) {
         // the lower half is the tiles whose top index bit (qubit N-1) is 0; a
         // mirror pass pairs tile tau with ~tau instead
-        const bool ok = geom.nh >= 1 && (z2 == Z2_LOWER ? geom.hpos[geom.nh - 1] == N - 1
-                                                        : tile.back() == N - 1 && (!cost || first || pre_beta));
+        const bool ok = geom.nh >= 1 && (z2 == Z2_LOWER ? geom.hpos[geom.nh - 1] == N - 1 : tile.back() == N - 1);
         if (!ok)
             return set_err(FQ_ERR_ARG, "internal: tile does not fit the half-state pass");
         a.ntiles = 1ull << (geom.nh - 1);
@@ -1279,6 +1300,22 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
             for (int i = 0; i + 1 < Q; ++i)
                 a.mirror_pm += 1ull << tile[i];
     }
+    a.ntab = a.ntiles;
+    return FQ_OK;
+}
+
+// Arguments as tile_pass.  The mirror pass may be a boundary pass too: the phase of a
+// mirror element is that of the N-qubit index it stands for (Cut(b) = Cut(~b)).
+static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
+                       fq_graph *g, double gamma, bool cost, bool first, int z2, const double *pre_beta, bool defer,
+                       MixPass &mp)
+{
+    const int N = st->N, A = mix_a_log(st->dtype, (int)tile.size());
+    MixArgs &a = mp.a;
+    if (int rc = pass_shape(N, tile, gates, A, mix_lane_bit, z2, a, mp.K, mp.lane))
+        return rc;
+    if (z2 >= Z2_MIRROR && cost && !first && !pre_beta)
+        return set_err(FQ_ERR_ARG, "internal: the mirror pass is no cost pass of its own");
     const PassFactor f = pass_factor(st, gates.size(), beta, pre_beta, cost, defer);
     a.t = f.t;
     a.pre_t = f.pre_t;
@@ -1289,18 +1326,9 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
     a.apply_scale = f.apply;
     if (cost) {
         // phase table of the layout the cost phase runs in: layout 0, or for a
-        // boundary pass the last one (thread bits = the tile bits outside it)
-        Geom cgeom = geom;
-        if (pre_beta && K > 0) {
-            std::vector<int> t2;
-            for (int i = 0; i < Q; ++i)
-                if (i < start(K) || i >= start(K) + A)
-                    t2.push_back(tile[i]);
-            for (int r = 0; r < A; ++r)
-                t2.push_back(tile[start(K) + r]);
-            cgeom = make_geom(N, t2, A);
-        }
+        // boundary pass the last one
         TileArgs &ca = mp.tab;
+        const Geom cgeom = layout_geom(N, tile, A, pre_beta ? mp.K : 0);
         geom_to_args(cgeom, ca);
         ca.ntiles_run = a.ntiles;
         if (int rc = get_plan(g, cgeom, &ca.plan, st->stream))
@@ -1311,8 +1339,6 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
         a.init_amp = st->init_amp;
     }
     mp.cost = cost;
-    a.ntab = a.ntiles;
-    mp.K = K;
     mp.kind = pre_beta ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
     mp.mir = z2 == Z2_MIRROR ? 1 : z2 == Z2_EXPAND ? 2 : 0;
     // a half-state pass reads and writes half the state; the expanding one
@@ -1333,14 +1359,16 @@ static int mix_table(fq_state *st, MixPass &mp)
 }
 
 // The phase tables of several passes in one launch where they are small and
-// of few geometries (*done); `done` false: each pass needs mix_table.
-static int mix_tables(fq_state *st, std::vector<MixPass> &mps, bool *done)
+// of few geometries (*done), with cuts also the table of exponents of each
+// geometry; `done` false: each pass needs its own launch.
+template <typename Pass>
+static int mix_tables(fq_state *st, std::vector<Pass> &mps, bool *done, bool cuts = false)
 {
     *done = false;
     TableJobs m;
-    size_t total = 0, most = 0;
+    size_t total = 0, most = 0, ncut = 0;
     int nj = 0, ng = 0;
-    for (const MixPass &mp : mps) {
+    for (const Pass &mp : mps) {
         if (!mp.cost)
             continue;
         if (nj == FQ_TABLE_JOBS)
@@ -1354,14 +1382,18 @@ static int mix_tables(fq_state *st, std::vector<MixPass> &mps, bool *done)
         g.ntiles = mp.tab.ntiles_run;
         g.plan = mp.tab.plan;
         int k = 0;
+        bool fresh = false;
         while (k < ng && memcmp(&m.geo[k], &g, sizeof(g)) != 0)
             ++k;
         if (k == ng) {
             if (ng == FQ_TABLE_GEOS)
                 return FQ_OK;
+            m.cut_offset[ng] = (uint32_t)ncut;
+            ncut += cuts ? mp.entries : 0;
             m.geo[ng++] = g;
+            fresh = true;
         }
-        m.job[nj++] = {mp.tab.gamma, (uint32_t)k, (uint32_t)total};
+        m.job[nj++] = {mp.tab.gamma, (uint16_t)k, (uint16_t)(cuts && fresh), (uint32_t)total};
         total += mp.entries;
         most = std::max(most, mp.entries);
         if (total * sizeof(double2) > FQ_TABLES_BYTES)
@@ -1369,13 +1401,17 @@ static int mix_tables(fq_state *st, std::vector<MixPass> &mps, bool *done)
     }
     if (nj < 2)
         return FQ_OK;
-    if (int rc = reserve_phases(st, total * sizeof(double2)))
+    if (int rc = reserve_phases(st, total * sizeof(double2) + ncut * sizeof(double)))
         return rc;
-    FQ_HIP(launch_phase_tables(m, nj, most, st->d_phase, st->stream));
+    double *cut = cuts ? (double *)(st->d_phase + total) : nullptr;
+    FQ_HIP(launch_phase_tables(m, nj, most, st->d_phase, cut, st->stream));
     nj = 0;
-    for (MixPass &mp : mps)
-        if (mp.cost)
-            mp.ptab = st->d_phase + m.job[nj++].offset;
+    for (Pass &mp : mps)
+        if (mp.cost) {
+            mp.ptab = st->d_phase + m.job[nj].offset;
+            mp.ctab = cuts ? cut + m.cut_offset[m.job[nj].geo] : nullptr;
+            ++nj;
+        }
     *done = true;
     return FQ_OK;
 }
@@ -1839,6 +1875,60 @@ static int chunk_log()
     return e ? atoi(e) : 27;
 }
 
+// Two passes of width Q: the low Q qubits, and the others over the lowest 2Q - N
+// (whose RX stays in pass 0).
+static std::vector<FusedPass> split_two(int N, int Q)
+{
+    FusedPass p0, p1;
+    p0.tile = low_tile(Q);
+    p0.gates = p0.tile;
+    p1.tile = low_tile(2 * Q - N);
+    for (int q = Q; q < N; ++q) {
+        p1.tile.push_back(q);
+        p1.gates.push_back(q);
+    }
+    return {p0, p1};
+}
+
+// Three passes of width Q (exec_plan): qubits above pass 0 that pass 1 takes (0:
+// they do not fit three passes).
+static int split_low(int N, int Q, int dtype, int least)
+{
+    const int rest = N - Q, most = Q - carriers_for(dtype);
+    const int n1 = std::max(least, rest - most);
+    return n1 <= most && n1 < rest ? n1 : 0;
+}
+
+// (lane_bit: whether RX can run on the thread bit below k exchanges' reach)
+static std::vector<FusedPass> split_three(int N, int Q, int n1, int A, bool (*lane_bit)(int, int, int))
+{
+    const int c1 = Q - n1, c2 = Q - (N - Q - n1);   // carried low qubits
+    // exchanges of a pass whose lowest gated tile bit is `low`; a lane bit counts 0.4
+    auto cost = [&](int low) {
+        const int nthr = Q - A, K = low < nthr ? (nthr - low + A - 1) / A : 0;
+        return K > 1 && low == nthr - (K - 1) * A - 1 && lane_bit(Q, A, K - 1) ? K - 0.6 : (double)K;
+    };
+    // the carried qubits' RX goes to pass 1, which is no boundary pass; of the
+    // other low ones pass 2 takes those below x that save more exchanges in
+    // pass 0 than they cost in pass 2
+    int x = c1;
+    for (int y = c1 + 1; y <= std::min(c2, Q - A); ++y)
+        if (cost(y) + cost(c1) < cost(x) + cost(x > c1 ? c1 : c2))
+            x = y;
+    FusedPass p0, p1, p2;
+    p0.tile = low_tile(Q);
+    p1.tile = low_tile(c1);
+    p2.tile = low_tile(c2);
+    for (int q = Q; q < N; ++q) {
+        FusedPass &p = q < Q + n1 ? p1 : p2;
+        p.tile.push_back(q);
+        p.gates.push_back(q);
+    }
+    for (int q = 0; q < Q; ++q)
+        (q < c1 ? p1 : q < x ? p2 : p0).gates.push_back(q);
+    return {p0, p1, p2};
+}
+
 // The plan fq_run uses for P layers: layer_plan's, except that a plan of three
 // passes splits the qubits otherwise: pass 1 takes the 9 qubits right above
 // pass 0's and pass 2 the top ones, and layers end alternately on passes 0 and
@@ -1872,15 +1962,7 @@ static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
                                std::max(dtype == FQ_C128 ? 9 : 10, (N + carriers_for(dtype) + 1) / 2));
         if (Q >= N)
             return lp;
-        FusedPass p0, p1;   // the carried qubits' RX stays in pass 0
-        p0.tile = low_tile(Q);
-        p0.gates = p0.tile;
-        p1.tile = low_tile(2 * Q - N);
-        for (int q = Q; q < N; ++q) {
-            p1.tile.push_back(q);
-            p1.gates.push_back(q);
-        }
-        lp.ps = {p0, p1};
+        lp.ps = split_two(N, Q);
         lp.end1 = 1;
         lp.split = true;
         lp.open0 = z2 && P % 2 == 0 ? 1 : 0;
@@ -1888,27 +1970,11 @@ static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
     }
     if (lp.ps.size() != 3)
         return lp;
-    const int Q = tile_max_q(dtype), rest = N - Q;
-    const int n1 = std::max(9, rest - (Q - carriers_for(dtype))), n2 = rest - n1;
-    if (n2 < 1)
+    const int Q = tile_max_q(dtype);
+    const int n1 = split_low(N, Q, dtype, 9);
+    if (n1 == 0)
         return lp;
-    const int c1 = Q - n1, c2 = Q - n2;   // carried low qubits
-    FusedPass p0, p1, p2;
-    p0.tile = low_tile(Q);
-    p1.tile = low_tile(c1);
-    p2.tile = low_tile(c2);
-    for (int q = Q; q < N; ++q) {
-        FusedPass &p = q < Q + n1 ? p1 : p2;
-        p.tile.push_back(q);
-        p.gates.push_back(q);
-    }
-    // the carried qubits' RX goes to pass 1, which is no boundary pass; the
-    // one that a single exchange of pass 0 does not reach to pass 2
-    for (int q = 0; q < Q; ++q) {
-        const bool reach = q >= Q - 2 * mix_a_log(dtype, Q);
-        (q < c1 ? p1 : !reach && q < c2 ? p2 : p0).gates.push_back(q);
-    }
-    lp.ps = {p0, p1, p2};
+    lp.ps = split_three(N, Q, n1, mix_a_log(dtype, Q), mix_lane_bit);
     lp.end1 = 2;
     lp.split = true;
     const int chunk = chunk_log() - elem_log;
@@ -1960,15 +2026,13 @@ static void layer_steps(const LayerPlan &lp, int p, int P, std::vector<Step> &ou
         out.push_back({e, STEP_BOUNDARY, p});
 }
 
-// The passes of a group, chunk by chunk (2^nlog chunks), alternate chunks on
-// two streams of the state: while one chunk's first pass reads from the HBM,
-// the other's later passes run from the cache.  Every pass has its phase table
-// (at most one of them is a cost pass) before the streams fork.
-static int run_chunks(fq_state *st, const MixPass *group, size_t n, int nlog)
+// n passes chunk by chunk (2^nlog chunks), alternate chunks on two streams of
+// the state: while one chunk's first pass reads from the HBM, the other's later
+// passes run from the cache.  launch(i, c, stream) queues chunk c of pass i.
+// Every pass has its phase table before the streams fork.
+template <typename F>
+static int run_chunks(fq_state *st, int kind, size_t n, double bytes, int nlog, F &&launch)
 {
-    double bytes = 0;
-    for (size_t i = 0; i < n; ++i)
-        bytes += group[i].bytes;
     for (int i = 0; i < 2; ++i) {
         if (!st->side[i])
             FQ_HIP(hipStreamCreateWithFlags(&st->side[i], hipStreamNonBlocking));
@@ -1977,20 +2041,13 @@ static int run_chunks(fq_state *st, const MixPass *group, size_t n, int nlog)
     }
     if (!st->forked)
         FQ_HIP(hipEventCreateWithFlags(&st->forked, hipEventDisableTiming));
-    return timed(st, FQ_K_FUSED, bytes, [&] {
+    return timed(st, kind, bytes, [&] {
         hipError_t e = hipEventRecord(st->forked, st->stream);
         for (int i = 0; i < 2 && e == hipSuccess; ++i)
             e = hipStreamWaitEvent(st->side[i], st->forked, 0);
         for (uint64_t c = 0; c < 1ull << nlog && e == hipSuccess; ++c)
-            for (size_t i = 0; i < n; ++i) {
-                const MixPass &mp = group[i];
-                MixArgs a = mp.a;
-                a.ntiles >>= nlog;
-                a.tile0 = c * a.ntiles;
-                e = launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, a, mp.ptab, st->side[c & 1]);
-                if (e != hipSuccess)
-                    break;
-            }
+            for (size_t i = 0; i < n && e == hipSuccess; ++i)
+                e = launch(i, c, st->side[c & 1]);
         // joined also after a failed launch: what was queued precedes the
         // stream's later work
         for (int i = 0; i < 2; ++i) {
@@ -2003,6 +2060,33 @@ static int run_chunks(fq_state *st, const MixPass *group, size_t n, int nlog)
     }, (int)n);
 }
 
+// Tiles of chunk c of 2^nlog.
+static MixArgs chunk_args(const MixArgs &whole, uint64_t c, int nlog)
+{
+    MixArgs a = whole;
+    a.ntiles >>= nlog;
+    a.tile0 = c * a.ntiles;
+    return a;
+}
+
+// Number of steps from seq[k] on that run chunk by chunk together: a run of
+// passes that stay within one chunk, with at most one cost phase among them (one
+// phase table); 1: a single pass over the whole state.
+static size_t chunk_group(const LayerPlan &lp, const std::vector<Step> &seq, size_t k)
+{
+    auto local = [&](const Step &s) {
+        const std::vector<int> &t = lp.ps[s.pass].tile;
+        return lp.chunk > 0 && *std::max_element(t.begin(), t.end()) < lp.chunk;
+    };
+    size_t n = 1;
+    if (local(seq[k])) {
+        bool c = seq[k].kind != STEP_PLAIN;
+        for (; k + n < seq.size() && local(seq[k + n]) && !(c && seq[k + n].kind != STEP_PLAIN); ++n)
+            c = c || seq[k + n].kind != STEP_PLAIN;
+    }
+    return n;
+}
+
 // Layers [p0, p1) of P.  expand: the last layer's mirror pass also writes the
 // upper half of the full state.
 static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, int p1, int P, const double *gammas,
@@ -2013,10 +2097,6 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
     std::vector<Step> seq;
     for (int p = p0; p < p1; ++p)
         layer_steps(lp, p, P, seq);
-    // a pass that stays within one chunk
-    auto local = [&](const Step &s) {
-        return lp.chunk > 0 && *std::max_element(ps[s.pass].tile.begin(), ps[s.pass].tile.end()) < lp.chunk;
-    };
     auto cost = [](const Step &s) { return s.kind != STEP_PLAIN; };
     // every pass on the compile-time kernel (the pass widths of tuning knobs
     // may have none): prepared first, and small phase tables made at once
@@ -2049,19 +2129,20 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
     if (int rc = mix_tables(st, mps, &tables))
         return rc;
     for (size_t k = 0; k < seq.size();) {
-        // passes of one group: a run of local ones with at most one cost
-        // phase among them (one phase table), else a single pass
-        size_t n = 1;
-        if (local(seq[k])) {
-            bool c = cost(seq[k]);
-            for (; k + n < seq.size() && local(seq[k + n]) && !(c && cost(seq[k + n])); ++n)
-                c = c || cost(seq[k + n]);
-        }
+        const size_t n = chunk_group(lp, seq, k);
         int rc = FQ_OK;
         for (size_t i = 0; i < n && !tables && rc == FQ_OK; ++i)
             rc = mix_table(st, mps[k + i]);
         if (rc == FQ_OK && n > 1) {
-            rc = run_chunks(st, &mps[k], n, (z2 ? st->N - 1 : st->N) - lp.chunk);
+            const int nlog = (z2 ? st->N - 1 : st->N) - lp.chunk;
+            double bytes = 0;
+            for (size_t i = 0; i < n; ++i)
+                bytes += mps[k + i].bytes;
+            rc = run_chunks(st, FQ_K_FUSED, n, bytes, nlog, [&](size_t i, uint64_t c, hipStream_t stream) {
+                const MixPass &mp = mps[k + i];
+                return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, chunk_args(mp.a, c, nlog), mp.ptab,
+                                  stream);
+            });
         } else if (rc == FQ_OK) {
             const MixPass &mp = mps[k];
             rc = timed(st, FQ_K_FUSED, mp.bytes, [&] {
@@ -2299,7 +2380,209 @@ static int ensure_aux(fq_state *st, size_t grad_slots)
     return FQ_OK;
 }
 
-// Reverse-uncompute gradient of <C> (fq_adjoint.hip).  The state must hold
+// lambda = Cut psi_P (on the half state from N = 3 on); sum |psi|^2 Cut and
+// sum |psi|^2 into d_grad.
+static int cut_lambda(fq_state *st, fq_graph *g)
+{
+    const int N = st->N, Q = std::min(12, N >= 3 ? N - 1 : N);
+    const int a_log = std::max(1, std::min(4, Q));
+    Geom geom = make_geom(N, low_tile(Q), a_log);
+    TileArgs a;
+    geom_to_args(geom, a);
+    if (N >= 3)
+        a.ntiles_run = 1ull << (geom.nh - 1);   // qubit N-1 is the top hidden bit
+    if (int rc = get_plan(g, geom, &a.plan, st->stream))
+        return rc;
+    FQ_HIP(launch_cut_mul(st->dtype, a_log, st->sv, st->aux, a, st->d_part, st->stream));
+    FQ_HIP(launch_finalize(st->d_part, run_tiles(a), st->d_grad, st->stream));
+    return FQ_OK;
+}
+
+// Partial sums of the pair passes (doubles) and the sums of `sums` of them after
+// d_grad's first two.
+static int ensure_pair_scratch(fq_state *st, size_t part, size_t sums)
+{
+    if (part > st->pair_cap) {
+        FQ_HIP(hipStreamSynchronize(st->stream));
+        hipFree(st->d_pair);
+        st->d_pair = nullptr;
+        st->pair_cap = 0;
+        if (hipMalloc(&st->d_pair, sizeof(double) * part) != hipSuccess)
+            return set_err(FQ_ERR_OOM, "gradient scratch allocation failed");
+        st->pair_cap = part;
+    }
+    return ensure_aux(st, 1 + (sums + 1) / 2);
+}
+
+// One pair pass of the walk back on compile-time phases (fq_pair.hip).
+struct PairPass {
+    PairArgs a;
+    int K = 0, kind = 0;
+    bool lane = false, mir = false, cost = false;
+    double weight = 1.0;   // of the pass's sums (the states' magnitude before it)
+    TileArgs tab;
+    size_t entries = 0;
+    const double2 *ptab = nullptr;
+    const double *ctab = nullptr;
+};
+
+// The passes of the pair walk back over an N-qubit half state: two of the
+// narrowest tiles, or three of full width, as exec_plan's; no passes where they do
+// not fit (very small and very large states) or a tuning knob is set.  Chunks hold
+// both states.
+static LayerPlan pair_plan(int N, int dtype)
+{
+    LayerPlan lp{{}, -1, 0, false, 0};
+    for (const char *k : {"FQ_TILE_Q", "FQ_PASS_BLOCK", "FQ_CARRIER_GATES", "FQ_LAYER_PIPE"})
+        if (getenv(k))
+            return lp;
+    const int Qmin = dtype == FQ_C128 ? 9 : 10, Qmax = dtype == FQ_C128 ? 12 : 13;
+    const int Q2 = std::max(Qmin, (N + carriers_for(dtype) + 1) / 2);
+    if (Q2 >= N)
+        return lp;
+    lp.split = true;
+    if (Q2 <= Qmax) {
+        lp.ps = split_two(N, Q2);
+        lp.end1 = 1;
+        return lp;
+    }
+    const int n1 = split_low(N, Qmax, dtype, 8);
+    if (n1 == 0)
+        return lp;
+    lp.ps = split_three(N, Qmax, n1, pair_a_log(dtype, Qmax), pair_lane_bit);
+    lp.end1 = 2;
+    const int elem_log = dtype == FQ_C128 ? 4 : 3, chunk = chunk_log() - 1 - elem_log;
+    if (N + elem_log > FQ_CACHE_LOG && chunk >= Qmax + n1 && chunk < N - 1)
+        lp.chunk = chunk;
+    return lp;
+}
+
+// The walk back over plan lp: <C> and the gradient sums of psi_P and lambda (both
+// on the half state, cut_lambda), not yet doubled.  Every RX is the
+// butterfly of rx_tform on both states, which grows them by (1 + t^2)^(1/2) a gate:
+// mag2 follows the inverse of what <lambda|psi> has taken on, each sum gets its
+// value as a weight, and each cost pass scales it back to 1.
+static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, const double *gammas, const double *betas,
+                     double *expect, double *grad_gammas, double *grad_betas)
+{
+    const int N = st->N, m = (int)lp.ps.size(), Q = (int)lp.ps[0].tile.size(), A = pair_a_log(st->dtype, Q);
+    std::vector<Step> seq;
+    for (int p = 0; p < P; ++p)
+        layer_steps(lp, p, P, seq);
+    std::reverse(seq.begin(), seq.end());
+    std::vector<PairPass> pp(seq.size());
+    double mag2 = 1.0;
+    for (size_t k = 0; k < seq.size(); ++k) {
+        const Step &s = seq[k];
+        PairPass &q = pp[k];
+        const bool bd = s.kind == STEP_BOUNDARY;
+        q.kind = bd ? PAIR_BOUNDARY : s.kind == STEP_PLAIN ? PAIR_PLAIN : PAIR_COST;
+        q.mir = s.pass + 1 == m;
+        q.cost = q.kind != PAIR_PLAIN;
+        memset(&q.a, 0, sizeof(q.a));
+        MixArgs &a = q.a.m;
+        if (int rc = pass_shape(N, lp.ps[s.pass].tile, lp.ps[s.pass].gates, A, pair_lane_bit,
+                                q.mir ? Z2_MIRROR : Z2_LOWER, a, q.K, q.lane))
+            return rc;
+        double sr, si, t1, t0;
+        const int later = bd ? s.layer + 1 : s.layer;
+        rx_tform(-betas[later], st->dtype, true, &t1, &sr, &si);
+        rx_tform(-betas[s.layer], st->dtype, true, &t0, &sr, &si);
+        a.pre_t = t1;
+        a.t = bd ? t0 : t1;
+        a.pre_tf = (float)a.pre_t;   // exact for complex64
+        a.tf = (float)a.t;
+        q.weight = mag2;
+        double w = 1.0;
+        auto gate = [&](bool on, double t, double &slot) {
+            slot = on ? w : 0.0;
+            w *= on ? 1.0 / (1.0 + t * t) : 1.0;
+        };
+        gate(q.lane, t1, q.a.up[PAIR_LANE]);
+        for (int i = 0; i < A * (q.K + 1); ++i)
+            gate((a.gates_w >> i) & 1u, t1, q.a.up[i]);
+        if (q.cost) {
+            q.a.phase = w;
+            a.scale_re = std::sqrt(mag2 * w);
+            w /= a.scale_re * a.scale_re;
+            TileArgs &ca = q.tab;
+            geom_to_args(layout_geom(N, lp.ps[s.pass].tile, A, q.K), ca);
+            ca.ntiles_run = a.ntiles;
+            if (int rc = get_plan(g, layout_geom(N, lp.ps[s.pass].tile, A, q.K), &ca.plan, st->stream))
+                return rc;
+            set_cost(ca, -gammas[later], st->init_amp);
+            q.entries = phase_table_entries(ca, A);
+        }
+        if (bd) {
+            for (int l = q.K; l >= 0; --l)
+                for (int r = 0; r < A; ++r)
+                    gate((a.gates_w >> (A * l + r)) & 1u, t0, q.a.down[A * l + r]);
+            gate(q.lane, t0, q.a.down[PAIR_LANE]);
+        }
+        mag2 *= w;
+    }
+    // partial sums of as many passes as fit 16 MiB at once
+    const uint64_t tiles = 1ull << (N - 1 - Q);
+    const size_t per = 3 * (size_t)tiles, batch = std::max<size_t>(1, std::min(pp.size(), ((size_t)2 << 20) / per));
+    if (int rc = ensure_pair_scratch(st, batch * per, 3 * pp.size()))
+        return rc;
+    bool tables = false;
+    if (int rc = mix_tables(st, pp, &tables, true))
+        return rc;
+    const double bytes = 2.0 * (double)st->bytes;   // two half states read and written
+    auto launch = [&](size_t k, const MixArgs &a, hipStream_t stream) {
+        PairArgs pa = pp[k].a;
+        pa.m = a;
+        return launch_pair_pass(st->dtype, pp[k].K, pp[k].lane, pp[k].kind, pp[k].mir, st->sv, st->aux, pa, pp[k].ptab,
+                                pp[k].ctab, st->d_pair + per * (k % batch), stream);
+    };
+    for (size_t k = 0; k < pp.size();) {
+        size_t n = chunk_group(lp, seq, k);
+        n = std::min(n, batch - k % batch);   // a group's sums stay within one batch
+        for (size_t i = 0; i < n && !tables; ++i)
+            if (pp[k + i].cost) {
+                double *ctab = nullptr;
+                if (int rc = prepare_phases(st, pp[k + i].tab, A, &ctab))
+                    return rc;
+                pp[k + i].ptab = st->d_phase;
+                pp[k + i].ctab = ctab;
+            }
+        int rc;
+        if (n > 1) {
+            const int nlog = N - 1 - lp.chunk;
+            rc = run_chunks(st, FQ_K_ADJOINT, n, bytes * (double)n, nlog, [&](size_t i, uint64_t c, hipStream_t stream) {
+                return launch(k + i, chunk_args(pp[k + i].a.m, c, nlog), stream);
+            });
+        } else {
+            rc = timed(st, FQ_K_ADJOINT, bytes, [&] { return launch(k, pp[k].a.m, st->stream); });
+        }
+        if (rc)
+            return rc;
+        k += n;
+        if (k % batch == 0 || k == pp.size()) {
+            const size_t first = (k - 1) / batch * batch;
+            FQ_HIP(launch_pair_sums(st->d_pair, tiles, (int)(k - first), st->d_grad + 2 + 3 * first, st->stream));
+        }
+    }
+    std::vector<double> sums(2 + 3 * pp.size());
+    FQ_HIP(hipMemcpyAsync(sums.data(), st->d_grad, sizeof(double) * sums.size(), hipMemcpyDeviceToHost, st->stream));
+    FQ_HIP(hipStreamSynchronize(st->stream));
+    *expect = sums[0];
+    const double *h = sums.data() + 2;
+    for (int k = 0; k < P; ++k)
+        grad_gammas[k] = grad_betas[k] = 0.0;
+    for (size_t k = 0; k < pp.size(); ++k) {
+        const int later = pp[k].kind == PAIR_BOUNDARY ? seq[k].layer + 1 : seq[k].layer;
+        grad_betas[later] += pp[k].weight * h[3 * k];
+        if (pp[k].cost)
+            grad_gammas[later] = -pp[k].weight * h[3 * k + 1];
+        if (pp[k].kind == PAIR_BOUNDARY)
+            grad_betas[seq[k].layer] += pp[k].weight * h[3 * k + 2];
+    }
+    return FQ_OK;
+}
+
+// Reverse-uncompute gradient of <C> (fq_adjoint.hip, fq_pair.hip).  The state must hold
 // psi_P of fq_run(FUSED or Z2) with the same graph and angles (identity qubit
 // map); it is consumed (for N >= 3 its lower half is walked back to |+>^N and
 // its upper half is left as it was).
@@ -2325,6 +2608,24 @@ extern "C" int fq_backward(fq_state *st, fq_graph *g, int P, const double *gamma
     // stale (the state is consumed).
     const bool z2 = N >= 3;
     const double mult = z2 ? 2.0 : 1.0;
+    if (const LayerPlan lp = pair_plan(N, st->dtype); !lp.ps.empty()) {
+        // (sums of 1 + P (m - 1) passes after the two of <C>)
+        const size_t passes = 1 + (size_t)P * (lp.ps.size() - 1);
+        if (int rc = ensure_aux(st, 1 + (3 * passes + 1) / 2))
+            return rc;
+        if (int rc = cut_lambda(st, g))
+            return rc;
+        double e = 0;
+        if (int rc = pair_walk(st, g, lp, P, gammas, betas, &e, grad_gammas, grad_betas))
+            return rc;
+        for (int k = 0; k < P; ++k) {
+            grad_gammas[k] *= mult;
+            grad_betas[k] *= mult;
+        }
+        if (expect)
+            *expect = mult * e;
+        return FQ_OK;
+    }
     // 2^12-amplitude tiles of psi and lambda share the LDS (2 x 68 KiB);
     // 512 threads x 8 amplitudes of each state
     const int Qb = std::min(12, z2 ? N - 1 : N);
@@ -2371,20 +2672,8 @@ extern "C" int fq_backward(fq_state *st, fq_graph *g, int P, const double *gamma
     if (int rc = ensure_aux(st, nslot))
         return rc;
 
-    // lambda = Cut * psi_P, <C> into slot 0
-    {
-        const int Q = Qb;
-        const int a_log = std::max(1, std::min(4, Q));
-        Geom geom = make_geom(N, low_tile(Q), a_log);
-        TileArgs a;
-        geom_to_args(geom, a);
-        if (z2)
-            a.ntiles_run = 1ull << (geom.nh - 1);   // qubit N-1 is the top hidden bit
-        if (int rc = get_plan(g, geom, &a.plan, st->stream))
-            return rc;
-        FQ_HIP(launch_cut_mul(st->dtype, a_log, st->sv, st->aux, a, st->d_part, st->stream));
-        FQ_HIP(launch_finalize(st->d_part, run_tiles(a), st->d_grad, st->stream));
-    }
+    if (int rc = cut_lambda(st, g))
+        return rc;
     // (launch index in fwd, first slot) of every launch, for the sums below
     std::vector<size_t> slot_of(fwd.size());
     {

@@ -87,6 +87,8 @@ struct TileArgs {
 
 // One pass of the compile-time tile kernel (fq_mix.hip).
 enum { MIX_PLAIN = 0, MIX_FIRST = 1, MIX_COST = 2, MIX_BOUNDARY = 3 };
+// The same of a pair pass of the gradient (fq_pair.hip).
+enum { PAIR_PLAIN = 0, PAIR_COST = 1, PAIR_BOUNDARY = 2 };
 struct MixArgs {
     int N, Q, nh;
     int has_rr;              // any register-register edge in the plan
@@ -103,6 +105,15 @@ struct MixArgs {
     double scale_re, scale_im;  // factor of the pass: in the cost phase, or before the
     int apply_scale;            // stores (apply_scale)
     double init_amp;
+};
+// One pair pass: t, pre_t and the real scale as above (a boundary pass undoes
+// RX(pre) first), and the weights of its sums: the inverse of the factor that
+// <lambda|X|psi> has taken in this pass when the sum is formed, for register bit r
+// of layout l at A l + r (0: not gated), the lane bit at PAIR_LANE, the phase.
+#define PAIR_LANE 16
+struct PairArgs {
+    MixArgs m;
+    double up[PAIR_LANE + 1], down[PAIR_LANE + 1], phase;
 };
 
 // Tiles a launch processes (a Z2-reduced state runs the lower half only).
@@ -122,11 +133,12 @@ struct TableGeo {
 };
 struct TableJob {
     double gamma;
-    uint32_t geo;
+    uint16_t geo, cut;       // cut: this job also writes the geometry's exponents
     uint32_t offset;         // entries
 };
 struct TableJobs {
     TableGeo geo[FQ_TABLE_GEOS];
+    uint32_t cut_offset[FQ_TABLE_GEOS];  // place of each geometry's exponents
     TableJob job[FQ_TABLE_JOBS];
 };
 
@@ -191,8 +203,10 @@ hipError_t launch_tile_mirror(int dtype, int a_log, bool expand, void *sv, const
 hipError_t launch_phase_table(const TileArgs &a, int a_log, double2 *tab, double *cut,
                               hipStream_t stream);
 size_t phase_table_entries(const TileArgs &a, int a_log);
-// njobs tables of at most `entries` entries each
-hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, hipStream_t stream);
+// njobs tables of at most `entries` entries each; cut not null: the exponents of
+// the geometries too
+hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, double *cut,
+                               hipStream_t stream);
 hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t stream);
 hipError_t launch_expect(int dtype, int a_log, const void *sv, const TileArgs &a, double *partials,
                          double *out2, hipStream_t stream);
@@ -219,6 +233,14 @@ hipError_t launch_pair(int dtype, int a_log, bool costbw, bool mirror, bool boun
 hipError_t launch_cut_mul(int dtype, int a_log, const void *psi, void *lam, const TileArgs &a,
                           double *partials, hipStream_t stream);
 size_t pair_lds_bytes(int dtype, int Q);
+// Pair passes of fq_pair.hip; arguments as launch_mix (register bits per thread
+// pair_a_log, 0: no instance for this tile width).  partials: three sums per tile.
+int pair_a_log(int dtype, int Q);
+bool pair_lane_bit(int Q, int A, int k);
+hipError_t launch_pair_pass(int dtype, int k, bool lane, int kind, bool mir, void *psi, void *lam, const PairArgs &a,
+                            const double2 *ptab, const double *ctab, double *partials, hipStream_t stream);
+// out[3 s ..] = the sums of pass s's n triples (partials + 3 n s)
+hipError_t launch_pair_sums(const double *partials, uint64_t n, int passes, double *out, hipStream_t stream);
 // packed slabs (fq_serve.hip)
 hipError_t launch_slab_phase_table(const TileArgs &local, int a_log, const SlotParams *slots, int nslots,
                                    double2 *tabs, size_t stride, hipStream_t stream);

@@ -64,7 +64,8 @@ __global__ void __launch_bounds__(256) k_phase_table(const TileArgs a, int a_log
 // The phase tables of several cost passes in one launch (blockIdx.y: the
 // pass).  A small state's passes take 5 to 20 us each; a table launch before
 // each of them took another 4 to 6 us, most of it latency.
-__global__ void __launch_bounds__(256) k_phase_tables(const TableJobs m, double2 *__restrict__ tab)
+__global__ void __launch_bounds__(256) k_phase_tables(const TableJobs m, double2 *__restrict__ tab,
+                                                      double *__restrict__ cut)
 {
     const TableJob &job = m.job[blockIdx.y];
     const TableGeo &g = m.geo[job.geo];
@@ -75,6 +76,8 @@ __global__ void __launch_bounds__(256) k_phase_tables(const TableJobs m, double2
     double sn, cs;
     sincos(job.gamma * coef, &sn, &cs);
     tab[job.offset + gid] = make_double2(cs, sn);
+    if (job.cut)
+        cut[m.cut_offset[job.geo] + gid] = coef;
 }
 
 __device__ __forceinline__ void zmul(double &x, double &y, double2 f)
@@ -1506,10 +1509,11 @@ hipError_t launch_phase_table(const TileArgs &a, int a_log, double2 *tab, double
     return hipGetLastError();
 }
 
-hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, hipStream_t stream)
+hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, double *cut,
+                               hipStream_t stream)
 {
     hipLaunchKernelGGL(k_phase_tables, dim3((unsigned)((entries + 255) / 256), (unsigned)njobs), dim3(256), 0, stream, m,
-                       tab);
+                       tab, cut);
     return hipGetLastError();
 }
 
