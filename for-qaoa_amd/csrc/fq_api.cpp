@@ -1760,6 +1760,64 @@ extern "C" int fq_multi_rx(fq_state *st, const int *targets, int gate_size, doub
     return rx_targets(st, t, beta);
 }
 
+// Qubit p changes places with qubit partner[p] (partner[partner[p]] == p).
+static int exchange_qubits(fq_state *st, const uint8_t *partner)
+{
+    const int N = st->N;
+    SwapArgs a;
+    memset(&a, 0, sizeof(a));
+    int moved = 0, least = N;   // pairs; the lowest upper qubit of one
+    for (int p = 0; p < N; ++p)
+        if (partner[p] > p) {
+            moved++;
+            least = std::min(least, (int)partner[p]);
+        }
+    // the tile takes qubits from the lowest up, each with its partner: 2^10
+    // complex128 and 2^12 complex64 amplitudes, two of them 32 and 64 KiB
+    // (complex64 N=27 13 qubits with 2^10 and 2^12: 462 and 450 us; below N=24, too
+    // few units for the chip: N=20 8 qubits 7.2 and 8.5)
+    const int most = std::min(N, st->dtype == FQ_C128 || N < 24 ? 10 : 12);
+    bool in[FQ_MAXN] = {false};
+    for (int p = 0; p < N; ++p) {
+        const int n = partner[p] == p ? 1 : 2;
+        if (!in[p] && a.tb + n <= most) {
+            in[p] = in[partner[p]] = true;
+            a.tb += n;
+        }
+    }
+    std::vector<int> lower, upper, rest;
+    int t = 0, bit[FQ_MAXN];
+    for (int p = 0; p < N; ++p) {
+        bit[p] = t;
+        if (in[p]) {
+            a.tpos[t++] = (uint8_t)p;
+        } else if (partner[p] > p) {
+            lower.push_back(p);
+            upper.push_back(partner[p]);
+        } else if (partner[p] == p) {
+            rest.push_back(p);
+        }
+    }
+    for (int i = 0; i < t; ++i)
+        a.partner[i] = (uint8_t)bit[partner[a.tpos[i]]];
+    auto runs = [](const std::vector<int> &pos, SwapRuns &r) {
+        for (size_t i = 0, j; i < pos.size(); i = j) {
+            for (j = i + 1; j < pos.size() && pos[j] == pos[j - 1] + 1; ++j)
+                ;
+            r.run[r.n++] = (uint32_t)i | ((uint32_t)(j - i) << 8) | ((uint32_t)pos[i] << 16);
+        }
+    };
+    runs(lower, a.lower);
+    runs(upper, a.upper);
+    runs(rest, a.rest);
+    a.nr = (int)rest.size();
+    a.npairs = (1ull << lower.size()) * ((1ull << lower.size()) + 1) / 2;
+    a.rest_fast = a.nr > 0 && rest[0] < least;
+    // an amplitude stays where the bits of each pair are equal
+    const double bytes = 2.0 * (double)st->bytes * (1.0 - std::ldexp(1.0, -moved));
+    return timed(st, FQ_K_SWAP, bytes, [&] { return launch_swap(st->dtype, st->sv, a, st->stream); });
+}
+
 extern "C" int fq_swap_conti(fq_state *st, int swap_out, int swap_in, int num_swap)
 {
     if (int rc = check_state(st))
@@ -1770,46 +1828,14 @@ extern "C" int fq_swap_conti(fq_state *st, int swap_out, int swap_in, int num_sw
                        swap_in, k, N);
     if (k == 0)
         return FQ_OK;
-    SwapArgs a;
-    memset(&a, 0, sizeof(a));
-    a.N = N;
-    a.out = swap_out;
-    a.in = swap_in;
-    a.k = k;
-    // out == 0 (the driver's case): pipelined LDS-tiled transpose with tiles
-    // of 2^10 (complex128) / 2^12 (complex64) amplitudes read as runs of
-    // >= 512 B where the blocks allow; one pair of sub-tiles per work-group
-    // for small blocks; otherwise one thread per pair.
-    a.t = -1;
-    if (swap_out == 0) {
-        const int tile_log = st->dtype == FQ_C128 ? 10 : 12;
-        const int t = std::min(k, tile_log / 2);
-        const int m = t == k ? std::max(0, std::min(tile_log - 2 * k, swap_in - k)) : 0;
-        if (2 * t + m == tile_log) {
-            a.pipe = 1;
-            a.t = t;
-            a.m = m;
-        } else if (k >= 3) {
-            a.t = std::min(k, 5);
-        }
-        if (a.t >= 0) {
-            const uint64_t mb = 1ull << (k - a.t);
-            a.npairs = mb * (mb + 1) / 2;
-        }
-    }
-    // rest bits: everything outside both blocks and the tile's rest bits
-    bool used[FQ_MAXN] = {false};
-    for (int i = 0; i < k; ++i)
-        used[swap_out + i] = used[swap_in + i] = true;
-    for (int i = 0; i < a.m; ++i)
-        used[k + i] = true;
+    uint8_t partner[FQ_MAXN];
     for (int p = 0; p < N; ++p)
-        if (!used[p])
-            a.rpos[a.nr++] = (uint8_t)p;
-    a.rest_fast = a.pipe && a.nr > 0 && a.rpos[0] < swap_in;
-    const double bytes = 2.0 * (double)st->bytes * (1.0 - std::ldexp(1.0, -k));
-    int rc = timed(st, FQ_K_SWAP, bytes, [&] { return launch_swap(st->dtype, st->sv, a, st->stream); });
-    if (rc)
+        partner[p] = (uint8_t)p;
+    for (int i = 0; i < k; ++i) {
+        partner[swap_out + i] = (uint8_t)(swap_in + i);
+        partner[swap_in + i] = (uint8_t)(swap_out + i);
+    }
+    if (int rc = exchange_qubits(st, partner))
         return rc;
     for (int i = 0; i < k; ++i)
         std::swap(st->qmap[swap_out + i], st->qmap[swap_in + i]);
@@ -2156,6 +2182,67 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
     return FQ_OK;
 }
 
+// FQ_SCHED_REFERENCE without its single steps: every layer applies RX(beta) to
+// each qubit once, wherever the transpositions have moved it, so the P layers are
+// those of the fused schedule in the labels of the start, followed by the
+// product of all transpositions.  That permutation of the qubits is a product of
+// two exchanges of disjoint pairs, each one pass over the state: a cycle
+// (c_0 .. c_{n-1}) is c_i <-> c_{-i}, then c_i <-> c_{1-i}.  N=28 P=3 complex128
+// C=12 with <C> on MI355X: 30.8 -> 12.6 ms (every step was a pass over the state,
+// bound by HBM: 6 a layer).
+static int reference_run(fq_state *st, fq_graph *g, const std::vector<int> &sizes, int P, const double *gammas,
+                         const double *betas)
+{
+    const int N = st->N;
+    if (P == 0)
+        return FQ_OK;
+    if (int rc = run_layers(st, g, exec_plan(N, st->dtype, false, P), 0, P, P, gammas, betas, false, true))
+        return rc;
+    int at[FQ_MAXN], to[FQ_MAXN], qmap[FQ_MAXN];   // position -> the position its qubit came from, and back
+    for (int p = 0; p < N; ++p)
+        at[p] = p;
+    for (int p = 0; p < P; ++p)
+        for (size_t i = 0, in = 0; i + 1 < sizes.size(); ++i) {
+            in += sizes[i];
+            for (int t = 0; t < sizes[i + 1]; ++t)
+                std::swap(at[t], at[in + t]);
+        }
+    uint8_t first[FQ_MAXN], second[FQ_MAXN];
+    bool seen[FQ_MAXN] = {false}, any[2] = {false, false};
+    for (int p = 0; p < N; ++p) {
+        to[at[p]] = p;
+        qmap[p] = st->qmap[at[p]];
+    }
+    for (int p = 0; p < N; ++p) {
+        std::vector<int> c;
+        for (int q = p; !seen[q]; q = to[q]) {
+            seen[q] = true;
+            c.push_back(q);
+        }
+        const int n = (int)c.size();
+        for (int i = 0; i < n; ++i) {
+            first[c[i]] = (uint8_t)c[(n - i) % n];
+            second[c[i]] = (uint8_t)c[(n + 1 - i) % n];
+            any[0] |= first[c[i]] != c[i];
+            any[1] |= second[c[i]] != c[i];
+        }
+    }
+    if (any[0])
+        if (int rc = exchange_qubits(st, first))
+            return rc;
+    if (any[1])
+        if (int rc = exchange_qubits(st, second))
+            return rc;
+    std::copy(qmap, qmap + N, st->qmap);
+    for (int p = 0; p < P; ++p)
+        for (size_t i = 0, in = 0; i + 1 < sizes.size(); ++i) {
+            in += sizes[i];
+            if (int rc = fq_graph_relabel(g, 0, (int)in, sizes[i + 1]))
+                return rc;
+        }
+    return FQ_OK;
+}
+
 extern "C" int fq_run(fq_state *st, fq_graph *g, int P, const double *gammas, const double *betas,
                       int schedule)
 {
@@ -2181,6 +2268,9 @@ extern "C" int fq_run(fq_state *st, fq_graph *g, int P, const double *gammas, co
         std::vector<int> sizes;
         for (int i = 0; i < N; i += st->C)
             sizes.push_back(std::min(st->C, N - i));
+        // (with class timing on, launch by launch, so that each class is timed)
+        if (!st->timing)
+            return reference_run(st, g, sizes, P, gammas, betas);
         for (int p = 0; p < P; ++p) {
             if (int rc = cost_pass(st, g, gammas[p], p == 0))
                 return rc;

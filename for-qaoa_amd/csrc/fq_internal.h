@@ -156,15 +156,23 @@ struct SlotParams {
     PlanDev eplan;           // cut plan of the <C> reduction geometry
 };
 
+#define FQ_SWAP_BITS 12     // qubits of an exchange tile: 2^12 complex64, 2^10 complex128
+
+// As BitRuns, for any set of positions.
+struct SwapRuns {
+    int n;
+    uint32_t run[FQ_MAXN / 2];
+};
+
+// Exchange of pairs of qubits (k_exchange).
 struct SwapArgs {
-    int N, out, in, k;
-    int t;                   // tiled: sub-tile log2 side (-1: one thread per pair)
-    int m;                   // pipelined: rest bits [k, k+m) inside the tile (t == k)
-    int pipe;                // pipelined persistent kernel (1) or one pair per work-group (0)
-    int rest_fast;           // pipelined: consecutive units step the rest index first
-    int nr;                  // number of rest bits (outside the tile)
-    uint8_t rpos[FQ_MAXN];   // rest bit -> physical position
-    uint64_t npairs;         // tiled: number of (X <= Y) sub-tile pairs
+    int tb;                          // tile qubits
+    int rest_fast;                   // consecutive units step the rest index first
+    int nr;                          // bits of the rest index
+    uint8_t tpos[FQ_SWAP_BITS];      // tile bit -> position (ascending)
+    uint8_t partner[FQ_SWAP_BITS];   // tile bit -> the tile bit it changes places with (itself if none)
+    SwapRuns lower, upper, rest;     // positions of the pairs outside the tile, and of the others
+    uint64_t npairs;                 // X <= Y
 };
 
 // Resident work-groups per CU of kernel fn at this block size and dynamic

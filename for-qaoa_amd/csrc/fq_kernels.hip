@@ -15,7 +15,7 @@
 //            are remapped into registers through padded LDS phases.
 //            Replaces _rotationCompressionWeighted_conti (src/rzz.cu:121-156)
 //            and _multirotateX_unroll (src/rx.cu:56-87).
-//  k_swap_tiled / k_swap_generic
+//  k_exchange
 //            in-place qubit-block exchange [out,out+k) <-> [in,in+k);
 //            replaces _swap_gate_conti (src/swap.cu:76-102) without the
 //            host-built pair table: 2^t x 2^t sub-tiles are transposed
@@ -801,56 +801,24 @@ __global__ void __launch_bounds__(1024) k_finalize(const double *__restrict__ pa
     }
 }
 
-// ---- block transposition ---------------------------------------------------
+// (the amplitude types as clang vectors)
+template <typename T> struct NativeVec;
+template <> struct NativeVec<double2> { typedef double type __attribute__((ext_vector_type(2))); };
+template <> struct NativeVec<float2> { typedef float type __attribute__((ext_vector_type(2))); };
 
-__device__ __forceinline__ uint64_t deposit_rest(uint64_t r, const SwapArgs &a)
-{
-    uint64_t o = 0;
-    for (int i = 0; i < a.nr; ++i)
-        o |= ((r >> i) & 1ull) << a.rpos[i];
-    return o;
-}
-
-// out == 0: the low block is contiguous.  Work-group = one pair of 2^t x 2^t
-// sub-tiles (X <= Y) of the 2^k x 2^k transpose for one rest index.
-template <typename T>
-__global__ void __launch_bounds__(256) k_swap_tiled(T *__restrict__ sv, const SwapArgs a)
-{
-    extern __shared__ __align__(16) unsigned char fq_smem[];
-    const int side = 1 << a.t;
-    const int stride = side + 1;
-    T *la = reinterpret_cast<T *>(fq_smem);
-    T *lb = la + side * stride;
-    const uint64_t lin = blockIdx.x;
-    const uint64_t p = lin % a.npairs;
-    const uint64_t r = lin / a.npairs;
-    // p -> (X <= Y): p = Y(Y+1)/2 + X
-    uint64_t Y = (uint64_t)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
-    while (Y * (Y + 1) / 2 > p)
-        --Y;
-    while ((Y + 1) * (Y + 2) / 2 <= p)
-        ++Y;
-    const uint64_t X = p - Y * (Y + 1) / 2;
-    const uint64_t base = deposit_rest(r, a);
-    const int n = side * side;
-    const int s = a.in;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int xr = i >> a.t, yc = i & (side - 1);
-        la[xr * stride + yc] = sv[base + ((X * side + xr) << s) + (Y * side + yc)];
-        if (X != Y)
-            lb[xr * stride + yc] = sv[base + ((Y * side + xr) << s) + (X * side + yc)];
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int xr = i >> a.t, yc = i & (side - 1);
-        if (X != Y) {
-            sv[base + ((X * side + xr) << s) + (Y * side + yc)] = lb[yc * stride + xr];
-            sv[base + ((Y * side + xr) << s) + (X * side + yc)] = la[yc * stride + xr];
-        } else {
-            sv[base + ((X * side + xr) << s) + (Y * side + yc)] = la[yc * stride + xr];
-        }
-    }
-}
+// ---- qubit exchange ---------------------------------------------------------
+//
+// Exchanges pairs of qubits in place: the amplitude at index i goes to the index
+// with the bits of every pair exchanged.  A tile is a set of 2^tb indices closed
+// under the exchange: the lowest qubits and their partners, so that it is read
+// and written in contiguous runs (512 B where half of its qubits are low ones).
+// It is permuted in LDS and written to the tile whose other bits are exchanged:
+// a unit is two such tiles (bits x on the lower qubits of the pairs outside the
+// tile and y on the upper ones, X < Y and Y, X), or one that maps to itself.
+// Memory-bound: one read and one write of what moves.  4.8 to 4.9 TB/s from N=27
+// for 4 to 14 qubit pairs in both types, wherever they lie (a block in the middle,
+// complex128 N=28 qubits 3..8 and 12..17: 1.75 ms; with one thread per pair of
+// amplitudes 4.7 ms).
 
 // Pair index p -> (X <= Y) with p = Y(Y+1)/2 + X.
 __device__ __forceinline__ void pair_of(uint64_t p, uint64_t &X, uint64_t &Y)
@@ -864,11 +832,21 @@ __device__ __forceinline__ void pair_of(uint64_t p, uint64_t &X, uint64_t &Y)
     X = p - y * (y + 1) / 2;
 }
 
-// Unit u of the pipelined transpose: the two tile origins and whether the
-// pair is on the diagonal (one tile, transposed in place).
-__device__ __forceinline__ void swap_unit(const SwapArgs &a, uint64_t u, uint64_t &pa, uint64_t &pb, bool &diag)
+__device__ __forceinline__ uint64_t deposit(uint64_t x, const SwapRuns &r)
 {
-    uint64_t p, r;
+    uint64_t o = 0;
+#pragma unroll 1
+    for (int k = 0; k < r.n; ++k) {
+        const uint32_t d = r.run[k];
+        o |= ((x >> (d & 0xff)) & ((1ull << ((d >> 8) & 0xff)) - 1ull)) << (d >> 16);
+    }
+    return o;
+}
+
+// Unit u: its two tiles (the same one twice on the diagonal).
+__device__ __forceinline__ void swap_unit(const SwapArgs &a, uint64_t u, uint64_t &pa, uint64_t &pb)
+{
+    uint64_t p, r, X, Y;
     if (a.rest_fast) {
         r = u & ((1ull << a.nr) - 1ull);
         p = u >> a.nr;
@@ -876,142 +854,96 @@ __device__ __forceinline__ void swap_unit(const SwapArgs &a, uint64_t u, uint64_
         p = u % a.npairs;
         r = u / a.npairs;
     }
-    uint64_t X, Y;
     pair_of(p, X, Y);
-    const uint64_t base = deposit_rest(r, a);
-    pa = base + ((Y << a.t) << a.in) + (X << a.t);
-    pb = base + ((X << a.t) << a.in) + (Y << a.t);
-    diag = X == Y;
+    const uint64_t base = deposit(r, a.rest);
+    pa = base | deposit(X, a.lower) | deposit(Y, a.upper);
+    pb = base | deposit(Y, a.lower) | deposit(X, a.upper);
 }
 
-// out == 0, persistent and pipelined.  A unit is a pair of tiles (X <= Y)
-// of 2^t x 2^m x 2^t amplitudes for one rest index: tile A has block-0 index
-// X*2^t + xc, rest bits [k, k+m) = rl and block-s index Y*2^t + yc; tile B
-// the same with X and Y exchanged.  Each side is read as 2^t runs of 2^(t+m)
-// contiguous amplitudes (m > 0 only when the whole block is in the tile,
-// t == k), exchanged through LDS (row stride 2^(m+t) + 1: conflict-free for
-// the transposed read) and written back to the other tile.  The next unit's
-// loads are issued before the current unit's LDS exchange.  256 threads,
-// E amplitudes per thread per tile.
-template <typename T> struct NativeVec;
-template <> struct NativeVec<double2> { typedef double type __attribute__((ext_vector_type(2))); };
-template <> struct NativeVec<float2> { typedef float type __attribute__((ext_vector_type(2))); };
-
+// Tiles of 2^TB amplitudes (TB = 8: or of fewer).  Persistent; the next unit's
+// loads are issued once the current one is in LDS, and the unit after that is
+// found behind them.
 // (register arrays of the clang vector type stay in VGPRs across the loop;
 // arrays of HIP_vector_type<double, 2> went to scratch here)
-template <typename T0, int E>
-__global__ void __launch_bounds__(256) k_swap_pipe(T0 *__restrict__ sv0, const SwapArgs a, uint64_t nunits)
+template <typename T0, int TB>
+__global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const SwapArgs a, uint64_t nunits)
 {
     typedef typename NativeVec<T0>::type T;
+    constexpr int E = 1 << (TB - 8), PAD = (TB + 1) / 2;
     T *__restrict__ sv = reinterpret_cast<T *>(sv0);
     extern __shared__ __align__(16) unsigned char fq_smem[];
-    const int t = a.t, m = a.m, s = a.in, k = a.k;
-    const int side = 1 << t;
-    const int R = (side << m) + 1;
-    T *la = reinterpret_cast<T *>(fq_smem);
-    T *lb = la + (size_t)side * R;
     const int tid = threadIdx.x;
-
-    // per-thread element coordinates (xc fastest, then rl, then yc)
-    uint64_t off_g[E];
-    int off_l[E], off_t[E];
+    const bool mine = TB > 8 || tid < 1 << a.tb;
+    // slot of element i: i + (i >> PAD)
+    T *la = reinterpret_cast<T *>(fq_smem);
+    T *lb = la + (1 << TB) + (1 << (TB - PAD));
+    const int to = tid + (tid >> PAD);
+    // an element's offset and the slot it is read from, by the bits of the
+    // thread and of the register
+    auto place = [&](int i, uint64_t &off, int &from) {
+        int f = 0;
+        off = 0;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int i = tid + e * 256;
-        const int xc = i & (side - 1);
-        const int rl = (i >> t) & ((1 << m) - 1);
-        const int yc = i >> (t + m);
-        off_g[e] = ((uint64_t)yc << s) + ((uint64_t)rl << k) + (uint64_t)xc;
-        off_l[e] = yc * R + rl * side + xc;  // natural slot
-        off_t[e] = xc * R + rl * side + yc;  // transposed slot
-    }
-
-
-    uint64_t u = blockIdx.x;
+        for (int k = 0; k < TB; ++k) {
+            const int on = (i >> k) & 1;
+            off |= (uint64_t)on << a.tpos[k];
+            f |= on << a.partner[k];
+        }
+        from = f + (f >> PAD);
+    };
+    uint64_t off_t, off_r[E];
+    int from_t, from_r[E];
+    place(tid, off_t, from_t);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        place(256 * e, off_r[e], from_r[e]);
     T va[E], vb[E];
-    uint64_t pa = 0, pb = 0;
-    bool diag = true;
-    if (u < nunits) {
-        swap_unit(a, u, pa, pb, diag);
+    auto load = [&](T (&x)[E], uint64_t base) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            va[e] = sv[pa + off_g[e]];
-        if (!diag) {
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                vb[e] = sv[pb + off_g[e]];
-        }
-    }
-    while (u < nunits) {
-        const uint64_t next = u + gridDim.x;
-        uint64_t na = 0, nb = 0;
-        bool ndiag = true;
-        T wa[E], wb[E];
-        if (next < nunits) {
-            swap_unit(a, next, na, nb, ndiag);
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                wa[e] = sv[na + off_g[e]];
-            if (!ndiag) {
-#pragma unroll
-                for (int e = 0; e < E; ++e)
-                    wb[e] = sv[nb + off_g[e]];
-            }
-        }
+            if (mine)
+                x[e] = sv[base + off_r[e] + off_t];
+    };
+    auto put = [&](const T (&x)[E], T *l) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            la[off_l[e]] = va[e];
-        if (!diag) {
+            if (mine)
+                l[to + 256 * e + ((256 * e) >> PAD)] = x[e];
+    };
+    auto store = [&](uint64_t base, const T *l) {
 #pragma unroll
-            for (int e = 0; e < E; ++e)
-                lb[off_l[e]] = vb[e];
-        }
+        for (int e = 0; e < E; ++e)
+            if (mine)
+                sv[base + off_r[e] + off_t] = l[from_t + from_r[e]];
+    };
+    const uint64_t G = gridDim.x;
+    uint64_t pa = 0, pb = 0, na = 0, nb = 0;
+    swap_unit(a, blockIdx.x, pa, pb);   // (the grid is not larger than nunits)
+    load(va, pa);
+    if (pa != pb)
+        load(vb, pb);
+    if (blockIdx.x + G < nunits)
+        swap_unit(a, blockIdx.x + G, na, nb);
+    for (uint64_t u = blockIdx.x; u < nunits; u += G) {
+        const uint64_t ca = na, cb = nb;
+        const bool more = u + G < nunits;
+        put(va, la);
+        if (more)
+            load(va, ca);
+        if (pa != pb)
+            put(vb, lb);
+        if (more && ca != cb)
+            load(vb, cb);
+        if (u + 2 * G < nunits)
+            swap_unit(a, u + 2 * G, na, nb);
         lds_barrier();
-        if (diag) {
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                sv[pa + off_g[e]] = la[off_t[e]];
-        } else {
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                sv[pa + off_g[e]] = lb[off_t[e]];
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                sv[pb + off_g[e]] = la[off_t[e]];
-        }
-        lds_barrier();  // the LDS reads finish before the next unit's writes
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            va[e] = wa[e];
-            vb[e] = wb[e];
-        }
-        u = next;
-        pa = na;
-        pb = nb;
-        diag = ndiag;
+        store(pa, pa != pb ? lb : la);
+        if (pa != pb)
+            store(pb, la);
+        lds_barrier();   // the LDS reads finish before the next unit's writes
+        pa = ca;
+        pb = cb;
     }
-}
-
-// Any out: one thread per (rest, x, y); the x < y threads swap their pair.
-template <typename T>
-__global__ void __launch_bounds__(256) k_swap_generic(T *__restrict__ sv, const SwapArgs a,
-                                                      uint64_t total)
-{
-    const uint64_t lin = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (lin >= total)
-        return;
-    const uint64_t km = (1ull << a.k) - 1;
-    const uint64_t y = lin & km;
-    const uint64_t x = (lin >> a.k) & km;
-    if (x >= y)
-        return;
-    const uint64_t r = lin >> (2 * a.k);
-    const uint64_t base = deposit_rest(r, a);
-    const uint64_t i0 = base + (x << a.in) + (y << a.out);
-    const uint64_t i1 = base + (y << a.in) + (x << a.out);
-    const T tmp = sv[i0];
-    sv[i0] = sv[i1];
-    sv[i1] = tmp;
 }
 
 // ---- top-k -----------------------------------------------------------------
@@ -1517,49 +1449,34 @@ hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, do
     return hipGetLastError();
 }
 
-template <typename T, int E>
-static hipError_t launch_swap_pipe(void *sv, const SwapArgs &a, hipStream_t stream)
+template <typename T, int TB> static hipError_t launch_swap_k(void *sv, const SwapArgs &a, hipStream_t stream)
 {
-    const int side = 1 << a.t;
-    const size_t lds = 2 * (size_t)side * (((size_t)side << a.m) + 1) * sizeof(T);
-    const void *fn = reinterpret_cast<const void *>(&k_swap_pipe<T, E>);
+    constexpr size_t lds = 2 * ((size_t)(1 << TB) + (1 << (TB - (TB + 1) / 2))) * sizeof(T);
+    const void *fn = reinterpret_cast<const void *>(&k_exchange<T, TB>);
     if (lds > 65536) {
         if (hipError_t e = allow_large_lds(fn))
             return e;
     }
-    const uint64_t nunits = a.npairs << a.nr;
-    const int per_cu = occupancy_per_cu(fn, 256, lds);
-    const uint64_t resident = (uint64_t)per_cu * device_cus();
-    const uint64_t grid = nunits < resident ? nunits : resident;
-    hipLaunchKernelGGL((k_swap_pipe<T, E>), dim3((unsigned)grid), dim3(256), lds, stream,
+    const uint64_t nunits = a.npairs << a.nr, resident = (uint64_t)occupancy_per_cu(fn, 256, lds) * device_cus();
+    hipLaunchKernelGGL((k_exchange<T, TB>), dim3((unsigned)std::min(nunits, resident)), dim3(256), lds, stream,
                        reinterpret_cast<T *>(sv), a, nunits);
     return hipGetLastError();
 }
 
-template <typename T>
-static hipError_t launch_swap_t(void *sv, const SwapArgs &a, hipStream_t stream)
+template <typename T> static hipError_t launch_swap_t(void *sv, const SwapArgs &a, hipStream_t stream)
 {
-    if (a.pipe) {
-        // tiles of 2^10 complex128 / 2^12 complex64 amplitudes
-        constexpr int E = sizeof(T) == 16 ? 4 : 16;
-        if ((1 << (2 * a.t + a.m)) != 256 * E)
-            return hipErrorInvalidValue;
-        return launch_swap_pipe<T, E>(sv, a, stream);
+    switch (std::max(8, a.tb)) {
+        case 8: return launch_swap_k<T, 8>(sv, a, stream);
+        case 9: return launch_swap_k<T, 9>(sv, a, stream);
+        case 10: return launch_swap_k<T, 10>(sv, a, stream);
     }
-    if (a.t >= 0) {
-        const uint64_t nrest = 1ull << a.nr;
-        const uint64_t blocks = a.npairs * nrest;
-        const int side = 1 << a.t;
-        const size_t lds = 2 * (size_t)side * (side + 1) * sizeof(T);
-        hipLaunchKernelGGL(k_swap_tiled<T>, dim3((unsigned)blocks), dim3(256), lds, stream,
-                           reinterpret_cast<T *>(sv), a);
-    } else {
-        const uint64_t total = 1ull << (a.nr + 2 * a.k);
-        const uint64_t blocks = (total + 255) / 256;
-        hipLaunchKernelGGL(k_swap_generic<T>, dim3((unsigned)blocks), dim3(256), 0, stream,
-                           reinterpret_cast<T *>(sv), a, total);
+    if constexpr (sizeof(T) == 8) {
+        switch (a.tb) {
+            case 11: return launch_swap_k<T, 11>(sv, a, stream);
+            case 12: return launch_swap_k<T, 12>(sv, a, stream);
+        }
     }
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t stream)

@@ -47,7 +47,9 @@ extern "C" {
 #define FQ_C64 1  /* complex64 amplitudes; cut values, phases, reductions in FP64 */
 
 /* layer schedules for fq_run */
-#define FQ_SCHED_REFERENCE 0 /* exactly src/Weighted.cpp:115-137: cost, R x RX chunk, R-1 x transposition */
+#define FQ_SCHED_REFERENCE 0 /* src/Weighted.cpp:115-137: cost, R x RX chunk, R-1 x transposition; the state, its
+                                layout and g end as these leave them.  Run step by step while timing is on
+                                (fq_timing_enable), otherwise as fused layers and the transpositions' product */
 #define FQ_SCHED_FUSED 1     /* cost fused into the first tile pass; high qubits by strided tiles, no transposition */
 #define FQ_SCHED_Z2 2        /* FQ_SCHED_FUSED on the half state z_{N-1} = 0 (psi(b) = psi(~b) for Max-Cut
                                 QAOA from |+>); RX on the top qubit pairs complementary tiles; the full
@@ -126,11 +128,11 @@ int fq_multi_rx(fq_state *st, const int *targets, int gate_size, double beta);
 int fq_swap_conti(fq_state *st, int swap_out, int swap_in, int num_swap);
 
 /* The driver loop (src/Weighted.cpp:97-137) for P layers with per-layer
- * angles gammas[p], betas[p].  FQ_SCHED_REFERENCE also relabels g after each
- * transposition exactly as the driver does (g ends in the state's physical
+ * angles gammas[p], betas[p].  FQ_SCHED_REFERENCE also relabels g for each
+ * transposition as the driver does (g ends in the state's physical
  * labels); FQ_SCHED_FUSED and FQ_SCHED_Z2 leave the layout and g unchanged.
- * With two or more passes per layer (three for FQ_SCHED_Z2) the fused
- * schedules pipeline the layers: the pass that ends layer p also applies the
+ * With two or more passes per layer (three for FQ_SCHED_Z2 from N = 24) the
+ * fused schedules pipeline the layers: the pass that ends layer p also applies the
  * cost phase and RX of layer p+1 on its qubits, so every layer after the
  * first runs one pass fewer (environment FQ_LAYER_PIPE=0 turns it off). */
 int fq_run(fq_state *st, fq_graph *g, int P, const double *gammas, const double *betas,
