@@ -3130,10 +3130,19 @@ struct SlotHost {
     int phase = 0;  // 0 free, 1 active, 2 finished (result pending collection)
     std::vector<double> gammas, betas;
     double amp_scale = 1.0;   // rx_norm_scale of the request
-    PlanDev plan{}, eplan{};  // cost and <C> plans of g, fetched at assignment
+    SlotPlans plans{};        // cost and <C> plans of g, fetched at assignment
+    bool fresh = false;       // not yet in device memory
     uint64_t gversion = 0;    // g->version the plans belong to
     uint64_t gepoch = 0;      // g->plan_epoch the plan pointers belong to
-    int has_rr = 0;
+    int has_rr[4] = {0, 0, 0, 0};
+};
+
+// One pass of a packed slab on the compile-time kernel (fq_mix.hip): its
+// launch arguments without the slots' factors.
+struct PackedPass {
+    MixArgs a;
+    int K = 0;
+    bool lane = false, mir = false;
 };
 
 // Launch arguments of one slab tile pass (fixed for the slab's lifetime).
@@ -3159,11 +3168,14 @@ struct fq_slab {
     void *sv = nullptr;
     hipStream_t stream = nullptr;
     std::vector<SlotHost> slots;
-    SlotParams *d_params = nullptr, *h_params = nullptr;
+    // a step's parameters, uploaded together: SlotParams [K], MixSlot [2 K],
+    // SlabJob [2 K], finishing slots [K]
+    char *d_step = nullptr, *h_step = nullptr;
+    SlotPlans *d_plans = nullptr, *h_plans = nullptr;
     double2 *d_tabs = nullptr;
     size_t tab_stride = 0;
     double *d_part = nullptr;
-    double *d_res = nullptr, *h_res = nullptr;
+    double *h_res = nullptr;   // results (pinned host memory that the kernels write)
     hipEvent_t done = nullptr;
     bool pending = false;  // a step was enqueued and not yet observed complete
     double init_amp = 0;
@@ -3174,6 +3186,14 @@ struct fq_slab {
     std::vector<SlabPass> pass_args;
     TileArgs exp_args{};       // <C> over the virtual state
     int exp_alog = 1, exp_shift = 0;
+    // packed: every step runs one pass of a two-pass plan on each slot, in one
+    // launch for all slots that do the same (fq_slab_step)
+    bool packed = false;
+    std::vector<PackedPass> pk;
+    Geom pk_geom[4];          // cost geometries, 2 * (boundary pass) + pass
+    SlabGeos pk_tab{};
+    size_t pk_entries = 0;    // of the largest table
+    int pk_end = 0;           // pass that ends the next step's layer
     // large slots: each slot runs the single-state tile passes of fq_run
     // (pipelined layers) over its own 2^N (or 2^(N-1)) amplitudes instead of
     // one packed launch; views[k] is slot k seen as a state (its amplitudes,
@@ -3183,6 +3203,12 @@ struct fq_slab {
     std::vector<fq_state *> views;
     int layers_per_step = 1;   // per_slot slabs: layers a step runs per slot
 };
+
+// Offsets of the arrays of a step's parameters.
+static size_t step_mix(int K) { return sizeof(SlotParams) * (size_t)K; }
+static size_t step_jobs(int K) { return step_mix(K) + sizeof(MixSlot) * 2 * (size_t)K; }
+static size_t step_fin(int K) { return step_jobs(K) + sizeof(SlabJob) * 2 * (size_t)K; }
+static size_t step_bytes(int K) { return step_fin(K) + sizeof(int) * (size_t)K; }
 
 static void slab_free(fq_slab *sb)
 {
@@ -3196,11 +3222,12 @@ static void slab_free(fq_slab *sb)
     if (sb->sv)
         budget_give(sb->bytes);
     hipFree(sb->sv);
-    hipFree(sb->d_params);
-    hipHostFree(sb->h_params);
+    hipFree(sb->d_step);
+    hipHostFree(sb->h_step);
+    hipFree(sb->d_plans);
+    hipHostFree(sb->h_plans);
     hipFree(sb->d_tabs);
     hipFree(sb->d_part);
-    hipFree(sb->d_res);
     hipHostFree(sb->h_res);
     if (sb->done)
         hipEventDestroy(sb->done);
@@ -3227,6 +3254,40 @@ static TileArgs slab_cost_args(const fq_slab *sb, Geom *gout)
     if (gout)
         *gout = g1;
     return a1;
+}
+
+// Passes and table geometries of a packed slab (two-pass plan lp).
+static int slab_build_packed(fq_slab *sb, const LayerPlan &lp)
+{
+    const int N = sb->N;
+    for (int i = 0; i < 2; ++i) {
+        const FusedPass &fp = lp.ps[i];
+        const int A = mix_a_log(sb->dtype, (int)fp.tile.size());
+        PackedPass p;
+        p.mir = sb->z2 && i == 1;
+        if (int rc = pass_shape(N, fp.tile, fp.gates, A, mix_lane_bit,
+                                !sb->z2 ? Z2_OFF : p.mir ? Z2_MIRROR : Z2_LOWER, p.a, p.K, p.lane))
+            return rc;
+        p.a.init_amp = sb->init_amp;
+        sb->pk.push_back(p);
+        for (int bd = 0; bd < 2; ++bd) {
+            const Geom g = layout_geom(N, fp.tile, A, bd ? p.K : 0);
+            sb->pk_geom[2 * bd + i] = g;
+            TileArgs ta;
+            geom_to_args(g, ta);
+            ta.ntiles_run = p.a.ntiles;
+            TableGeo &tg = sb->pk_tab.geo[2 * bd + i];
+            tg.Q = ta.Q;
+            tg.nthr = ta.nthr;
+            tg.nh = ta.nh;
+            tg.a_log = A;
+            tg.ntiles = p.a.ntiles;
+            sb->pk_entries = std::max(sb->pk_entries, phase_table_entries(ta, A));
+        }
+    }
+    sb->slot_plan = lp;
+    sb->tab_stride = 2 * sb->pk_entries;   // a slot's first layer has two tables
+    return FQ_OK;
 }
 
 // Tile-pass and <C> launch arguments of a slab (its virtual state: the Ns
@@ -3268,37 +3329,49 @@ static int slab_build_args(fq_slab *sb)
     sb->exp_geom = make_geom(N, low_tile(Qe), sb->exp_alog);
     geom_to_args(make_geom(Ns + sb->s, low_tile(Qe), sb->exp_alog), sb->exp_args);
     sb->exp_shift = Ns - Qe;
-    // at least 1024 tiles per slot in the first pass: the persistent
-    // single-state tile kernel per slot (register prefetch, compile-time tile
-    // widths) fills the device on its own
+    const LayerPlan lp = exec_plan(N, sb->dtype, sb->z2, 1);
+    sb->packed = lp.split && lp.ps.size() == 2 && (int)lp.ps[0].tile.size() < tile_max_q(sb->dtype);
+    if (sb->packed)
+        return slab_build_packed(sb, lp);
+    // passes that fill the device on one slot: one slot after the other (three
+    // passes, or tiles of full width, which take no packed launches)
     const int Q1 = (int)sb->passes[0].tile.size();
-    sb->per_slot = Ns - Q1 >= 10;
-    if (sb->per_slot)
-        sb->slot_plan = layer_plan(N, sb->dtype, sb->z2);
+    sb->per_slot = lp.split || Ns - Q1 >= 10;   // (or 1,024 tiles)
+    if (sb->per_slot) {
+        sb->slot_plan = lp;
+        sb->slot_plan.chunk = 0;   // a step is one layer, launched pass by pass
+    }
     return FQ_OK;
 }
 
-// Per-slot state views of a per-slot slab (after its amplitudes and stream
-// exist), each with a phase-table buffer for the largest cost pass of the
-// layer plan, so no step allocates.
+// Per-slot state views of a slab (after its amplitudes and stream exist); of a
+// per-slot slab each with a phase-table buffer, so no step allocates.
 static int slab_make_views(fq_slab *sb)
 {
     const LayerPlan &lp = sb->slot_plan;
     const int m = (int)lp.ps.size();
-    size_t need = 0;
-    for (int i = 0; i < m; ++i) {
+    size_t need = 0;   // the tables of the first layer's two cost passes
+    for (int i = 0; i < m && sb->per_slot; ++i) {
         if (i != 0 && i != lp.end1)
             continue;
-        // pass 0 runs as the write-only layer-0 pass too, possibly with
-        // another register width (tile_a_log)
-        for (int first = 0; first <= (i == 0 ? 1 : 0); ++first) {
-            TileArgs a;
+        TileArgs a;
+        size_t most = 0;
+        if (const int A = mix_a_log(sb->dtype, (int)lp.ps[i].tile.size())) {
+            geom_to_args(layout_geom(sb->N, lp.ps[i].tile, A, 0), a);
+            a.ntiles_run = sb->z2 ? 1ull << (a.nh - 1) : 0;
+            most = phase_table_entries(a, A);
+        } else {
             Geom geom;
             const int z2 = !sb->z2 ? Z2_OFF : i + 1 < m ? Z2_LOWER : Z2_MIRROR;
-            if (int rc = pass_args(sb->N, sb->dtype, lp.ps[i].tile, lp.ps[i].gates, true, z2, a, geom, 0, first != 0))
-                return rc;
-            need = std::max(need, phase_table_entries(a, geom.a_log) * sizeof(double2));
+            // pass 0 runs as the write-only layer-0 pass too, possibly with
+            // another register width (tile_a_log)
+            for (int first = 0; first <= (i == 0 ? 1 : 0); ++first) {
+                if (int rc = pass_args(sb->N, sb->dtype, lp.ps[i].tile, lp.ps[i].gates, true, z2, a, geom, 0, first != 0))
+                    return rc;
+                most = std::max(most, phase_table_entries(a, geom.a_log));
+            }
         }
+        need += most * sizeof(double2);
     }
     for (int k = 0; k < sb->K; ++k) {
         fq_state *v = new fq_state();
@@ -3311,8 +3384,9 @@ static int slab_make_views(fq_slab *sb)
         for (int q = 0; q < FQ_MAXN; ++q)
             v->qmap[q] = q;
         v->init_amp = sb->init_amp;
+        v->in_run = true;   // a slot runs fq_run's layers on a QAOA state
         sb->views.push_back(v);
-        if (hipMalloc(&v->d_phase, need) != hipSuccess) {
+        if (need && hipMalloc(&v->d_phase, need) != hipSuccess) {
             hipGetLastError();
             v->d_phase = nullptr;
             return set_err(FQ_ERR_OOM, "slab phase-table allocation failed");
@@ -3325,14 +3399,17 @@ static int slab_make_views(fq_slab *sb)
 // Cost and <C> plans of a slot's graph (again after the graph changed).
 static int slab_slot_plans(fq_slab *sb, SlotHost &h)
 {
-    if (int rc = get_plan(h.g, sb->cost_geom, &h.plan, sb->stream))
+    for (int i = 0; i < (sb->packed ? 4 : 1); ++i) {
+        if (int rc = get_plan(h.g, sb->packed ? sb->pk_geom[i] : sb->cost_geom, &h.plans.cost[i], sb->stream))
+            return rc;
+        h.has_rr[i] = 0;
+        for (int j = 0; j < FQ_MAX_REGS; ++j)
+            if (h.plans.cost[i].rr[j] != 0)
+                h.has_rr[i] = 1;
+    }
+    if (int rc = get_plan(h.g, sb->exp_geom, &h.plans.expect, sb->stream))
         return rc;
-    if (int rc = get_plan(h.g, sb->exp_geom, &h.eplan, sb->stream))
-        return rc;
-    h.has_rr = 0;
-    for (int j = 0; j < FQ_MAX_REGS; ++j)
-        if (h.plan.rr[j] != 0)
-            h.has_rr = 1;
+    h.fresh = true;
     h.gversion = h.g->version;
     h.gepoch = h.g->plan_epoch;
     return FQ_OK;
@@ -3401,11 +3478,12 @@ extern "C" int fq_slab_create_sched(int N, int nslots, int dtype, int schedule, 
         slab_free(sb);
         return set_err(FQ_ERR_OOM, "slab allocation of %zu bytes failed", (size_t)(((size_t)1 << N) * (dtype == FQ_C128 ? 16 : 8) * nslots));
     }
-    ok = hipMalloc(&sb->d_params, sizeof(SlotParams) * nslots) == hipSuccess &&
-         hipHostMalloc(&sb->h_params, sizeof(SlotParams) * nslots, hipHostMallocDefault) == hipSuccess &&
+    ok = hipMalloc(&sb->d_step, step_bytes(nslots)) == hipSuccess &&
+         hipHostMalloc(&sb->h_step, step_bytes(nslots), hipHostMallocDefault) == hipSuccess &&
+         hipMalloc(&sb->d_plans, sizeof(SlotPlans) * nslots) == hipSuccess &&
+         hipHostMalloc(&sb->h_plans, sizeof(SlotPlans) * nslots, hipHostMallocDefault) == hipSuccess &&
          hipMalloc(&sb->d_tabs, sizeof(double2) * sb->tab_stride * nslots) == hipSuccess &&
          hipMalloc(&sb->d_part, sizeof(double) * 2 * etiles) == hipSuccess &&
-         hipMalloc(&sb->d_res, sizeof(double) * 2 * nslots) == hipSuccess &&
          hipHostMalloc(&sb->h_res, sizeof(double) * 2 * nslots, hipHostMallocDefault) == hipSuccess &&
          hipStreamCreateWithFlags(&sb->stream, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&sb->done, hipEventDisableTiming) == hipSuccess;
@@ -3416,12 +3494,12 @@ extern "C" int fq_slab_create_sched(int N, int nslots, int dtype, int schedule, 
     }
     own_stream(sb->stream, true);
     sb->layers_per_step = slab_layers_default();
-    if (sb->per_slot)
+    if (sb->per_slot || sb->packed)
         if (int rc = slab_make_views(sb)) {
             slab_free(sb);
             return rc;
         }
-    memset(sb->h_params, 0, sizeof(SlotParams) * nslots);
+    memset(sb->h_step, 0, step_bytes(nslots));
     *out = sb;
     return FQ_OK;
 }
@@ -3504,6 +3582,82 @@ extern "C" int fq_slab_poll(fq_slab *sb, int *busy)
     return FQ_OK;
 }
 
+// One layer of every active slot of a packed slab.  The slots go in step: a step
+// ends their layers on one of the two passes (pk_end, alternately) with a
+// boundary pass, which opens the next layer there, or with a plain one where the
+// request is done; a slot that enters first writes its state in the other pass.
+// Each of the three is one launch over its slots, and one launch makes all
+// phase tables.  48 requests of N=16..26, complex64 half states, on MI355X: 13.3
+// -> 10.7 ms (5.2 where fewer of them are of N=26), the device's time 14 -> 7.2 ms
+// for the latter: the general kernel ran two full-width passes per layer, one
+// work-group per CU.
+static int slab_step_packed(fq_slab *sb)
+{
+    const int K = sb->K, e = sb->pk_end;
+    MixSlot *h = (MixSlot *)(sb->h_step + step_mix(K));
+    SlabJob *jobs = (SlabJob *)(sb->h_step + step_jobs(K));
+    const MixSlot *d = (const MixSlot *)(sb->d_step + step_mix(K));
+    int n = 0, nj = 0, at[4] = {0, 0, 0, 0};
+    MixArgs args[3];
+    enum { FIRST = 0, BOUNDARY = 1, PLAIN = 2 };
+    for (int kind = FIRST; kind <= PLAIN; ++kind) {
+        const int pass = kind == FIRST ? 1 - e : e;
+        const PackedPass &pp = sb->pk[pass];
+        args[kind] = pp.a;
+        for (int k = 0; k < K; ++k) {
+            SlotHost &s = sb->slots[k];
+            if (s.phase != 1)
+                continue;
+            const int L = s.layer;
+            const bool last = L + 1 == s.P;
+            if (kind == FIRST ? L != 0 : last != (kind == PLAIN))
+                continue;
+            fq_state *v = sb->views[k];
+            if (kind == FIRST) {
+                v->pending_re = 1.0;
+                v->pending_im = 0.0;
+            }
+            const int open = kind == BOUNDARY ? L + 1 : L;
+            const PassFactor f = pass_factor(v, sb->slot_plan.ps[pass].gates.size(), s.betas[open],
+                                             kind == BOUNDARY ? &s.betas[L] : nullptr, kind != PLAIN, false);
+            MixSlot &m = h[n++];
+            m.t = f.t;
+            m.pre_t = f.pre_t;
+            m.tf = (float)f.t;
+            m.pre_tf = (float)f.pre_t;
+            m.scale_re = f.re;
+            m.scale_im = f.im;
+            m.base = (sb->slot_bytes / sb->elem) * (uint64_t)k;
+            m.table = 0;
+            m.has_rr = 0;
+            args[kind].apply_scale = f.apply;
+            if (kind != PLAIN) {
+                const int geo = 2 * (kind == BOUNDARY) + pass;
+                m.table = (uint32_t)(sb->tab_stride * k + sb->pk_entries * (kind == BOUNDARY));
+                m.has_rr = s.has_rr[geo];
+                jobs[nj++] = {s.gammas[open], (uint32_t)k, (uint32_t)geo, m.table, 0};
+            }
+        }
+        at[kind + 1] = n;
+    }
+    FQ_HIP(hipMemcpyAsync(sb->d_step, sb->h_step, step_bytes(K), hipMemcpyHostToDevice, sb->stream));
+    if (nj > 0)
+        FQ_HIP(launch_slab_tables(sb->pk_tab, (const SlabJob *)(sb->d_step + step_jobs(K)), nj, sb->pk_entries, sb->d_plans,
+                                  sb->d_tabs, sb->stream));
+    for (int kind = FIRST; kind <= PLAIN; ++kind) {
+        const int ns = at[kind + 1] - at[kind];
+        if (ns == 0)
+            continue;
+        const PackedPass &pp = sb->pk[kind == FIRST ? 1 - e : e];
+        args[kind].slots = d + at[kind];
+        args[kind].nslots = ns;
+        FQ_HIP(launch_mix(sb->dtype, pp.K, pp.lane, kind == FIRST ? MIX_FIRST : kind == BOUNDARY ? MIX_BOUNDARY : MIX_PLAIN,
+                          pp.mir ? 1 : 0, sb->sv, args[kind], sb->d_tabs, sb->stream));
+    }
+    sb->pk_end = 1 - e;
+    return FQ_OK;
+}
+
 // Advance every active slot by one layer: one packed launch per tile pass.
 // Slots that complete their last layer also get <C> reduced; their results
 // are read with fq_slab_collect once fq_slab_poll reports the step done.
@@ -3531,73 +3685,79 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
     }
     // layers of this step per slot (per_slot slabs may run several)
     std::vector<int> nl(K, 0);
+    SlotParams *params = (SlotParams *)sb->h_step;
+    int *fin = (int *)(sb->h_step + step_fin(K));
     int nact = 0, nfin = 0;
     for (int k = 0; k < K; ++k) {
         SlotHost &h = sb->slots[k];
-        SlotParams &sp = sb->h_params[k];
+        SlotParams &sp = params[k];
         memset(&sp, 0, sizeof(sp));
         if (h.phase != 1)
             continue;
+        if (h.fresh) {
+            sb->h_plans[k] = h.plans;
+            FQ_HIP(hipMemcpyAsync(sb->d_plans + k, sb->h_plans + k, sizeof(SlotPlans), hipMemcpyHostToDevice, sb->stream));
+            h.fresh = false;
+        }
         nl[k] = sb->per_slot ? std::min(sb->layers_per_step, h.P - h.layer) : 1;
         const int L = h.layer;
         rx_coeffs(h.betas[L], sb->dtype, &sp.rx_c, &sp.rx_s);
         sp.gamma = h.gammas[L];
-        // the packed kernels apply RX with rx_coeffs (norm factor amp_scale);
-        // per-slot slots run fq_run's passes, whose RX factors are exact
-        sp.init_amp = sb->init_amp * (sb->per_slot ? 1.0 : h.amp_scale);
+        // the general kernel applies RX with rx_coeffs (norm factor amp_scale);
+        // the others run fq_run's passes, whose RX factors are exact
+        sp.init_amp = sb->init_amp * (sb->per_slot || sb->packed ? 1.0 : h.amp_scale);
         sp.active = 1;
         sp.cost_first = L == 0;
-        sp.want_expect = L + nl[k] == h.P;
         sp.ptab = sb->d_tabs + sb->tab_stride * (size_t)k;
-        sp.plan = h.plan;
-        sp.eplan = h.eplan;
-        sp.has_rr = h.has_rr;
+        sp.has_rr = h.has_rr[0];
         ++nact;
-        nfin += sp.want_expect;
+        if (L + nl[k] == h.P)
+            fin[nfin++] = k;
     }
     if (nfinishing)
         *nfinishing = nfin;
     if (nact == 0)
         return FQ_OK;
-    FQ_HIP(hipMemcpyAsync(sb->d_params, sb->h_params, sizeof(SlotParams) * K, hipMemcpyHostToDevice,
-                          sb->stream));
+    if (sb->packed) {
+        if (int rc = slab_step_packed(sb))
+            return rc;
+    } else {
+        FQ_HIP(hipMemcpyAsync(sb->d_step, sb->h_step, step_bytes(K), hipMemcpyHostToDevice, sb->stream));
+    }
     if (sb->per_slot) {
         // each slot nl[k] layers of fq_run's pipelined schedule on its own
         // amplitudes (the slots' layers interleaved on the slab's stream)
         const int most = *std::max_element(nl.begin(), nl.end());
         for (int rep = 0; rep < most; ++rep) {
             for (int k = 0; k < K; ++k) {
-                const SlotParams &sp = sb->h_params[k];
-                if (!sp.active || rep >= nl[k])
+                if (!params[k].active || rep >= nl[k])
                     continue;
                 SlotHost &h = sb->slots[k];
                 fq_state *v = sb->views[k];
                 const int L = h.layer + rep;
-                v->init_amp = sp.init_amp;
                 if (L == 0) {
                     v->pending_re = 1.0;
                     v->pending_im = 0.0;
                 }
-                v->in_run = true;   // a slot runs fq_run's layers on a QAOA state
                 if (int rc = run_layers(v, h.g, sb->slot_plan, L, L + 1, h.P, h.gammas.data(), h.betas.data(), sb->z2,
                                         false))
                     return rc;
             }
         }
-    } else {
-        FQ_HIP(launch_slab_phase_table(sb->cost_args, sb->cost_geom.a_log, sb->d_params, K, sb->d_tabs,
-                                       sb->tab_stride, sb->stream));
+    } else if (!sb->packed) {
+        const SlotParams *d = (const SlotParams *)sb->d_step;
+        FQ_HIP(launch_slab_phase_table(sb->cost_args, sb->cost_geom.a_log, d, sb->d_plans, K, sb->d_tabs, sb->tab_stride,
+                                       sb->stream));
         for (size_t i = 0; i < sb->pass_args.size(); ++i) {
             const SlabPass &sp = sb->pass_args[i];
-            FQ_HIP(launch_slab_pass(sb->dtype, sp.a_log, i == 0, sp.mirror, sb->sv, sp.args, sb->d_params,
-                                    sp.slot_shift, sb->stream));
+            FQ_HIP(launch_slab_pass(sb->dtype, sp.a_log, i == 0, sp.mirror, sb->sv, sp.args, d, sp.slot_shift,
+                                    sb->stream));
         }
     }
-    if (nfin > 0) {
-        FQ_HIP(launch_slab_expect(sb->dtype, sb->exp_alog, sb->sv, sb->exp_args, sb->d_params, sb->exp_shift, K,
-                                  sb->d_part, sb->d_res, sb->stream));
-        FQ_HIP(hipMemcpyAsync(sb->h_res, sb->d_res, sizeof(double) * 2 * K, hipMemcpyDeviceToHost, sb->stream));
-    }
+    if (nfin > 0)
+        FQ_HIP(launch_slab_expect(sb->dtype, sb->exp_alog, sb->sv, sb->exp_args, sb->d_plans,
+                                  (const int *)(sb->d_step + step_fin(K)), nfin, sb->exp_shift, sb->d_part, sb->h_res,
+                                  sb->stream));
     FQ_HIP(hipEventRecord(sb->done, sb->stream));
     sb->pending = true;
     for (int k = 0; k < K; ++k) {
@@ -3653,6 +3813,34 @@ extern "C" int fq_slab_collect(fq_slab *sb, int *slots, double *expect, double *
     return FQ_OK;
 }
 
+// A running slot's amplitudes after the layers it has run, at tmp: its last
+// boundary pass has also opened the next layer, which is undone there.
+static int slab_close_layer(fq_slab *sb, int slot, void *tmp)
+{
+    const SlotHost &h = sb->slots[slot];
+    const LayerPlan &lp = sb->slot_plan;
+    const int L = h.layer, e = sb->packed ? 1 - sb->pk_end : (L - 1) % 2 == 0 ? lp.end1 : 0;
+    fq_state v;
+    v.N = sb->N;
+    v.dtype = sb->dtype;
+    v.elem = sb->elem;
+    v.bytes = sb->slot_bytes;
+    v.sv = tmp;
+    v.stream = sb->stream;
+    v.in_run = true;
+    for (int q = 0; q < FQ_MAXN; ++q)
+        v.qmap[q] = q;
+    v.init_amp = sb->init_amp;
+    const double pre = -h.betas[L];
+    const int mode = !sb->z2 ? Z2_OFF : e + 1 < (int)lp.ps.size() ? Z2_LOWER : Z2_MIRROR;
+    const int rc = tile_pass(&v, lp.ps[e].tile, lp.ps[e].gates, 0.0, h.g, -h.gammas[L], true, false, FQ_K_FUSED, mode,
+                             &pre, false);
+    hipStreamSynchronize(sb->stream);
+    hipFree(v.d_phase);
+    v.sv = nullptr;
+    return rc;
+}
+
 // Amplitudes of one slot (identity layout) to host memory.  Waits.
 extern "C" int fq_slab_copy_out(fq_slab *sb, int slot, void *host, size_t bytes)
 {
@@ -3661,9 +3849,27 @@ extern "C" int fq_slab_copy_out(fq_slab *sb, int slot, void *host, size_t bytes)
     const size_t full = ((size_t)1 << sb->N) * sb->elem;
     if (slot < 0 || slot >= sb->K || bytes != full)
         return set_err(FQ_ERR_ARG, "bad slot or size (%zu bytes expected)", full);
-    FQ_HIP(hipMemcpyAsync(host, (char *)sb->sv + sb->slot_bytes * (size_t)slot, sb->slot_bytes,
-                          hipMemcpyDeviceToHost, sb->stream));
-    FQ_HIP(hipStreamSynchronize(sb->stream));
+    const char *src = (const char *)sb->sv + sb->slot_bytes * (size_t)slot;
+    const SlotHost &h = sb->slots[slot];
+    void *tmp = nullptr;
+    int rc = FQ_OK;
+    if ((sb->packed || sb->per_slot) && sb->slot_plan.end1 >= 0 && h.phase == 1 && h.layer > 0) {
+        if (hipMalloc(&tmp, sb->slot_bytes) != hipSuccess) {
+            hipGetLastError();
+            return set_err(FQ_ERR_OOM, "scratch for a running slot's amplitudes failed");
+        }
+        if (hipMemcpyAsync(tmp, src, sb->slot_bytes, hipMemcpyDeviceToDevice, sb->stream) == hipSuccess)
+            rc = slab_close_layer(sb, slot, tmp);
+        else
+            rc = set_err(FQ_ERR_DEVICE, "copy of a running slot's amplitudes failed");
+    }
+    if (rc == FQ_OK && (hipMemcpyAsync(host, tmp ? (const char *)tmp : src, sb->slot_bytes, hipMemcpyDeviceToHost,
+                                       sb->stream) != hipSuccess ||
+                        hipStreamSynchronize(sb->stream) != hipSuccess))
+        rc = set_err(FQ_ERR_DEVICE, "copy of a slot's amplitudes failed");
+    hipFree(tmp);
+    if (rc)
+        return rc;
     sb->pending = false;
     if (sb->z2) {
         // psi(b) = psi(~b): the upper half is the stored half reversed

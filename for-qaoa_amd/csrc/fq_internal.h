@@ -89,6 +89,16 @@ struct TileArgs {
 enum { MIX_PLAIN = 0, MIX_FIRST = 1, MIX_COST = 2, MIX_BOUNDARY = 3 };
 // The same of a pair pass of the gradient (fq_pair.hip).
 enum { PAIR_PLAIN = 0, PAIR_COST = 1, PAIR_BOUNDARY = 2 };
+// One slot of a packed launch: its first amplitude, its factors (as in MixArgs)
+// and its phase table's first entry.
+struct MixSlot {
+    double t, pre_t;
+    double scale_re, scale_im;
+    float tf, pre_tf;
+    uint64_t base;
+    uint32_t table;
+    int has_rr;
+};
 struct MixArgs {
     int N, Q, nh;
     int has_rr;              // any register-register edge in the plan
@@ -105,6 +115,8 @@ struct MixArgs {
     double scale_re, scale_im;  // factor of the pass: in the cost phase, or before the
     int apply_scale;            // stores (apply_scale)
     double init_amp;
+    const MixSlot *slots;    // packed launch (blockIdx.y: the slot), else null
+    int nslots;
 };
 // One pair pass: t, pre_t and the real scale as above (a boundary pass undoes
 // RX(pre) first), and the weights of its sums: the inverse of the factor that
@@ -142,7 +154,13 @@ struct TableJobs {
     TableJob job[FQ_TABLE_JOBS];
 };
 
-// Per-slot parameters of a packed (slab) step, in device memory.
+// Device plans of a slot's graph: the cost passes' geometries (the general
+// kernel uses the first; the packed passes 2 * (boundary pass) + pass), <C>.
+struct SlotPlans {
+    PlanDev cost[4];
+    PlanDev expect;
+};
+// Per-slot parameters of a step of the general kernel, in device memory.
 struct SlotParams {
     double rx_c, rx_s;       // RX(beta) of the slot's current layer
     double gamma;            // cost angle of the slot's current layer
@@ -150,10 +168,16 @@ struct SlotParams {
     int active;              // the slot runs this step
     int cost_first;          // layer 0: launch-control write, no read
     int has_rr;
-    int want_expect;         // the slot finishes this step: reduce <C>
     const double2 *ptab;     // the slot's phase table for this step
-    PlanDev plan;            // cut plan of the first (contiguous) tile pass
-    PlanDev eplan;           // cut plan of the <C> reduction geometry
+};
+// Phase tables of a packed step: the geometries (plan unused) and, per table,
+// angle, slot, geometry and first entry.
+struct SlabGeos {
+    TableGeo geo[4];
+};
+struct SlabJob {
+    double gamma;
+    uint32_t slot, geo, offset, pad;
 };
 
 #define FQ_SWAP_BITS 12     // qubits of an exchange tile: 2^12 complex64, 2^10 complex128
@@ -250,12 +274,16 @@ hipError_t launch_pair_pass(int dtype, int k, bool lane, int kind, bool mir, voi
 // out[3 s ..] = the sums of pass s's n triples (partials + 3 n s)
 hipError_t launch_pair_sums(const double *partials, uint64_t n, int passes, double *out, hipStream_t stream);
 // packed slabs (fq_serve.hip)
-hipError_t launch_slab_phase_table(const TileArgs &local, int a_log, const SlotParams *slots, int nslots,
-                                   double2 *tabs, size_t stride, hipStream_t stream);
+hipError_t launch_slab_phase_table(const TileArgs &local, int a_log, const SlotParams *slots, const SlotPlans *plans,
+                                   int nslots, double2 *tabs, size_t stride, hipStream_t stream);
+hipError_t launch_slab_tables(const SlabGeos &g, const SlabJob *jobs, int njobs, size_t entries, const SlotPlans *plans,
+                              double2 *tabs, hipStream_t stream);
 hipError_t launch_slab_pass(int dtype, int a_log, bool cost, bool mirror, void *sv, const TileArgs &a,
                             const SlotParams *slots, int slot_shift, hipStream_t stream);
-hipError_t launch_slab_expect(int dtype, int a_log, const void *sv, const TileArgs &a, const SlotParams *slots,
-                              int slot_shift, int nslots, double *partials, double *out, hipStream_t stream);
+// <C> and sum |psi|^2 of the nfin slots fin[] into out[2 slot]
+hipError_t launch_slab_expect(int dtype, int a_log, const void *sv, const TileArgs &a, const SlotPlans *plans,
+                              const int *fin, int nfin, int slot_shift, double *partials, double *out,
+                              hipStream_t stream);
 int tile_max_q(int dtype);
 size_t tile_lds_bytes(int dtype, int Q);
 

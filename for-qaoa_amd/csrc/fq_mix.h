@@ -75,6 +75,9 @@ __device__ __forceinline__ void mix_phase(T (&v)[1 << A], const R (&fx)[A], cons
     }
 }
 
+// Whether the instances of this width take packed launches.
+template <typename R> static constexpr bool mix_packs(int Q) { return Q < (sizeof(R) == 4 ? 14 : 13); }
+
 // One work-group per tile: with two of them on a CU the dispatcher's order keeps
 // loads and butterflies apart better than persistent groups with a range of
 // tiles each (N=30 complex128 13.64 -> 13.37 ms per layer).
@@ -91,7 +94,7 @@ __device__ __forceinline__ void mix_phase(T (&v)[1 << A], const R (&fx)[A], cons
 // by lane operations.
 template <typename R, int Q, int A, int K, int KIND, int MIR, bool LG>
 __global__ void __launch_bounds__(1 << (Q - A), 4)
-    k_mix(typename CT<R>::T *__restrict__ sv, const MixArgs a, const double2 *__restrict__ ptab)
+    k_mix(typename CT<R>::T *__restrict__ sv0, const MixArgs a, const double2 *__restrict__ ptab0)
 {
     typedef typename CT<R>::T T;
     typedef MixLay<R, Q, A, K> Lay;
@@ -121,11 +124,27 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
         for (int l = 0; l <= K; ++l)
             sb[l] += on ? Lay::w(Lay::p(l, k)) : 0;
     }
+    // a packed launch's slot has its own amplitudes, factors and phase table
+    // (not at full width, which large states run at: there this cost 1.5%)
+    typename CT<R>::T *__restrict__ sv = sv0;
+    const double2 *__restrict__ ptab = ptab0;
+    R rt = sizeof(R) == 4 ? (R)a.tf : (R)a.t;
+    R pt = sizeof(R) == 4 ? (R)a.pre_tf : (R)a.pre_t;
+    double scale_re = a.scale_re, scale_im = a.scale_im;
+    int has_rr = a.has_rr;
+    if (mix_packs<R>(Q) && a.slots) {
+        const MixSlot &s = a.slots[blockIdx.y];
+        sv += s.base;
+        ptab += s.table;
+        rt = sizeof(R) == 4 ? (R)s.tf : (R)s.t;
+        pt = sizeof(R) == 4 ? (R)s.pre_tf : (R)s.pre_t;
+        scale_re = s.scale_re;
+        scale_im = s.scale_im;
+        has_rr = s.has_rr;
+    }
     const uint64_t q1 = Q + 1;
     const double2 *thr_tab = COST ? ptab + a.ntab * q1 : nullptr;
     const double2 *rr_tab = COST ? thr_tab + ((size_t)(1 + A) << NT) : nullptr;
-    const R rt = sizeof(R) == 4 ? (R)a.tf : (R)a.t;
-    const R pt = sizeof(R) == 4 ? (R)a.pre_tf : (R)a.pre_t;
 
     const uint64_t tile = a.tile0 + blockIdx.x;
     const uint64_t base = unpack_runs_uniform(tile, a.hruns);
@@ -168,8 +187,8 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
             x = on ? nx : x;
             y = on ? ny : y;
         }
-        mul(KIND == MIX_FIRST ? make_double2(a.init_amp * a.scale_re, a.init_amp * a.scale_im)
-                              : make_double2(a.scale_re, a.scale_im));
+        mul(KIND == MIX_FIRST ? make_double2(a.init_amp * scale_re, a.init_amp * scale_im)
+                              : make_double2(scale_re, scale_im));
         const R x0 = (R)x, y0 = (R)y;
         R fx[A], fy[A];
         __builtin_amdgcn_sched_barrier(0);
@@ -182,7 +201,7 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
         }
         mix_phase<T, R, A, A, KIND == MIX_FIRST>(v, fx, fy, x0, y0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        if (a.has_rr) {
+        if (has_rr) {
 #pragma unroll
             for (int j = 0; j < N; ++j) {
                 const double2 f = rr_tab[j];
@@ -204,7 +223,7 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
     if (!COST && a.apply_scale) {
 #pragma unroll
         for (int j = 0; j < N; ++j)
-            cmul_by(v[j], (R)a.scale_re, (R)a.scale_im);
+            cmul_by(v[j], (R)scale_re, (R)scale_im);
     }
     uint64_t ro[N];
     reg_offsets<N, NB>(LS == 0 ? a.rpos0_w : a.rposk_w, ro);
@@ -244,12 +263,14 @@ static hipError_t launch_mix_t(void *sv, const MixArgs &a, const double2 *ptab, 
     constexpr unsigned threads = 1u << (Q - A);
     constexpr size_t lds = K > 0 ? sizeof(R) * (size_t)MixLay<R, Q, A, K>::slots() : 0;
     const void *fn = reinterpret_cast<const void *>(&k_mix<R, Q, A, K, KIND, MIR, LG>);
+    if (a.slots && !mix_packs<R>(Q))
+        return hipErrorInvalidValue;
     if (lds > 65536) {
         if (hipError_t e = allow_large_lds(fn))
             return e;
     }
-    hipLaunchKernelGGL((k_mix<R, Q, A, K, KIND, MIR, LG>), dim3((unsigned)a.ntiles), dim3(threads), lds, stream,
-                       reinterpret_cast<T *>(sv), a, ptab);
+    hipLaunchKernelGGL((k_mix<R, Q, A, K, KIND, MIR, LG>), dim3((unsigned)a.ntiles, a.slots ? (unsigned)a.nslots : 1u),
+                       dim3(threads), lds, stream, reinterpret_cast<T *>(sv), a, ptab);
     return hipGetLastError();
 }
 

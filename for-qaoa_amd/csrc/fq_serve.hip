@@ -1,12 +1,16 @@
 // fq_serve.hip -- packed execution of many QAOA evaluations of one size N.
 //
 // No reference counterpart (the reference runs one evaluation per process).
-// A slab holds K = 2^s state slots of 2^N amplitudes in one allocation; seen
-// as one virtual state of N + s qubits whose top s bits select the slot, a
-// single persistent tile-pass launch covers every active slot.  Each slot has
-// its own graph, angles and current layer (per-slot parameters in device
-// memory), so requests of different depth P advance together one layer per
-// step and a request can enter a free slot at any layer boundary.
+// A slab holds K = 2^s state slots of 2^N amplitudes in one allocation.  Each
+// slot has its own graph, angles and current layer (per-slot parameters in
+// device memory), so requests of different depth P advance together one layer
+// per step and a request can enter a free slot at any layer boundary.
+//
+// Slots of 10 to 22 qubits run the tile passes of fq_mix.h, one launch for all
+// slots that run the same pass; here are their phase tables and <C>.  k_slab_pass
+// is the general kernel, for smaller slots and the plans of tuning knobs: the
+// slab is one virtual state of N + s qubits whose top s bits select the slot, and
+// one persistent launch covers every active slot.
 #include "forqaoa.h"
 #include "fq_device.h"
 #include "fq_internal.h"
@@ -19,6 +23,7 @@ namespace fq {
 // slot * stride).  Grid: (entries, slots).
 __global__ void __launch_bounds__(256) k_slab_phase_table(const TileArgs a, int a_log,
                                                           const SlotParams *__restrict__ slots,
+                                                          const SlotPlans *__restrict__ plans,
                                                           double2 *__restrict__ tabs, size_t stride)
 {
     const SlotParams &sp = slots[blockIdx.y];
@@ -26,12 +31,28 @@ __global__ void __launch_bounds__(256) k_slab_phase_table(const TileArgs a, int 
         return;
     const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     double coef;
-    if (!phase_coef(a.Q, run_tiles(a), a.nthr, a.nh, sp.plan, a_log, gid, coef))
+    if (!phase_coef(a.Q, run_tiles(a), a.nthr, a.nh, plans[blockIdx.y].cost[0], a_log, gid, coef))
         return;
     const double angle = sp.gamma * coef;
     double sn, cs;
     sincos(angle, &sn, &cs);
     tabs[stride * blockIdx.y + gid] = make_double2(cs, sn);
+}
+
+// The phase tables of a packed step (blockIdx.y: the table), one launch for all
+// its slots and passes.
+__global__ void __launch_bounds__(256) k_slab_tables(const SlabGeos geos, const SlabJob *__restrict__ jobs,
+                                                     const SlotPlans *__restrict__ plans, double2 *__restrict__ tabs)
+{
+    const SlabJob &job = jobs[blockIdx.y];
+    const TableGeo &g = geos.geo[job.geo];
+    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    double coef;
+    if (!phase_coef(g.Q, g.ntiles, g.nthr, g.nh, plans[job.slot].cost[job.geo], g.a_log, gid, coef))
+        return;
+    double sn, cs;
+    sincos(job.gamma * coef, &sn, &cs);
+    tabs[job.offset + gid] = make_double2(cs, sn);
 }
 
 // First tile at or after tl (below end) that the pass processes: its slot is
@@ -237,12 +258,13 @@ __global__ void __launch_bounds__(1024) k_slab_pass(typename CT<R>::T *__restric
     }
 }
 
-// <C> and sum |psi|^2 of the slots with want_expect; per-tile partials.
+// <C> and sum |psi|^2 of the slots fin[] (blockIdx.y); per-tile partials.
 template <typename R, int A_LOG>
 __global__ void __launch_bounds__(256) k_slab_expect(const typename CT<R>::T *__restrict__ sv,
                                                      const TileArgs a,
-                                                     const SlotParams *__restrict__ slots,
-                                                     int slot_shift, double *__restrict__ partials)
+                                                     const SlotPlans *__restrict__ plans,
+                                                     const int *__restrict__ fin, int slot_shift,
+                                                     double *__restrict__ partials0)
 {
     typedef typename CT<R>::T T;
     constexpr int A = 1 << A_LOG;
@@ -252,17 +274,10 @@ __global__ void __launch_bounds__(256) k_slab_expect(const typename CT<R>::T *__
     __shared__ double s_p[256];
     const int t = threadIdx.x;
     const int nthreads = blockDim.x;
-    const uint64_t tile = blockIdx.x;
-    const SlotParams &sp = slots[tile >> slot_shift];
-    if (!sp.want_expect) {
-        if (t == 0) {
-            partials[2 * tile] = 0.0;
-            partials[2 * tile + 1] = 0.0;
-        }
-        return;
-    }
-    const PlanDev &p = sp.eplan;
-    const uint64_t lt = tile & ((1ull << slot_shift) - 1ull);
+    const int slot = fin[blockIdx.y];
+    const PlanDev &p = plans[slot].expect;
+    const uint64_t lt = blockIdx.x, tile = ((uint64_t)slot << slot_shift) + lt;
+    double *const partials = partials0 + 2 * ((uint64_t)blockIdx.y << slot_shift);
     const uint64_t base = unpack_runs(tile, a.hruns) + unpack_runs((uint64_t)t, a.truns);
     cut_tile_prologue(p, a.Q, slot_shift, lt, s_c, &s_K, t, nthreads);
     __syncthreads();
@@ -303,21 +318,18 @@ __global__ void __launch_bounds__(256) k_slab_expect(const typename CT<R>::T *__
         __syncthreads();
     }
     if (t == 0) {
-        partials[2 * tile] = s_pc[0];
-        partials[2 * tile + 1] = s_p[0];
+        partials[2 * lt] = s_pc[0];
+        partials[2 * lt + 1] = s_p[0];
     }
 }
 
-// One work-group per slot: sum that slot's tile partials in a fixed order.
+// One work-group per finishing slot: sum its tile partials in a fixed order.
 // Only slots reduced in this step are written, so an earlier result stays
 // until it is collected.
 __global__ void __launch_bounds__(256) k_slab_finalize(const double *__restrict__ partials,
-                                                       uint64_t tiles_per_slot,
-                                                       const SlotParams *__restrict__ slots,
+                                                       uint64_t tiles_per_slot, const int *__restrict__ fin,
                                                        double *__restrict__ out)
 {
-    if (!slots[blockIdx.x].want_expect)
-        return;
     __shared__ double s_a[256];
     __shared__ double s_b[256];
     const int t = threadIdx.x;
@@ -338,19 +350,28 @@ __global__ void __launch_bounds__(256) k_slab_finalize(const double *__restrict_
         __syncthreads();
     }
     if (t == 0) {
-        out[2 * blockIdx.x] = s_a[0];
-        out[2 * blockIdx.x + 1] = s_b[0];
+        out[2 * fin[blockIdx.x]] = s_a[0];
+        out[2 * fin[blockIdx.x] + 1] = s_b[0];
     }
 }
 
 // ---- launchers -----------------------------------------------------------------
 
-hipError_t launch_slab_phase_table(const TileArgs &local, int a_log, const SlotParams *slots, int nslots,
-                                   double2 *tabs, size_t stride, hipStream_t stream)
+hipError_t launch_slab_phase_table(const TileArgs &local, int a_log, const SlotParams *slots, const SlotPlans *plans,
+                                   int nslots, double2 *tabs, size_t stride, hipStream_t stream)
 {
     const size_t n = phase_table_entries(local, a_log);
     const dim3 grid((unsigned)((n + 255) / 256), (unsigned)nslots);
-    hipLaunchKernelGGL(k_slab_phase_table, grid, dim3(256), 0, stream, local, a_log, slots, tabs, stride);
+    hipLaunchKernelGGL(k_slab_phase_table, grid, dim3(256), 0, stream, local, a_log, slots, plans, tabs,
+                       stride);
+    return hipGetLastError();
+}
+
+hipError_t launch_slab_tables(const SlabGeos &g, const SlabJob *jobs, int njobs, size_t entries, const SlotPlans *plans,
+                              double2 *tabs, hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_slab_tables, dim3((unsigned)((entries + 255) / 256), (unsigned)njobs), dim3(256), 0, stream, g,
+                       jobs, plans, tabs);
     return hipGetLastError();
 }
 
@@ -402,14 +423,14 @@ hipError_t launch_slab_pass(int dtype, int a_log, bool cost, bool mirror, void *
 #undef FQ_SP
 }
 
-hipError_t launch_slab_expect(int dtype, int a_log, const void *sv, const TileArgs &a, const SlotParams *slots,
-                              int slot_shift, int nslots, double *partials, double *out, hipStream_t stream)
+hipError_t launch_slab_expect(int dtype, int a_log, const void *sv, const TileArgs &a, const SlotPlans *plans,
+                              const int *fin, int nfin, int slot_shift, double *partials, double *out,
+                              hipStream_t stream)
 {
-    const uint64_t tiles = 1ull << a.nh;
-    const dim3 g((unsigned)tiles), b(1u << a.nthr);
+    const dim3 g(1u << slot_shift, (unsigned)nfin), b(1u << a.nthr);
 #define FQ_SE(R, AL)                                                                                  \
     hipLaunchKernelGGL((k_slab_expect<R, AL>), g, b, 0, stream,                                      \
-                       reinterpret_cast<const typename CT<R>::T *>(sv), a, slots, slot_shift, partials); \
+                       reinterpret_cast<const typename CT<R>::T *>(sv), a, plans, fin, slot_shift, partials); \
     break;
     if (dtype == 0) {
         switch (a_log) {
@@ -432,8 +453,7 @@ hipError_t launch_slab_expect(int dtype, int a_log, const void *sv, const TileAr
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return e;
-    hipLaunchKernelGGL(k_slab_finalize, dim3(nslots), dim3(256), 0, stream, partials,
-                       tiles / (uint64_t)nslots, slots, out);
+    hipLaunchKernelGGL(k_slab_finalize, dim3(nfin), dim3(256), 0, stream, partials, 1ull << slot_shift, fin, out);
     return hipGetLastError();
 }
 

@@ -194,8 +194,7 @@ int fq_set_memory_budget(size_t bytes);
 int fq_memory_in_use(size_t *bytes);
 
 /* A slab packs nslots (a power of two) evaluations of the same N into one
- * allocation: its slots form one virtual state whose top bits select the
- * slot, so each tile pass is one launch over every active slot.  Slots are
+ * allocation; a tile pass is one launch over every slot that runs it.  Slots are
  * assigned requests (graph, P, angles) independently; fq_slab_step advances
  * every active slot by one fused layer (slots at different layers and with
  * different P run together); a slot finishing its last layer gets <C> reduced
@@ -214,9 +213,9 @@ int fq_slab_assign(fq_slab *sb, int slot, fq_graph *g, int P, const double *gamm
 /* Enqueue one layer for every active slot (waits for the previous step first);
  * nfinishing (may be NULL) receives the number of slots finishing with it. */
 int fq_slab_step(fq_slab *sb, int *nfinishing);
-/* Layers a step runs per slot in a slab of large slots (2^10 or more
- * first-pass tiles per slot, whose slots run fq_run's tile passes one after
- * the other): up to `layers` (>= 1, default 1), fewer for a slot that has
+/* Layers a step runs per slot in a slab of large slots (half states from about
+ * N = 22 complex128, 23 complex64, whose slots run fq_run's tile passes one
+ * after the other): up to `layers` (>= 1, default 1), fewer for a slot that has
  * fewer left.  Slabs of small slots (one packed launch per pass) keep one
  * layer per step. */
 int fq_slab_set_layers_per_step(fq_slab *sb, int layers);
@@ -224,7 +223,8 @@ int fq_slab_set_layers_per_step(fq_slab *sb, int layers);
 int fq_slab_poll(fq_slab *sb, int *busy);
 /* Finished slots: indices, <C>, sum |psi|^2; frees them.  Waits. */
 int fq_slab_collect(fq_slab *sb, int *slots, double *expect, double *norm2, int *n);
-/* Amplitudes of one slot (logical = physical order).  Waits. */
+/* Amplitudes of one slot after the layers it has run (logical = physical
+ * order).  Waits. */
 int fq_slab_copy_out(fq_slab *sb, int slot, void *host, size_t bytes);
 
 /* The tile passes that cover one layer of FQ_SCHED_FUSED or FQ_SCHED_Z2 for N
