@@ -184,6 +184,60 @@ static bool is_own_stream(hipStream_t s)
     return g_own_streams.count(s) != 0;
 }
 
+// A state's stream and a page of pinned host memory that its kernels write results
+// to.  Both outlive it: up to FQ_LANES idle ones are kept for the next states
+// (making a stream takes 60 to 130 us; a state was made in 78 to 143 us, and now in 8
+// to 16).  A result that the kernels write themselves needs no copy behind them:
+// <C> at N=16 28 -> 20 us, with its sums added up by the last work-group.
+#define FQ_LANES 16
+#define FQ_LANE_DOUBLES 512
+struct Lane {
+    hipStream_t stream = nullptr;
+    double *host = nullptr;
+    int device = -1;
+};
+static std::mutex g_lanes_mu;
+static std::vector<Lane> g_lanes;
+
+static bool lane_take(Lane &l)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess)
+        return false;
+    {
+        std::lock_guard<std::mutex> lk(g_lanes_mu);
+        for (size_t i = 0; i < g_lanes.size(); ++i)
+            if (g_lanes[i].device == dev) {
+                l = g_lanes[i];
+                g_lanes.erase(g_lanes.begin() + i);
+                return true;
+            }
+    }
+    l.device = dev;
+    if (hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking) != hipSuccess)
+        return false;
+    if (hipHostMalloc(&l.host, sizeof(double) * FQ_LANE_DOUBLES, hipHostMallocDefault) != hipSuccess) {
+        hipStreamDestroy(l.stream);
+        l.stream = nullptr;
+        return false;
+    }
+    return true;
+}
+
+// (its work is done)
+static void lane_give(const Lane &l)
+{
+    {
+        std::lock_guard<std::mutex> lk(g_lanes_mu);
+        if (g_lanes.size() < FQ_LANES) {
+            g_lanes.push_back(l);
+            return;
+        }
+    }
+    hipStreamDestroy(l.stream);
+    hipHostFree(l.host);
+}
+
 // ---- handles -------------------------------------------------------------------
 
 struct PlanEntry {
@@ -234,7 +288,8 @@ struct fq_state {
     int N = 0, D = 0, B = 0, C = 0, dtype = 0;
     size_t elem = 16, bytes = 0;
     void *sv = nullptr;
-    hipStream_t own = nullptr, stream = nullptr;
+    Lane lane;
+    hipStream_t stream = nullptr;   // the lane's, or a caller's
     // chunked runs (run_chunks): two streams forked from and joined to `stream`
     hipStream_t side[2] = {nullptr, nullptr};
     hipEvent_t forked = nullptr, joined[2] = {nullptr, nullptr};
@@ -248,7 +303,7 @@ struct fq_state {
     bool in_run = false;
     double *d_part = nullptr;  // expect partials
     size_t part_cap = 0;
-    double *d_out2 = nullptr;
+    unsigned *d_count = nullptr;   // of launch_expect
     double *d_cand_p = nullptr;
     uint64_t *d_cand_i = nullptr;
     int cand_blocks = 0;
@@ -859,17 +914,18 @@ extern "C" int fq_state_create(int N, int D, int B, int C, int dtype, fq_state *
     st->part_cap = (size_t)1 << (N - Qr);
     st->cand_blocks = (int)std::min<uint64_t>(1024, std::max<uint64_t>(1, ((uint64_t)1 << N) / 4096));
     bool ok = hipMalloc(&st->d_part, sizeof(double) * 2 * st->part_cap) == hipSuccess &&
-              hipMalloc(&st->d_out2, sizeof(double) * 2) == hipSuccess &&
+              hipMalloc(&st->d_count, sizeof(unsigned)) == hipSuccess &&
               hipMalloc(&st->d_cand_p, sizeof(double) * FQ_TOPK_MAX * st->cand_blocks) == hipSuccess &&
               hipMalloc(&st->d_cand_i, sizeof(uint64_t) * FQ_TOPK_MAX * st->cand_blocks) == hipSuccess &&
-              hipStreamCreateWithFlags(&st->own, hipStreamNonBlocking) == hipSuccess;
+              lane_take(st->lane) &&
+              hipMemsetAsync(st->d_count, 0, sizeof(unsigned), st->lane.stream) == hipSuccess;
     if (!ok) {
         hipGetLastError();
         fq_state_destroy(st);
         return set_err(FQ_ERR_OOM, "scratch allocation failed");
     }
-    own_stream(st->own, true);
-    st->stream = st->own;
+    own_stream(st->lane.stream, true);
+    st->stream = st->lane.stream;
     *out = st;
     return FQ_OK;
 }
@@ -890,7 +946,7 @@ extern "C" int fq_state_destroy(fq_state *st)
         budget_give(st->bytes);
     hipFree(st->sv);
     hipFree(st->d_part);
-    hipFree(st->d_out2);
+    hipFree(st->d_count);
     hipFree(st->d_cand_p);
     hipFree(st->d_cand_i);
     hipFree(st->d_phase);
@@ -907,9 +963,10 @@ extern "C" int fq_state_destroy(fq_state *st)
     }
     if (st->forked)
         hipEventDestroy(st->forked);
-    if (st->own) {
-        own_stream(st->own, false);
-        hipStreamDestroy(st->own);
+    if (st->lane.stream) {
+        hipStreamSynchronize(st->lane.stream);   // (a state on a caller's stream)
+        own_stream(st->lane.stream, false);
+        lane_give(st->lane);
     }
     delete st;
     return FQ_OK;
@@ -945,7 +1002,7 @@ extern "C" int fq_state_set_stream(fq_state *st, void *hip_stream)
     if (int rc = check_state(st))
         return rc;
     FQ_HIP(hipStreamSynchronize(st->stream));
-    st->stream = hip_stream ? (hipStream_t)hip_stream : st->own;
+    st->stream = hip_stream ? (hipStream_t)hip_stream : st->lane.stream;
     return FQ_OK;
 }
 
@@ -2348,13 +2405,12 @@ extern "C" int fq_expect_cut(fq_state *st, fq_graph *g, double *expect, double *
     if (int rc = get_plan(g, geom, &a.plan, st->stream))
         return rc;
     int rc = timed(st, FQ_K_REDUCE, (double)st->bytes, [&] {
-        return launch_expect(st->dtype, a_log, st->sv, a, st->d_part, st->d_out2, st->stream);
+        return launch_expect(st->dtype, a_log, st->sv, a, st->d_part, st->d_count, st->lane.host, st->stream);
     });
     if (rc)
         return rc;
-    double h[2];
-    FQ_HIP(hipMemcpyAsync(h, st->d_out2, sizeof(h), hipMemcpyDeviceToHost, st->stream));
     FQ_HIP(hipStreamSynchronize(st->stream));
+    const double *h = st->lane.host;
     *expect = h[0];
     if (norm2)
         *norm2 = h[1];
@@ -2434,7 +2490,7 @@ extern "C" int fq_expect_cut_static(fq_state *st, fq_graph *g, double *expect, d
     // the previous call on this stream may still read the plan: stream order
     // keeps this upload behind it
     FQ_HIP(hipMemcpyAsync(plan_mem, pb.bytes.data(), pb.bytes.size(), hipMemcpyHostToDevice, st->stream));
-    FQ_HIP(launch_expect(st->dtype, a_log, st->sv, a, part, out2, st->stream));
+    FQ_HIP(launch_expect(st->dtype, a_log, st->sv, a, part, nullptr, out2, st->stream));
     double h[2];
     FQ_HIP(hipMemcpyAsync(h, out2, sizeof(h), hipMemcpyDeviceToHost, st->stream));
     FQ_HIP(hipStreamSynchronize(st->stream));
@@ -2471,8 +2527,8 @@ static int ensure_aux(fq_state *st, size_t grad_slots)
 }
 
 // lambda = Cut psi_P (on the half state from N = 3 on); sum |psi|^2 Cut and
-// sum |psi|^2 into d_grad.
-static int cut_lambda(fq_state *st, fq_graph *g)
+// sum |psi|^2 into out.
+static int cut_lambda(fq_state *st, fq_graph *g, double *out)
 {
     const int N = st->N, Q = std::min(12, N >= 3 ? N - 1 : N);
     const int a_log = std::max(1, std::min(4, Q));
@@ -2484,13 +2540,12 @@ static int cut_lambda(fq_state *st, fq_graph *g)
     if (int rc = get_plan(g, geom, &a.plan, st->stream))
         return rc;
     FQ_HIP(launch_cut_mul(st->dtype, a_log, st->sv, st->aux, a, st->d_part, st->stream));
-    FQ_HIP(launch_finalize(st->d_part, run_tiles(a), st->d_grad, st->stream));
+    FQ_HIP(launch_finalize(st->d_part, run_tiles(a), out, st->stream));
     return FQ_OK;
 }
 
-// Partial sums of the pair passes (doubles) and the sums of `sums` of them after
-// d_grad's first two.
-static int ensure_pair_scratch(fq_state *st, size_t part, size_t sums)
+// Partial sums of the pair passes (doubles).
+static int ensure_pair_scratch(fq_state *st, size_t part)
 {
     if (part > st->pair_cap) {
         FQ_HIP(hipStreamSynchronize(st->stream));
@@ -2501,7 +2556,7 @@ static int ensure_pair_scratch(fq_state *st, size_t part, size_t sums)
             return set_err(FQ_ERR_OOM, "gradient scratch allocation failed");
         st->pair_cap = part;
     }
-    return ensure_aux(st, 1 + (sums + 1) / 2);
+    return FQ_OK;
 }
 
 // One pair pass of the walk back on compile-time phases (fq_pair.hip).
@@ -2548,12 +2603,13 @@ static LayerPlan pair_plan(int N, int dtype)
 }
 
 // The walk back over plan lp: <C> and the gradient sums of psi_P and lambda (both
-// on the half state, cut_lambda), not yet doubled.  Every RX is the
+// on the half state, cut_lambda), not yet doubled.  out: the passes' sums after
+// those of <C>, in the lane's page or d_grad.  Every RX is the
 // butterfly of rx_tform on both states, which grows them by (1 + t^2)^(1/2) a gate:
 // mag2 follows the inverse of what <lambda|psi> has taken on, each sum gets its
 // value as a weight, and each cost pass scales it back to 1.
 static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, const double *gammas, const double *betas,
-                     double *expect, double *grad_gammas, double *grad_betas)
+                     double *out, double *expect, double *grad_gammas, double *grad_betas)
 {
     const int N = st->N, m = (int)lp.ps.size(), Q = (int)lp.ps[0].tile.size(), A = pair_a_log(st->dtype, Q);
     std::vector<Step> seq;
@@ -2614,7 +2670,7 @@ static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, cons
     // partial sums of as many passes as fit 16 MiB at once
     const uint64_t tiles = 1ull << (N - 1 - Q);
     const size_t per = 3 * (size_t)tiles, batch = std::max<size_t>(1, std::min(pp.size(), ((size_t)2 << 20) / per));
-    if (int rc = ensure_pair_scratch(st, batch * per, 3 * pp.size()))
+    if (int rc = ensure_pair_scratch(st, batch * per))
         return rc;
     bool tables = false;
     if (int rc = mix_tables(st, pp, &tables, true))
@@ -2651,12 +2707,15 @@ static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, cons
         k += n;
         if (k % batch == 0 || k == pp.size()) {
             const size_t first = (k - 1) / batch * batch;
-            FQ_HIP(launch_pair_sums(st->d_pair, tiles, (int)(k - first), st->d_grad + 2 + 3 * first, st->stream));
+            FQ_HIP(launch_pair_sums(st->d_pair, tiles, (int)(k - first), out + 2 + 3 * first, st->stream));
         }
     }
     std::vector<double> sums(2 + 3 * pp.size());
-    FQ_HIP(hipMemcpyAsync(sums.data(), st->d_grad, sizeof(double) * sums.size(), hipMemcpyDeviceToHost, st->stream));
+    if (out == st->d_grad)
+        FQ_HIP(hipMemcpyAsync(sums.data(), out, sizeof(double) * sums.size(), hipMemcpyDeviceToHost, st->stream));
     FQ_HIP(hipStreamSynchronize(st->stream));
+    if (out != st->d_grad)
+        std::copy(out, out + sums.size(), sums.begin());
     *expect = sums[0];
     const double *h = sums.data() + 2;
     for (int k = 0; k < P; ++k)
@@ -2699,14 +2758,16 @@ extern "C" int fq_backward(fq_state *st, fq_graph *g, int P, const double *gamma
     const bool z2 = N >= 3;
     const double mult = z2 ? 2.0 : 1.0;
     if (const LayerPlan lp = pair_plan(N, st->dtype); !lp.ps.empty()) {
-        // (sums of 1 + P (m - 1) passes after the two of <C>)
-        const size_t passes = 1 + (size_t)P * (lp.ps.size() - 1);
-        if (int rc = ensure_aux(st, 1 + (3 * passes + 1) / 2))
+        // the sums of <C>, then of 1 + P (m - 1) passes: in the lane's page, or
+        // copied from device memory where they do not fit
+        const size_t nsums = 2 + 3 * (1 + (size_t)P * (lp.ps.size() - 1));
+        if (int rc = ensure_aux(st, (nsums + 1) / 2))
             return rc;
-        if (int rc = cut_lambda(st, g))
+        double *out = nsums <= FQ_LANE_DOUBLES ? st->lane.host : st->d_grad;
+        if (int rc = cut_lambda(st, g, out))
             return rc;
         double e = 0;
-        if (int rc = pair_walk(st, g, lp, P, gammas, betas, &e, grad_gammas, grad_betas))
+        if (int rc = pair_walk(st, g, lp, P, gammas, betas, out, &e, grad_gammas, grad_betas))
             return rc;
         for (int k = 0; k < P; ++k) {
             grad_gammas[k] *= mult;
@@ -2762,7 +2823,7 @@ extern "C" int fq_backward(fq_state *st, fq_graph *g, int P, const double *gamma
     if (int rc = ensure_aux(st, nslot))
         return rc;
 
-    if (int rc = cut_lambda(st, g))
+    if (int rc = cut_lambda(st, g, st->d_grad))
         return rc;
     // (launch index in fwd, first slot) of every launch, for the sums below
     std::vector<size_t> slot_of(fwd.size());
