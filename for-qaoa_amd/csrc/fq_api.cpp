@@ -1361,19 +1361,12 @@ static int pass_shape(int N, const std::vector<int> &tile, const std::vector<int
     return FQ_OK;
 }
 
-// Arguments as tile_pass.  The mirror pass may be a boundary pass too: the phase of a
-// mirror element is that of the N-qubit index it stands for (Cut(b) = Cut(~b)).
-static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, double beta,
-                       fq_graph *g, double gamma, bool cost, bool first, int z2, const double *pre_beta, bool defer,
-                       MixPass &mp)
+// The factors of a prepared pass and its angle: what differs between the layers.
+static void mix_factors(fq_state *st, size_t ngates, double beta, double gamma, const double *pre_beta, bool defer,
+                        MixPass &mp)
 {
-    const int N = st->N, A = mix_a_log(st->dtype, (int)tile.size());
     MixArgs &a = mp.a;
-    if (int rc = pass_shape(N, tile, gates, A, mix_lane_bit, z2, a, mp.K, mp.lane))
-        return rc;
-    if (z2 >= Z2_MIRROR && cost && !first && !pre_beta)
-        return set_err(FQ_ERR_ARG, "internal: the mirror pass is no cost pass of its own");
-    const PassFactor f = pass_factor(st, gates.size(), beta, pre_beta, cost, defer);
+    const PassFactor f = pass_factor(st, ngates, beta, pre_beta, mp.cost, defer);
     a.t = f.t;
     a.pre_t = f.pre_t;
     a.tf = (float)f.t;   // exact for complex64 (rx_tform rounds t to FP32)
@@ -1381,22 +1374,37 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
     a.scale_re = f.re;
     a.scale_im = f.im;
     a.apply_scale = f.apply;
+    mp.tab.gamma = gamma;
+}
+
+// A pass without its factors (mix_factors); arguments as tile_pass.  The mirror pass
+// may be a boundary pass too: the phase of a mirror element is that of the N-qubit
+// index it stands for (Cut(b) = Cut(~b)).
+static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::vector<int> &gates, fq_graph *g, bool cost,
+                       bool first, int z2, bool boundary, MixPass &mp)
+{
+    const int N = st->N, A = mix_a_log(st->dtype, (int)tile.size());
+    MixArgs &a = mp.a;
+    if (int rc = pass_shape(N, tile, gates, A, mix_lane_bit, z2, a, mp.K, mp.lane))
+        return rc;
+    if (z2 >= Z2_MIRROR && cost && !first && !boundary)
+        return set_err(FQ_ERR_ARG, "internal: the mirror pass is no cost pass of its own");
     if (cost) {
         // phase table of the layout the cost phase runs in: layout 0, or for a
         // boundary pass the last one
         TileArgs &ca = mp.tab;
-        const Geom cgeom = layout_geom(N, tile, A, pre_beta ? mp.K : 0);
+        const Geom cgeom = layout_geom(N, tile, A, boundary ? mp.K : 0);
         geom_to_args(cgeom, ca);
         ca.ntiles_run = a.ntiles;
         if (int rc = get_plan(g, cgeom, &ca.plan, st->stream))
             return rc;
-        set_cost(ca, gamma, st->init_amp);
+        set_cost(ca, 0.0, st->init_amp);
         mp.entries = phase_table_entries(ca, A);
         a.has_rr = ca.has_rr;
         a.init_amp = st->init_amp;
     }
     mp.cost = cost;
-    mp.kind = pre_beta ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
+    mp.kind = boundary ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
     mp.mir = z2 == Z2_MIRROR ? 1 : z2 == Z2_EXPAND ? 2 : 0;
     // a half-state pass reads and writes half the state; the expanding one
     // writes the whole state
@@ -1478,8 +1486,9 @@ static int mix_pass(fq_state *st, const std::vector<int> &tile, const std::vecto
                     bool defer)
 {
     MixPass mp;
-    if (int rc = mix_prepare(st, tile, gates, beta, g, gamma, cost, first, z2, pre_beta, defer, mp))
+    if (int rc = mix_prepare(st, tile, gates, g, cost, first, z2, pre_beta != nullptr, mp))
         return rc;
+    mix_factors(st, gates.size(), beta, gamma, pre_beta, defer, mp);
     if (int rc = mix_table(st, mp))
         return rc;
     return timed(st, kind, mp.bytes, [&] {
@@ -2033,14 +2042,15 @@ static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
         if (getenv(k))
             return lp;
     const int elem_log = dtype == FQ_C128 ? 4 : 3, Ns = z2 ? N - 1 : N;
-    if (lp.ps.size() == 2 && (!z2 || N < 24)) {
+    if (lp.ps.size() <= 2 && (!z2 || N < 24)) {
         // Two passes of the narrowest tiles that cover N with 128 B runs: a
         // full-width tile leaves most CUs of a small state idle (16 tiles at
         // N=17) and takes a pass's whole latency for its 128 KiB.  Per layer,
         // with one phase-table launch a run (mix_tables), full-width tiles and
         // a launch per table before: N=14 complex128 17.6 -> 6.1 us, N=18 22.3
         // -> 10.2, N=20 30.6 -> 16.7; half state N=20 complex64 31.1 -> 10.8
-        // (also one pass per layer instead of two).
+        // (also one pass per layer instead of two), and against one tile of full
+        // width: N=13 complex128 8.7 -> 4.5, N=14 complex64 13.0 -> 5.7.
         const int Q = std::min(tile_max_q(dtype),
                                std::max(dtype == FQ_C128 ? 9 : 10, (N + carriers_for(dtype) + 1) / 2));
         if (Q >= N)
@@ -2185,6 +2195,7 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
     // may have none): prepared first, and small phase tables made at once
     const bool mix = mix_a_log(st->dtype, (int)ps[0].tile.size()) > 0;
     std::vector<MixPass> mps(mix ? seq.size() : 0);
+    std::vector<int> modes(mps.size());
     bool tables = false;
     for (size_t k = 0; k < seq.size(); ++k) {
         const Step &s = seq[k];
@@ -2200,12 +2211,22 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
         const double *pre = bd ? &betas[s.layer] : nullptr;
         // plain passes leave their RX factor to the next cost pass, except
         // the run's very last pass, which leaves the state exact
-        const int rc = mix ? mix_prepare(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, mode,
-                                         pre, !last, mps[k])
-                           : tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST,
-                                       FQ_K_FUSED, mode, pre, !last);
-        if (rc)
+        if (!mix) {
+            if (int rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, FQ_K_FUSED,
+                                   mode, pre, !last))
+                return rc;
+            continue;
+        }
+        // the passes of a layer repeat: prepared once, with each layer's factors
+        size_t same = 0;
+        while (same < k && !(seq[same].pass == s.pass && seq[same].kind == s.kind && modes[same] == mode))
+            ++same;
+        modes[k] = mode;
+        if (same < k)
+            mps[k] = mps[same];
+        else if (int rc = mix_prepare(st, fp.tile, fp.gates, g, cost(s), s.kind == STEP_FIRST, mode, bd, mps[k]))
             return rc;
+        mix_factors(st, fp.gates.size(), betas[L], gamma, pre, !last, mps[k]);
     }
     if (!mix)
         return FQ_OK;
@@ -2239,6 +2260,74 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
     return FQ_OK;
 }
 
+// P layers of a state that is one tile (k_solo), FQ_SOLO_LAYERS a launch, and one
+// launch for their phase tables.  done false: not such a state, or a plan of tuning
+// knobs is asked for.
+static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, const double *betas, bool *done)
+{
+    const int N = st->N;
+    *done = false;
+    if (N < solo_min(st->dtype) || N > solo_max(st->dtype))
+        return FQ_OK;
+    for (const char *k : {"FQ_TILE_Q", "FQ_PASS_BLOCK", "FQ_CARRIER_GATES", "FQ_LAYER_PIPE"})
+        if (getenv(k))
+            return FQ_OK;
+    *done = true;
+    const std::vector<int> tile = low_tile(N);
+    const int A = mix_a_log(st->dtype, N);
+    for (int p0 = 0; p0 < P; p0 += FQ_SOLO_LAYERS) {
+        const int n = std::min(FQ_SOLO_LAYERS, P - p0);
+        std::vector<MixPass> mps(n);
+        SoloArgs a;
+        memset(&a, 0, sizeof(a));
+        a.P = n;
+        a.first = p0 == 0;
+        a.init_amp = st->init_amp;
+        // odd layers go down the layouts and take their cost phase in the last one
+        TileArgs tab[2];
+        for (int i = 0; i < std::min(n, 2); ++i) {
+            const Geom geom = layout_geom(N, tile, A, i ? 2 : 0);
+            geom_to_args(geom, tab[i]);
+            tab[i].ntiles_run = 1;
+            if (int rc = get_plan(g, geom, &tab[i].plan, st->stream))
+                return rc;
+            set_cost(tab[i], 0.0, st->init_amp);
+            a.has_rr |= tab[i].has_rr;
+        }
+        MixArgs shape;
+        int K = 0;
+        bool lane = false;
+        if (int rc = pass_shape(N, tile, tile, A, mix_lane_bit, Z2_OFF, shape, K, lane))
+            return rc;
+        if (K != 2 || lane)
+            return set_err(FQ_ERR_ARG, "internal: a state of %d qubits takes %d exchanges", N, K);
+        a.gates_w = shape.gates_w;
+        for (int i = 0; i < n; ++i) {
+            MixPass &mp = mps[i];
+            const PassFactor f = pass_factor(st, N, betas[p0 + i], nullptr, true, false);
+            a.t[i] = f.t;
+            a.scale_re[i] = f.re;
+            a.scale_im[i] = f.im;
+            mp.cost = true;
+            mp.tab = tab[i & 1];
+            mp.tab.gamma = gammas[p0 + i];
+            mp.entries = phase_table_entries(mp.tab, A);
+        }
+        bool tables = false;
+        if (int rc = mix_tables(st, mps, &tables))
+            return rc;
+        if (!tables)   // (one layer)
+            if (int rc = prepare_phases(st, mps[0].tab, A))
+                return rc;
+        for (int i = 0; i < n; ++i)
+            a.table[i] = tables ? (uint32_t)(mps[i].ptab - st->d_phase) : 0;
+        const double bytes = (a.first ? 1.0 : 2.0) * (double)st->bytes;
+        if (int rc = timed(st, FQ_K_FUSED, bytes, [&] { return launch_solo(st->dtype, N, st->sv, a, st->d_phase, st->stream); }))
+            return rc;
+    }
+    return FQ_OK;
+}
+
 // FQ_SCHED_REFERENCE without its single steps: every layer applies RX(beta) to
 // each qubit once, wherever the transpositions have moved it, so the P layers are
 // those of the fused schedule in the labels of the start, followed by the
@@ -2253,8 +2342,12 @@ static int reference_run(fq_state *st, fq_graph *g, const std::vector<int> &size
     const int N = st->N;
     if (P == 0)
         return FQ_OK;
-    if (int rc = run_layers(st, g, exec_plan(N, st->dtype, false, P), 0, P, P, gammas, betas, false, true))
+    bool done = false;
+    if (int rc = solo_run(st, g, P, gammas, betas, &done))
         return rc;
+    if (!done)
+        if (int rc = run_layers(st, g, exec_plan(N, st->dtype, false, P), 0, P, P, gammas, betas, false, true))
+            return rc;
     int at[FQ_MAXN], to[FQ_MAXN], qmap[FQ_MAXN];   // position -> the position its qubit came from, and back
     for (int p = 0; p < N; ++p)
         at[p] = p;
@@ -2355,10 +2448,18 @@ extern "C" int fq_run(fq_state *st, fq_graph *g, int P, const double *gammas, co
         // half z_{N-1} = 0 and the other half is written once at the end.
         if (N < 3)
             return set_err(FQ_ERR_ARG, "the half-state schedule needs N >= 3");
+        bool done = false;   // (a small state as a whole: the same amplitudes)
+        const int rc = solo_run(st, g, P, gammas, betas, &done);
+        if (rc || done)
+            return rc;
         return run_layers(st, g, exec_plan(N, st->dtype, true, P), 0, P, P, gammas, betas, true, true);
     }
     if (schedule != FQ_SCHED_FUSED)
         return set_err(FQ_ERR_ARG, "unknown schedule %d", schedule);
+    bool done = false;
+    const int rc = solo_run(st, g, P, gammas, betas, &done);
+    if (rc || done)
+        return rc;
     return run_layers(st, g, exec_plan(N, st->dtype, false, P), 0, P, P, gammas, betas, false, true);
 }
 
@@ -2622,14 +2723,30 @@ static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, cons
         const Step &s = seq[k];
         PairPass &q = pp[k];
         const bool bd = s.kind == STEP_BOUNDARY;
-        q.kind = bd ? PAIR_BOUNDARY : s.kind == STEP_PLAIN ? PAIR_PLAIN : PAIR_COST;
-        q.mir = s.pass + 1 == m;
-        q.cost = q.kind != PAIR_PLAIN;
-        memset(&q.a, 0, sizeof(q.a));
+        // the passes of a layer repeat: prepared once, with each layer's angles
+        size_t same = 0;
+        while (same < k && (seq[same].pass != s.pass || seq[same].kind != s.kind))
+            ++same;
         MixArgs &a = q.a.m;
-        if (int rc = pass_shape(N, lp.ps[s.pass].tile, lp.ps[s.pass].gates, A, pair_lane_bit,
-                                q.mir ? Z2_MIRROR : Z2_LOWER, a, q.K, q.lane))
-            return rc;
+        if (same < k) {
+            q = pp[same];
+        } else {
+            memset(&q.a, 0, sizeof(q.a));
+            q.kind = bd ? PAIR_BOUNDARY : s.kind == STEP_PLAIN ? PAIR_PLAIN : PAIR_COST;
+            q.mir = s.pass + 1 == m;
+            q.cost = q.kind != PAIR_PLAIN;
+            if (int rc = pass_shape(N, lp.ps[s.pass].tile, lp.ps[s.pass].gates, A, pair_lane_bit,
+                                    q.mir ? Z2_MIRROR : Z2_LOWER, a, q.K, q.lane))
+                return rc;
+            if (q.cost) {
+                const Geom geom = layout_geom(N, lp.ps[s.pass].tile, A, q.K);
+                geom_to_args(geom, q.tab);
+                q.tab.ntiles_run = a.ntiles;
+                if (int rc = get_plan(g, geom, &q.tab.plan, st->stream))
+                    return rc;
+                q.entries = phase_table_entries(q.tab, A);
+            }
+        }
         double sr, si, t1, t0;
         const int later = bd ? s.layer + 1 : s.layer;
         rx_tform(-betas[later], st->dtype, true, &t1, &sr, &si);
@@ -2651,13 +2768,7 @@ static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, cons
             q.a.phase = w;
             a.scale_re = std::sqrt(mag2 * w);
             w /= a.scale_re * a.scale_re;
-            TileArgs &ca = q.tab;
-            geom_to_args(layout_geom(N, lp.ps[s.pass].tile, A, q.K), ca);
-            ca.ntiles_run = a.ntiles;
-            if (int rc = get_plan(g, layout_geom(N, lp.ps[s.pass].tile, A, q.K), &ca.plan, st->stream))
-                return rc;
-            set_cost(ca, -gammas[later], st->init_amp);
-            q.entries = phase_table_entries(ca, A);
+            set_cost(q.tab, -gammas[later], st->init_amp);
         }
         if (bd) {
             for (int l = q.K; l >= 0; --l)

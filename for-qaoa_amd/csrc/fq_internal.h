@@ -118,6 +118,16 @@ struct MixArgs {
     const MixSlot *slots;    // packed launch (blockIdx.y: the slot), else null
     int nslots;
 };
+// Layers of a small state (k_solo): per layer the place of its phase table, its
+// factors as above.
+#define FQ_SOLO_LAYERS 64
+struct SoloArgs {
+    int P, first, has_rr;
+    uint32_t gates_w;
+    double init_amp;
+    uint32_t table[FQ_SOLO_LAYERS];
+    double t[FQ_SOLO_LAYERS], scale_re[FQ_SOLO_LAYERS], scale_im[FQ_SOLO_LAYERS];
+};
 // One pair pass: t, pre_t and the real scale as above (a boundary pass undoes
 // RX(pre) first), and the weights of its sums: the inverse of the factor that
 // <lambda|X|psi> has taken in this pass when the sum is formed, for register bit r
@@ -269,6 +279,10 @@ hipError_t launch_pair(int dtype, int a_log, bool costbw, bool mirror, bool boun
 hipError_t launch_cut_mul(int dtype, int a_log, const void *psi, void *lam, const TileArgs &a,
                           double *partials, hipStream_t stream);
 size_t pair_lds_bytes(int dtype, int Q);
+// Qubits of a state that k_solo takes: [solo_min, solo_max].
+inline int solo_min(int dtype) { return dtype == 0 ? 9 : 10; }
+inline int solo_max(int) { return 12; }
+hipError_t launch_solo(int dtype, int N, void *sv, const SoloArgs &a, const double2 *ptab, hipStream_t stream);
 // Pair passes of fq_pair.hip; arguments as launch_mix (register bits per thread
 // pair_a_log, 0: no instance for this tile width).  partials: three sums per tile.
 int pair_a_log(int dtype, int Q);

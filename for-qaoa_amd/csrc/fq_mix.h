@@ -75,6 +75,61 @@ __device__ __forceinline__ void mix_phase(T (&v)[1 << A], const R (&fx)[A], cons
     }
 }
 
+// The cost phase times (sx, sy) on a thread's amplitudes (SET: of a state of ones):
+// the tile's row of the table (entry i in lane i, broadcast by readlane), the
+// thread's entry f_thr, the thread's register entries and the
+// register-register ones.
+template <typename T, typename R, int Q, int A, bool SET>
+__device__ __forceinline__ void mix_cost(T (&v)[1 << A], double2 f_row, double2 f_thr, const double2 *thr_tab,
+                                         const double2 *rr_tab, int has_rr, double sx, double sy, int t)
+{
+    constexpr int NT = Q - A, N = 1 << A;
+    // all loads at once, behind the products of the thread's factor (each of them in
+    // its turn took 1 us of a small state's pass: N=20 complex128 14.2 -> 13.9 us, and
+    // N=24 139 -> 132)
+    double2 f_reg[A];
+#pragma unroll
+    for (int r = 0; r < A; ++r)
+        f_reg[r] = thr_tab[((1 + r) << NT) + t];
+    __builtin_amdgcn_sched_barrier(0);
+    double x = f_thr.x, y = f_thr.y;
+    auto mul = [&](double2 f) {
+        const double nx = x * f.x - y * f.y;
+        y = x * f.y + y * f.x;
+        x = nx;
+    };
+    mul(lane_bcast(f_row, Q));
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const double2 f = lane_bcast(f_row, i);
+        const double nx = x * f.x - y * f.y;
+        const double ny = x * f.y + y * f.x;
+        const bool on = (t >> i) & 1;
+        x = on ? nx : x;
+        y = on ? ny : y;
+    }
+    mul(make_double2(sx, sy));
+    const R x0 = (R)x, y0 = (R)y;
+    R fx[A], fy[A];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < A; ++r) {
+        const double2 f = lane_bcast(f_row, NT + r), g = f_reg[r];
+        fx[r] = (R)(g.x * f.x - g.y * f.y);
+        fy[r] = (R)(g.x * f.y + g.y * f.x);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    mix_phase<T, R, A, A, SET>(v, fx, fy, x0, y0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (has_rr) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const double2 f = rr_tab[j];
+            cmul_by(v[j], (R)f.x, (R)f.y);
+        }
+    }
+}
+
 // Whether the instances of this width take packed launches.
 template <typename R> static constexpr bool mix_packs(int Q) { return Q < (sizeof(R) == 4 ? 14 : 13); }
 
@@ -171,43 +226,10 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
         }
     }
     auto cost = [&]() {
-        double x = f_thr.x, y = f_thr.y;
-        auto mul = [&](double2 f) {
-            const double nx = x * f.x - y * f.y;
-            y = x * f.y + y * f.x;
-            x = nx;
-        };
-        mul(lane_bcast(f_row, Q));
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            const double2 f = lane_bcast(f_row, i);
-            const double nx = x * f.x - y * f.y;
-            const double ny = x * f.y + y * f.x;
-            const bool on = (t >> i) & 1;
-            x = on ? nx : x;
-            y = on ? ny : y;
-        }
-        mul(KIND == MIX_FIRST ? make_double2(a.init_amp * scale_re, a.init_amp * scale_im)
-                              : make_double2(scale_re, scale_im));
-        const R x0 = (R)x, y0 = (R)y;
-        R fx[A], fy[A];
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int r = 0; r < A; ++r) {
-            const double2 f = lane_bcast(f_row, NT + r), g = thr_tab[((1 + r) << NT) + t];
-            fx[r] = (R)(g.x * f.x - g.y * f.y);
-            fy[r] = (R)(g.x * f.y + g.y * f.x);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        mix_phase<T, R, A, A, KIND == MIX_FIRST>(v, fx, fy, x0, y0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (has_rr) {
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const double2 f = rr_tab[j];
-                cmul_by(v[j], (R)f.x, (R)f.y);
-            }
-        }
+        const bool first = KIND == MIX_FIRST;
+        mix_cost<T, R, Q, A, KIND == MIX_FIRST>(v, f_row, f_thr, thr_tab, rr_tab, has_rr,
+                                                first ? a.init_amp * scale_re : scale_re,
+                                                first ? a.init_amp * scale_im : scale_im, t);
     };
     if constexpr (KIND == MIX_FIRST || KIND == MIX_COST)
         cost();
@@ -246,6 +268,87 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
                 pm[half - ro[j - AH]] = v[j - AH];
         }
     }
+}
+
+// ---- small states ------------------------------------------------------------
+
+// Layers of a state that is one tile, in one launch of one work-group: the
+// amplitudes stay in registers, the layers go through the layouts up and down
+// in turn, each with its cost phase where it begins.  A layer takes the latency of
+// its table entries and of K exchanges, instead of that of a launch, a load and
+// a store besides: per layer on MI355X 4.0 us at N=12 and 2.8 at N=10 complex128
+// (a launch each: 7.1 and 5.4), 3.7 and 2.9 complex64 (6.9 and 5.5).  One
+// work-group's butterflies set the limit: at N=13 complex64 it took 6.7 us, two
+// narrow passes 5.7.
+template <typename R, int Q, int A, int K>
+__global__ void __launch_bounds__(1 << (Q - A), 1)
+    k_solo(typename CT<R>::T *__restrict__ sv, const SoloArgs a, const double2 *__restrict__ ptab)
+{
+    typedef typename CT<R>::T T;
+    typedef MixLay<R, Q, A, K> Lay;
+    constexpr int N = 1 << A, NT = Q - A;
+    static_assert(K % 2 == 0, "the exchanges of a layer start with the real parts");
+    extern __shared__ __align__(16) unsigned char fq_smem_1[];
+    R *lds = reinterpret_cast<R *>(fq_smem_1);
+    const int t = threadIdx.x;
+    int sb[K + 1], soff = 0;
+#pragma unroll
+    for (int l = 0; l <= K; ++l)
+        sb[l] = 0;
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        const int on = (t >> k) & 1;
+        soff |= on << Lay::p(K, k);
+#pragma unroll
+        for (int l = 0; l <= K; ++l)
+            sb[l] += on * Lay::w(Lay::p(l, k));
+    }
+    T v[N];
+    if (a.first) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            v[j].x = (R)a.init_amp;
+            v[j].y = 0;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            v[j] = sv[t + (j << NT)];
+    }
+    const uint32_t gates = a.gates_w;
+    auto cost = [&](int p) {
+        const double2 *tab = ptab + a.table[p], *thr = tab + (Q + 1);
+        const double2 f_row = tab[(t & 63) % (Q + 1)], f_thr = thr[t];
+        mix_cost<T, R, Q, A, false>(v, f_row, f_thr, thr, thr + ((1 + A) << NT), a.has_rr, a.scale_re[p], a.scale_im[p], t);
+    };
+    bool up = true;
+    for (int p = 0; p < a.P; ++p, up = !up) {
+        cost(p);
+        if (up)
+            mix_up<Lay, T, R, A, K, 0, 0, -1>(v, lds, sb, gates, (R)a.t[p]);
+        else
+            mix_down<Lay, T, R, A, K, K, 0, -1>(v, lds, sb, gates, (R)a.t[p]);
+    }
+    if (up) {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            sv[t + (j << NT)] = v[j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+            sv[soff + (j << Lay::start(K))] = v[j];
+    }
+}
+
+template <typename R, int Q, int A>
+static hipError_t launch_solo_q(void *sv, const SoloArgs &a, const double2 *ptab, hipStream_t stream)
+{
+    constexpr int K = 2;
+    constexpr size_t lds = sizeof(R) * (size_t)MixLay<R, Q, A, K>::slots();
+    static_assert(lds <= 65536, "static limit of dynamic LDS");
+    hipLaunchKernelGGL((k_solo<R, Q, A, K>), dim3(1), dim3(1u << (Q - A)), lds, stream,
+                       reinterpret_cast<typename CT<R>::T *>(sv), a, ptab);
+    return hipGetLastError();
 }
 
 // ---- launchers ---------------------------------------------------------------

@@ -40,4 +40,18 @@ bool mix_lane_bit(int Q, int A, int k)
     return k > 0 && (b == 4 || b == 3 || b == 1 || b == 0);
 }
 
+hipError_t launch_solo_c128(int N, void *sv, const SoloArgs &a, const double2 *ptab, hipStream_t stream);
+
+hipError_t launch_solo(int dtype, int N, void *sv, const SoloArgs &a, const double2 *ptab, hipStream_t stream)
+{
+    if (dtype == 0)
+        return launch_solo_c128(N, sv, a, ptab, stream);
+    switch (N) {
+        case 12: return launch_solo_q<float, 12, 4>(sv, a, ptab, stream);
+        case 11: return launch_solo_q<float, 11, 4>(sv, a, ptab, stream);
+        case 10: return launch_solo_q<float, 10, 4>(sv, a, ptab, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 }  // namespace fq
