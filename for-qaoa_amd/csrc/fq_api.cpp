@@ -491,24 +491,17 @@ static std::string geom_key(const Geom &g)
 }
 
 // RX groups: gate bits among the thread bits, a_log per LDS phase.
-// lane_swap: thread bits 4 and 5 (gated) are exchanged with register bits 1
-// and 0 by cross-lane swaps and get their RX there; the LDS phases take the
-// other gated thread bits.
-static int set_gates(TileArgs &a, const Geom &g, uint32_t gate_mask, bool lane_swap = false)
+static int set_gates(TileArgs &a, const Geom &g, uint32_t gate_mask)
 {
     a.gate_mask = gate_mask;
-    a.lane_swap = lane_swap ? 1u : 0u;
-    // gated thread bits, lowest first: the last LDS phase gets the highest
-    // ones, so that it usually holds none of the six lane bits and the tile
-    // can be stored straight from its layout (direct_store)
+    // gated thread bits, lowest first
     std::vector<int> pend;
     for (int i = 0; i < g.nthr; ++i)
-        if (((gate_mask >> i) & 1u) && !(lane_swap && (i == 4 || i == 5)))
+        if ((gate_mask >> i) & 1u)
             pend.push_back(i);
     a.ngroups = 0;
     a.grp_mask_w = 0;
     a.grp_gates_w = 0;
-    a.direct_store = 0;
     size_t pos = 0;
     while (pos < pend.size()) {
         if (a.ngroups >= FQ_MAX_GROUPS)
@@ -538,14 +531,6 @@ static int set_gates(TileArgs &a, const Geom &g, uint32_t gate_mask, bool lane_s
             a.grp_mask_w |= (uint64_t)gm << (16 * a.ngroups);
         a.grp_gates_w |= (uint32_t)(gg & 0x1f) << (5 * a.ngroups);
         a.ngroups++;
-    }
-    a.dpos_w = 0;
-    if (a.ngroups > 0 && g.nthr >= 6 && (a.grp_mask[a.ngroups - 1] & 0x3f) == 0) {
-        a.direct_store = 1;
-        // register r of the last phase is its r-th lowest tile bit
-        for (int i = 0, r = 0; i < g.Q; ++i)
-            if ((a.grp_mask[a.ngroups - 1] >> i) & 1u)
-                a.dpos_w |= (uint32_t)g.tpos[i] << (6 * r++);
     }
     return FQ_OK;
 }
@@ -808,64 +793,11 @@ static int check_state(const fq_state *st)
     return FQ_OK;
 }
 
-// FQ_WIDE_REGS=0 (environment, read per call): the contiguous 14-qubit
-// complex64 tile passes always run 1024 threads x 16 amplitudes (tile_a_log).
-static bool wide_regs()
-{
-    const char *e = getenv("FQ_WIDE_REGS");
-    return e ? atoi(e) != 0 : true;
-}
-
-// Register bits per thread of a packed slab pass.
-static int slab_a_log(int dtype, int Q)
+// Register bits per thread of a general tile pass.
+static int tile_a_log(int dtype, int Q)
 {
     const int want = dtype == FQ_C128 ? 3 : 4;
     return std::max(1, std::min(want, Q));
-}
-
-// Register bits per thread of a tile pass.  The contiguous full-width
-// complex64 tile (qubits 0..13, 128 KiB of LDS) can run 512 threads x 32
-// amplitudes instead of 1024 x 16: five register bits per LDS phase, and the
-// 256 VGPRs of a 512-thread group hold the 32 amplitudes plus the next tile's
-// prefetch.  It is used where it needs fewer LDS phases than four bits would
-// (N=34: RX on qubits 4..13 in one phase instead of two, one of them half
-// filler), which measured on MI355X: boundary pass 61.6 -> 55.6 ms, plain
-// 48.4 -> 47.1 ms, layer-0 pass 37 -> 34 ms, 8.27 -> 8.39 layers/s.  With the
-// same number of phases the wider tile only adds filler butterflies and
-// halves the waves per CU (N=30: 130.2 vs 127.9 layers/s), and the strided
-// tiles measured slower with it (N=34 plain strided pass 55.4 -> 60.5 ms).
-// Only the write-only layer-0 pass (first) keeps it where qubits 4 and 5 are
-// gated: at 1024 x 16 the layer-boundary pass then gets their RX by lane
-// swaps and needs one LDS phase, and the other passes drop the half-filled
-// last phase's filler butterflies; N=34 boundary pass 0 57.3-58.3 -> 50.8 ms,
-// plain pass 0 46.9 -> 45.6 ms, while the layer-0 pass at 1024 x 16 took
-// 35.5 ms against 33.6-34.2.
-static int tile_a_log(int dtype, const std::vector<int> &tile, const std::vector<int> &gates, bool first = false)
-{
-    const int Q = (int)tile.size();
-    bool low = true;
-    for (int i = 0; i < Q; ++i)
-        low = low && tile[i] == i;
-    if (dtype == FQ_C64 && Q == 14 && low && wide_regs()) {
-        // gated thread bits (tile position = qubit here) and the LDS phases they need
-        int g4 = 0, g5 = 0;
-        bool l4 = false, l5 = false;
-        for (int q : gates) {
-            g4 += q < 10;
-            g5 += q < 9;
-            l4 = l4 || q == 4;
-            l5 = l5 || q == 5;
-        }
-        if ((g5 + 4) / 5 < (g4 + 3) / 4 && (first || !(l4 && l5)))
-            return 5;
-    }
-    // the complex128 write-only layer-0 pass as 512 threads x 16 amplitudes
-    // (183 VGPRs, no prefetch to hold): its RX on qubits 5..12 takes one LDS
-    // phase of four register bits instead of two of three; N=30 3.55-3.62 ->
-    // 2.88 ms (5.96 TB/s written), 68.9-69.1 -> 69.5-69.6 layers/s
-    if (dtype == FQ_C128 && Q == 13 && low && first && wide_regs())
-        return 4;
-    return slab_a_log(dtype, Q);
 }
 
 extern "C" int fq_state_create(int N, int D, int B, int C, int dtype, fq_state **out)
@@ -1190,10 +1122,11 @@ enum { Z2_OFF = 0, Z2_LOWER = 1, Z2_MIRROR = 2, Z2_EXPAND = 3 };
 // Launch arguments of one tile pass of an N-qubit state: tile positions
 // (thread bits first), RX gate positions and the half-state mode.
 static int pass_args(int N, int dtype, const std::vector<int> &tile, const std::vector<int> &gates, bool cost,
-                     int z2, TileArgs &a, Geom &geom, int a_log_override = 0, bool first = false)
+                     int z2, TileArgs &a, Geom &geom, int a_log = 0)
 {
     const int Q = (int)tile.size();
-    const int a_log = a_log_override > 0 ? a_log_override : tile_a_log(dtype, tile, gates, first);
+    if (a_log == 0)
+        a_log = tile_a_log(dtype, Q);
     geom = make_geom(N, tile, a_log);
     if (geom_runs(geom) > FQ_MAX_RUNS)
         return set_err(FQ_ERR_ARG, "internal: tile geometry needs more than %d bit runs", FQ_MAX_RUNS);
@@ -1518,20 +1451,9 @@ static int tile_pass(fq_state *st, const std::vector<int> &tile, const std::vect
         return set_err(FQ_ERR_ARG, "internal: no mirror boundary pass at this tile width");
     TileArgs a;
     Geom geom;
-    if (int rc = pass_args(st->N, st->dtype, tile, gates, cost, z2, a, geom, 0, first))
+    if (int rc = pass_args(st->N, st->dtype, tile, gates, cost, z2, a, geom))
         return rc;
     const int a_log = geom.a_log;
-    // complex64 layer-boundary passes on 1024 x 16 tiles whose lane bits 4
-    // and 5 are gated: RX on those two by swaps between lanes and registers,
-    // one LDS phase fewer (at least one must remain: the pass applies its
-    // cost phase in the last phase's layout)
-    if (st->dtype == FQ_C64 && a_log == 4 && geom.Q == 14 && z2 < Z2_MIRROR && pre_beta &&
-        ((a.gate_mask >> 4) & 3u) == 3u) {
-        uint32_t rest = a.gate_mask & ((1u << geom.nthr) - 1u) & ~0x30u;
-        if (rest != 0)
-            if (int rc = set_gates(a, geom, a.gate_mask, true))
-                return rc;
-    }
     // the pass's factor: sigma^(#gates) per RX set, times what is pending
     double sr = st->pending_re, si = st->pending_im;
     auto absorb = [&](double b, double *t) {
@@ -1678,7 +1600,7 @@ static std::vector<FusedPass> cover_passes(int N, int Qmax, int dtype, int bound
             std::vector<int> &nw = news[k2];
             std::sort(nw.begin(), nw.end());
             const int c = Qmax - want[k2];
-            const int a_log = slab_a_log(dtype, Qmax);
+            const int a_log = tile_a_log(dtype, Qmax);
             // lane order: the 64 lanes of a wave are the tile's first six
             // positions; past the carriers they take the pass's lowest new
             // qubits whose byte-address bit is outside [19, hi] (one load
@@ -1708,7 +1630,7 @@ static std::vector<FusedPass> cover_passes(int N, int Qmax, int dtype, int bound
                 if (std::find(lane_q.begin(), lane_q.end(), q) == lane_q.end())
                     p.tile.push_back(q);
             p.gates = nw;
-            fits = fits && geom_runs(make_geom(N, p.tile, slab_a_log(dtype, Qmax))) <= FQ_MAX_RUNS;
+            fits = fits && geom_runs(make_geom(N, p.tile, tile_a_log(dtype, Qmax))) <= FQ_MAX_RUNS;
             more.push_back(p);
         }
         if (fits || blk >= rest) {
@@ -1783,7 +1705,7 @@ static int rx_targets_once(fq_state *st, std::vector<int> targets, double beta)
                 if (std::find(chunk.begin(), chunk.end(), p) == chunk.end())
                     tile.push_back(p);
             std::sort(tile.begin(), tile.end());
-            const int a_log = tile_a_log(st->dtype, tile, chunk);
+            const int a_log = tile_a_log(st->dtype, (int)tile.size());
             if (chunk.size() == 1 || geom_runs(make_geom(N, tile, a_log)) <= FQ_MAX_RUNS)
                 break;
             chunk.pop_back();  // scattered targets: fewer per pass
@@ -3418,7 +3340,7 @@ static int slab_qe(const fq_slab *sb) { return std::min(12, sb->z2 ? sb->N - 1 :
 static TileArgs slab_cost_args(const fq_slab *sb, Geom *gout)
 {
     const int Q1 = (int)sb->passes[0].tile.size();
-    Geom g1 = make_geom(sb->N, sb->passes[0].tile, slab_a_log(sb->dtype, Q1));
+    Geom g1 = make_geom(sb->N, sb->passes[0].tile, tile_a_log(sb->dtype, Q1));
     TileArgs a1;
     geom_to_args(g1, a1);
     if (sb->z2)
@@ -3474,7 +3396,7 @@ static int slab_build_args(fq_slab *sb)
         const FusedPass &ps = sb->passes[i];
         const int Q = (int)ps.tile.size();
         SlabPass sp;
-        sp.a_log = slab_a_log(sb->dtype, Q);
+        sp.a_log = tile_a_log(sb->dtype, Q);
         sp.mirror = sb->z2 && i + 1 == sb->passes.size();
         std::vector<int> tile = ps.tile;
         if (sp.mirror)
@@ -3535,13 +3457,9 @@ static int slab_make_views(fq_slab *sb)
         } else {
             Geom geom;
             const int z2 = !sb->z2 ? Z2_OFF : i + 1 < m ? Z2_LOWER : Z2_MIRROR;
-            // pass 0 runs as the write-only layer-0 pass too, possibly with
-            // another register width (tile_a_log)
-            for (int first = 0; first <= (i == 0 ? 1 : 0); ++first) {
-                if (int rc = pass_args(sb->N, sb->dtype, lp.ps[i].tile, lp.ps[i].gates, true, z2, a, geom, 0, first != 0))
-                    return rc;
-                most = std::max(most, phase_table_entries(a, geom.a_log));
-            }
+            if (int rc = pass_args(sb->N, sb->dtype, lp.ps[i].tile, lp.ps[i].gates, true, z2, a, geom))
+                return rc;
+            most = phase_table_entries(a, geom.a_log);
         }
         need += most * sizeof(double2);
     }

@@ -75,34 +75,9 @@ __device__ __forceinline__ void rx_registers_t(T *v, unsigned mask, R t)
     }
 }
 
-// RX on register bits 0..K-1 only (compile time): the last LDS phase of a
-// pass whose gated bits are its K lowest register bits, the others filling
-// the phase, runs no identity butterflies on the fillers.
-template <typename T, typename R, int A_LOG, int K>
-__device__ __forceinline__ void rx_registers_low(T *v, R t)
-{
-    constexpr int A = 1 << A_LOG;
-#pragma unroll
-    for (int r = 0; r < K; ++r) {
-#pragma unroll
-        for (int j = 0; j < A; ++j)
-            if (!((j >> r) & 1))
-                rx_pair_t<T, R>(v[j], v[j | (1 << r)], t);
-    }
-}
-
-// Exchange of a wave's lanes 32..63 of a with lanes 0..31 of b
-// (v_permlane32_swap): for a pair of registers a = v[j], b = v[j | 2^r]
-// this exchanges lane bit 5 with register bit r.
-__device__ __forceinline__ void lane_xchg32(float &a, float &b)
-{
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-    a = __uint_as_float(r[0]);
-    b = __uint_as_float(r[1]);
-}
-
-// The same for lane bit 4 (v_permlane16_swap: the odd 16-lane rows of a
-// with the even rows of b).
+// Exchange of a wave's odd 16-lane rows of a with the even rows of b
+// (v_permlane16_swap): for a pair of registers a = v[j], b = v[j | 2^r] this
+// exchanges lane bit 4 with register bit r.
 __device__ __forceinline__ void lane_xchg16(float &a, float &b)
 {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);

@@ -194,8 +194,8 @@ __device__ __forceinline__ void mix_natural(T (&v)[1 << A_LOG], const TileArgs &
 // Persistent tile pass.  Each work-group walks tiles blockIdx.x,
 // blockIdx.x + gridDim.x, ...; while a tile goes through its cost phase and
 // LDS phases, the next tile's amplitudes are already loading into registers.
-// QT > 0 fixes the tile width at compile time (the fused passes' full-width
-// tiles); QT == 0 reads it from the arguments.
+// QT > 0 fixes the tile width at compile time (the cost phase alone); QT == 0
+// reads it from the arguments: tiles below the widths of fq_mix.h.
 // PRE: the pass that ends one layer and opens the next applies RX of the
 // previous layer (pre_t) on the same gate positions before the cost phase
 // (COST, not FIRST, MIRROR 0 only).
@@ -204,22 +204,8 @@ __device__ __forceinline__ void mix_natural(T (&v)[1 << A_LOG], const TileArgs &
 // passes that left theirs pending) as a.scale_re + i a.scale_im, which a cost
 // pass folds into its FP64 phase factor and a pass without the cost phase
 // multiplies in before its stores when a.apply_scale is set.
-// KL > 0: the last LDS phase's gated bits are its KL lowest register bits
-// (the host launches this instance only then), and its RX runs on those
-// alone instead of running identity butterflies on the filler bits.
-// LS (the complex64 layer-boundary pass at 1024 x 16, a.lane_swap): thread
-// bits 4 and 5, both gated, are exchanged with register bits 1 and 0 by
-// v_permlane16_swap / v_permlane32_swap right after the natural layout's RX,
-// get their RX there, and go to the LDS in that exchanged layout; the LDS
-// phases take the other gated thread bits, and after the second RX set the
-// swaps bring the natural layout back for the stores.  At N=34 that turns
-// the strided boundary pass's two LDS phases (4 + 2 bits) into one (strided
-// boundary pass 65.6 -> 58.3 ms).  The plain passes do not use it: with
-// their last phase's registers on other qubits their direct stores measured
-// far slower (N=34 plain strided pass 51.2 -> 75.6 ms).
-template <typename R, int A_LOG, int QT, bool COST, bool FIRST, bool GATES, int MIRROR = 0, bool PRE = false,
-          int KL = 0, bool LS = false>
-__global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LOG >= 4) ? 512 : 1024) : 256)
+template <typename R, int A_LOG, int QT, bool COST, bool FIRST, bool GATES, int MIRROR = 0, bool PRE = false>
+__global__ void __launch_bounds__(GATES ? 1024 : 256)
     k_tile(typename CT<R>::T *__restrict__ sv, const TileArgs a, const double2 *__restrict__ ptab)
 {
     typedef typename CT<R>::T T;
@@ -245,35 +231,12 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
     // per-thread LDS slots of every remapping phase (padded), once per launch;
     // lds_pad is additive over disjoint bit sets: pad(x | y) = pad(x) + pad(y)
     int etp[MAXG];
-    const int nat = LS ? lds_pad((t & ~0x30) | (((t >> 5) & 1) << (QT - A_LOG)) | (((t >> 4) & 1) << (QT - A_LOG + 1)))
-                       : lds_pad(t);
+    const int nat = lds_pad(t);
     if (GATES) {
         const unsigned qmask = (1u << Q) - 1u;
 #pragma unroll
         for (int g = 0; g < MAXG; ++g)
             etp[g] = g < a.ngroups ? lds_pad(deposit<QT>(t, qmask & ~(unsigned)a.grp_mask[g], Q)) : 0;
-    }
-    // Direct store: when the last LDS phase holds none of the six lane bits,
-    // the tile is stored straight from that phase's registers (no write-back
-    // and re-read of the natural layout).  Element e of the tile lives at
-    // tile_base + phys(e); phys is additive over disjoint bits: the thread's
-    // part (pe_last) is computed once per launch, the part of each register
-    // (the phase's register bits sit at the positions packed in a.dpos_w) at
-    // the stores, as reg_offsets does for the natural layout.
-    // (full-width tiles only, and not in the read-write cost passes, whose
-    // registers are full with the prefetch and the phase factors)
-    const bool direct = GATES && MIRROR == 0 && QT > 0 && (FIRST || !COST) && a.direct_store && a.ngroups > 0;
-    uint64_t pe_last = 0;
-    if (direct) {
-        const unsigned qmask = (1u << Q) - 1u;
-        const unsigned gm = (unsigned)a.grp_mask[a.ngroups - 1];
-        const unsigned tmask = (1u << nthr) - 1u;
-        const unsigned et = (unsigned)deposit<QT>(t, qmask & ~gm, Q);
-        pe_last = unpack_runs((uint64_t)(et & tmask), a.truns);
-#pragma unroll
-        for (int r = 0; r < A_LOG; ++r)
-            if ((et >> (nthr + r)) & 1u)
-                pe_last |= 1ull << a.rpos[r];
     }
     const uint64_t q1 = (uint64_t)Q + 1;
     const double2 *thr_tab = COST ? ptab + (ntiles * q1) : nullptr;
@@ -288,17 +251,9 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
     // bytes per lane, and both passes fit their 128 VGPRs without spills
     // when they read the row with scalar loads instead)
     constexpr bool ROWPF = COST && QT > 0 && !(sizeof(R) == 4 && !FIRST);
-    // When the next tile's loads are issued (measured on MI355X; a tile's
-    // loads and the previous tile's stores issued back to back left the
-    // memory pipe idle through the compute between them):
-    // * the complex64 boundary pass at 1024 threads issues half of them
-    //   before its cost phase and half after it (N=34: strided boundary
-    //   pass 72.5 -> 66.2 ms, 8.31 -> 8.56 layers/s);
-    // * the passes without the cost phase issue them after their first LDS
-    //   phase instead of at the top of the iteration (N=34 c64 8.58 -> 8.82
-    //   layers/s, N=30 c64 130.2 -> 131.7, half state 247 -> 250; complex128
-    //   unchanged).
-    constexpr bool SPLITPF = PRE && sizeof(R) == 4 && A_LOG == 4;
+    // the passes without the cost phase issue the next tile's loads after their
+    // first LDS phase: issued back to back with the previous tile's stores they
+    // left the memory idle through the compute between them
     constexpr bool LATEPF = !COST;
     const int row_lane = (t & 63) % (QT + 1);
     double2 fcur = make_double2(0.0, 0.0), fnext = make_double2(0.0, 0.0);
@@ -405,27 +360,6 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
         };
         T w[A];
         // the next tile's loads (issued after the cost phase: few registers live)
-        // registers [j0, j1) of the next tile (part of prefetch)
-        auto prefetch_part = [&](int j0, int j1) {
-            if (ROWPF && j0 == 0 && next < ntiles)
-                fnext = ptab[next * q1 + row_lane];
-            if (!FIRST && next < ntiles) {
-                uint64_t roff[A];
-                reg_offsets<A, NB>(rpos_w, roff);
-                const T *p1 = sv + (tile_base(a, next) + toff);
-#pragma unroll
-                for (int j = 0; j < AH; ++j)
-                    if (j >= j0 && j < j1)
-                        w[j] = p1[roff[j]];
-                if (MIRROR && j1 > AH) {
-                    const T *pm = sv + (tile_base(a, ~next & hmask) + a.mirror_pm - toff);
-#pragma unroll
-                    for (int j = AH; j < A; ++j)
-                        if (j >= j0 && j < j1)
-                            w[j] = pm[-(int64_t)roff[j - AH]];
-                }
-            }
-        };
         auto prefetch = [&]() {
             if (ROWPF && next < ntiles)
                 fnext = ptab[next * q1 + row_lane];
@@ -478,64 +412,25 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
                 lds_opaque(eg);
             rx_registers_t<T, R, A_LOG>(v, group_gates(a, g), tt);
         };
-        // the last LDS phase of a KL instance
-        auto phase_read_last = [&](int g, int &eg, R tt) {
-            eg = phase_slots(g);
-#pragma unroll
-            for (int j = 0; j < A; ++j)
-                v[j] = lds[eg + ej[j]];
-            if (COST && sizeof(R) == 4)
-                lds_opaque(eg);
-            rx_registers_low<T, R, A_LOG, (KL > 0 ? KL : A_LOG)>(v, tt);
-        };
         auto phase_write = [&](int eg) {
 #pragma unroll
             for (int j = 0; j < A; ++j)
                 lds[eg + ej[j]] = v[j];
             lds_barrier();
         };
-        // LS: element (t, j) of the exchanged layout is tile element
-        // (t without bits 4, 5) | t4 << (nthr + 1) | t5 << nthr | j0 << 5 |
-        // j1 << 4 | (j >> 2) << (nthr + 2); lds_pad is additive over disjoint
-        // bits, so the thread's part (nat) and register j's (a constant) add
-        auto reg_slot = [&](int j) -> int {
-            if constexpr (LS)
-                return lds_pad(((j & 1) << 5) | (((j >> 1) & 1) << 4) | ((j >> 2) << (QT - A_LOG + 2)));
-            else
-                return lds_pad(j << nthr);
-        };
         auto natural_write = [&]() {
             // own slots: the previous tile's final read used the same slots,
             // so no barrier is needed before this write
 #pragma unroll
             for (int j = 0; j < A; ++j)
-                lds[nat + reg_slot(j)] = v[j];
+                lds[nat + lds_pad(j << nthr)] = v[j];
             lds_barrier();
         };
         auto natural_read = [&]() {
 #pragma unroll
             for (int j = 0; j < A; ++j)
-                v[j] = lds[nat + reg_slot(j)];
+                v[j] = lds[nat + lds_pad(j << nthr)];
         };
-        // LS: exchange thread bit 5 with register bit 0 and thread bit 4 with
-        // register bit 1 (each swap is its own inverse, and the two commute)
-        auto lane_swap = [&]() {
-            if constexpr (LS) {
-#pragma unroll
-                for (int j = 0; j < A; ++j)
-                    if (!(j & 1)) {
-                        lane_xchg32(v[j].x, v[j | 1].x);
-                        lane_xchg32(v[j].y, v[j | 1].y);
-                    }
-#pragma unroll
-                for (int j = 0; j < A; ++j)
-                    if (!(j & 2)) {
-                        lane_xchg16(v[j].x, v[j | 2].x);
-                        lane_xchg16(v[j].y, v[j | 2].y);
-                    }
-            }
-        };
-
         if constexpr (PRE && sizeof(R) == 4) {
             // complex64 layer-boundary pass: RX(pre) through its LDS phases, the cost
             // phase applied in the last phase's layout (with the phase table
@@ -547,42 +442,21 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
             const R pt = a.pre_tf, rt = a.rx_tf;
             const int G = a.ngroups;
             rx_registers_t<T, R, A_LOG>(v, a.gate_mask >> nthr, pt);
-            if constexpr (LS) {
-                lane_swap();
-                rx_registers_low<T, R, A_LOG, 2>(v, pt);
-            }
             int eg = 0;
             if (G > 0) {
                 natural_write();
-                if constexpr (KL > 0) {
 #pragma unroll 1
-                    for (int g = 0; g + 1 < G; ++g) {
-                        phase_read_rx(g, eg, pt);
-                        phase_write(eg);
-                    }
-                    phase_read_last(G - 1, eg, pt);
-                } else {
-#pragma unroll 1
-                    for (int g = 0; g < G; ++g) {
-                        phase_read_rx(g, eg, pt);
-                        if (g + 1 == G)
-                            break;
-                        phase_write(eg);
-                    }
+                for (int g = 0; g < G; ++g) {
+                    phase_read_rx(g, eg, pt);
+                    if (g + 1 == G)
+                        break;
+                    phase_write(eg);
                 }
             }
-            if constexpr (SPLITPF)
-                prefetch_part(0, A / 2);
             apply_cost();
-            if constexpr (SPLITPF)
-                prefetch_part(A / 2, A);
-            else
-                prefetch();
+            prefetch();
             if (G > 0) {
-                if constexpr (KL > 0)
-                    rx_registers_low<T, R, A_LOG, KL>(v, rt);
-                else
-                    rx_registers_t<T, R, A_LOG>(v, group_gates(a, G - 1), rt);
+                rx_registers_t<T, R, A_LOG>(v, group_gates(a, G - 1), rt);
                 eg = phase_slots(G - 1);
                 phase_write(eg);
 #pragma unroll 1
@@ -591,10 +465,6 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
                     phase_write(eg);
                 }
                 natural_read();
-            }
-            if constexpr (LS) {
-                rx_registers_low<T, R, A_LOG, 2>(v, rt);
-                lane_swap();
             }
             rx_registers_t<T, R, A_LOG>(v, a.gate_mask >> nthr, rt);
         } else {
@@ -607,8 +477,7 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
                 apply_cost();
             if (!LATEPF)
                 prefetch();
-            // LATEPF: after the first LDS phase's write-back, or after the
-            // RX where that phase is stored directly or there is none
+            // LATEPF: after the first LDS phase's write-back, or after the RX
             bool pf_left = LATEPF;
             auto prefetch_rest = [&]() {
                 if (LATEPF && pf_left) {
@@ -624,38 +493,14 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
                     // rolled loop: unrolling lets the compiler hoist every
                     // phase's addresses out of the tile loop and spill
                     int eg = 0;
-                    if constexpr (KL > 0) {
-                        const int G = a.ngroups;
 #pragma unroll 1
-                        for (int g = 0; g + 1 < G; ++g) {
-                            phase_read_rx(g, eg, rt);
-                            phase_write(eg);
-                            if (g == 0)
-                                prefetch_rest();
-                        }
-                        // (KL instances run with two or more phases: the
-                        // loads went out after the first)
-                        phase_read_last(G - 1, eg, rt);
-                        if (!direct)
-                            phase_write(eg);
-                    } else {
-#pragma unroll 1
-                        for (int g = 0; g < a.ngroups; ++g) {
-                            phase_read_rx(g, eg, rt);
-                            if (direct && g == a.ngroups - 1)
-                                break;
-                            phase_write(eg);
-                            if (g == 0)
-                                prefetch_rest();
-                        }
+                    for (int g = 0; g < a.ngroups; ++g) {
+                        phase_read_rx(g, eg, rt);
+                        phase_write(eg);
+                        if (g == 0)
+                            prefetch_rest();
                     }
-                    if (direct) {
-                        // every thread has read its last-phase elements before
-                        // the next tile's first LDS writes
-                        lds_barrier();
-                    } else {
-                        natural_read();
-                    }
+                    natural_read();
                 }
             }
             prefetch_rest();
@@ -667,14 +512,7 @@ __global__ void __launch_bounds__(GATES ? (A_LOG >= 5 || (sizeof(R) == 8 && A_LO
                 cmul_by(v[j], (R)a.scale_re, (R)a.scale_im);
         }
 
-        if (direct) {
-            uint64_t doff[A];
-            reg_offsets<A, A_LOG>(a.dpos_w, doff);
-            T *const ps = sv + (tile_base(a, tile) + pe_last);
-#pragma unroll
-            for (int j = 0; j < A; ++j)
-                ps[doff[j]] = v[j];
-        } else {
+        {
             uint64_t roff[A];
             reg_offsets<A, NB>(rpos_w, roff);
             T *const p0 = sv + (tile_base(a, tile) + toff);
@@ -1195,15 +1033,14 @@ int occupancy_per_cu(const void *fn, int threads, size_t lds)
     return per_cu;
 }
 
-template <typename R, int A_LOG, int QT, bool COST, bool FIRST, bool GATES, bool PRE = false, int KL = 0,
-          bool LS = false>
+template <typename R, int A_LOG, int QT, bool COST, bool FIRST, bool GATES, bool PRE = false>
 static hipError_t launch_tile_t(void *sv, const TileArgs &a, const double2 *ptab, hipStream_t stream)
 {
     typedef typename CT<R>::T T;
     const unsigned threads = 1u << a.nthr;
     const uint64_t tiles = run_tiles(a);
     const size_t lds = GATES && a.ngroups > 0 ? tile_lds_bytes(sizeof(R) == 8 ? 0 : 1, a.Q) : 0;
-    const void *fn = reinterpret_cast<const void *>(&k_tile<R, A_LOG, QT, COST, FIRST, GATES, 0, PRE, KL, LS>);
+    const void *fn = reinterpret_cast<const void *>(&k_tile<R, A_LOG, QT, COST, FIRST, GATES, 0, PRE>);
     if (lds > 65536) {
         if (hipError_t e = allow_large_lds(fn))
             return e;
@@ -1216,19 +1053,19 @@ static hipError_t launch_tile_t(void *sv, const TileArgs &a, const double2 *ptab
     TileArgs la = a;
     if (la.order == 1 && grid % 8 != 0)
         la.order = 0;
-    hipLaunchKernelGGL((k_tile<R, A_LOG, QT, COST, FIRST, GATES, 0, PRE, KL, LS>), dim3((unsigned)grid), dim3(threads),
+    hipLaunchKernelGGL((k_tile<R, A_LOG, QT, COST, FIRST, GATES, 0, PRE>), dim3((unsigned)grid), dim3(threads),
                        lds, stream, reinterpret_cast<T *>(sv), la, ptab);
     return hipGetLastError();
 }
 
-template <typename R, int A_LOG, int QT, int MIRROR>
+template <typename R, int A_LOG, int MIRROR>
 static hipError_t launch_mirror_m(void *sv, const TileArgs &a, hipStream_t stream)
 {
     typedef typename CT<R>::T T;
     const unsigned threads = 1u << a.nthr;
     const uint64_t tiles = a.ntiles_run;
     const size_t lds = a.ngroups > 0 ? tile_lds_bytes(sizeof(R) == 8 ? 0 : 1, a.Q) : 0;
-    const void *fn = reinterpret_cast<const void *>(&k_tile<R, A_LOG, QT, false, false, true, MIRROR>);
+    const void *fn = reinterpret_cast<const void *>(&k_tile<R, A_LOG, 0, false, false, true, MIRROR>);
     if (lds > 65536) {
         if (hipError_t e = allow_large_lds(fn))
             return e;
@@ -1239,15 +1076,15 @@ static hipError_t launch_mirror_m(void *sv, const TileArgs &a, hipStream_t strea
     TileArgs la = a;
     if (la.order == 1 && grid % 8 != 0)
         la.order = 0;
-    hipLaunchKernelGGL((k_tile<R, A_LOG, QT, false, false, true, MIRROR>), dim3((unsigned)grid), dim3(threads),
+    hipLaunchKernelGGL((k_tile<R, A_LOG, 0, false, false, true, MIRROR>), dim3((unsigned)grid), dim3(threads),
                        lds, stream, reinterpret_cast<T *>(sv), la, nullptr);
     return hipGetLastError();
 }
 
-template <typename R, int A_LOG, int QT>
+template <typename R, int A_LOG>
 static hipError_t launch_mirror_t(bool expand, void *sv, const TileArgs &a, hipStream_t stream)
 {
-    return expand ? launch_mirror_m<R, A_LOG, QT, 2>(sv, a, stream) : launch_mirror_m<R, A_LOG, QT, 1>(sv, a, stream);
+    return expand ? launch_mirror_m<R, A_LOG, 2>(sv, a, stream) : launch_mirror_m<R, A_LOG, 1>(sv, a, stream);
 }
 
 hipError_t launch_tile_mirror(int dtype, int a_log, bool expand, void *sv, const TileArgs &a, hipStream_t stream)
@@ -1255,24 +1092,18 @@ hipError_t launch_tile_mirror(int dtype, int a_log, bool expand, void *sv, const
     if (a.ntiles_run == 0)
         return hipErrorInvalidValue;
     if (dtype == 0) {
-        if (a_log == 3 && a.Q == 13)
-            return launch_mirror_t<double, 3, 13>(expand, sv, a, stream);
         switch (a_log) {
-            case 1: return launch_mirror_t<double, 1, 0>(expand, sv, a, stream);
-            case 2: return launch_mirror_t<double, 2, 0>(expand, sv, a, stream);
-            case 3: return launch_mirror_t<double, 3, 0>(expand, sv, a, stream);
+            case 1: return launch_mirror_t<double, 1>(expand, sv, a, stream);
+            case 2: return launch_mirror_t<double, 2>(expand, sv, a, stream);
+            case 3: return launch_mirror_t<double, 3>(expand, sv, a, stream);
             default: return hipErrorInvalidValue;
         }
     }
-    if (a_log == 5 && a.Q == 14)
-        return launch_mirror_t<float, 5, 14>(expand, sv, a, stream);
-    if (a_log == 4 && a.Q == 14)
-        return launch_mirror_t<float, 4, 14>(expand, sv, a, stream);
     switch (a_log) {
-        case 1: return launch_mirror_t<float, 1, 0>(expand, sv, a, stream);
-        case 2: return launch_mirror_t<float, 2, 0>(expand, sv, a, stream);
-        case 3: return launch_mirror_t<float, 3, 0>(expand, sv, a, stream);
-        case 4: return launch_mirror_t<float, 4, 0>(expand, sv, a, stream);
+        case 1: return launch_mirror_t<float, 1>(expand, sv, a, stream);
+        case 2: return launch_mirror_t<float, 2>(expand, sv, a, stream);
+        case 3: return launch_mirror_t<float, 3>(expand, sv, a, stream);
+        case 4: return launch_mirror_t<float, 4>(expand, sv, a, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1287,30 +1118,15 @@ static hipError_t launch_cost_only(bool first, void *sv, const TileArgs &a, cons
                  : launch_tile_t<R, A_LOG, QT, true, false, false>(sv, a, ptab, stream);
 }
 
-// The last LDS phase gates its two lowest register bits only (the complex64
-// strided passes' 14 = 4 + 4 + 4 + 2 and 10 = 4 + 4 + 2 gates): the KL = 2
-// instances skip the butterflies of its two filler bits (N=34 complex64:
-// strided boundary pass 67.9 -> 64.8 ms, plain strided pass 52.5 -> 50.8 ms).
-static bool last_phase_low2(const TileArgs &a)
-{
-    return a.ngroups >= 2 && a.grp_gates[a.ngroups - 1] == 3u;
-}
-
 // Gated passes, with or without the cost phase.
-template <typename R, int A_LOG, int QT>
+template <typename R, int A_LOG>
 static hipError_t launch_gated(bool cost, bool first, void *sv, const TileArgs &a, const double2 *ptab,
                                hipStream_t stream)
 {
-    if (!cost) {
-        if (a.lane_swap)
-            return hipErrorInvalidValue;
-        if constexpr (sizeof(R) == 4 && A_LOG == 4 && QT == 14)
-            if (last_phase_low2(a))
-                return launch_tile_t<R, A_LOG, QT, false, false, true, false, 2>(sv, a, ptab, stream);
-        return launch_tile_t<R, A_LOG, QT, false, false, true>(sv, a, ptab, stream);
-    }
-    return first ? launch_tile_t<R, A_LOG, QT, true, true, true>(sv, a, ptab, stream)
-                 : launch_tile_t<R, A_LOG, QT, true, false, true>(sv, a, ptab, stream);
+    if (!cost)
+        return launch_tile_t<R, A_LOG, 0, false, false, true>(sv, a, ptab, stream);
+    return first ? launch_tile_t<R, A_LOG, 0, true, true, true>(sv, a, ptab, stream)
+                 : launch_tile_t<R, A_LOG, 0, true, false, true>(sv, a, ptab, stream);
 }
 
 template <typename R>
@@ -1328,36 +1144,16 @@ static hipError_t launch_tile_r(int a_log, bool cost, bool first, bool gates, vo
             default: return hipErrorInvalidValue;
         }
     }
-    // compile-time tile widths for the full-width tiles of the fused passes;
-    // anything else takes the generic instance.  Register bits per thread:
-    // up to 3 for complex128, 4 for complex64 (5 in the 14-qubit tiles).
-    if constexpr (sizeof(R) == 8) {
-        if (a_log == 3 && a.Q == 13)
-            return launch_gated<R, 3, 13>(cost, first, sv, a, ptab, stream);
-        if (a_log == 4 && a.Q == 13 && cost && first)
-            return launch_tile_t<R, 4, 13, true, true, true>(sv, a, ptab, stream);
-        if (a_log == 3 && a.Q == 12)
-            return launch_gated<R, 3, 12>(cost, first, sv, a, ptab, stream);
-        switch (a_log) {
-            case 1: return launch_gated<R, 1, 0>(cost, first, sv, a, ptab, stream);
-            case 2: return launch_gated<R, 2, 0>(cost, first, sv, a, ptab, stream);
-            case 3: return launch_gated<R, 3, 0>(cost, first, sv, a, ptab, stream);
-            default: return hipErrorInvalidValue;
-        }
-    } else {
-        if (a_log == 5 && a.Q == 14)
-            return launch_gated<R, 5, 14>(cost, first, sv, a, ptab, stream);
-        if (a_log == 4 && a.Q == 14)
-            return launch_gated<R, 4, 14>(cost, first, sv, a, ptab, stream);
-        if (a_log == 4 && a.Q == 13)
-            return launch_gated<R, 4, 13>(cost, first, sv, a, ptab, stream);
-        switch (a_log) {
-            case 1: return launch_gated<R, 1, 0>(cost, first, sv, a, ptab, stream);
-            case 2: return launch_gated<R, 2, 0>(cost, first, sv, a, ptab, stream);
-            case 3: return launch_gated<R, 3, 0>(cost, first, sv, a, ptab, stream);
-            case 4: return launch_gated<R, 4, 0>(cost, first, sv, a, ptab, stream);
-            default: return hipErrorInvalidValue;
-        }
+    // register bits per thread: up to 3 for complex128, 4 for complex64
+    switch (a_log) {
+        case 1: return launch_gated<R, 1>(cost, first, sv, a, ptab, stream);
+        case 2: return launch_gated<R, 2>(cost, first, sv, a, ptab, stream);
+        case 3: return launch_gated<R, 3>(cost, first, sv, a, ptab, stream);
+        case 4:
+            if constexpr (sizeof(R) == 4)
+                return launch_gated<R, 4>(cost, first, sv, a, ptab, stream);
+            return hipErrorInvalidValue;
+        default: return hipErrorInvalidValue;
     }
 }
 
@@ -1374,23 +1170,6 @@ hipError_t launch_tile(int dtype, int a_log, bool cost, bool first, bool gates, 
 template <typename R>
 static hipError_t launch_pre_r(int a_log, void *sv, const TileArgs &a, const double2 *ptab, hipStream_t stream)
 {
-    if constexpr (sizeof(R) == 8) {
-        if (a_log == 3 && a.Q == 13)
-            return launch_tile_t<R, 3, 13, true, false, true, true>(sv, a, ptab, stream);
-        if (a_log == 3 && a.Q == 12)
-            return launch_tile_t<R, 3, 12, true, false, true, true>(sv, a, ptab, stream);
-    } else {
-        if (a_log == 5 && a.Q == 14)
-            return launch_tile_t<R, 5, 14, true, false, true, true>(sv, a, ptab, stream);
-        if (a_log == 4 && a.Q == 14) {
-            if (a.lane_swap)
-                return launch_tile_t<R, 4, 14, true, false, true, true, 0, true>(sv, a, ptab, stream);
-            return last_phase_low2(a) ? launch_tile_t<R, 4, 14, true, false, true, true, 2>(sv, a, ptab, stream)
-                                      : launch_tile_t<R, 4, 14, true, false, true, true>(sv, a, ptab, stream);
-        }
-        if (a_log == 4 && a.Q == 13)
-            return launch_tile_t<R, 4, 13, true, false, true, true>(sv, a, ptab, stream);
-    }
     switch (a_log) {
         case 1: return launch_tile_t<R, 1, 0, true, false, true, true>(sv, a, ptab, stream);
         case 2: return launch_tile_t<R, 2, 0, true, false, true, true>(sv, a, ptab, stream);
