@@ -241,10 +241,10 @@ static void lane_give(const Lane &l)
 // ---- handles -------------------------------------------------------------------
 
 struct PlanEntry {
-    void *dmem = nullptr;
-    size_t cap = 0;               // bytes of dmem and staging
+    char *dmem = nullptr;         // in a block of the graph, as staging
+    size_t cap = 0;               // bytes of both
     PlanDev dev{};
-    void *staging = nullptr;      // pinned copy of the blob (asynchronous upload)
+    char *staging = nullptr;      // pinned copy of the blob (asynchronous upload)
     hipEvent_t ready = nullptr;   // upload done
     hipStream_t stream = nullptr; // stream the upload was queued on
     std::vector<hipStream_t> users; // streams the plan was handed to
@@ -252,16 +252,13 @@ struct PlanEntry {
     uint64_t last_use = 0;        // fq_graph::use_clock at the last lookup
 };
 
-// Releases a plan's memory; the caller has synchronized the device (hipFree
-// waits for the whole device anyway).
-static void plan_free(PlanEntry &e)
-{
-    hipFree(e.dmem);
-    hipHostFree(e.staging);
-    if (e.ready)
-        hipEventDestroy(e.ready);
-    e = PlanEntry();
-}
+// Memory of a graph's plans: device and pinned memory in blocks (a pinned
+// allocation for each plan took 30 us and more, and a slab's graph has five plans).
+#define FQ_PLAN_BLOCK ((size_t)64 << 10)
+struct PlanBlock {
+    char *dmem = nullptr, *staging = nullptr;
+    size_t used = 0, size = 0;
+};
 
 // Plans cached per graph; beyond this the least recently used plan's buffers
 // are reused for the next one.
@@ -272,10 +269,48 @@ struct fq_graph {
     std::vector<double> W;  // N*N, W[min*N+max], current labels
     // key: tile geometry + the bytes of W, so a hit is an exact content match
     std::map<std::string, PlanEntry> plans;
+    std::vector<PlanBlock> blocks;
     uint64_t version = 1;       // bumped by every change of W
     uint64_t plan_epoch = 0;    // bumped when a cached plan is dropped or reused
     uint64_t use_clock = 0;
 };
+
+// Drops all plans of a graph; the caller has synchronized the device (hipFree
+// waits for the whole device anyway).
+static void plans_free(fq_graph *G)
+{
+    for (auto &kv : G->plans)
+        if (kv.second.ready)
+            hipEventDestroy(kv.second.ready);
+    G->plans.clear();
+    for (PlanBlock &b : G->blocks) {
+        hipFree(b.dmem);
+        hipHostFree(b.staging);
+    }
+    G->blocks.clear();
+}
+
+// cap bytes of both memories for a plan, from the last block or a new one.
+static bool plan_memory(fq_graph *G, size_t cap, PlanEntry &e)
+{
+    if (G->blocks.empty() || G->blocks.back().size - G->blocks.back().used < cap) {
+        PlanBlock b;
+        b.size = std::max(cap, FQ_PLAN_BLOCK);
+        if (hipMalloc(&b.dmem, b.size) != hipSuccess)
+            return false;
+        if (hipHostMalloc(&b.staging, b.size, hipHostMallocDefault) != hipSuccess) {
+            hipFree(b.dmem);
+            return false;
+        }
+        G->blocks.push_back(b);
+    }
+    PlanBlock &b = G->blocks.back();
+    e.dmem = b.dmem + b.used;
+    e.staging = b.staging + b.used;
+    e.cap = cap;
+    b.used += cap;
+    return true;
+}
 
 struct TimingRec {
     int kind;
@@ -726,9 +761,7 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
             // every cached plan is smaller than this one: drop them all (rare;
             // hipFree waits for the device in any case)
             FQ_HIP(hipDeviceSynchronize());
-            for (auto &kv : G->plans)
-                plan_free(kv.second);
-            G->plans.clear();
+            plans_free(G);
         } else {
             pe = victim->second;
             G->plans.erase(victim);
@@ -755,12 +788,10 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
         size_t cap = 4096;
         while (cap < total)
             cap *= 2;
-        pe.cap = cap;
-        if (hipMalloc(&pe.dmem, cap) != hipSuccess ||
-            hipHostMalloc(&pe.staging, cap, hipHostMallocDefault) != hipSuccess ||
-            hipEventCreateWithFlags(&pe.ready, hipEventDisableTiming) != hipSuccess) {
+        if (hipEventCreateWithFlags(&pe.ready, hipEventDisableTiming) != hipSuccess || !plan_memory(G, cap, pe)) {
             hipGetLastError();
-            plan_free(pe);
+            if (pe.ready)
+                hipEventDestroy(pe.ready);
             return set_err(FQ_ERR_OOM, "plan allocation of %zu bytes failed", cap);
         }
     }
@@ -770,7 +801,7 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
         hipEventRecord(pe.ready, stream) != hipSuccess) {
         hipGetLastError();
         hipStreamSynchronize(stream);
-        plan_free(pe);
+        hipEventDestroy(pe.ready);   // (its memory stays with the graph)
         return set_err(FQ_ERR_DEVICE, "plan upload failed");
     }
     const PlanDev dev = place_plan(pb, (char *)pe.dmem);
@@ -993,10 +1024,9 @@ extern "C" int fq_graph_destroy(fq_graph *g)
 {
     if (!g)
         return FQ_OK;
-    if (!g->plans.empty()) {
+    if (!g->blocks.empty()) {
         hipDeviceSynchronize();
-        for (auto &kv : g->plans)
-            plan_free(kv.second);
+        plans_free(g);
     }
     delete g;
     return FQ_OK;
@@ -3319,10 +3349,8 @@ static void slab_free(fq_slab *sb)
     hipFree(sb->d_step);
     hipHostFree(sb->h_step);
     hipFree(sb->d_plans);
-    hipHostFree(sb->h_plans);
     hipFree(sb->d_tabs);
     hipFree(sb->d_part);
-    hipHostFree(sb->h_res);
     if (sb->done)
         hipEventDestroy(sb->done);
     if (sb->stream) {
@@ -3568,13 +3596,13 @@ extern "C" int fq_slab_create_sched(int N, int nslots, int dtype, int schedule, 
         slab_free(sb);
         return set_err(FQ_ERR_OOM, "slab allocation of %zu bytes failed", (size_t)(((size_t)1 << N) * (dtype == FQ_C128 ? 16 : 8) * nslots));
     }
+    // one pinned allocation: a step's parameters, the plans, the results
+    const size_t o_plans = (step_bytes(nslots) + 63) & ~(size_t)63, o_res = o_plans + sizeof(SlotPlans) * nslots;
     ok = hipMalloc(&sb->d_step, step_bytes(nslots)) == hipSuccess &&
-         hipHostMalloc(&sb->h_step, step_bytes(nslots), hipHostMallocDefault) == hipSuccess &&
+         hipHostMalloc(&sb->h_step, o_res + sizeof(double) * 2 * nslots, hipHostMallocDefault) == hipSuccess &&
          hipMalloc(&sb->d_plans, sizeof(SlotPlans) * nslots) == hipSuccess &&
-         hipHostMalloc(&sb->h_plans, sizeof(SlotPlans) * nslots, hipHostMallocDefault) == hipSuccess &&
          hipMalloc(&sb->d_tabs, sizeof(double2) * sb->tab_stride * nslots) == hipSuccess &&
          hipMalloc(&sb->d_part, sizeof(double) * 2 * etiles) == hipSuccess &&
-         hipHostMalloc(&sb->h_res, sizeof(double) * 2 * nslots, hipHostMallocDefault) == hipSuccess &&
          hipStreamCreateWithFlags(&sb->stream, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&sb->done, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
@@ -3590,6 +3618,8 @@ extern "C" int fq_slab_create_sched(int N, int nslots, int dtype, int schedule, 
             return rc;
         }
     memset(sb->h_step, 0, step_bytes(nslots));
+    sb->h_plans = (SlotPlans *)(sb->h_step + o_plans);
+    sb->h_res = (double *)(sb->h_step + o_res);
     *out = sb;
     return FQ_OK;
 }
