@@ -1229,6 +1229,12 @@ static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const do
 // or more, its table's launch is under 2% of it.
 #define FQ_TABLES_BYTES ((size_t)8 << 20)
 
+// The memory-side cache: 256 MiB.
+#define FQ_CACHE_LOG 28
+#define FQ_CACHE_BYTES ((size_t)1 << FQ_CACHE_LOG)
+
+static int carriers_for(int dtype);
+
 // A tile pass on the compile-time kernel (fq_mix.hip), ready to launch over
 // all its tiles or a range of them.
 struct MixPass {
@@ -1366,6 +1372,14 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
         a.has_rr = ca.has_rr;
         a.init_amp = st->init_amp;
     }
+    // runs of 128 B from HBM: neighbouring tiles, which share DRAM pages, on one XCD.
+    // Per layer on MI355X, N=34 complex64 fused 125 -> 104 ms (8 ranges of tiles
+    // instead of 64: 102), N=33 complex128 122 -> 101; RX on the top 10 qubits at
+    // N=34 113 -> 71 (8 ranges 113); no difference at N=30 complex128.
+    int carried = 0;
+    while (carried < (int)tile.size() && tile[carried] == carried)
+        ++carried;
+    a.by_xcd = carried <= carriers_for(st->dtype) && a.ntiles >= 2048 && st->bytes > FQ_CACHE_BYTES;
     mp.cost = cost;
     mp.kind = boundary ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
     mp.mir = z2 == Z2_MIRROR ? 1 : z2 == Z2_EXPAND ? 2 : 0;
@@ -1986,7 +2000,6 @@ static std::vector<FusedPass> split_three(int N, int Q, int n1, int A, bool (*la
 // 12.80 and 13.07 ms with 7, 8, 9 and 10; N=32 complex64 30.6, 30.6, 27.9 and
 // 29.0; half state N=30 complex128 7.62, 6.79, 6.66 and 6.88.  Where the plan
 // of tuning knobs is asked for, layer_plan's passes run as they are.
-#define FQ_CACHE_LOG 28
 static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
 {
     LayerPlan lp = layer_plan(N, dtype, z2);
@@ -2017,7 +2030,12 @@ static LayerPlan exec_plan(int N, int dtype, bool z2, int P)
         return lp;
     const int Q = tile_max_q(dtype);
     const int n1 = split_low(N, Q, dtype, 9);
-    if (n1 == 0)
+    // A pass 2 that carries no more than 128 B runs (complex64 from N=33, complex128
+    // from N=32) has 1,024 of them, each in another region of 2^22 amplitudes or
+    // more: such a boundary pass took 113 ms at N=34 complex64 (58 with the qubits
+    // dealt out as layer_plan does).  Per layer there, split 136 ms, dealt out 102;
+    // N=33 56.3 and 54.3.
+    if (n1 == 0 || N - Q - n1 == Q - carriers_for(dtype))
         return lp;
     lp.ps = split_three(N, Q, n1, mix_a_log(dtype, Q), mix_lane_bit);
     lp.end1 = 2;
@@ -2111,6 +2129,7 @@ static MixArgs chunk_args(const MixArgs &whole, uint64_t c, int nlog)
     MixArgs a = whole;
     a.ntiles >>= nlog;
     a.tile0 = c * a.ntiles;
+    a.by_xcd = 0;   // (cached)
     return a;
 }
 

@@ -112,6 +112,7 @@ struct MixArgs {
     double scale_re, scale_im;  // factor of the pass: in the cost phase, or before the
     int apply_scale;            // stores (apply_scale)
     double init_amp;
+    int by_xcd;              // tile order (a multiple of 64 tiles)
     const MixSlot *slots;    // packed launch (blockIdx.y: the slot), else null
     int nslots;
 };

@@ -201,7 +201,10 @@ __global__ void __launch_bounds__(1 << (Q - A), 4)
     const double2 *thr_tab = COST ? ptab + a.ntab * q1 : nullptr;
     const double2 *rr_tab = COST ? thr_tab + ((size_t)(1 + A) << NT) : nullptr;
 
-    const uint64_t tile = a.tile0 + blockIdx.x;
+    // by_xcd: work-groups go round the 8 XCDs in turn; an XCD takes consecutive
+    // tiles from 8 of 64 ranges
+    const uint32_t b = blockIdx.x;
+    const uint64_t tile = a.tile0 + (a.by_xcd ? (b & 63u) * (gridDim.x >> 6) + (b >> 6) : b);
     const uint64_t base = unpack_runs_uniform(tile, a.hruns);
     // cost phase: the tile's row of the table, entry i in lane i (broadcast by
     // readlane), and the thread's entry, loaded ahead of the amplitudes
