@@ -354,7 +354,7 @@ def main():
     traffic = traffic_from_profiles() if args.workload == "n30_gnp05" and args.dtype == "c128" else None
     roof = dict(bound="hbm", achieved=dom.get("gbs"), peak=HBM_PEAK_GBS, unit="GB/s",
                 frac=(dom.get("gbs") or 0) / HBM_PEAK_GBS, traffic=traffic,
-                kernel=("k_tile (fused tile pass: cost phase + RX through LDS)" if dom_name == "fused"
+                kernel=("k_mix (fused tile pass: cost phase + RX through LDS)" if dom_name == "fused"
                         else "k_tile (cost phase)"),
                 bytes_per_launch=dom.get("bytes_per_launch"), avg_launch_ms=dom.get("avg_ms"))
     if stream and stream.get("inplace_gbs"):
