@@ -194,10 +194,13 @@ static bool is_own_stream(hipStream_t s)
 struct Lane {
     hipStream_t stream = nullptr;
     double *host = nullptr;
+    bool shared = false;   // host is one of g_pages
     int device = -1;
 };
 static std::mutex g_lanes_mu;
 static std::vector<Lane> g_lanes;
+static std::vector<double *> g_pages;   // free ones of the first FQ_LANES, allocated together
+static bool g_pages_made = false;
 
 static bool lane_take(Lane &l)
 {
@@ -216,6 +219,22 @@ static bool lane_take(Lane &l)
     l.device = dev;
     if (hipStreamCreateWithFlags(&l.stream, hipStreamNonBlocking) != hipSuccess)
         return false;
+    {
+        std::lock_guard<std::mutex> lk(g_lanes_mu);
+        double *m = nullptr;
+        if (!g_pages_made &&
+            hipHostMalloc(&m, sizeof(double) * FQ_LANE_DOUBLES * FQ_LANES, hipHostMallocPortable) == hipSuccess) {
+            g_pages_made = true;
+            for (int i = 0; i < FQ_LANES; ++i)
+                g_pages.push_back(m + (size_t)FQ_LANE_DOUBLES * i);
+        }
+        if (!g_pages.empty()) {
+            l.host = g_pages.back();
+            l.shared = true;
+            g_pages.pop_back();
+            return true;
+        }
+    }
     if (hipHostMalloc(&l.host, sizeof(double) * FQ_LANE_DOUBLES, hipHostMallocDefault) != hipSuccess) {
         hipStreamDestroy(l.stream);
         l.stream = nullptr;
@@ -233,9 +252,12 @@ static void lane_give(const Lane &l)
             g_lanes.push_back(l);
             return;
         }
+        if (l.shared)
+            g_pages.push_back(l.host);
     }
     hipStreamDestroy(l.stream);
-    hipHostFree(l.host);
+    if (!l.shared)
+        hipHostFree(l.host);
 }
 
 // ---- handles -------------------------------------------------------------------
@@ -1235,7 +1257,7 @@ static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const do
 
 static int carriers_for(int dtype);
 
-// A tile pass on the compile-time kernel (fq_mix.hip), ready to launch over
+// A tile pass on the compile-time kernel (fq_mix.h), ready to launch over
 // all its tiles or a range of them.
 struct MixPass {
     MixArgs a;
@@ -3280,7 +3302,7 @@ struct SlotHost {
     int has_rr[4] = {0, 0, 0, 0};
 };
 
-// One pass of a packed slab on the compile-time kernel (fq_mix.hip): its
+// One pass of a packed slab on the compile-time kernel (fq_mix.h): its
 // launch arguments without the slots' factors.
 struct PackedPass {
     MixArgs a;

@@ -82,7 +82,7 @@ struct TileArgs {
     PlanDev plan;
 };
 
-// One pass of the compile-time tile kernel (fq_mix.hip).
+// One pass of the compile-time tile kernel (fq_mix.h).
 enum { MIX_PLAIN = 0, MIX_FIRST = 1, MIX_COST = 2, MIX_BOUNDARY = 3 };
 // The same of a pair pass of the gradient (fq_pair.hip).
 enum { PAIR_PLAIN = 0, PAIR_COST = 1, PAIR_BOUNDARY = 2 };
@@ -223,7 +223,7 @@ hipError_t launch_tile(int dtype, int a_log, bool cost, bool first, bool gates, 
 // Layer-boundary pass: RX(pre) on the pass's qubits, cost phase, RX(rx).
 hipError_t launch_tile_pre(int dtype, int a_log, void *sv, const TileArgs &a, const double2 *ptab,
                            hipStream_t stream);
-// Tile passes of fq_mix.hip.  mix_a_log: register bits per thread of its
+// Tile passes of fq_mix.h.  mix_a_log: register bits per thread of its
 // instance for tiles of 2^Q amplitudes (0: none).  k: exchanges one way (they
 // reach the tile bits from Q - (k + 1) A up), lane: RX also on the bit below
 // those, where mix_lane_bit says there is such an instance; kind MIX_*, mir:

@@ -14,12 +14,12 @@
 //            Register bits are butterflied in registers; the other gate bits
 //            are remapped into registers through padded LDS phases.
 //            Replaces _rotationCompressionWeighted_conti (src/rzz.cu:121-156)
-//            and _multirotateX_unroll (src/rx.cu:56-87).
+//            and, at widths that fq_mix.h has no instance of,
+//            _multirotateX_unroll (src/rx.cu:56-87).
 //  k_exchange
-//            in-place qubit-block exchange [out,out+k) <-> [in,in+k);
-//            replaces _swap_gate_conti (src/swap.cu:76-102) without the
-//            host-built pair table: 2^t x 2^t sub-tiles are transposed
-//            through LDS so both sides are read and written coalesced.
+//            in-place exchange of qubit pairs; replaces _swap_gate_conti
+//            (src/swap.cu:76-102) without the host-built pair table: tiles are
+//            permuted through LDS so both sides are read and written coalesced.
 //  k_expect / k_finalize   <C> and sum|psi|^2, FP64, fixed reduction order.
 //  k_topk    per-block top-16 candidates (bitonic sort in LDS).
 #include "fq_device.h"
