@@ -283,7 +283,7 @@ struct PlanBlock {
 };
 
 // Plans cached per graph; beyond this the least recently used plan's buffers
-// are reused for the next one.
+// are reused for the next one, unless it is held (PlanHold).
 #define FQ_PLAN_CACHE 64
 
 struct fq_graph {
@@ -295,6 +295,27 @@ struct fq_graph {
     uint64_t version = 1;       // bumped by every change of W
     uint64_t plan_epoch = 0;    // bumped when a cached plan is dropped or reused
     uint64_t use_clock = 0;
+    int holds = 0;              // PlanHold's alive
+    uint64_t held_from = 0;     // use_clock when the first of them was made
+};
+
+// While one is alive, plans of the graph that get_plan hands out stay as they are: for
+// a caller that looks up several plans before it launches what reads the first.
+struct PlanHold {
+    fq_graph *g;
+    explicit PlanHold(fq_graph *graph) : g(graph)
+    {
+        if (g->holds++ == 0)
+            g->held_from = g->use_clock;
+    }
+    PlanHold(PlanHold &&o) noexcept : g(o.g) { o.g = nullptr; }
+    PlanHold(const PlanHold &) = delete;
+    PlanHold &operator=(const PlanHold &) = delete;
+    ~PlanHold()
+    {
+        if (g)
+            --g->holds;
+    }
 };
 
 // Drops all plans of a graph; the caller has synchronized the device (hipFree
@@ -741,8 +762,12 @@ static PlanDev place_plan(const PlanBlob &pb, char *base)
 // are large enough is replaced: `stream` first waits (on the device, through
 // an event) for the work queued so far on every stream that plan was handed
 // to, so no launch still reading it sees the new contents, and the host
-// blocks on nothing but that plan's own earlier upload.
-static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream)
+// blocks on nothing but that plan's own earlier upload.  A held plan is not
+// replaced; if all that are large enough are held, the cache grows by the new one
+// (at most by the plans of one holder: they are the next one's to replace).
+// entry, if not null, receives the plan's entry, which lives until the graph's
+// plan_epoch changes.
+static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream, PlanEntry **entry = nullptr)
 {
     std::string key = geom_key(g);
     key.append(reinterpret_cast<const char *>(G->W.data()), G->W.size() * sizeof(double));
@@ -767,6 +792,8 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
             }
         }
         *out = e.dev;
+        if (entry)
+            *entry = &e;
         return FQ_OK;
     }
     PlanBlob pb;
@@ -776,15 +803,22 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
     bool reused = false;
     if (G->plans.size() >= FQ_PLAN_CACHE) {
         auto victim = G->plans.end();
-        for (auto v = G->plans.begin(); v != G->plans.end(); ++v)
+        bool held = false;
+        for (auto v = G->plans.begin(); v != G->plans.end(); ++v) {
+            if (G->holds > 0 && v->second.last_use > G->held_from) {
+                held = true;
+                continue;
+            }
             if (v->second.cap >= total && (victim == G->plans.end() || v->second.last_use < victim->second.last_use))
                 victim = v;
-        if (victim == G->plans.end()) {
+        }
+        if (victim == G->plans.end() && !held) {
             // every cached plan is smaller than this one: drop them all (rare;
             // hipFree waits for the device in any case)
             FQ_HIP(hipDeviceSynchronize());
             plans_free(G);
-        } else {
+            G->plan_epoch++;
+        } else if (victim != G->plans.end()) {
             pe = victim->second;
             G->plans.erase(victim);
             reused = true;
@@ -803,8 +837,8 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
             }
             pe.users.clear();
             pe.foreign = false;
+            G->plan_epoch++;
         }
-        G->plan_epoch++;
     }
     if (!reused) {
         size_t cap = 4096;
@@ -834,6 +868,8 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
     ne = pe;
     note_user(ne);
     *out = dev;
+    if (entry)
+        *entry = &ne;
     return FQ_OK;
 }
 
@@ -2178,6 +2214,7 @@ static size_t chunk_group(const LayerPlan &lp, const std::vector<Step> &seq, siz
 static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, int p1, int P, const double *gammas,
                       const double *betas, bool z2, bool expand)
 {
+    const PlanHold hold(g);   // the passes' plans, until their tables are queued
     const std::vector<FusedPass> &ps = lp.ps;
     const int m = (int)ps.size();
     std::vector<Step> seq;
@@ -2266,6 +2303,7 @@ static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, cons
         if (getenv(k))
             return FQ_OK;
     *done = true;
+    const PlanHold hold(g);
     const std::vector<int> tile = low_tile(N);
     const int A = mix_a_log(st->dtype, N);
     for (int p0 = 0; p0 < P; p0 += FQ_SOLO_LAYERS) {
@@ -2705,6 +2743,7 @@ static LayerPlan pair_plan(int N, int dtype)
 static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, const double *gammas, const double *betas,
                      double *out, double *expect, double *grad_gammas, double *grad_betas)
 {
+    const PlanHold hold(g);
     const int N = st->N, m = (int)lp.ps.size(), Q = (int)lp.ps[0].tile.size(), A = pair_a_log(st->dtype, Q);
     std::vector<Step> seq;
     for (int p = 0; p < P; ++p)
@@ -3299,6 +3338,7 @@ struct SlotHost {
     bool fresh = false;       // not yet in device memory
     uint64_t gversion = 0;    // g->version the plans belong to
     uint64_t gepoch = 0;      // g->plan_epoch the plan pointers belong to
+    PlanEntry *entries[5] = {nullptr};   // of the plans, while that is the graph's epoch
     int has_rr[4] = {0, 0, 0, 0};
 };
 
@@ -3558,15 +3598,17 @@ static int slab_make_views(fq_slab *sb)
 // Cost and <C> plans of a slot's graph (again after the graph changed).
 static int slab_slot_plans(fq_slab *sb, SlotHost &h)
 {
+    const PlanHold hold(h.g);   // (so that none of them replaces another)
     for (int i = 0; i < (sb->packed ? 4 : 1); ++i) {
-        if (int rc = get_plan(h.g, sb->packed ? sb->pk_geom[i] : sb->cost_geom, &h.plans.cost[i], sb->stream))
+        if (int rc = get_plan(h.g, sb->packed ? sb->pk_geom[i] : sb->cost_geom, &h.plans.cost[i], sb->stream,
+                              &h.entries[i]))
             return rc;
         h.has_rr[i] = 0;
         for (int j = 0; j < FQ_MAX_REGS; ++j)
             if (h.plans.cost[i].rr[j] != 0)
                 h.has_rr[i] = 1;
     }
-    if (int rc = get_plan(h.g, sb->exp_geom, &h.plans.expect, sb->stream))
+    if (int rc = get_plan(h.g, sb->exp_geom, &h.plans.expect, sb->stream, &h.entries[4]))
         return rc;
     h.fresh = true;
     h.gversion = h.g->version;
@@ -3831,16 +3873,28 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
         sb->pending = false;
     }
     const int K = sb->K;
+    // the slots' plans stay until the step is queued: the passes of large slots look
+    // up plans of their own, and <C> comes after them
+    std::vector<PlanHold> holds;
+    for (const SlotHost &h : sb->slots)
+        if (h.phase == 1)
+            holds.emplace_back(h.g);
     // refresh plans of changed graphs; a refresh can release a graph's plan
     // cache, so repeat until every active slot's plans are current
     for (bool again = true; again;) {
         again = false;
         for (int k = 0; k < K; ++k) {
             SlotHost &h = sb->slots[k];
-            if (h.phase == 1 && slab_slot_stale(h)) {
+            if (h.phase != 1)
+                continue;
+            if (slab_slot_stale(h)) {
                 if (int rc = slab_slot_plans(sb, h))
                     return rc;
                 again = true;
+            } else {
+                for (PlanEntry *e : h.entries)
+                    if (e)
+                        e->last_use = ++h.g->use_clock;
             }
         }
     }

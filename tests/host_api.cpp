@@ -1,0 +1,346 @@
+// host_api.cpp -- fq_api.cpp on the CPU: device memory is host memory, copies
+// happen at once, and the launchers look at their arguments instead of launching.
+// So what the host side hands to the kernels can be checked without a GPU:
+//
+//   plans   every cost plan that a launch reads, when it is launched, is a plan of the
+//           graph as it then is (build_plan's bytes), and lies in live memory.
+//
+// Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
+#include <hip/hip_runtime.h>
+#define __align__(n) __attribute__((aligned(n)))
+#define HIP_SYMBOL(x) (&x)
+
+#include "fq_api.cpp"
+
+#include <sys/mman.h>
+
+// ---- device memory and streams --------------------------------------------------
+
+static std::map<char *, size_t> g_live;   // device and pinned allocations
+static std::vector<char *> g_freed;       // (kept, poisoned: a late read is seen, not undefined)
+
+static bool live(const void *p, size_t n)
+{
+    auto it = g_live.upper_bound((char *)p);
+    if (it == g_live.begin())
+        return false;
+    --it;
+    return (char *)p >= it->first && (char *)p + n <= it->first + it->second;
+}
+
+static hipError_t take(void **p, size_t n)
+{
+    // (a state's pages are never touched)
+    void *m = mmap(nullptr, n, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+    if (m == MAP_FAILED)
+        return hipErrorOutOfMemory;
+    g_live[(char *)m] = n;
+    *p = m;
+    return hipSuccess;
+}
+
+static hipError_t give(void *p)
+{
+    auto it = g_live.find((char *)p);
+    if (it == g_live.end())
+        return p ? hipErrorInvalidValue : hipSuccess;
+    if (it->second <= (size_t)64 << 20)
+        memset(p, 0xff, it->second);
+    g_live.erase(it);
+    return hipSuccess;
+}
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n); }
+hipError_t hipFree(void *p) { return give(p); }
+hipError_t hipHostFree(void *p) { return give(p); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t)
+{
+    memset(d, v, n);
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d)
+{
+    *d = 0;
+    return hipSuccess;
+}
+static hipError_t handle(void **h)
+{
+    static size_t n = 0;
+    *h = (void *)(16 * ++n);
+    return hipSuccess;
+}
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle((void **)s); }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { return handle((void **)e); }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return handle((void **)e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
+{
+    *ms = 1.0f;
+    return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipGetSymbolAddress(void **p, const void *s)
+{
+    *p = (void *)s;
+    return hipSuccess;
+}
+}
+
+// ---- plans ------------------------------------------------------------------------
+
+static fq_graph *g_graph = nullptr;        // the graph of the program
+static std::vector<Geom> g_geoms;          // the geometries its launches may use
+static long g_checked = 0, g_wrong = 0;
+
+template <typename T> static bool same(const PlanBlob &pb, size_t o, const T *at, size_t n)
+{
+    return n == 0 || (live(at, n * sizeof(T)) && memcmp(at, pb.bytes.data() + o, n * sizeof(T)) == 0);
+}
+
+// Whether p holds the plan of the graph for a geometry with these widths.
+static bool plan_ok(const PlanDev &p, int Q, int nthr, int nh)
+{
+    for (const Geom &g : g_geoms) {
+        if (g.Q != Q || g.nthr != nthr || g.nh != nh)
+            continue;
+        PlanBlob pb;
+        build_plan(g_graph, g, pb);
+        const int nnz = ((const int *)(pb.bytes.data() + pb.o_off))[Q];
+        // (the scalars, which the caller holds, tell geometries of equal widths apart)
+        if (pb.dev.n_hh == p.n_hh && pb.dev.wtot == p.wtot && memcmp(pb.dev.rr, p.rr, sizeof(p.rr)) == 0 &&
+            same(pb, pb.o_cH, p.cH, Q) && same(pb, pb.o_om, p.omega, nh) && same(pb, pb.o_off, p.csr_off, Q + 1) &&
+            same(pb, pb.o_ch, p.csr_h, nnz) && same(pb, pb.o_cw, p.csr_w, nnz) && same(pb, pb.o_hw, p.hh_w, p.n_hh) &&
+            same(pb, pb.o_hu, p.hh_u, p.n_hh) && same(pb, pb.o_hv, p.hh_v, p.n_hh) &&
+            same(pb, pb.o_thr, p.thr, (size_t)(1 + g.a_log) << nthr))
+            return true;
+    }
+    return false;
+}
+
+static void check(const PlanDev &p, int Q, int nthr, int nh)
+{
+    ++g_checked;
+    if (!plan_ok(p, Q, nthr, nh))
+        ++g_wrong;
+}
+
+// ---- launchers ----------------------------------------------------------------------
+
+namespace fq {
+int tile_max_q(int dtype) { return dtype == 0 ? 13 : 14; }
+size_t tile_lds_bytes(int, int) { return 0; }
+int mix_a_log(int dtype, int Q)
+{
+    if (dtype == 0)
+        return Q >= 10 && Q <= 13 ? 4 : Q == 9 ? 3 : 0;
+    return Q == 13 || Q == 14 ? 5 : Q >= 10 && Q <= 12 ? 4 : 0;
+}
+bool mix_lane_bit(int Q, int A, int k)
+{
+    const int b = Q - A - k * A - 1;
+    return k > 0 && (b == 4 || b == 3 || b == 1 || b == 0);
+}
+int pair_a_log(int dtype, int Q)
+{
+    if (dtype == 0)
+        return Q >= 9 && Q <= 12 ? 3 : 0;
+    return Q >= 10 && Q <= 13 ? 4 : 0;
+}
+bool pair_lane_bit(int Q, int A, int k)
+{
+    const int b = Q - A - k * A - 1;
+    return k > 0 && (b == 3 || b == 1 || b == 0);
+}
+size_t phase_table_entries(const TileArgs &a, int a_log)
+{
+    return (size_t)run_tiles(a) * (size_t)(a.Q + 1) + ((size_t)(1 + a_log) << a.nthr) + FQ_MAX_REGS;
+}
+hipError_t launch_phase_table(const TileArgs &a, int, double2 *, double *, hipStream_t)
+{
+    check(a.plan, a.Q, a.nthr, a.nh);
+    return hipSuccess;
+}
+hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t, double2 *, double *, hipStream_t)
+{
+    for (int j = 0; j < njobs; ++j) {
+        const TableGeo &g = m.geo[m.job[j].geo];
+        check(g.plan, g.Q, g.nthr, g.nh);
+    }
+    return hipSuccess;
+}
+hipError_t launch_slab_phase_table(const TileArgs &a, int, const SlotParams *slots, const SlotPlans *plans, int nslots,
+                                   double2 *, size_t, hipStream_t)
+{
+    for (int k = 0; k < nslots; ++k)
+        if (slots[k].active)
+            check(plans[k].cost[0], a.Q, a.nthr, a.nh);
+    return hipSuccess;
+}
+hipError_t launch_slab_tables(const SlabGeos &g, const SlabJob *jobs, int njobs, size_t, const SlotPlans *plans,
+                              double2 *, hipStream_t)
+{
+    for (int j = 0; j < njobs; ++j) {
+        const TableGeo &t = g.geo[jobs[j].geo];
+        check(plans[jobs[j].slot].cost[jobs[j].geo], t.Q, t.nthr, t.nh);
+    }
+    return hipSuccess;
+}
+hipError_t launch_slab_expect(int, int a_log, const void *, const TileArgs &a, const SlotPlans *plans, const int *fin,
+                              int nfin, int slot_shift, double *, double *, hipStream_t)
+{
+    for (int i = 0; i < nfin; ++i)
+        check(plans[fin[i]].expect, a.Q, a.Q - a_log, g_graph->N - a.Q);
+    (void)slot_shift;
+    return hipSuccess;
+}
+hipError_t launch_expect(int, int, const void *, const TileArgs &a, double *, unsigned *, double *, hipStream_t)
+{
+    check(a.plan, a.Q, a.nthr, a.nh);
+    return hipSuccess;
+}
+hipError_t launch_cut_mul(int, int, const void *, void *, const TileArgs &a, double *, hipStream_t)
+{
+    check(a.plan, a.Q, a.nthr, a.nh);
+    return hipSuccess;
+}
+hipError_t launch_tile(int, int, bool, bool, bool, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
+hipError_t launch_tile_pre(int, int, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
+hipError_t launch_tile_mirror(int, int, bool, void *, const TileArgs &, hipStream_t) { return hipSuccess; }
+hipError_t launch_mix(int, int, bool, int, int, void *, const MixArgs &, const double2 *, hipStream_t) { return hipSuccess; }
+hipError_t launch_solo(int, int, void *, const SoloArgs &, const double2 *, hipStream_t) { return hipSuccess; }
+hipError_t launch_pair_pass(int, int, bool, int, bool, void *, void *, const PairArgs &, const double2 *, const double *,
+                            double *, hipStream_t) { return hipSuccess; }
+hipError_t launch_pair_sums(const double *, uint64_t, int, double *, hipStream_t) { return hipSuccess; }
+hipError_t launch_pair(int, int, bool, bool, bool, void *, void *, const TileArgs &, const double2 *, const double *,
+                       double *, unsigned *grid, hipStream_t)
+{
+    *grid = 1;
+    return hipSuccess;
+}
+hipError_t launch_finalize(const double *, uint64_t, double *, hipStream_t) { return hipSuccess; }
+hipError_t launch_swap(int, void *, const SwapArgs &, hipStream_t) { return hipSuccess; }
+hipError_t launch_topk(int, const void *, int, int, double *, uint64_t *, hipStream_t) { return hipSuccess; }
+hipError_t launch_gather(int, const void *, const uint64_t *, size_t, double *, hipStream_t) { return hipSuccess; }
+hipError_t launch_fill_zero_one(int, void *, int, hipStream_t) { return hipSuccess; }
+hipError_t launch_stream(void *, size_t, int, float *, hipStream_t) { return hipSuccess; }
+hipError_t launch_slab_pass(int, int, bool, bool, void *, const TileArgs &, const SlotParams *, int, hipStream_t)
+{
+    return hipSuccess;
+}
+}  // namespace fq
+
+// ---- programs -----------------------------------------------------------------------
+
+static void ok(int rc)
+{
+    if (rc) {
+        fprintf(stderr, "failed (%d): %s\n", rc, fq_last_error());
+        exit(1);
+    }
+}
+
+static void add_plan_geoms(int N, const LayerPlan &lp, int A)
+{
+    for (const FusedPass &p : lp.ps)
+        for (int K = 0; K <= 3; ++K)
+            g_geoms.push_back(layout_geom(N, p.tile, A, K));
+}
+
+static fq_graph *dense_graph(int N)
+{
+    fq_graph *g = nullptr;
+    ok(fq_graph_create(N, &g));
+    for (int i = 0; i < N; ++i)
+        for (int j = i + 1; j < N; ++j)
+            ok(fq_graph_add_edge(g, i, j, 0.25 + 0.01 * i + 0.001 * j));
+    g_graph = g;
+    return g;
+}
+
+// Every geometry that the calls on N qubits use.
+static void all_geoms(int N, int dtype)
+{
+    for (int z2 = 0; z2 < 2; ++z2) {
+        const LayerPlan lp = exec_plan(N, dtype, z2 != 0, 1);
+        add_plan_geoms(N, lp, mix_a_log(dtype, (int)lp.ps[0].tile.size()));
+        const int Q = std::min(12, N - z2);
+        g_geoms.push_back(make_geom(N, low_tile(Q), std::min(4, Q)));
+        const int Qs = std::min(tile_max_q(dtype), N - z2);
+        g_geoms.push_back(make_geom(N, low_tile(Qs), tile_a_log(dtype, Qs)));
+    }
+    const LayerPlan lp = pair_plan(N, dtype);
+    if (!lp.ps.empty())
+        add_plan_geoms(N, lp, pair_a_log(dtype, (int)lp.ps[0].tile.size()));
+    if (N >= solo_min(dtype) && N <= solo_max(dtype))
+        for (int K = 0; K <= 2; K += 2)
+            g_geoms.push_back(layout_geom(N, low_tile(N), mix_a_log(dtype, N), K));
+}
+
+// plans <call> N dtype P small: `small` cost plans of other weights (of <C>, the
+// smallest there are), then the call on new weights, four times.
+static int plans(const std::string &call, int N, int dtype, int P, int small)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_state *st = nullptr;
+    ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+    std::vector<double> gm(P, 0.3), bt(P, 0.2), gg(P), gb(P);
+    int step = 0;
+    auto change = [&] { ok(fq_graph_add_edge(g, 0, N - 1, 1.0 + ++step)); };
+    for (int i = 0; i < small; ++i) {
+        change();
+        double e;
+        ok(fq_expect_cut(st, g, &e, nullptr));
+    }
+    fq_slab *sb = nullptr;
+    if (call == "slab" || call == "slab_z2")
+        ok(fq_slab_create_sched(N, 2, dtype, call == "slab" ? FQ_SCHED_FUSED : FQ_SCHED_Z2, &sb));
+    for (int rep = 0; rep < 4; ++rep) {
+        change();
+        if (sb) {
+            for (int k = 0; k < 2; ++k)
+                ok(fq_slab_assign(sb, k, g, P, gm.data(), bt.data()));
+            for (int p = 0; p < P; ++p)
+                ok(fq_slab_step(sb, nullptr));
+            int n = 0;
+            ok(fq_slab_collect(sb, nullptr, nullptr, nullptr, &n));
+        } else if (call == "backward") {
+            double e;
+            ok(fq_backward(st, g, P, gm.data(), bt.data(), &e, gg.data(), gb.data()));
+        } else {
+            ok(fq_run(st, g, P, gm.data(), bt.data(), call == "z2" ? FQ_SCHED_Z2 : FQ_SCHED_FUSED));
+        }
+    }
+    // the cache stays bounded: the plans of a call beyond its limit at most
+    printf("cached %zu\n", g->plans.size());
+    if (sb)
+        ok(fq_slab_destroy(sb));
+    ok(fq_state_destroy(st));
+    return 0;
+}
+
+int main(int argc, char **argv)
+{
+    const std::string what = argc > 1 ? argv[1] : "";
+    auto num = [&](int i) { return i < argc ? atoi(argv[i]) : 0; };
+    int rc = 2;
+    if (what == "plans" && argc == 7)
+        rc = plans(argv[2], num(3), num(4), num(5), num(6));
+    printf("checked %ld wrong %ld\n", g_checked, g_wrong);
+    return rc;
+}

@@ -1,0 +1,42 @@
+"""The host side of the library on the CPU (tests/host_api.cpp): fq_api.cpp compiled
+against host memory and launchers that check what they are given."""
+import os
+import re
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="session")
+def host_api(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("host_api") / "host_api")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", f"-I{ROCM}/include",
+                           f"-I{ROOT}/include", f"-I{ROOT}/for-qaoa_amd/csrc", f"{ROOT}/tests/host_api.cpp",
+                           "-o", exe])
+
+    def run(*args):
+        r = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stderr
+        return dict((k, int(v)) for k, v in re.findall(r"(\w+) (-?\d+)", r.stdout))
+
+    return run
+
+
+@pytest.mark.parametrize("call,N,dtype,P,small", [
+    # 64 plans are kept; the <C> plans that fill the cache are smaller than the calls'
+    ("run", 22, 0, 3, 62), ("run", 22, 0, 3, 63), ("run", 24, 0, 5, 63), ("run", 23, 1, 3, 63), ("run", 28, 1, 2, 63),
+    ("z2", 24, 0, 3, 63), ("z2", 28, 1, 3, 62), ("run", 12, 0, 3, 63), ("run", 20, 1, 3, 64),
+    ("backward", 22, 0, 3, 62), ("backward", 26, 1, 2, 62), ("backward", 24, 0, 3, 63),
+    ("slab", 16, 0, 3, 63), ("slab_z2", 23, 1, 3, 62), ("slab_z2", 24, 0, 3, 63), ("slab", 25, 1, 3, 63),
+    # plans of equal size: the least recently used ones are replaced throughout
+    ("run", 16, 0, 3, 70), ("slab", 20, 1, 3, 70), ("slab_z2", 8, 0, 3, 70),
+])
+def test_plans_stay_until_they_are_read(host_api, call, N, dtype, P, small):
+    """A full plan cache: no plan that a call has looked up is replaced before the
+    launches that read it, and the cache stays bounded."""
+    r = host_api("plans", call, N, dtype, P, small)
+    assert r["checked"] > small and r["wrong"] == 0
+    assert r["cached"] <= 64 + 5   # (a call's own plans at most beyond the limit)
