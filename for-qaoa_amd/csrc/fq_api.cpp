@@ -3339,6 +3339,7 @@ struct SlotHost {
     uint64_t gversion = 0;    // g->version the plans belong to
     uint64_t gepoch = 0;      // g->plan_epoch the plan pointers belong to
     PlanEntry *entries[5] = {nullptr};   // of the plans, while that is the graph's epoch
+    std::vector<double> W;    // the weights that gversion stands for
     int has_rr[4] = {0, 0, 0, 0};
 };
 
@@ -3613,7 +3614,53 @@ static int slab_slot_plans(fq_slab *sb, SlotHost &h)
     h.fresh = true;
     h.gversion = h.g->version;
     h.gepoch = h.g->plan_epoch;
+    h.W = h.g->W;
     return FQ_OK;
+}
+
+// Whether a step's last pass also opens the next layer of a slot that goes on.
+static bool slab_opens_ahead(const fq_slab *sb)
+{
+    return (sb->packed || sb->per_slot) && sb->slot_plan.end1 >= 0;
+}
+
+// The pass that ended a running slot's last layer (and opened the next one).
+static int slab_ended_on(const fq_slab *sb, const SlotHost &h)
+{
+    return sb->packed ? 1 - sb->pk_end : (h.layer - 1) % 2 == 0 ? sb->slot_plan.end1 : 0;
+}
+
+// That pass again on v (the slot, or a copy of it): RX(pre), the phase of gamma with
+// weights W, RX(beta).  Waits.
+static int slab_again(fq_slab *sb, const SlotHost &h, fq_state *v, const std::vector<double> &W, double pre, double gamma,
+                      double beta)
+{
+    const LayerPlan &lp = sb->slot_plan;
+    const int e = slab_ended_on(sb, h);
+    const int mode = !sb->z2 ? Z2_OFF : e + 1 < (int)lp.ps.size() ? Z2_LOWER : Z2_MIRROR;
+    fq_graph g;   // (plans of its own: none of the slot's graph goes for them)
+    g.N = sb->N;
+    g.W = W;
+    const int rc = tile_pass(v, lp.ps[e].tile, lp.ps[e].gates, beta, &g, gamma, true, false, FQ_K_FUSED, mode, &pre, false);
+    const hipError_t done = hipStreamSynchronize(sb->stream);
+    plans_free(&g);
+    return rc == FQ_OK && done != hipSuccess ? set_err(FQ_ERR_DEVICE, "slab: %s", hipGetErrorString(done)) : rc;
+}
+
+// A graph that changes while a request runs counts from the next layer on.  That
+// layer is open already (with the old weights): RX off, the phase of the difference,
+// RX on again.
+static int slab_reopen(fq_slab *sb, int slot)
+{
+    const SlotHost &h = sb->slots[slot];
+    const int L = h.layer;
+    std::vector<double> W = h.g->W;
+    bool any = false;
+    for (size_t i = 0; i < W.size(); ++i) {
+        W[i] -= h.W[i];
+        any |= W[i] != 0;
+    }
+    return any ? slab_again(sb, h, sb->views[slot], W, -h.betas[L], h.gammas[L], h.betas[L]) : FQ_OK;
 }
 
 static bool slab_slot_stale(const SlotHost &h)
@@ -3888,6 +3935,9 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
             if (h.phase != 1)
                 continue;
             if (slab_slot_stale(h)) {
+                if (h.layer > 0 && h.g->version != h.gversion && slab_opens_ahead(sb))
+                    if (int rc = slab_reopen(sb, k))
+                        return rc;
                 if (int rc = slab_slot_plans(sb, h))
                     return rc;
                 again = true;
@@ -4033,8 +4083,6 @@ extern "C" int fq_slab_collect(fq_slab *sb, int *slots, double *expect, double *
 static int slab_close_layer(fq_slab *sb, int slot, void *tmp)
 {
     const SlotHost &h = sb->slots[slot];
-    const LayerPlan &lp = sb->slot_plan;
-    const int L = h.layer, e = sb->packed ? 1 - sb->pk_end : (L - 1) % 2 == 0 ? lp.end1 : 0;
     fq_state v;
     v.N = sb->N;
     v.dtype = sb->dtype;
@@ -4046,11 +4094,7 @@ static int slab_close_layer(fq_slab *sb, int slot, void *tmp)
     for (int q = 0; q < FQ_MAXN; ++q)
         v.qmap[q] = q;
     v.init_amp = sb->init_amp;
-    const double pre = -h.betas[L];
-    const int mode = !sb->z2 ? Z2_OFF : e + 1 < (int)lp.ps.size() ? Z2_LOWER : Z2_MIRROR;
-    const int rc = tile_pass(&v, lp.ps[e].tile, lp.ps[e].gates, 0.0, h.g, -h.gammas[L], true, false, FQ_K_FUSED, mode,
-                             &pre, false);
-    hipStreamSynchronize(sb->stream);
+    const int rc = slab_again(sb, h, &v, h.W, -h.betas[h.layer], -h.gammas[h.layer], 0.0);
     hipFree(v.d_phase);
     v.sv = nullptr;
     return rc;
@@ -4068,7 +4112,7 @@ extern "C" int fq_slab_copy_out(fq_slab *sb, int slot, void *host, size_t bytes)
     const SlotHost &h = sb->slots[slot];
     void *tmp = nullptr;
     int rc = FQ_OK;
-    if ((sb->packed || sb->per_slot) && sb->slot_plan.end1 >= 0 && h.phase == 1 && h.layer > 0) {
+    if (slab_opens_ahead(sb) && h.phase == 1 && h.layer > 0) {
         if (hipMalloc(&tmp, sb->slot_bytes) != hipSuccess) {
             hipGetLastError();
             return set_err(FQ_ERR_OOM, "scratch for a running slot's amplitudes failed");

@@ -199,7 +199,9 @@ int fq_memory_in_use(size_t *bytes);
  * every active slot by one fused layer (slots at different layers and with
  * different P run together); a slot finishing its last layer gets <C> reduced
  * and is collected with fq_slab_collect, after which it is free for the next
- * request.  Calls on one slab run in order on the slab's own HIP stream. */
+ * request.  A graph that changes while a request on it runs counts from the
+ * request's next layer on.  Calls on one slab run in order on the slab's own HIP
+ * stream. */
 typedef struct fq_slab fq_slab;
 int fq_slab_create(int N, int nslots, int dtype, fq_slab **out);
 /* As fq_slab_create with a layer schedule: FQ_SCHED_FUSED (what
