@@ -387,6 +387,7 @@ struct fq_state {
     int cand_blocks = 0;
     double2 *d_phase = nullptr;  // per-launch cost phase factors
     size_t phase_cap = 0;        // bytes
+    std::vector<double2 *> old_phase;   // smaller ones before it (reserve_phases)
     void *aux = nullptr;         // adjoint state (lambda), allocated on first use
     double *d_grad = nullptr;    // adjoint per-pass sums
     size_t grad_cap = 0;
@@ -399,6 +400,16 @@ struct fq_state {
     int64_t t_cnt[FQ_K_COUNT] = {0};
     double t_bytes[FQ_K_COUNT] = {0};
 };
+
+static void free_phases(fq_state *st)
+{
+    for (double2 *p : st->old_phase)
+        hipFree(p);
+    st->old_phase.clear();
+    hipFree(st->d_phase);
+    st->d_phase = nullptr;
+    st->phase_cap = 0;
+}
 
 // ---- timing ------------------------------------------------------------------
 
@@ -970,7 +981,7 @@ extern "C" int fq_state_destroy(fq_state *st)
     hipFree(st->d_count);
     hipFree(st->d_cand_p);
     hipFree(st->d_cand_i);
-    hipFree(st->d_phase);
+    free_phases(st);
     if (st->aux)
         budget_give(st->bytes);
     hipFree(st->aux);
@@ -1153,19 +1164,41 @@ static void set_cost(TileArgs &a, double gamma, double init_amp)
             a.has_rr = 1;
 }
 
-// Grows the state's phase-table buffer (a larger one needs the previous
-// launches that read the old one to finish).
-static int reserve_phases(fq_state *st, size_t need)
+// Phase tables of one run made by one launch: up to this size together.  At
+// N=22 complex128 five of them are 1.3 MB; where a pass takes some hundred us
+// or more, its table's launch is under 2% of it.
+#define FQ_TABLES_BYTES ((size_t)8 << 20)
+
+// A first buffer holds the tables of any depth where they stay below this: from 2 MiB
+// on an allocation takes 7 us instead of 0.7, and its free the same.
+#define FQ_TABLES_FIRST (((size_t)2 << 20) - 4096)
+
+// Whether work queued on the stream is being captured into a graph.
+static bool is_capturing(hipStream_t stream)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &c) == hipSuccess && c != hipStreamCaptureStatusNone;
+}
+
+// Phase-table buffer of at least `need` bytes (`want` where it is made).  A smaller one
+// before it stays with the state: launches in flight and captured graphs read it.  Up to
+// FQ_TABLES_BYTES each is at least twice the one before; larger ones differ only by the
+// kind of call (run, cost layer, gradient).
+static int reserve_phases(fq_state *st, size_t need, size_t want = 0)
 {
     if (need <= st->phase_cap)
         return FQ_OK;
-    FQ_HIP(hipStreamSynchronize(st->stream));
-    hipFree(st->d_phase);
-    st->d_phase = nullptr;
-    st->phase_cap = 0;
-    if (hipMalloc(&st->d_phase, need) != hipSuccess)
-        return set_err(FQ_ERR_OOM, "phase table allocation of %zu bytes failed", need);
-    st->phase_cap = need;
+    const size_t twice = 2 * st->phase_cap <= FQ_TABLES_BYTES ? 2 * st->phase_cap : 0;
+    const size_t cap = std::max({need, want, twice});
+    void *m = nullptr;
+    if (hipMalloc(&m, cap) != hipSuccess) {
+        hipGetLastError();
+        return set_err(FQ_ERR_OOM, "phase table allocation of %zu bytes failed", cap);
+    }
+    if (st->d_phase)
+        st->old_phase.push_back(st->d_phase);
+    st->d_phase = (double2 *)m;
+    st->phase_cap = cap;
     return FQ_OK;
 }
 
@@ -1281,11 +1314,6 @@ static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const do
     st->pending_im = keep ? si : 0.0;
     return f;
 }
-
-// Phase tables of one run made by one launch: up to this size together.  At
-// N=22 complex128 five of them are 1.3 MB; where a pass takes some hundred us
-// or more, its table's launch is under 2% of it.
-#define FQ_TABLES_BYTES ((size_t)8 << 20)
 
 // The memory-side cache: 256 MiB.
 #define FQ_CACHE_LOG 28
@@ -1501,7 +1529,12 @@ static int mix_tables(fq_state *st, std::vector<Pass> &mps, bool *done, bool cut
     }
     if (nj < 2)
         return FQ_OK;
-    if (int rc = reserve_phases(st, total * sizeof(double2) + ncut * sizeof(double)))
+    const size_t need = total * sizeof(double2) + ncut * sizeof(double);
+    // (a graph under capture cannot wait for memory: a table for each pass)
+    if (need > st->phase_cap && is_capturing(st->stream))
+        return FQ_OK;
+    if (int rc = reserve_phases(st, need, std::min(FQ_TABLE_JOBS * most * sizeof(double2) + ncut * sizeof(double),
+                                                   FQ_TABLES_FIRST)))
         return rc;
     double *cut = cuts ? (double *)(st->d_phase + total) : nullptr;
     FQ_HIP(launch_phase_tables(m, nj, most, st->d_phase, cut, st->stream));
@@ -2347,6 +2380,8 @@ static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, cons
         bool tables = false;
         if (int rc = mix_tables(st, mps, &tables))
             return rc;
+        if (!tables && n > 1)
+            return set_err(FQ_ERR_OOM, "no memory for phase tables under capture: the same call before it makes it");
         if (!tables)   // (one layer)
             if (int rc = prepare_phases(st, mps[0].tab, A))
                 return rc;
@@ -3421,7 +3456,7 @@ static void slab_free(fq_slab *sb)
     if (sb->stream)
         hipStreamSynchronize(sb->stream);
     for (fq_state *v : sb->views) {
-        hipFree(v->d_phase);
+        free_phases(v);
         delete v;
     }
     sb->views.clear();
@@ -4095,7 +4130,7 @@ static int slab_close_layer(fq_slab *sb, int slot, void *tmp)
         v.qmap[q] = q;
     v.init_amp = sb->init_amp;
     const int rc = slab_again(sb, h, &v, h.W, -h.betas[h.layer], -h.gammas[h.layer], 0.0);
-    hipFree(v.d_phase);
+    free_phases(&v);
     v.sv = nullptr;
     return rc;
 }

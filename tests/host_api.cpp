@@ -4,6 +4,8 @@
 //
 //   plans   every cost plan that a launch reads, when it is launched, is a plan of the
 //           graph as it then is (build_plan's bytes), and lies in live memory.
+//   capture a run on a captured stream neither allocates nor waits, and the phase tables
+//           that its launches read stay where they are while the state lives.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
 #include <hip/hip_runtime.h>
@@ -50,10 +52,19 @@ static hipError_t give(void *p)
     return hipSuccess;
 }
 
+// While a stream is captured, allocations and waits are refused.
+static bool g_capturing = false;
+static hipError_t refuse(hipError_t e) { return g_capturing ? hipErrorStreamCaptureUnsupported : e; }
+
 extern "C" {
-hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return take(p, n); }
-hipError_t hipFree(void *p) { return give(p); }
+hipError_t hipMalloc(void **p, size_t n) { return g_capturing ? refuse(hipSuccess) : take(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return g_capturing ? refuse(hipSuccess) : take(p, n); }
+hipError_t hipFree(void *p) { return g_capturing ? refuse(hipSuccess) : give(p); }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c)
+{
+    *c = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipHostFree(void *p) { return give(p); }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
@@ -78,9 +89,9 @@ static hipError_t handle(void **h)
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle((void **)s); }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return refuse(hipSuccess); }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return refuse(hipSuccess); }
 hipError_t hipEventCreate(hipEvent_t *e) { return handle((void **)e); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return handle((void **)e); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -137,6 +148,14 @@ static void check(const PlanDev &p, int Q, int nthr, int nh)
     ++g_checked;
     if (!plan_ok(p, Q, nthr, nh))
         ++g_wrong;
+}
+
+// Phase tables that captured launches read (and write).
+static std::vector<const void *> g_captured;
+static void note(const void *tab)
+{
+    if (g_capturing && tab)
+        g_captured.push_back(tab);
 }
 
 // ---- launchers ----------------------------------------------------------------------
@@ -221,8 +240,16 @@ hipError_t launch_cut_mul(int, int, const void *, void *, const TileArgs &a, dou
 hipError_t launch_tile(int, int, bool, bool, bool, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
 hipError_t launch_tile_pre(int, int, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
 hipError_t launch_tile_mirror(int, int, bool, void *, const TileArgs &, hipStream_t) { return hipSuccess; }
-hipError_t launch_mix(int, int, bool, int, int, void *, const MixArgs &, const double2 *, hipStream_t) { return hipSuccess; }
-hipError_t launch_solo(int, int, void *, const SoloArgs &, const double2 *, hipStream_t) { return hipSuccess; }
+hipError_t launch_mix(int, int, bool, int, int, void *, const MixArgs &, const double2 *tab, hipStream_t)
+{
+    note(tab);
+    return hipSuccess;
+}
+hipError_t launch_solo(int, int, void *, const SoloArgs &, const double2 *tab, hipStream_t)
+{
+    note(tab);
+    return hipSuccess;
+}
 hipError_t launch_pair_pass(int, int, bool, int, bool, void *, void *, const PairArgs &, const double2 *, const double *,
                             double *, hipStream_t) { return hipSuccess; }
 hipError_t launch_pair_sums(const double *, uint64_t, int, double *, hipStream_t) { return hipSuccess; }
@@ -334,6 +361,40 @@ static int plans(const std::string &call, int N, int dtype, int P, int small)
     return 0;
 }
 
+// capture N dtype schedule P0 P1 P2: a run of P0 layers, one of P1 captured, one of P2,
+// a cost layer and a gradient.
+static int capture(int N, int dtype, int sched, int P0, int P1, int P2)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_state *st = nullptr;
+    ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+    const int most = std::max({P0, P1, P2});
+    std::vector<double> gm(most, 0.3), bt(most, 0.2), gg(most), gb(most);
+    auto run = [&](int P) { ok(fq_run(st, g, P, gm.data(), bt.data(), sched)); };
+    run(P0);
+    g_capturing = true;
+    run(P1);
+    g_capturing = false;
+    run(P2);
+    double e;
+    ok(fq_backward(st, g, P2, gm.data(), bt.data(), &e, gg.data(), gb.data()));
+    ok(fq_cost_layer(st, g, 0.3, 1));
+    for (const void *p : g_captured) {
+        ++g_checked;
+        g_wrong += !live(p, sizeof(double2));
+    }
+    const size_t before = g_live.size();
+    ok(fq_state_destroy(st));
+    // (the stream and its page stay with the library)
+    printf("freed %d\n", (int)(before - g_live.size()));
+    size_t lost = 0;
+    for (const void *p : g_captured)
+        lost += live(p, 1);
+    printf("kept %zu\n", lost);
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
@@ -341,6 +402,8 @@ int main(int argc, char **argv)
     int rc = 2;
     if (what == "plans" && argc == 7)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
+    if (what == "capture" && argc == 8)
+        rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
     printf("checked %ld wrong %ld\n", g_checked, g_wrong);
     return rc;
 }

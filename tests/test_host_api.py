@@ -40,3 +40,17 @@ def test_plans_stay_until_they_are_read(host_api, call, N, dtype, P, small):
     r = host_api("plans", call, N, dtype, P, small)
     assert r["checked"] > small and r["wrong"] == 0
     assert r["cached"] <= 64 + 5   # (a call's own plans at most beyond the limit)
+
+
+@pytest.mark.parametrize("N,dtype,schedule,depths", [
+    # one launch of all layers; all tables at once, in a first buffer that holds them and
+    # in one that does not; a table for each pass, with and without chunks
+    (12, 0, 1, (4, 64, 70)), (16, 0, 1, (4, 30, 64)), (20, 1, 1, (4, 30, 64)), (22, 0, 1, (4, 40, 64)),
+    (22, 0, 2, (5, 41, 64)), (25, 1, 1, (4, 9, 20)), (28, 1, 1, (3, 6, 9)), (26, 0, 2, (5, 7, 8)),
+])
+def test_captured_runs_keep_their_tables(host_api, N, dtype, schedule, depths):
+    """A run that is captured, deeper than the one before it, allocates nothing, and the
+    tables its launches read outlive what grows after it, as long as the state."""
+    r = host_api("capture", N, dtype, schedule, *depths)
+    assert r["checked"] > 0 and r["wrong"] == 0
+    assert r["kept"] == 0
