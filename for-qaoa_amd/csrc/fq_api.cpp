@@ -1936,6 +1936,7 @@ static int exchange_qubits(fq_state *st, const uint8_t *partner)
     a.nr = (int)rest.size();
     a.npairs = (1ull << lower.size()) * ((1ull << lower.size()) + 1) / 2;
     a.rest_fast = a.nr > 0 && rest[0] < least;
+    a.large = st->bytes > FQ_CACHE_BYTES;
     // an amplitude stays where the bits of each pair are equal
     const double bytes = 2.0 * (double)st->bytes * (1.0 - std::ldexp(1.0, -moved));
     return timed(st, FQ_K_SWAP, bytes, [&] { return launch_swap(st->dtype, st->sv, a, st->stream); });

@@ -201,6 +201,7 @@ struct SwapArgs {
     int tb;                          // tile qubits
     int rest_fast;                   // consecutive units step the rest index first
     int nr;                          // bits of the rest index
+    int large;                       // the state exceeds the memory-side cache
     uint8_t tpos[FQ_SWAP_BITS];      // tile bit -> position (ascending)
     uint8_t partner[FQ_SWAP_BITS];   // tile bit -> the tile bit it changes places with (itself if none)
     SwapRuns lower, upper, rest;     // positions of the pairs outside the tile, and of the others

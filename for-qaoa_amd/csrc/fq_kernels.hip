@@ -681,9 +681,9 @@ template <> struct NativeVec<float2> { typedef float type __attribute__((ext_vec
 // It is permuted in LDS and written to the tile whose other bits are exchanged:
 // a unit is two such tiles (bits x on the lower qubits of the pairs outside the
 // tile and y on the upper ones, X < Y and Y, X), or one that maps to itself.
-// Memory-bound: one read and one write of what moves.  4.8 to 4.9 TB/s from N=27
-// for 4 to 14 qubit pairs in both types, wherever they lie (a block in the middle,
-// complex128 N=28 qubits 3..8 and 12..17: 1.75 ms; with one thread per pair of
+// Memory-bound: one read and one write of what moves.  5.0 to 5.3 TB/s from N=27
+// for 8 to 14 qubit pairs in both types, wherever they lie (a block in the middle,
+// complex128 N=28 qubits 3..8 and 12..17: 1.56 ms; with one thread per pair of
 // amplitudes 4.7 ms).
 
 // Pair index p -> (X <= Y) with p = Y(Y+1)/2 + X.
@@ -727,11 +727,11 @@ __device__ __forceinline__ void swap_unit(const SwapArgs &a, uint64_t u, uint64_
 }
 
 // Tiles of 2^TB amplitudes (TB = 8: or of fewer).  Persistent; the next unit's
-// loads are issued once the current one is in LDS, and the unit after that is
-// found behind them.
+// loads are issued once the current one is in LDS (DEEP: before that, into registers of
+// their own), and the unit after that is found behind them.
 // (register arrays of the clang vector type stay in VGPRs across the loop;
 // arrays of HIP_vector_type<double, 2> went to scratch here)
-template <typename T0, int TB>
+template <typename T0, int TB, bool DEEP>
 __global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const SwapArgs a, uint64_t nunits)
 {
     typedef typename NativeVec<T0>::type T;
@@ -793,13 +793,25 @@ __global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const Sw
     for (uint64_t u = blockIdx.x; u < nunits; u += G) {
         const uint64_t ca = na, cb = nb;
         const bool more = u + G < nunits;
-        put(va, la);
-        if (more)
-            load(va, ca);
-        if (pa != pb)
-            put(vb, lb);
-        if (more && ca != cb)
-            load(vb, cb);
+        T wa[E], wb[E];
+        if (DEEP) {
+            if (more) {
+                load(wa, ca);
+                if (ca != cb)
+                    load(wb, cb);
+            }
+            put(va, la);
+            if (pa != pb)
+                put(vb, lb);
+        } else {
+            put(va, la);
+            if (more)
+                load(va, ca);
+            if (pa != pb)
+                put(vb, lb);
+            if (more && ca != cb)
+                load(vb, cb);
+        }
         if (u + 2 * G < nunits)
             swap_unit(a, u + 2 * G, na, nb);
         lds_barrier();
@@ -807,6 +819,13 @@ __global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const Sw
         if (pa != pb)
             store(pb, la);
         lds_barrier();   // the LDS reads finish before the next unit's writes
+        if (DEEP) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                va[e] = wa[e];
+                vb[e] = wb[e];
+            }
+        }
         pa = ca;
         pb = cb;
     }
@@ -1256,18 +1275,40 @@ hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, do
     return hipGetLastError();
 }
 
-template <typename T, int TB> static hipError_t launch_swap_k(void *sv, const SwapArgs &a, hipStream_t stream)
+template <typename T, int TB, bool DEEP> static hipError_t launch_swap_d(void *sv, const SwapArgs &a, hipStream_t stream)
 {
     constexpr size_t lds = 2 * ((size_t)(1 << TB) + (1 << (TB - (TB + 1) / 2))) * sizeof(T);
-    const void *fn = reinterpret_cast<const void *>(&k_exchange<T, TB>);
+    const void *fn = reinterpret_cast<const void *>(&k_exchange<T, TB, DEEP>);
     if (lds > 65536) {
         if (hipError_t e = allow_large_lds(fn))
             return e;
     }
-    const uint64_t nunits = a.npairs << a.nr, resident = (uint64_t)occupancy_per_cu(fn, 256, lds) * device_cus();
-    hipLaunchKernelGGL((k_exchange<T, TB>), dim3((unsigned)std::min(nunits, resident)), dim3(256), lds, stream,
-                       reinterpret_cast<T *>(sv), a, nunits);
+    const uint64_t nunits = a.npairs << a.nr;
+    uint64_t grid = (uint64_t)occupancy_per_cu(fn, 256, lds) * device_cus();
+    // States beyond the memory-side cache: fewer than one work-group per CU, and not a
+    // power of two of them, so that the units in flight are not all at the same offset of
+    // their DRAM pages.  Of 256 CUs, complex128 N=28 exchanges of the lowest qubits with
+    // those from 13 on, 2, 3 and 8 of them: 1,024 work-groups 1,890, 1,830, 2,057 us; 256
+    // 1,648, 1,875, 1,748; 240 1,599, 1,590, 1,725.  complex64 N=29, from qubit 14 on, 2
+    // and 8 of them, DEEP: 256 1,696, 1,704; 248 1,693, 1,678; 240 1,727, 1,671.
+    if (a.large)
+        grid = device_cus() - device_cus() / (DEEP ? 32 : 16);
+    hipLaunchKernelGGL((k_exchange<T, TB, DEEP>), dim3((unsigned)std::min(nunits, std::max<uint64_t>(grid, 1))), dim3(256), lds,
+                       stream, reinterpret_cast<T *>(sv), a, nunits);
     return hipGetLastError();
+}
+
+// DEEP for complex64 tiles of large states, where one work-group per CU leaves the
+// registers: N=29, 8 qubits with those from 14 on 1,840 -> 1,678 us (with 240
+// work-groups and without), 10 with those from 12 on 1,557 -> 1,510; a cached state has
+// two per CU, which hide the loads better (N=25 2 qubits 80 us, DEEP 98); complex128 N=28
+// 2 qubits 1,599 us, DEEP 1,811.
+template <typename T, int TB> static hipError_t launch_swap_k(void *sv, const SwapArgs &a, hipStream_t stream)
+{
+    if constexpr (TB == FQ_SWAP_BITS)
+        if (a.large)
+            return launch_swap_d<T, TB, true>(sv, a, stream);
+    return launch_swap_d<T, TB, false>(sv, a, stream);
 }
 
 template <typename T> static hipError_t launch_swap_t(void *sv, const SwapArgs &a, hipStream_t stream)
