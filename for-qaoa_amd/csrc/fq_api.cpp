@@ -1319,6 +1319,9 @@ static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const do
 #define FQ_CACHE_LOG 28
 #define FQ_CACHE_BYTES ((size_t)1 << FQ_CACHE_LOG)
 
+// States whose plans deal the qubits out instead of splitting them (exec_plan).
+#define FQ_DEALT_BYTES ((size_t)64 << 30)
+
 static int carriers_for(int dtype);
 
 // A tile pass on the compile-time kernel (fq_mix.h), ready to launch over
@@ -1462,10 +1465,15 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
     // Per layer on MI355X, N=34 complex64 fused 125 -> 104 ms (8 ranges of tiles
     // instead of 64: 102), N=33 complex128 122 -> 101; RX on the top 10 qubits at
     // N=34 113 -> 71 (8 ranges 113); no difference at N=30 complex128.
+    // From 64 GiB on, where the plans deal the qubits out (exec_plan), every pass:
+    // N=33 complex64 half state 34.8 -> 31.8 ms per layer (33.9 by the general kernel's
+    // order, one range of tiles for each of its work-groups), N=32 complex128 34.0 ->
+    // 31.2 (32.7), N=34 complex64 fused 111 -> 107.
     int carried = 0;
     while (carried < (int)tile.size() && tile[carried] == carried)
         ++carried;
-    a.by_xcd = carried <= carriers_for(st->dtype) && a.ntiles >= 2048 && st->bytes > FQ_CACHE_BYTES;
+    a.by_xcd = (carried <= carriers_for(st->dtype) || st->bytes >= FQ_DEALT_BYTES) && a.ntiles >= 2048 &&
+               st->bytes > FQ_CACHE_BYTES;
     mp.cost = cost;
     mp.kind = boundary ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
     mp.mir = z2 == Z2_MIRROR ? 1 : z2 == Z2_EXPAND ? 2 : 0;
