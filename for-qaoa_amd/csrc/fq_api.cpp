@@ -1833,8 +1833,13 @@ static int rx_targets_once(fq_state *st, std::vector<int> targets, double beta)
     std::sort(targets.begin(), targets.end());
     if (targets.empty())
         return FQ_OK;
-    if (targets.back() < Ceff)
-        return tile_pass(st, low_tile(Ceff), targets, beta, nullptr, 0, false, false, FQ_K_RX);
+    if (targets.back() < Ceff) {
+        // complex64 beyond the memory-side cache: 2^11 amplitudes at least (N=28, RX on
+        // 10 qubits: a work-group per 2^10 is one wave, 935 us, the general kernel 872,
+        // 2^11 788, 2^12 790; complex128, whose 2^9 is as many bytes, 1,638 and 2^11 1,650)
+        const int Q = st->dtype == FQ_C64 && st->bytes > FQ_CACHE_BYTES ? std::max(Ceff, 11) : Ceff;
+        return tile_pass(st, low_tile(Q), targets, beta, nullptr, 0, false, false, FQ_K_RX);
+    }
     const int Qmax = std::min(pass_tile_q(st->dtype), N);
     const int per = std::max(1, Qmax - std::min(carriers_for(st->dtype), Qmax - 1));
     size_t pos = 0;
