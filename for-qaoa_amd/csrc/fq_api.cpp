@@ -188,7 +188,7 @@ static bool is_own_stream(hipStream_t s)
 // to.  Both outlive it: up to FQ_LANES idle ones are kept for the next states
 // (making a stream takes 60 to 130 us; a state was made in 78 to 143 us, and now in 8
 // to 16).  A result that the kernels write themselves needs no copy behind them:
-// <C> at N=16 28 -> 20 us, with its sums added up by the last work-group.
+// <C> at N=16 27 -> 18.5 us.
 #define FQ_LANES 16
 #define FQ_LANE_DOUBLES 512
 struct Lane {
@@ -381,7 +381,6 @@ struct fq_state {
     bool in_run = false;
     double *d_part = nullptr;  // expect partials
     size_t part_cap = 0;
-    unsigned *d_count = nullptr;   // of launch_expect
     double *d_cand_p = nullptr;
     uint64_t *d_cand_i = nullptr;
     int cand_blocks = 0;
@@ -946,11 +945,9 @@ extern "C" int fq_state_create(int N, int D, int B, int C, int dtype, fq_state *
     st->part_cap = (size_t)1 << (N - Qr);
     st->cand_blocks = (int)std::min<uint64_t>(1024, std::max<uint64_t>(1, ((uint64_t)1 << N) / 4096));
     bool ok = hipMalloc(&st->d_part, sizeof(double) * 2 * st->part_cap) == hipSuccess &&
-              hipMalloc(&st->d_count, sizeof(unsigned)) == hipSuccess &&
               hipMalloc(&st->d_cand_p, sizeof(double) * FQ_TOPK_MAX * st->cand_blocks) == hipSuccess &&
               hipMalloc(&st->d_cand_i, sizeof(uint64_t) * FQ_TOPK_MAX * st->cand_blocks) == hipSuccess &&
-              lane_take(st->lane) &&
-              hipMemsetAsync(st->d_count, 0, sizeof(unsigned), st->lane.stream) == hipSuccess;
+              lane_take(st->lane);
     if (!ok) {
         hipGetLastError();
         fq_state_destroy(st);
@@ -978,7 +975,6 @@ extern "C" int fq_state_destroy(fq_state *st)
         budget_give(st->bytes);
     hipFree(st->sv);
     hipFree(st->d_part);
-    hipFree(st->d_count);
     hipFree(st->d_cand_p);
     hipFree(st->d_cand_i);
     free_phases(st);
@@ -2588,7 +2584,7 @@ extern "C" int fq_expect_cut(fq_state *st, fq_graph *g, double *expect, double *
     if (int rc = get_plan(g, geom, &a.plan, st->stream))
         return rc;
     int rc = timed(st, FQ_K_REDUCE, (double)st->bytes, [&] {
-        return launch_expect(st->dtype, a_log, st->sv, a, st->d_part, st->d_count, st->lane.host, st->stream);
+        return launch_expect(st->dtype, a_log, st->sv, a, st->d_part, st->lane.host, true, st->stream);
     });
     if (rc)
         return rc;
@@ -2673,7 +2669,7 @@ extern "C" int fq_expect_cut_static(fq_state *st, fq_graph *g, double *expect, d
     // the previous call on this stream may still read the plan: stream order
     // keeps this upload behind it
     FQ_HIP(hipMemcpyAsync(plan_mem, pb.bytes.data(), pb.bytes.size(), hipMemcpyHostToDevice, st->stream));
-    FQ_HIP(launch_expect(st->dtype, a_log, st->sv, a, part, nullptr, out2, st->stream));
+    FQ_HIP(launch_expect(st->dtype, a_log, st->sv, a, part, out2, false, st->stream));
     double h[2];
     FQ_HIP(hipMemcpyAsync(h, out2, sizeof(h), hipMemcpyDeviceToHost, st->stream));
     FQ_HIP(hipStreamSynchronize(st->stream));

@@ -249,12 +249,13 @@ size_t phase_table_entries(const TileArgs &a, int a_log);
 hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, double *cut,
                                hipStream_t stream);
 hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t stream);
-// count: a zeroed counter of this stream's own (its last work-group finishes <C>
-// where there are at most FQ_EXPECT_LAST of them: each one's fence and atomic cost
-// more than a second launch where there are many), or null
-#define FQ_EXPECT_LAST 1024
+// one: the sums of a state that is one tile come from the first launch alone.  (More
+// tiles take a second launch of one work-group: the last of them adding up instead, by a
+// fence and an atomic of each, took N=16 18.4 us instead of 18.5, N=20 22.9 instead of
+// 19.4, N=22 46 instead of 28.5, and N=3, whose work-group is one thread, 135 instead
+// of 15.)
 hipError_t launch_expect(int dtype, int a_log, const void *sv, const TileArgs &a, double *partials,
-                         unsigned *count, double *out2, hipStream_t stream);
+                         double *out2, bool one, hipStream_t stream);
 hipError_t launch_topk(int dtype, const void *sv, int N, int nblocks, double *cand_p,
                        uint64_t *cand_i, hipStream_t stream);
 hipError_t launch_gather(int dtype, const void *sv, const uint64_t *idx, size_t n, double *out,

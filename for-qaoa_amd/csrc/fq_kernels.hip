@@ -548,50 +548,17 @@ __global__ void __launch_bounds__(GATES ? 1024 : 256)
 
 // ---- <C> reduction ---------------------------------------------------------
 
-// Sums of n partial pairs, in one order for k_finalize and the last work-group
-// of k_expect: thread t of 1024 takes every 1024th, then a tree.
-__device__ __forceinline__ void finalize_pairs(const double *__restrict__ partials, uint64_t n, double *s_a, double *s_b,
-                                               double *__restrict__ out)
-{
-    const int t = threadIdx.x, nt = blockDim.x;
-    for (int v = t; v < 1024; v += nt) {
-        double a = 0.0, b = 0.0;
-        for (uint64_t i = v; i < n; i += 1024) {
-            a += partials[2 * i];
-            b += partials[2 * i + 1];
-        }
-        s_a[v] = a;
-        s_b[v] = b;
-    }
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        for (int v = t; v < w; v += nt) {
-            s_a[v] += s_a[v + w];
-            s_b[v] += s_b[v + w];
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        out[0] = s_a[0];
-        out[1] = s_b[0];
-    }
-}
-
-// count (zero before and after a launch): the work-group that finishes last adds
-// up the partials into out, so that <C> of a small state is one launch; null: the
-// partials are left to k_finalize.
+// Per-tile sums into partials.
 template <typename R, int A_LOG>
 __global__ void __launch_bounds__(256) k_expect(const typename CT<R>::T *__restrict__ sv,
-                                                const TileArgs a, double *__restrict__ partials,
-                                                unsigned *__restrict__ count, double *__restrict__ out)
+                                                const TileArgs a, double *__restrict__ partials)
 {
     typedef typename CT<R>::T T;
     constexpr int A = 1 << A_LOG;
     __shared__ double s_c[FQ_MAXQ + 2];
     __shared__ double s_K;
-    __shared__ double s_pc[1024];
-    __shared__ double s_p[1024];
-    __shared__ unsigned s_last;
+    __shared__ double s_pc[256];
+    __shared__ double s_p[256];
     const int t = threadIdx.x;
     const int nthreads = blockDim.x;
     const uint64_t tile = blockIdx.x;
@@ -644,19 +611,6 @@ __global__ void __launch_bounds__(256) k_expect(const typename CT<R>::T *__restr
         partials[2 * tile] = s_pc[0];
         partials[2 * tile + 1] = s_p[0];
     }
-    if (!count)
-        return;
-    if (t == 0) {
-        __threadfence();
-        s_last = atomicAdd(count, 1u) == gridDim.x - 1;
-    }
-    __syncthreads();
-    if (!s_last)
-        return;
-    __threadfence();
-    finalize_pairs(partials, gridDim.x, s_pc, s_p, out);
-    if (t == 0)
-        *count = 0;
 }
 
 __global__ void __launch_bounds__(1024) k_finalize(const double *__restrict__ partials,
@@ -664,7 +618,26 @@ __global__ void __launch_bounds__(1024) k_finalize(const double *__restrict__ pa
 {
     __shared__ double s_a[1024];
     __shared__ double s_b[1024];
-    finalize_pairs(partials, n, s_a, s_b, out);
+    const int t = threadIdx.x;
+    double a = 0.0, b = 0.0;
+    for (uint64_t i = t; i < n; i += 1024) {
+        a += partials[2 * i];
+        b += partials[2 * i + 1];
+    }
+    s_a[t] = a;
+    s_b[t] = b;
+    __syncthreads();
+    for (int w = 512; w > 0; w >>= 1) {
+        if (t < w) {
+            s_a[t] += s_a[t + w];
+            s_b[t] += s_b[t + w];
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        out[0] = s_a[0];
+        out[1] = s_b[0];
+    }
 }
 
 // the amplitude types as clang vectors
@@ -1333,15 +1306,14 @@ hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t strea
 }
 
 template <typename R, int A_LOG>
-static hipError_t launch_expect_t(const void *sv, const TileArgs &a, double *partials, unsigned *count, double *out2,
-                                  hipStream_t stream)
+static hipError_t launch_expect_t(const void *sv, const TileArgs &a, double *partials, double *out2, hipStream_t stream)
 {
     typedef typename CT<R>::T T;
     const uint64_t tiles = run_tiles(a);
     hipLaunchKernelGGL((k_expect<R, A_LOG>), dim3((unsigned)tiles), dim3(1u << a.nthr), 0, stream,
-                       reinterpret_cast<const T *>(sv), a, partials, count, out2);
+                       reinterpret_cast<const T *>(sv), a, partials);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || count)
+    if (e != hipSuccess || partials == out2)
         return e;
     hipLaunchKernelGGL(k_finalize, dim3(1), dim3(1024), 0, stream, partials, tiles, out2);
     return hipGetLastError();
@@ -1354,16 +1326,16 @@ hipError_t launch_finalize(const double *partials, uint64_t n, double *out2, hip
 }
 
 hipError_t launch_expect(int dtype, int a_log, const void *sv, const TileArgs &a, double *partials,
-                         unsigned *count, double *out2, hipStream_t stream)
+                         double *out2, bool one, hipStream_t stream)
 {
-    if (run_tiles(a) > FQ_EXPECT_LAST)
-        count = nullptr;
+    if (one && run_tiles(a) == 1)
+        partials = out2;
 #define FQ_EXP(R)                                                              \
     switch (a_log) {                                                           \
-        case 1: return launch_expect_t<R, 1>(sv, a, partials, count, out2, stream); \
-        case 2: return launch_expect_t<R, 2>(sv, a, partials, count, out2, stream); \
-        case 3: return launch_expect_t<R, 3>(sv, a, partials, count, out2, stream); \
-        case 4: return launch_expect_t<R, 4>(sv, a, partials, count, out2, stream); \
+        case 1: return launch_expect_t<R, 1>(sv, a, partials, out2, stream);   \
+        case 2: return launch_expect_t<R, 2>(sv, a, partials, out2, stream);   \
+        case 3: return launch_expect_t<R, 3>(sv, a, partials, out2, stream);   \
+        case 4: return launch_expect_t<R, 4>(sv, a, partials, out2, stream);   \
         default: return hipErrorInvalidValue;                                  \
     }
     if (dtype == 0) {
