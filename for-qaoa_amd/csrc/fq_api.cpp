@@ -3386,7 +3386,7 @@ struct SlotHost {
     uint64_t gversion = 0;    // g->version the plans belong to
     uint64_t gepoch = 0;      // g->plan_epoch the plan pointers belong to
     PlanEntry *entries[5] = {nullptr};   // of the plans, while that is the graph's epoch
-    std::vector<double> W;    // the weights that gversion stands for
+    std::vector<double> W;    // the weights of the open layer's phase
     int has_rr[4] = {0, 0, 0, 0};
 };
 
@@ -3699,7 +3699,7 @@ static int slab_again(fq_slab *sb, const SlotHost &h, fq_state *v, const std::ve
 // RX on again.
 static int slab_reopen(fq_slab *sb, int slot)
 {
-    const SlotHost &h = sb->slots[slot];
+    SlotHost &h = sb->slots[slot];
     const int L = h.layer;
     std::vector<double> W = h.g->W;
     bool any = false;
@@ -3707,7 +3707,11 @@ static int slab_reopen(fq_slab *sb, int slot)
         W[i] -= h.W[i];
         any |= W[i] != 0;
     }
-    return any ? slab_again(sb, h, sb->views[slot], W, -h.betas[L], h.gammas[L], h.betas[L]) : FQ_OK;
+    if (any)
+        if (int rc = slab_again(sb, h, sb->views[slot], W, -h.betas[L], h.gammas[L], h.betas[L]))
+            return rc;
+    h.W = h.g->W;   // (now, not with the new plans: a step that fails on those is called again)
+    return FQ_OK;
 }
 
 static bool slab_slot_stale(const SlotHost &h)

@@ -6,6 +6,8 @@
 //           graph as it then is (build_plan's bytes), and lies in live memory.
 //   capture a run on a captured stream neither allocates nor waits, and the phase tables
 //           that its launches read stay where they are while the state lives.
+//   reopen  a slab's step whose plans cannot be made after its graph changed, called
+//           again: the slot's open layer takes the change once.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
 #include <hip/hip_runtime.h>
@@ -93,7 +95,14 @@ hipError_t hipStreamSynchronize(hipStream_t) { return refuse(hipSuccess); }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return refuse(hipSuccess); }
 hipError_t hipEventCreate(hipEvent_t *e) { return handle((void **)e); }
-hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return handle((void **)e); }
+static int g_events_left = -1;   // events that can still be made (-1: any number)
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    if (g_events_left == 0)
+        return hipErrorOutOfMemory;
+    g_events_left -= g_events_left > 0;
+    return handle((void **)e);
+}
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
@@ -240,9 +249,11 @@ hipError_t launch_cut_mul(int, int, const void *, void *, const TileArgs &a, dou
 hipError_t launch_tile(int, int, bool, bool, bool, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
 hipError_t launch_tile_pre(int, int, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
 hipError_t launch_tile_mirror(int, int, bool, void *, const TileArgs &, hipStream_t) { return hipSuccess; }
-hipError_t launch_mix(int, int, bool, int, int, void *, const MixArgs &, const double2 *tab, hipStream_t)
+static int g_boundaries = 0;   // boundary passes on single states
+hipError_t launch_mix(int, int, bool, int kind, int, void *, const MixArgs &a, const double2 *tab, hipStream_t)
 {
     note(tab);
+    g_boundaries += kind == MIX_BOUNDARY && !a.slots;
     return hipSuccess;
 }
 hipError_t launch_solo(int, int, void *, const SoloArgs &, const double2 *tab, hipStream_t)
@@ -395,6 +406,28 @@ static int capture(int N, int dtype, int sched, int P0, int P1, int P2)
     return 0;
 }
 
+// reopen N dtype schedule
+static int reopen(int N, int dtype, int sched)
+{
+    fq_graph *g = dense_graph(N);
+    fq_slab *sb = nullptr;
+    ok(fq_slab_create_sched(N, 2, dtype, sched, &sb));
+    std::vector<double> gm(4, 0.3), bt(4, 0.2);
+    ok(fq_slab_assign(sb, 0, g, 4, gm.data(), bt.data()));
+    ok(fq_slab_step(sb, nullptr));
+    ok(fq_graph_add_edge(g, 0, 1, 2.0));
+    g_boundaries = 0;
+    g_events_left = 1;   // (the phase of the difference has one plan)
+    printf("failed %d\n", (int)(fq_slab_step(sb, nullptr) != FQ_OK));
+    g_events_left = -1;
+    printf("reopened %d\n", g_boundaries);
+    const bool own = !sb->packed;   // the step itself then runs such a pass
+    ok(fq_slab_step(sb, nullptr));
+    printf("again %d\n", g_boundaries - own);
+    ok(fq_slab_destroy(sb));
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
@@ -404,6 +437,8 @@ int main(int argc, char **argv)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
     if (what == "capture" && argc == 8)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
+    if (what == "reopen" && argc == 5)
+        rc = reopen(num(2), num(3), num(4));
     printf("checked %ld wrong %ld\n", g_checked, g_wrong);
     return rc;
 }

@@ -54,3 +54,11 @@ def test_captured_runs_keep_their_tables(host_api, N, dtype, schedule, depths):
     r = host_api("capture", N, dtype, schedule, *depths)
     assert r["checked"] > 0 and r["wrong"] == 0
     assert r["kept"] == 0
+
+
+@pytest.mark.parametrize("N,dtype,schedule", [(14, 0, 1), (16, 1, 2), (23, 1, 2), (25, 0, 2)])
+def test_open_layer_takes_a_change_once(host_api, N, dtype, schedule):
+    """A step that fails once the open layer has the new weights does not add the
+    difference again when it is called again."""
+    r = host_api("reopen", N, dtype, schedule)
+    assert r["failed"] == 1 and r["reopened"] == 1 and r["again"] == 1
