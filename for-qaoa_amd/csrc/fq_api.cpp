@@ -3719,6 +3719,38 @@ static bool slab_slot_stale(const SlotHost &h)
     return h.g->version != h.gversion || h.g->plan_epoch != h.gepoch;
 }
 
+// A slab without its launch arguments, memory or stream.
+static fq_slab *slab_shape(int N, int nslots, int s, int dtype, bool z2)
+{
+    fq_slab *sb = new fq_slab();
+    sb->N = N;
+    sb->K = nslots;
+    sb->s = s;
+    sb->dtype = dtype;
+    sb->z2 = z2;
+    sb->elem = dtype == FQ_C128 ? 16 : 8;
+    sb->slot_bytes = ((size_t)1 << (z2 ? N - 1 : N)) * sb->elem;
+    sb->bytes = sb->slot_bytes * nslots;
+    sb->slots.resize(nslots);
+    sb->init_amp = pow(1. / sqrt(2.), N);
+    sb->passes = cover_passes(N, std::min(tile_max_q(dtype), z2 ? N - 1 : N), dtype);
+    return sb;
+}
+
+extern "C" int fq_slab_passes(int N, int dtype, int schedule, int P, int *npass)
+{
+    if (N < 1 || N > 36 || (dtype != FQ_C128 && dtype != FQ_C64) || P < 1 || !npass)
+        return set_err(FQ_ERR_ARG, "bad N, dtype or layer count, or null output");
+    if (schedule != FQ_SCHED_FUSED && (schedule != FQ_SCHED_Z2 || N < 3))
+        return set_err(FQ_ERR_ARG, "slab schedule must be FQ_SCHED_FUSED or FQ_SCHED_Z2 (N >= 3)");
+    fq_slab *sb = slab_shape(N, 1, 0, dtype, schedule == FQ_SCHED_Z2);
+    const int rc = slab_build_args(sb);
+    const int m = (int)(sb->packed || sb->per_slot ? sb->slot_plan.ps : sb->passes).size();
+    *npass = slab_opens_ahead(sb) ? 1 + P * (m - 1) : P * m;
+    delete sb;
+    return rc;
+}
+
 extern "C" int fq_slab_create(int N, int nslots, int dtype, fq_slab **out)
 {
     return fq_slab_create_sched(N, nslots, dtype, FQ_SCHED_FUSED, out);
@@ -3743,18 +3775,7 @@ extern "C" int fq_slab_create_sched(int N, int nslots, int dtype, int schedule, 
     const bool z2 = schedule == FQ_SCHED_Z2;
     if (z2 && N < 3)
         return set_err(FQ_ERR_ARG, "the half-state schedule needs N >= 3");
-    fq_slab *sb = new fq_slab();
-    sb->N = N;
-    sb->K = nslots;
-    sb->s = s;
-    sb->dtype = dtype;
-    sb->z2 = z2;
-    sb->elem = dtype == FQ_C128 ? 16 : 8;
-    sb->slot_bytes = ((size_t)1 << (z2 ? N - 1 : N)) * sb->elem;
-    sb->bytes = sb->slot_bytes * nslots;
-    sb->slots.resize(nslots);
-    sb->init_amp = pow(1. / sqrt(2.), N);
-    sb->passes = cover_passes(N, std::min(tile_max_q(dtype), z2 ? N - 1 : N), dtype);
+    fq_slab *sb = slab_shape(N, nslots, s, dtype, z2);
     if (!budget_take(sb->bytes)) {
         delete sb;
         return set_err(FQ_ERR_BUDGET, "slab of %d x 2^%d amplitudes exceeds the memory budget", nslots, N);

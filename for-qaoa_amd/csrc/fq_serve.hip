@@ -6,9 +6,10 @@
 // device memory), so requests of different depth P advance together one layer
 // per step and a request can enter a free slot at any layer boundary.
 //
-// Slots of 10 to 22 qubits run the tile passes of fq_mix.h, one launch for all
-// slots that run the same pass; here are their phase tables and <C>.  k_slab_pass
-// is the general kernel, for smaller slots and the plans of tuning knobs: the
+// Slots of 10 to 21 qubits (complex64 11 to 22) run the tile passes of fq_mix.h, one
+// launch for all slots that run the same pass; here are their phase tables and <C>.
+// k_slab_pass is the general kernel, for smaller slots, for half states of 24 qubits
+// in complex64, which no two-pass plan takes, and for the plans of tuning knobs: the
 // slab is one virtual state of N + s qubits whose top s bits select the slot, and
 // one persistent launch covers every active slot.
 #include "forqaoa.h"

@@ -321,27 +321,15 @@ def latency_stats(done):
 
 def bytes_floor(stream, requests, dtype="c64", schedule="fused"):
     """Algorithmic HBM bytes of the slab schedule for these requests: the
-    tile passes each request's slot runs (layer 0's first pass writes the
+    tile passes each request's slot runs (fq_slab_passes; the first writes the
     stored state once, every other pass reads and writes it) plus one <C>
-    read.  A half-state slab stores and moves half of each state.  Slots of
-    at least 2^10 first-pass tiles run fq_run's pipelined layers (1 + P(m-1)
-    passes for m passes per layer, when m >= 2 (full) or 3 (half state));
-    smaller slots run P*m packed passes."""
-    from . import layer_passes
-
+    read.  A half-state slab stores and moves half of each state."""
     elem = 16 if DTYPES[dtype] == FQ_C128 else 8
-    qmax = 13 if DTYPES[dtype] == FQ_C128 else 14
-    m_of = {}
     tot = 0.0
+    n = ctypes.c_int()
     for r in requests:
         half = schedule == "z2" and r.N >= 3
-        ns = r.N - 1 if half else r.N
-        S = (1 << ns) * elem
-        if r.N not in m_of:
-            m_of[r.N] = len(layer_passes(r.N, dtype, "z2" if half else "fused"))
-        m = m_of[r.N]
-        per_slot = ns - min(qmax, ns) >= 10
-        piped = per_slot and m >= (3 if half else 2)
-        npass = 1 + r.P * (m - 1) if piped else r.P * m
-        tot += S * (2 * npass - 1) + S
+        S = (1 << (r.N - 1 if half else r.N)) * elem
+        check(lib().fq_slab_passes(r.N, DTYPES[dtype], SCHEDULES["z2" if half else "fused"], r.P, ctypes.byref(n)))
+        tot += S * (2 * n.value - 1) + S
     return tot

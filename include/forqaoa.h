@@ -215,9 +215,9 @@ int fq_slab_assign(fq_slab *sb, int slot, fq_graph *g, int P, const double *gamm
 /* Enqueue one layer for every active slot (waits for the previous step first);
  * nfinishing (may be NULL) receives the number of slots finishing with it. */
 int fq_slab_step(fq_slab *sb, int *nfinishing);
-/* Layers a step runs per slot in a slab of large slots (half states from about
- * N = 22 complex128, 23 complex64, whose slots run fq_run's tile passes one
- * after the other): up to `layers` (>= 1, default 1), fewer for a slot that has
+/* Layers a step runs per slot in a slab of large slots (from N = 22 complex128, 23
+ * complex64, but not half states of N = 24 complex64; their slots run fq_run's tile
+ * passes one after the other): up to `layers` (>= 1, default 1), fewer for a slot that has
  * fewer left.  Slabs of small slots (one packed launch per pass) keep one
  * layer per step. */
 int fq_slab_set_layers_per_step(fq_slab *sb, int layers);
@@ -229,11 +229,19 @@ int fq_slab_collect(fq_slab *sb, int *slots, double *expect, double *norm2, int 
  * order).  Waits. */
 int fq_slab_copy_out(fq_slab *sb, int slot, void *host, size_t bytes);
 
+/* Tile passes that a slot of such a slab runs for a request of P layers; the first
+ * writes the stored state, the others read and write it (host-only, no device
+ * needed). */
+int fq_slab_passes(int N, int dtype, int schedule, int P, int *npass);
+
 /* The tile passes that cover one layer of FQ_SCHED_FUSED or FQ_SCHED_Z2 for N
- * qubits (no counterpart in the reference; host-only, no device needed; fq_run
- * launches as many, but with three passes it may deal the qubits above pass 0
- * out differently and run passes that stay within a part of the state part by
- * part, environment FQ_CHUNK):
+ * qubits (no counterpart in the reference; host-only, no device needed).  fq_run
+ * runs exactly these where a tuning knob is set (environment FQ_TILE_Q,
+ * FQ_PASS_BLOCK, FQ_CARRIER_GATES, FQ_LAYER_PIPE).  Without one it runs other
+ * passes where they are faster: all layers in one launch for states of 9 (FQ_C64:
+ * 10) to 12 qubits, two passes of narrower tiles for those after them, and with
+ * three passes another split of the qubits above pass 0, passes that stay within a
+ * part of the state part by part (environment FQ_CHUNK):
  * *npass passes of *tile_q positions each; pass p's tile positions (thread
  * bits first, the last ones register bits) in tiles[16*p .. 16*p+15] (-1
  * padded) and its RX targets as the bit mask gates[p].  In layer order pass

@@ -8,6 +8,7 @@
 //           that its launches read stay where they are while the state lives.
 //   reopen  a slab's step whose plans cannot be made after its graph changed, called
 //           again: the slot's open layer takes the change once.
+//   passes  the launches of a slab's request, and what fq_slab_passes says.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
 #include <hip/hip_runtime.h>
@@ -246,14 +247,28 @@ hipError_t launch_cut_mul(int, int, const void *, void *, const TileArgs &a, dou
     check(a.plan, a.Q, a.nthr, a.nh);
     return hipSuccess;
 }
-hipError_t launch_tile(int, int, bool, bool, bool, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
-hipError_t launch_tile_pre(int, int, void *, const TileArgs &, const double2 *, hipStream_t) { return hipSuccess; }
-hipError_t launch_tile_mirror(int, int, bool, void *, const TileArgs &, hipStream_t) { return hipSuccess; }
 static int g_boundaries = 0;   // boundary passes on single states
+static int g_passes = 0;       // tile passes
 hipError_t launch_mix(int, int, bool, int kind, int, void *, const MixArgs &a, const double2 *tab, hipStream_t)
 {
     note(tab);
+    ++g_passes;
     g_boundaries += kind == MIX_BOUNDARY && !a.slots;
+    return hipSuccess;
+}
+hipError_t launch_tile(int, int, bool, bool, bool, void *, const TileArgs &, const double2 *, hipStream_t)
+{
+    ++g_passes;
+    return hipSuccess;
+}
+hipError_t launch_tile_pre(int, int, void *, const TileArgs &, const double2 *, hipStream_t)
+{
+    ++g_passes;
+    return hipSuccess;
+}
+hipError_t launch_tile_mirror(int, int, bool, void *, const TileArgs &, hipStream_t)
+{
+    ++g_passes;
     return hipSuccess;
 }
 hipError_t launch_solo(int, int, void *, const SoloArgs &, const double2 *tab, hipStream_t)
@@ -278,6 +293,7 @@ hipError_t launch_fill_zero_one(int, void *, int, hipStream_t) { return hipSucce
 hipError_t launch_stream(void *, size_t, int, float *, hipStream_t) { return hipSuccess; }
 hipError_t launch_slab_pass(int, int, bool, bool, void *, const TileArgs &, const SlotParams *, int, hipStream_t)
 {
+    ++g_passes;
     return hipSuccess;
 }
 }  // namespace fq
@@ -428,6 +444,23 @@ static int reopen(int N, int dtype, int sched)
     return 0;
 }
 
+// passes N dtype schedule P
+static int passes(int N, int dtype, int sched, int P)
+{
+    fq_graph *g = dense_graph(N);
+    fq_slab *sb = nullptr;
+    ok(fq_slab_create_sched(N, 2, dtype, sched, &sb));
+    const std::vector<double> gm(P, 0.3), bt(P, 0.2);
+    ok(fq_slab_assign(sb, 1, g, P, gm.data(), bt.data()));
+    for (int p = 0; p < P; ++p)
+        ok(fq_slab_step(sb, nullptr));
+    int told = 0;
+    ok(fq_slab_passes(N, dtype, sched, P, &told));
+    printf("launched %d told %d\n", g_passes, told);
+    ok(fq_slab_destroy(sb));
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     const std::string what = argc > 1 ? argv[1] : "";
@@ -437,6 +470,8 @@ int main(int argc, char **argv)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
     if (what == "capture" && argc == 8)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
+    if (what == "passes" && argc == 6)
+        rc = passes(num(2), num(3), num(4), num(5));
     if (what == "reopen" && argc == 5)
         rc = reopen(num(2), num(3), num(4));
     printf("checked %ld wrong %ld\n", g_checked, g_wrong);

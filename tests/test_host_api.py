@@ -62,3 +62,22 @@ def test_open_layer_takes_a_change_once(host_api, N, dtype, schedule):
     difference again when it is called again."""
     r = host_api("reopen", N, dtype, schedule)
     assert r["failed"] == 1 and r["reopened"] == 1 and r["again"] == 1
+
+
+@pytest.mark.parametrize("N,dtype,schedule", [
+    # general, packed, one by one; the half states of 24 qubits in between
+    (3, 0, 2), (9, 0, 1), (10, 0, 1), (10, 1, 2), (11, 1, 2), (21, 0, 2), (22, 0, 2), (22, 1, 1), (23, 1, 2), (24, 1, 2),
+    (24, 0, 1), (25, 0, 1), (25, 1, 2), (30, 1, 2),
+])
+@pytest.mark.parametrize("P", [1, 2, 5])
+def test_slab_passes_are_those_launched(host_api, N, dtype, schedule, P):
+    r = host_api("passes", N, dtype, schedule, P)
+    assert r["launched"] == r["told"] > 0
+
+
+def test_serving_floor_counts_the_passes_that_run():
+    # packed slots of N=16 run 1 + P passes of a half state, not 2 P
+    from forqaoa.serve import Request, Stream, bytes_floor
+    r = Request(0, 16, 5, 0, [0.1] * 5, [0.2] * 5)
+    S = (1 << 15) * 8
+    assert bytes_floor(Stream({}, [r]), [r], "c64", "z2") == S * (2 * 6 - 1) + S
