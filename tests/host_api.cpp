@@ -8,6 +8,8 @@
 //           that its launches read stay where they are while the state lives.
 //   reopen  a slab's step whose plans cannot be made after its graph changed, called
 //           again: the slot's open layer takes the change once.
+//   cover   the plans of fq_run and of the gradient: per layer one RX on each qubit, after
+//           the layer's phase and before the next one's, on passes that have an instance.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
@@ -444,6 +446,100 @@ static int reopen(int N, int dtype, int sched)
     return 0;
 }
 
+// Plan lp of an N-qubit state and its launches for P layers; a_log, lane_bit: of its kernels.
+static void cover_plan(int N, const LayerPlan &lp, bool z2, int P, int (*a_log)(int, int), bool (*lane_bit)(int, int, int),
+                       int dtype)
+{
+    auto need = [&](bool good, const char *what) {
+        ++g_checked;
+        if (!good) {
+            ++g_wrong;
+            fprintf(stderr, "N=%d dtype=%d z2=%d P=%d: %s\n", N, dtype, z2, P, what);
+        }
+    };
+    const int m = (int)lp.ps.size(), Q = (int)lp.ps[0].tile.size(), A = a_log(dtype, Q);
+    std::vector<int> gated(N, 0);
+    for (int i = 0; i < m; ++i) {
+        const FusedPass &fp = lp.ps[i];
+        need((int)fp.tile.size() == Q, "tiles of one width");
+        need(std::set<int>(fp.tile.begin(), fp.tile.end()).size() == fp.tile.size(), "distinct positions");
+        for (int q : fp.tile)
+            need(q >= 0 && q < N, "a position of the state");
+        for (int q : fp.gates) {
+            gated[q]++;
+            need(std::count(fp.tile.begin(), fp.tile.end(), q) == 1, "a gated qubit in the tile");
+        }
+        if (z2) {
+            const bool top = std::count(fp.tile.begin(), fp.tile.end(), N - 1) > 0;
+            need(top == (i + 1 == m) && (!top || fp.tile.back() == N - 1), "the top qubit on the last register bit");
+        }
+        if (A == 0) {
+            need(geom_runs(make_geom(N, fp.tile, tile_a_log(dtype, Q))) <= FQ_MAX_RUNS, "bit runs");
+            continue;
+        }
+        MixArgs a;
+        int K = 0;
+        bool lane = false;
+        ok(pass_shape(N, fp.tile, fp.gates, A, lane_bit, !z2 ? Z2_OFF : i + 1 == m ? Z2_MIRROR : Z2_LOWER, a, K, lane));
+        need(K == 0 || Q - A > (K - 1) * A, "an instance with as many exchanges");
+        int rx = lane;
+        for (uint32_t w = a.gates_w; w; w &= w - 1)
+            ++rx;
+        need(rx == (int)fp.gates.size(), "every gated qubit in a layout");
+    }
+    for (int q = 0; q < N; ++q)
+        need(gated[q] == 1, "one RX on each qubit");
+    std::vector<Step> seq;
+    for (int p = 0; p < P; ++p)
+        layer_steps(lp, p, P, seq);
+    std::vector<int> rx(N, -1);   // the last layer whose RX a qubit has had
+    int phase = -1;               // the last layer whose phase has run
+    for (const Step &s : seq) {
+        auto apply = [&](int layer) {
+            need(phase == layer, "RX after its layer's phase");
+            for (int q : lp.ps[s.pass].gates) {
+                need(rx[q] == layer - 1, "RX in order");
+                rx[q] = layer;
+            }
+        };
+        if (s.kind == STEP_BOUNDARY)
+            apply(s.layer);
+        if (s.kind != STEP_PLAIN) {
+            ++phase;
+            need(std::count(rx.begin(), rx.end(), phase - 1) == N, "the phase after the layer before");
+        }
+        apply(s.kind == STEP_BOUNDARY ? s.layer + 1 : s.layer);
+    }
+    need(std::count(rx.begin(), rx.end(), P - 1) == N, "all layers");
+    need(!z2 || (seq.back().kind == STEP_PLAIN && seq.back().pass + 1 == m) || a_log == pair_a_log,
+         "the mirror pass last");
+    for (size_t k = 0, n; k < seq.size(); k += n) {
+        n = chunk_group(lp, seq, k);
+        int cost = 0;
+        for (size_t i = k; i < k + n && n > 1; ++i) {
+            cost += seq[i].kind != STEP_PLAIN;
+            for (int q : lp.ps[seq[i].pass].tile)
+                need(q < lp.chunk && lp.chunk < N - z2, "a pass within a chunk");
+        }
+        need(cost <= 1, "one phase table a chunk");
+    }
+}
+
+// cover N0 N1: states of N0 to N1 qubits
+static int cover(int N0, int N1)
+{
+    for (int N = N0; N <= N1; ++N)
+        for (int dtype = 0; dtype < 2; ++dtype)
+            for (int P = 1; P <= 4; ++P) {
+                for (int z2 = 0; z2 < (N >= 3 ? 2 : 1); ++z2)
+                    cover_plan(N, exec_plan(N, dtype, z2 != 0, P), z2 != 0, P, mix_a_log, mix_lane_bit, dtype);
+                const LayerPlan lp = pair_plan(N, dtype);
+                if (!lp.ps.empty())
+                    cover_plan(N, lp, true, P, pair_a_log, pair_lane_bit, dtype);
+            }
+    return 0;
+}
+
 // passes N dtype schedule P
 static int passes(int N, int dtype, int sched, int P)
 {
@@ -470,6 +566,8 @@ int main(int argc, char **argv)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
     if (what == "capture" && argc == 8)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
+    if (what == "cover" && argc == 4)
+        rc = cover(num(2), num(3));
     if (what == "passes" && argc == 6)
         rc = passes(num(2), num(3), num(4), num(5));
     if (what == "reopen" && argc == 5)

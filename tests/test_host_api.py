@@ -81,3 +81,10 @@ def test_serving_floor_counts_the_passes_that_run():
     r = Request(0, 16, 5, 0, [0.1] * 5, [0.2] * 5)
     S = (1 << 15) * 8
     assert bytes_floor(Stream({}, [r]), [r], "c64", "z2") == S * (2 * 6 - 1) + S
+
+
+def test_default_plans_cover_every_layer(host_api):
+    """The plans that fq_run and the gradient run without tuning knobs, for every N, both
+    types, the full and the half state."""
+    r = host_api("cover", 1, 36)
+    assert r["checked"] > 10000 and r["wrong"] == 0
