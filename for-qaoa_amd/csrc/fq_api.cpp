@@ -2254,6 +2254,22 @@ static size_t chunk_group(const LayerPlan &lp, const std::vector<Step> &seq, siz
     return n;
 }
 
+// End of the steps from seq[k] on that are prepared together: whole groups
+// (chunk_group) with at most FQ_TABLE_JOBS cost passes, so that a deep run needs no more
+// host memory than one of that many layers.
+static size_t window_end(const LayerPlan &lp, const std::vector<Step> &seq, size_t k)
+{
+    int jobs = 0;
+    for (size_t n; k < seq.size(); k += n) {
+        n = chunk_group(lp, seq, k);
+        for (size_t i = k; i < k + n; ++i)
+            jobs += seq[i].kind != STEP_PLAIN;
+        if (jobs > FQ_TABLE_JOBS)
+            break;
+    }
+    return k;
+}
+
 // Layers [p0, p1) of P.  expand: the last layer's mirror pass also writes the
 // upper half of the full state.
 static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, int p1, int P, const double *gammas,
@@ -2269,68 +2285,77 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
     // every pass on the compile-time kernel (the pass widths of tuning knobs
     // may have none): prepared first, and small phase tables made at once
     const bool mix = mix_a_log(st->dtype, (int)ps[0].tile.size()) > 0;
-    std::vector<MixPass> mps(mix ? seq.size() : 0);
-    std::vector<int> modes(mps.size());
-    bool tables = false;
-    for (size_t k = 0; k < seq.size(); ++k) {
-        const Step &s = seq[k];
-        const FusedPass &fp = ps[s.pass];
-        const bool last = s.layer + 1 == P && k + 1 == seq.size();
-        const int mode = !z2 ? (int)Z2_OFF
-                         : s.pass + 1 < m ? (int)Z2_LOWER
-                                          : s.layer + 1 == P && s.kind == STEP_PLAIN && expand ? (int)Z2_EXPAND
-                                                                                                : (int)Z2_MIRROR;
-        const bool bd = s.kind == STEP_BOUNDARY;
-        const int L = bd ? s.layer + 1 : s.layer;
-        const double gamma = cost(s) ? gammas[L] : 0.0;
-        const double *pre = bd ? &betas[s.layer] : nullptr;
-        // plain passes leave their RX factor to the next cost pass, except
-        // the run's very last pass, which leaves the state exact
-        if (!mix) {
-            if (int rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST, FQ_K_FUSED,
-                                   mode, pre, !last))
+    // the passes of a layer repeat: prepared once, with each layer's factors
+    struct Prepared {
+        int pass, kind, mode;
+        MixPass mp;
+    };
+    std::vector<Prepared> made;
+    std::vector<MixPass> mps;
+    for (size_t k0 = 0; k0 < seq.size();) {
+        const size_t k1 = mix ? window_end(lp, seq, k0) : seq.size();
+        mps.clear();
+        for (size_t k = k0; k < k1; ++k) {
+            const Step &s = seq[k];
+            const FusedPass &fp = ps[s.pass];
+            const bool last = s.layer + 1 == P && k + 1 == seq.size();
+            const int mode = !z2 ? (int)Z2_OFF
+                             : s.pass + 1 < m ? (int)Z2_LOWER
+                                              : s.layer + 1 == P && s.kind == STEP_PLAIN && expand ? (int)Z2_EXPAND
+                                                                                                    : (int)Z2_MIRROR;
+            const bool bd = s.kind == STEP_BOUNDARY;
+            const int L = bd ? s.layer + 1 : s.layer;
+            const double gamma = cost(s) ? gammas[L] : 0.0;
+            const double *pre = bd ? &betas[s.layer] : nullptr;
+            // plain passes leave their RX factor to the next cost pass, except
+            // the run's very last pass, which leaves the state exact
+            if (!mix) {
+                if (int rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST,
+                                       FQ_K_FUSED, mode, pre, !last))
+                    return rc;
+                continue;
+            }
+            size_t i = 0;
+            while (i < made.size() && !(made[i].pass == s.pass && made[i].kind == s.kind && made[i].mode == mode))
+                ++i;
+            if (i == made.size()) {
+                made.push_back({s.pass, s.kind, mode, {}});
+                if (int rc = mix_prepare(st, fp.tile, fp.gates, g, cost(s), s.kind == STEP_FIRST, mode, bd, made[i].mp))
+                    return rc;
+            }
+            mps.push_back(made[i].mp);
+            mix_factors(st, fp.gates.size(), betas[L], gamma, pre, !last, mps.back());
+        }
+        bool tables = false;
+        if (int rc = mix_tables(st, mps, &tables))
+            return rc;
+        for (size_t k = k0; mix && k < k1;) {
+            const size_t n = chunk_group(lp, seq, k);
+            MixPass *const group = &mps[k - k0];
+            int rc = FQ_OK;
+            for (size_t i = 0; i < n && !tables && rc == FQ_OK; ++i)
+                rc = mix_table(st, group[i]);
+            if (rc == FQ_OK && n > 1) {
+                const int nlog = (z2 ? st->N - 1 : st->N) - lp.chunk;
+                double bytes = 0;
+                for (size_t i = 0; i < n; ++i)
+                    bytes += group[i].bytes;
+                rc = run_chunks(st, FQ_K_FUSED, n, bytes, nlog, [&](size_t i, uint64_t c, hipStream_t stream) {
+                    const MixPass &mp = group[i];
+                    return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, chunk_args(mp.a, c, nlog),
+                                      mp.ptab, stream);
+                });
+            } else if (rc == FQ_OK) {
+                const MixPass &mp = group[0];
+                rc = timed(st, FQ_K_FUSED, mp.bytes, [&] {
+                    return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, mp.a, mp.ptab, st->stream);
+                });
+            }
+            if (rc)
                 return rc;
-            continue;
+            k += n;
         }
-        // the passes of a layer repeat: prepared once, with each layer's factors
-        size_t same = 0;
-        while (same < k && !(seq[same].pass == s.pass && seq[same].kind == s.kind && modes[same] == mode))
-            ++same;
-        modes[k] = mode;
-        if (same < k)
-            mps[k] = mps[same];
-        else if (int rc = mix_prepare(st, fp.tile, fp.gates, g, cost(s), s.kind == STEP_FIRST, mode, bd, mps[k]))
-            return rc;
-        mix_factors(st, fp.gates.size(), betas[L], gamma, pre, !last, mps[k]);
-    }
-    if (!mix)
-        return FQ_OK;
-    if (int rc = mix_tables(st, mps, &tables))
-        return rc;
-    for (size_t k = 0; k < seq.size();) {
-        const size_t n = chunk_group(lp, seq, k);
-        int rc = FQ_OK;
-        for (size_t i = 0; i < n && !tables && rc == FQ_OK; ++i)
-            rc = mix_table(st, mps[k + i]);
-        if (rc == FQ_OK && n > 1) {
-            const int nlog = (z2 ? st->N - 1 : st->N) - lp.chunk;
-            double bytes = 0;
-            for (size_t i = 0; i < n; ++i)
-                bytes += mps[k + i].bytes;
-            rc = run_chunks(st, FQ_K_FUSED, n, bytes, nlog, [&](size_t i, uint64_t c, hipStream_t stream) {
-                const MixPass &mp = mps[k + i];
-                return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, chunk_args(mp.a, c, nlog), mp.ptab,
-                                  stream);
-            });
-        } else if (rc == FQ_OK) {
-            const MixPass &mp = mps[k];
-            rc = timed(st, FQ_K_FUSED, mp.bytes, [&] {
-                return launch_mix(st->dtype, mp.K, mp.lane, mp.kind, mp.mir, st->sv, mp.a, mp.ptab, st->stream);
-            });
-        }
-        if (rc)
-            return rc;
-        k += n;
+        k0 = k1;
     }
     return FQ_OK;
 }
@@ -2743,7 +2768,6 @@ struct PairPass {
     PairArgs a;
     int K = 0, kind = 0;
     bool lane = false, mir = false, cost = false;
-    double weight = 1.0;   // of the pass's sums (the states' magnitude before it)
     TileArgs tab;
     size_t entries = 0;
     const double2 *ptab = nullptr;
@@ -2796,111 +2820,121 @@ static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, cons
     for (int p = 0; p < P; ++p)
         layer_steps(lp, p, P, seq);
     std::reverse(seq.begin(), seq.end());
-    std::vector<PairPass> pp(seq.size());
-    double mag2 = 1.0;
-    for (size_t k = 0; k < seq.size(); ++k) {
-        const Step &s = seq[k];
-        PairPass &q = pp[k];
-        const bool bd = s.kind == STEP_BOUNDARY;
-        // the passes of a layer repeat: prepared once, with each layer's angles
-        size_t same = 0;
-        while (same < k && (seq[same].pass != s.pass || seq[same].kind != s.kind))
-            ++same;
-        MixArgs &a = q.a.m;
-        if (same < k) {
-            q = pp[same];
-        } else {
-            memset(&q.a, 0, sizeof(q.a));
-            q.kind = bd ? PAIR_BOUNDARY : s.kind == STEP_PLAIN ? PAIR_PLAIN : PAIR_COST;
-            q.mir = s.pass + 1 == m;
-            q.cost = q.kind != PAIR_PLAIN;
-            if (int rc = pass_shape(N, lp.ps[s.pass].tile, lp.ps[s.pass].gates, A, pair_lane_bit,
-                                    q.mir ? Z2_MIRROR : Z2_LOWER, a, q.K, q.lane))
-                return rc;
-            if (q.cost) {
-                const Geom geom = layout_geom(N, lp.ps[s.pass].tile, A, q.K);
-                geom_to_args(geom, q.tab);
-                q.tab.ntiles_run = a.ntiles;
-                if (int rc = get_plan(g, geom, &q.tab.plan, st->stream))
-                    return rc;
-                q.entries = phase_table_entries(q.tab, A);
-            }
-        }
-        double sr, si, t1, t0;
-        const int later = bd ? s.layer + 1 : s.layer;
-        rx_tform(-betas[later], st->dtype, true, &t1, &sr, &si);
-        rx_tform(-betas[s.layer], st->dtype, true, &t0, &sr, &si);
-        a.pre_t = t1;
-        a.t = bd ? t0 : t1;
-        a.pre_tf = (float)a.pre_t;   // exact for complex64
-        a.tf = (float)a.t;
-        q.weight = mag2;
-        double w = 1.0;
-        auto gate = [&](bool on, double t, double &slot) {
-            slot = on ? w : 0.0;
-            w *= on ? 1.0 / (1.0 + t * t) : 1.0;
-        };
-        gate(q.lane, t1, q.a.up[PAIR_LANE]);
-        for (int i = 0; i < A * (q.K + 1); ++i)
-            gate((a.gates_w >> i) & 1u, t1, q.a.up[i]);
-        if (q.cost) {
-            q.a.phase = w;
-            a.scale_re = std::sqrt(mag2 * w);
-            w /= a.scale_re * a.scale_re;
-            set_cost(q.tab, -gammas[later], st->init_amp);
-        }
-        if (bd) {
-            for (int l = q.K; l >= 0; --l)
-                for (int r = 0; r < A; ++r)
-                    gate((a.gates_w >> (A * l + r)) & 1u, t0, q.a.down[A * l + r]);
-            gate(q.lane, t0, q.a.down[PAIR_LANE]);
-        }
-        mag2 *= w;
-    }
     // partial sums of as many passes as fit 16 MiB at once
     const uint64_t tiles = 1ull << (N - 1 - Q);
-    const size_t per = 3 * (size_t)tiles, batch = std::max<size_t>(1, std::min(pp.size(), ((size_t)2 << 20) / per));
+    const size_t per = 3 * (size_t)tiles, batch = std::max<size_t>(1, std::min(seq.size(), ((size_t)2 << 20) / per));
     if (int rc = ensure_pair_scratch(st, batch * per))
         return rc;
-    bool tables = false;
-    if (int rc = mix_tables(st, pp, &tables, true))
-        return rc;
     const double bytes = 2.0 * (double)st->bytes;   // two half states read and written
-    auto launch = [&](size_t k, const MixArgs &a, hipStream_t stream) {
-        PairArgs pa = pp[k].a;
-        pa.m = a;
-        return launch_pair_pass(st->dtype, pp[k].K, pp[k].lane, pp[k].kind, pp[k].mir, st->sv, st->aux, pa, pp[k].ptab,
-                                pp[k].ctab, st->d_pair + per * (k % batch), stream);
+    std::vector<double> weight(seq.size());   // of each pass's sums (the states' magnitude before it)
+    // the passes of a layer repeat: prepared once, with each layer's angles
+    struct Prepared {
+        int pass, kind;
+        PairPass q;
     };
-    for (size_t k = 0; k < pp.size();) {
-        size_t n = chunk_group(lp, seq, k);
-        n = std::min(n, batch - k % batch);   // a group's sums stay within one batch
-        for (size_t i = 0; i < n && !tables; ++i)
-            if (pp[k + i].cost) {
-                double *ctab = nullptr;
-                if (int rc = prepare_phases(st, pp[k + i].tab, A, &ctab))
+    std::vector<Prepared> made;
+    std::vector<PairPass> pp;
+    double mag2 = 1.0;
+    for (size_t k0 = 0; k0 < seq.size();) {
+        const size_t k1 = std::min(window_end(lp, seq, k0), k0 + batch);
+        pp.clear();
+        for (size_t k = k0; k < k1; ++k) {
+            const Step &s = seq[k];
+            const bool bd = s.kind == STEP_BOUNDARY;
+            size_t i = 0;
+            while (i < made.size() && (made[i].pass != s.pass || made[i].kind != s.kind))
+                ++i;
+            if (i == made.size()) {
+                made.push_back({s.pass, s.kind, {}});
+                PairPass &q = made[i].q;
+                MixArgs &a = q.a.m;
+                memset(&q.a, 0, sizeof(q.a));
+                q.kind = bd ? PAIR_BOUNDARY : s.kind == STEP_PLAIN ? PAIR_PLAIN : PAIR_COST;
+                q.mir = s.pass + 1 == m;
+                q.cost = q.kind != PAIR_PLAIN;
+                if (int rc = pass_shape(N, lp.ps[s.pass].tile, lp.ps[s.pass].gates, A, pair_lane_bit,
+                                        q.mir ? Z2_MIRROR : Z2_LOWER, a, q.K, q.lane))
                     return rc;
-                pp[k + i].ptab = st->d_phase;
-                pp[k + i].ctab = ctab;
+                if (q.cost) {
+                    const Geom geom = layout_geom(N, lp.ps[s.pass].tile, A, q.K);
+                    geom_to_args(geom, q.tab);
+                    q.tab.ntiles_run = a.ntiles;
+                    if (int rc = get_plan(g, geom, &q.tab.plan, st->stream))
+                        return rc;
+                    q.entries = phase_table_entries(q.tab, A);
+                }
             }
-        int rc;
-        if (n > 1) {
-            const int nlog = N - 1 - lp.chunk;
-            rc = run_chunks(st, FQ_K_ADJOINT, n, bytes * (double)n, nlog, [&](size_t i, uint64_t c, hipStream_t stream) {
-                return launch(k + i, chunk_args(pp[k + i].a.m, c, nlog), stream);
-            });
-        } else {
-            rc = timed(st, FQ_K_ADJOINT, bytes, [&] { return launch(k, pp[k].a.m, st->stream); });
+            pp.push_back(made[i].q);
+            PairPass &q = pp.back();
+            MixArgs &a = q.a.m;
+            double sr, si, t1, t0;
+            const int later = bd ? s.layer + 1 : s.layer;
+            rx_tform(-betas[later], st->dtype, true, &t1, &sr, &si);
+            rx_tform(-betas[s.layer], st->dtype, true, &t0, &sr, &si);
+            a.pre_t = t1;
+            a.t = bd ? t0 : t1;
+            a.pre_tf = (float)a.pre_t;   // exact for complex64
+            a.tf = (float)a.t;
+            weight[k] = mag2;
+            double w = 1.0;
+            auto gate = [&](bool on, double t, double &slot) {
+                slot = on ? w : 0.0;
+                w *= on ? 1.0 / (1.0 + t * t) : 1.0;
+            };
+            gate(q.lane, t1, q.a.up[PAIR_LANE]);
+            for (int i = 0; i < A * (q.K + 1); ++i)
+                gate((a.gates_w >> i) & 1u, t1, q.a.up[i]);
+            if (q.cost) {
+                q.a.phase = w;
+                a.scale_re = std::sqrt(mag2 * w);
+                w /= a.scale_re * a.scale_re;
+                set_cost(q.tab, -gammas[later], st->init_amp);
+            }
+            if (bd) {
+                for (int l = q.K; l >= 0; --l)
+                    for (int r = 0; r < A; ++r)
+                        gate((a.gates_w >> (A * l + r)) & 1u, t0, q.a.down[A * l + r]);
+                gate(q.lane, t0, q.a.down[PAIR_LANE]);
+            }
+            mag2 *= w;
         }
-        if (rc)
+        bool tables = false;
+        if (int rc = mix_tables(st, pp, &tables, true))
             return rc;
-        k += n;
-        if (k % batch == 0 || k == pp.size()) {
-            const size_t first = (k - 1) / batch * batch;
-            FQ_HIP(launch_pair_sums(st->d_pair, tiles, (int)(k - first), out + 2 + 3 * first, st->stream));
+        auto launch = [&](size_t k, const MixArgs &a, hipStream_t stream) {
+            const PairPass &q = pp[k - k0];
+            PairArgs pa = q.a;
+            pa.m = a;
+            return launch_pair_pass(st->dtype, q.K, q.lane, q.kind, q.mir, st->sv, st->aux, pa, q.ptab, q.ctab,
+                                    st->d_pair + per * (k - k0), stream);
+        };
+        for (size_t k = k0; k < k1;) {
+            const size_t n = std::min(chunk_group(lp, seq, k), k1 - k);   // (its sums fit)
+            for (size_t i = k - k0; i < k - k0 + n && !tables; ++i)
+                if (pp[i].cost) {
+                    double *ctab = nullptr;
+                    if (int rc = prepare_phases(st, pp[i].tab, A, &ctab))
+                        return rc;
+                    pp[i].ptab = st->d_phase;
+                    pp[i].ctab = ctab;
+                }
+            int rc;
+            if (n > 1) {
+                const int nlog = N - 1 - lp.chunk;
+                rc = run_chunks(st, FQ_K_ADJOINT, n, bytes * (double)n, nlog, [&](size_t i, uint64_t c, hipStream_t stream) {
+                    return launch(k + i, chunk_args(pp[k - k0 + i].a.m, c, nlog), stream);
+                });
+            } else {
+                rc = timed(st, FQ_K_ADJOINT, bytes, [&] { return launch(k, pp[k - k0].a.m, st->stream); });
+            }
+            if (rc)
+                return rc;
+            k += n;
         }
+        FQ_HIP(launch_pair_sums(st->d_pair, tiles, (int)(k1 - k0), out + 2 + 3 * k0, st->stream));
+        k0 = k1;
     }
-    std::vector<double> sums(2 + 3 * pp.size());
+    std::vector<double> sums(2 + 3 * seq.size());
     if (out == st->d_grad)
         FQ_HIP(hipMemcpyAsync(sums.data(), out, sizeof(double) * sums.size(), hipMemcpyDeviceToHost, st->stream));
     FQ_HIP(hipStreamSynchronize(st->stream));
@@ -2910,13 +2944,14 @@ static int pair_walk(fq_state *st, fq_graph *g, const LayerPlan &lp, int P, cons
     const double *h = sums.data() + 2;
     for (int k = 0; k < P; ++k)
         grad_gammas[k] = grad_betas[k] = 0.0;
-    for (size_t k = 0; k < pp.size(); ++k) {
-        const int later = pp[k].kind == PAIR_BOUNDARY ? seq[k].layer + 1 : seq[k].layer;
-        grad_betas[later] += pp[k].weight * h[3 * k];
-        if (pp[k].cost)
-            grad_gammas[later] = -pp[k].weight * h[3 * k + 1];
-        if (pp[k].kind == PAIR_BOUNDARY)
-            grad_betas[seq[k].layer] += pp[k].weight * h[3 * k + 2];
+    for (size_t k = 0; k < seq.size(); ++k) {
+        const bool bd = seq[k].kind == STEP_BOUNDARY;
+        const int later = bd ? seq[k].layer + 1 : seq[k].layer;
+        grad_betas[later] += weight[k] * h[3 * k];
+        if (seq[k].kind != STEP_PLAIN)
+            grad_gammas[later] = -weight[k] * h[3 * k + 1];
+        if (bd)
+            grad_betas[seq[k].layer] += weight[k] * h[3 * k + 2];
     }
     return FQ_OK;
 }

@@ -10,6 +10,7 @@
 //           again: the slot's open layer takes the change once.
 //   cover   the plans of fq_run and of the gradient: per layer one RX on each qubit, after
 //           the layer's phase and before the next one's, on passes that have an instance.
+//   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
@@ -525,6 +526,38 @@ static void cover_plan(int N, const LayerPlan &lp, bool z2, int P, int (*a_log)(
     }
 }
 
+// deep <call> N dtype P: the growth of resident memory
+static int deep(const std::string &call, int N, int dtype, int P)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_state *st = nullptr;
+    ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+    const std::vector<double> gm(P, 0.3), bt(P, 0.2);
+    std::vector<double> gg(P), gb(P);
+    auto run = [&](int p) {
+        double e;
+        if (call == "backward")
+            ok(fq_backward(st, g, p, gm.data(), bt.data(), &e, gg.data(), gb.data()));
+        else
+            ok(fq_run(st, g, p, gm.data(), bt.data(), call == "z2" ? FQ_SCHED_Z2 : FQ_SCHED_FUSED));
+    };
+    auto kib = [] {   // (ru_maxrss would be the parent's where that is larger)
+        long k = 0;
+        FILE *f = fopen("/proc/self/status", "r");
+        for (char line[256]; f && fgets(line, sizeof(line), f);)
+            sscanf(line, "VmHWM: %ld", &k);
+        fclose(f);
+        return k;
+    };
+    run(256);   // (scratch as large as it gets)
+    const long before = kib();
+    run(P);
+    printf("bytes_per_layer %ld\n", (kib() - before) * 1024 / P);
+    ok(fq_state_destroy(st));
+    return 0;
+}
+
 // cover N0 N1: states of N0 to N1 qubits
 static int cover(int N0, int N1)
 {
@@ -566,6 +599,8 @@ int main(int argc, char **argv)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
     if (what == "capture" && argc == 8)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
+    if (what == "deep" && argc == 6)
+        rc = deep(argv[2], num(3), num(4), num(5));
     if (what == "cover" && argc == 4)
         rc = cover(num(2), num(3));
     if (what == "passes" && argc == 6)

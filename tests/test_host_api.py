@@ -88,3 +88,11 @@ def test_default_plans_cover_every_layer(host_api):
     types, the full and the half state."""
     r = host_api("cover", 1, 36)
     assert r["checked"] > 10000 and r["wrong"] == 0
+
+
+@pytest.mark.parametrize("call,N,dtype", [("run", 11, 0), ("run", 14, 0), ("z2", 25, 1), ("run", 27, 0),
+                                          ("backward", 14, 1), ("backward", 25, 0)])
+def test_deep_runs_stay_small(host_api, call, N, dtype):
+    """A run keeps some tens of bytes of host memory for each layer (the list of its
+    passes, a gradient's sums), not the launch arguments of all passes."""
+    assert host_api("deep", call, N, dtype, 4000)["bytes_per_layer"] < 256
