@@ -1185,9 +1185,9 @@ static int reserve_phases(fq_state *st, size_t need, size_t want = 0)
     if (need <= st->phase_cap)
         return FQ_OK;
     const size_t twice = 2 * st->phase_cap <= FQ_TABLES_BYTES ? 2 * st->phase_cap : 0;
-    const size_t cap = std::max({need, want, twice});
+    size_t cap = std::max({need, want, twice});
     void *m = nullptr;
-    if (hipMalloc(&m, cap) != hipSuccess) {
+    if (hipMalloc(&m, cap) != hipSuccess && (cap == need || hipMalloc(&m, cap = need) != hipSuccess)) {
         hipGetLastError();
         return set_err(FQ_ERR_OOM, "phase table allocation of %zu bytes failed", cap);
     }
@@ -1536,12 +1536,11 @@ static int mix_tables(fq_state *st, std::vector<Pass> &mps, bool *done, bool cut
     if (nj < 2)
         return FQ_OK;
     const size_t need = total * sizeof(double2) + ncut * sizeof(double);
-    // (a graph under capture cannot wait for memory: a table for each pass)
+    // a table for each pass where there is no memory, or a captured stream cannot get any
     if (need > st->phase_cap && is_capturing(st->stream))
         return FQ_OK;
-    if (int rc = reserve_phases(st, need, std::min(FQ_TABLE_JOBS * most * sizeof(double2) + ncut * sizeof(double),
-                                                   FQ_TABLES_FIRST)))
-        return rc;
+    if (reserve_phases(st, need, std::min(FQ_TABLE_JOBS * most * sizeof(double2) + ncut * sizeof(double), FQ_TABLES_FIRST)))
+        return FQ_OK;
     double *cut = cuts ? (double *)(st->d_phase + total) : nullptr;
     FQ_HIP(launch_phase_tables(m, nj, most, st->d_phase, cut, st->stream));
     nj = 0;
@@ -2376,8 +2375,9 @@ static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, cons
     const PlanHold hold(g);
     const std::vector<int> tile = low_tile(N);
     const int A = mix_a_log(st->dtype, N);
-    for (int p0 = 0; p0 < P; p0 += FQ_SOLO_LAYERS) {
-        const int n = std::min(FQ_SOLO_LAYERS, P - p0);
+    int most = FQ_SOLO_LAYERS;
+    for (int p0 = 0, n; p0 < P; p0 += n) {
+        n = std::min(most, P - p0);
         std::vector<MixPass> mps(n);
         SoloArgs a;
         memset(&a, 0, sizeof(a));
@@ -2417,9 +2417,12 @@ static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, cons
         bool tables = false;
         if (int rc = mix_tables(st, mps, &tables))
             return rc;
-        if (!tables && n > 1)
-            return set_err(FQ_ERR_OOM, "no memory for phase tables under capture: the same call before it makes it");
-        if (!tables)   // (one layer)
+        if (!tables && n > 1) {   // no memory for them: a layer each, in the room of one table
+            most = 1;
+            n = 0;
+            continue;
+        }
+        if (!tables)
             if (int rc = prepare_phases(st, mps[0].tab, A))
                 return rc;
         for (int i = 0; i < n; ++i)

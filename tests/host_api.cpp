@@ -10,6 +10,7 @@
 //           again: the slot's open layer takes the change once.
 //   cover   the plans of fq_run and of the gradient: per layer one RX on each qubit, after
 //           the layer's phase and before the next one's, on passes that have an instance.
+//   nomem   a run where no device memory for all its phase tables is left.
 //   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
 //
@@ -58,12 +59,17 @@ static hipError_t give(void *p)
     return hipSuccess;
 }
 
+static size_t g_largest = SIZE_MAX;   // device allocation that succeeds
+
 // While a stream is captured, allocations and waits are refused.
 static bool g_capturing = false;
 static hipError_t refuse(hipError_t e) { return g_capturing ? hipErrorStreamCaptureUnsupported : e; }
 
 extern "C" {
-hipError_t hipMalloc(void **p, size_t n) { return g_capturing ? refuse(hipSuccess) : take(p, n); }
+hipError_t hipMalloc(void **p, size_t n)
+{
+    return g_capturing ? refuse(hipSuccess) : n > g_largest ? hipErrorOutOfMemory : take(p, n);
+}
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return g_capturing ? refuse(hipSuccess) : take(p, n); }
 hipError_t hipFree(void *p) { return g_capturing ? refuse(hipSuccess) : give(p); }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c)
@@ -526,6 +532,21 @@ static void cover_plan(int N, const LayerPlan &lp, bool z2, int P, int (*a_log)(
     }
 }
 
+// nomem N dtype schedule P KiB: the largest allocation that succeeds once the state is made
+static int nomem(int N, int dtype, int sched, int P, int kib)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_state *st = nullptr;
+    ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+    const std::vector<double> gm(P, 0.3), bt(P, 0.2);
+    g_largest = (size_t)kib << 10;
+    ok(fq_run(st, g, P, gm.data(), bt.data(), sched));
+    g_largest = SIZE_MAX;
+    ok(fq_state_destroy(st));
+    return 0;
+}
+
 // deep <call> N dtype P: the growth of resident memory
 static int deep(const std::string &call, int N, int dtype, int P)
 {
@@ -599,6 +620,8 @@ int main(int argc, char **argv)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
     if (what == "capture" && argc == 8)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
+    if (what == "nomem" && argc == 7)
+        rc = nomem(num(2), num(3), num(4), num(5), num(6));
     if (what == "deep" && argc == 6)
         rc = deep(argv[2], num(3), num(4), num(5));
     if (what == "cover" && argc == 4)

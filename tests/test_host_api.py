@@ -47,6 +47,8 @@ def test_plans_stay_until_they_are_read(host_api, call, N, dtype, P, small):
     # in one that does not; a table for each pass, with and without chunks
     (12, 0, 1, (4, 64, 70)), (16, 0, 1, (4, 30, 64)), (20, 1, 1, (4, 30, 64)), (22, 0, 1, (4, 40, 64)),
     (22, 0, 2, (5, 41, 64)), (25, 1, 1, (4, 9, 20)), (28, 1, 1, (3, 6, 9)), (26, 0, 2, (5, 7, 8)),
+    # a first run of one layer makes the room of one table
+    (12, 0, 1, (1, 3, 64)), (11, 1, 2, (1, 66, 2)), (16, 0, 1, (1, 3, 64)), (22, 1, 1, (1, 4, 2)),
 ])
 def test_captured_runs_keep_their_tables(host_api, N, dtype, schedule, depths):
     """A run that is captured, deeper than the one before it, allocates nothing, and the
@@ -96,3 +98,11 @@ def test_deep_runs_stay_small(host_api, call, N, dtype):
     """A run keeps some tens of bytes of host memory for each layer (the list of its
     passes, a gradient's sums), not the launch arguments of all passes."""
     assert host_api("deep", call, N, dtype, 4000)["bytes_per_layer"] < 256
+
+
+@pytest.mark.parametrize("N,dtype,schedule,P,kib", [(12, 0, 1, 30, 64), (11, 1, 2, 67, 64), (16, 0, 1, 30, 64),
+                                                    (21, 1, 2, 30, 256)])
+def test_runs_without_memory_for_all_tables(host_api, N, dtype, schedule, P, kib):
+    """A table at a time, as before all of a run's tables were made at once."""
+    r = host_api("nomem", N, dtype, schedule, P, kib)
+    assert r["checked"] == P and r["wrong"] == 0
