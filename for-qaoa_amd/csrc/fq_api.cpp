@@ -765,6 +765,13 @@ static PlanDev place_plan(const PlanBlob &pb, char *base)
     return dev;
 }
 
+// Whether work queued on the stream is being captured into a graph.
+static bool is_capturing(hipStream_t stream)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(stream, &c) == hipSuccess && c != hipStreamCaptureStatusNone;
+}
+
 // Device cut plan of graph G for tile geometry g, cached per (geometry, W
 // content).  A new plan is uploaded asynchronously on `stream`; a cached plan
 // whose upload was queued on another stream makes `stream` wait for it.
@@ -775,6 +782,9 @@ static PlanDev place_plan(const PlanBlob &pb, char *base)
 // blocks on nothing but that plan's own earlier upload.  A held plan is not
 // replaced; if all that are large enough are held, the cache grows by the new one
 // (at most by the plans of one holder: they are the next one's to replace).
+// A new plan on a captured stream is uploaded by the captured graph, on each replay,
+// from memory of its own that stays with G: it is not cached, since no call outside
+// that graph can know when it is there.
 // entry, if not null, receives the plan's entry, which lives until the graph's
 // plan_epoch changes.
 static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream, PlanEntry **entry = nullptr)
@@ -810,6 +820,18 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
     build_plan(G, g, pb);
     const size_t total = pb.bytes.size();
     PlanEntry pe;
+    if (is_capturing(stream)) {
+        if (!plan_memory(G, align16(total), pe)) {
+            hipGetLastError();
+            return set_err(FQ_ERR_OOM, "no memory for a new plan under capture: the same call before it makes it");
+        }
+        memcpy(pe.staging, pb.bytes.data(), total);
+        FQ_HIP(hipMemcpyAsync(pe.dmem, pe.staging, total, hipMemcpyHostToDevice, stream));
+        *out = place_plan(pb, pe.dmem);
+        if (entry)
+            *entry = nullptr;
+        return FQ_OK;
+    }
     bool reused = false;
     if (G->plans.size() >= FQ_PLAN_CACHE) {
         auto victim = G->plans.end();
@@ -1168,13 +1190,6 @@ static void set_cost(TileArgs &a, double gamma, double init_amp)
 // A first buffer holds the tables of any depth where they stay below this: from 2 MiB
 // on an allocation takes 7 us instead of 0.7, and its free the same.
 #define FQ_TABLES_FIRST (((size_t)2 << 20) - 4096)
-
-// Whether work queued on the stream is being captured into a graph.
-static bool is_capturing(hipStream_t stream)
-{
-    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(stream, &c) == hipSuccess && c != hipStreamCaptureStatusNone;
-}
 
 // Phase-table buffer of at least `need` bytes (`want` where it is made).  A smaller one
 // before it stays with the state: launches in flight and captured graphs read it.  Up to
@@ -2375,7 +2390,9 @@ static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, cons
     const PlanHold hold(g);
     const std::vector<int> tile = low_tile(N);
     const int A = mix_a_log(st->dtype, N);
-    int most = FQ_SOLO_LAYERS;
+    // odd layers go down the layouts and take their cost phase in the last one
+    TileArgs tab[2];
+    int ntab = 0, most = FQ_SOLO_LAYERS;
     for (int p0 = 0, n; p0 < P; p0 += n) {
         n = std::min(most, P - p0);
         std::vector<MixPass> mps(n);
@@ -2384,15 +2401,16 @@ static int solo_run(fq_state *st, fq_graph *g, int P, const double *gammas, cons
         a.P = n;
         a.first = p0 == 0;
         a.init_amp = st->init_amp;
-        // odd layers go down the layouts and take their cost phase in the last one
-        TileArgs tab[2];
         for (int i = 0; i < std::min(n, 2); ++i) {
-            const Geom geom = layout_geom(N, tile, A, i ? 2 : 0);
-            geom_to_args(geom, tab[i]);
-            tab[i].ntiles_run = 1;
-            if (int rc = get_plan(g, geom, &tab[i].plan, st->stream))
-                return rc;
-            set_cost(tab[i], 0.0, st->init_amp);
+            if (i == ntab) {
+                const Geom geom = layout_geom(N, tile, A, i ? 2 : 0);
+                geom_to_args(geom, tab[i]);
+                tab[i].ntiles_run = 1;
+                if (int rc = get_plan(g, geom, &tab[i].plan, st->stream))
+                    return rc;
+                set_cost(tab[i], 0.0, st->init_amp);
+                ++ntab;
+            }
             a.has_rr |= tab[i].has_rr;
         }
         MixArgs shape;

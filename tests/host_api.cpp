@@ -10,6 +10,8 @@
 //           again: the slot's open layer takes the change once.
 //   cover   the plans of fq_run and of the gradient: per layer one RX on each qubit, after
 //           the layer's phase and before the next one's, on passes that have an instance.
+//   newplan a captured run whose plans are not there yet: eager runs before and between
+//           the replays make their own.
 //   nomem   a run where no device memory for all its phase tables is left.
 //   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
@@ -21,6 +23,7 @@
 
 #include "fq_api.cpp"
 
+#include <functional>
 #include <sys/mman.h>
 
 // ---- device memory and streams --------------------------------------------------
@@ -61,8 +64,17 @@ static hipError_t give(void *p)
 
 static size_t g_largest = SIZE_MAX;   // device allocation that succeeds
 
-// While a stream is captured, allocations and waits are refused.
+// While a stream is captured, allocations and waits are refused, and what is queued
+// happens when the graph is replayed.
 static bool g_capturing = false;
+static std::vector<std::function<void()>> g_nodes;
+static void now(std::function<void()> f)
+{
+    if (g_capturing)
+        g_nodes.push_back(f);
+    else
+        f();
+}
 static hipError_t refuse(hipError_t e) { return g_capturing ? hipErrorStreamCaptureUnsupported : e; }
 
 extern "C" {
@@ -80,7 +92,7 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c)
 hipError_t hipHostFree(void *p) { return give(p); }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
-    memcpy(d, s, n);
+    now([=] { memcpy(d, s, n); });
     return hipSuccess;
 }
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t)
@@ -164,9 +176,11 @@ static bool plan_ok(const PlanDev &p, int Q, int nthr, int nh)
 
 static void check(const PlanDev &p, int Q, int nthr, int nh)
 {
-    ++g_checked;
-    if (!plan_ok(p, Q, nthr, nh))
-        ++g_wrong;
+    now([=] {
+        ++g_checked;
+        if (!plan_ok(p, Q, nthr, nh))
+            ++g_wrong;
+    });
 }
 
 // Phase tables that captured launches read (and write).
@@ -532,6 +546,30 @@ static void cover_plan(int N, const LayerPlan &lp, bool z2, int P, int (*a_log)(
     }
 }
 
+// newplan N dtype schedule P
+static int newplan(int N, int dtype, int sched, int P)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_state *st = nullptr;
+    ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+    const std::vector<double> gm(P, 0.3), bt(P, 0.2);
+    auto run = [&] { ok(fq_run(st, g, P, gm.data(), bt.data(), sched)); };
+    run();
+    ok(fq_graph_add_edge(g, 0, 1, 3.0));
+    g_capturing = true;
+    run();
+    g_capturing = false;
+    for (int rep = 0; rep < 2; ++rep) {
+        run();
+        for (auto &f : g_nodes)
+            f();
+    }
+    printf("nodes %zu\n", g_nodes.size());
+    ok(fq_state_destroy(st));
+    return 0;
+}
+
 // nomem N dtype schedule P KiB: the largest allocation that succeeds once the state is made
 static int nomem(int N, int dtype, int sched, int P, int kib)
 {
@@ -620,6 +658,8 @@ int main(int argc, char **argv)
         rc = plans(argv[2], num(3), num(4), num(5), num(6));
     if (what == "capture" && argc == 8)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
+    if (what == "newplan" && argc == 6)
+        rc = newplan(num(2), num(3), num(4), num(5));
     if (what == "nomem" && argc == 7)
         rc = nomem(num(2), num(3), num(4), num(5), num(6));
     if (what == "deep" && argc == 6)

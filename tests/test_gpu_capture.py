@@ -57,3 +57,44 @@ def test_captured_run(N, dtype, schedule, P):
     st.destroy()
     gr.destroy()
     other.destroy()
+
+
+@pytest.mark.parametrize("N,dtype,schedule,P", [
+    # a layer a launch, as an eager run of one layer left room for one table; two passes
+    (12, "c128", "fused", 5), (11, "c64", "z2", 4), (14, "c128", "fused", 5), (16, "c64", "z2", 4),
+])
+def test_captured_run_on_weights_not_seen_before(N, dtype, schedule, P):
+    """Its plans are uploaded by each replay; eager runs on the same weights, before the
+    first replay and between them, have their own."""
+    print(f"captured run with new plans N={N} {dtype} {schedule} P={P}", flush=True)
+    edges = G.gnp(N, 0.4, 9600 + N, "uniform")
+    u, v, w = edges[0]
+    changed = [(u, v, w + 0.75)] + list(edges[1:])
+    g, b = G.angles(P, 9700 + N)
+    alone, fresh = State(N, C=10, dtype=dtype), Graph(N, changed)
+    alone.run(fresh, g, b, schedule)
+    want = alone.copy_out().astype(np.complex128)
+    alone.destroy()
+    fresh.destroy()
+    st, gr = State(N, C=10, dtype=dtype), Graph(N, edges)
+    s = torch.cuda.Stream()
+    st.set_stream(s.cuda_stream)
+    st.run(gr, g[:1], b[:1], schedule)
+    st.sync()
+    gr.addEdgeTo2DGraph(u, v, w + 0.75)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        st.run(gr, g, b, schedule)
+    for rep in range(3):
+        st.run(gr, g, b, schedule)
+        got = st.copy_out().astype(np.complex128)
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) < TOL[dtype], rep
+        st.run(gr, g[:1], b[:1], schedule)
+        with torch.cuda.stream(s):
+            graph.replay()
+        s.synchronize()
+        got = st.copy_out().astype(np.complex128)
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) < TOL[dtype], rep
+    del graph
+    st.destroy()
+    gr.destroy()

@@ -106,3 +106,10 @@ def test_runs_without_memory_for_all_tables(host_api, N, dtype, schedule, P, kib
     """A table at a time, as before all of a run's tables were made at once."""
     r = host_api("nomem", N, dtype, schedule, P, kib)
     assert r["checked"] == P and r["wrong"] == 0
+
+
+@pytest.mark.parametrize("N,dtype,schedule", [(12, 0, 1), (14, 0, 1), (16, 1, 2), (9, 1, 1)])
+def test_plans_first_made_under_capture(host_api, N, dtype, schedule):
+    """Their upload happens on each replay, so only the captured run may count on them."""
+    r = host_api("newplan", N, dtype, schedule, 3)
+    assert r["checked"] > 0 and r["nodes"] > 0 and r["wrong"] == 0
