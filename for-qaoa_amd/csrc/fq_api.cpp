@@ -1487,6 +1487,10 @@ static int mix_prepare(fq_state *st, const std::vector<int> &tile, const std::ve
     // order 241; 1 GiB 467 and 442; 2 GiB 944 and 997; 4 GiB 1,885 and 2,068.
     a.by_xcd = (carried <= carriers_for(st->dtype) || st->bytes >= FQ_DEALT_BYTES) && a.ntiles >= 2048 &&
                st->bytes >= 8 * FQ_CACHE_BYTES;
+    // complex64 of 2 GiB only with the top qubits in the tile (RX on qubits 10..19 of N=28
+    // 1,078 us, in order 863, by the general kernel 908; N=29 1,630 and 1,721).
+    if (st->dtype == FQ_C64 && st->bytes == 8 * FQ_CACHE_BYTES && *std::max_element(tile.begin(), tile.end()) != N - 1)
+        a.by_xcd = 0;
     mp.cost = cost;
     mp.kind = boundary ? MIX_BOUNDARY : first ? MIX_FIRST : cost ? MIX_COST : MIX_PLAIN;
     mp.mir = z2 == Z2_MIRROR ? 1 : z2 == Z2_EXPAND ? 2 : 0;
@@ -1836,6 +1840,27 @@ static int rx_targets(fq_state *st, std::vector<int> targets, double beta)
     return rx_targets_once(st, targets, beta);
 }
 
+// Tile width of an RX pass with n targets outside the low chunk (FQ_MAXQ: the full one).
+// Few targets in full tiles took longer than in the general kernel, whose work-groups
+// walk ranges of tiles: MI355X, complex64 N=28, 1 target in the middle and 5 at the top,
+// general kernel 892 and 877 us, 2^14 901 and 919, 2^12 778 and 792; complex128 N=28, 1
+// and 5 at the top, general kernel 1,605 and 1,755, 2^13 1,765 and 1,685, 2^11 1,589 and
+// 1,632.  Which width is best turns on the addresses in flight at a time, and differs
+// once the state exceeds the memory-side cache (N=24, 4 and 5 at the top, complex128:
+// general 94 and 95, 2^13 98 and 101, 2^11 97 and 109, 2^10 90 and 92): taken where it
+// was faster for targets in the middle and at the top, from 32 MiB to 8 GiB.
+static int rx_width(const fq_state *st, int n)
+{
+    if (st->bytes < (size_t)32 << 20)
+        return FQ_MAXQ;
+    const bool large = st->bytes > FQ_CACHE_BYTES;
+    if (n == 6 && st->bytes >= FQ_CACHE_BYTES)
+        return st->dtype == FQ_C64 ? 13 : 12;
+    if (st->dtype == FQ_C64)
+        return n <= 2 ? 12 : n == 3 ? 10 : n == 5 ? 11 + large : FQ_MAXQ;
+    return n == 4 ? 10 : n == 5 ? 10 + large : !large || n > 3 ? FQ_MAXQ : n == 1 ? 11 : 12;
+}
+
 static int rx_targets_once(fq_state *st, std::vector<int> targets, double beta)
 {
     const int N = st->N;
@@ -1844,20 +1869,25 @@ static int rx_targets_once(fq_state *st, std::vector<int> targets, double beta)
     if (targets.empty())
         return FQ_OK;
     if (targets.back() < Ceff) {
-        // complex64 beyond the memory-side cache: 2^11 amplitudes at least (N=28, RX on
-        // 10 qubits: a work-group per 2^10 is one wave, 935 us, the general kernel 872,
-        // 2^11 788, 2^12 790; complex128, whose 2^9 is as many bytes, 1,638 and 2^11 1,650)
-        const int Q = st->dtype == FQ_C64 && st->bytes > FQ_CACHE_BYTES ? std::max(Ceff, 11) : Ceff;
+        // complex64: no wider than it takes, but 2^11 amplitudes (a work-group per 2^10 is
+        // one wave: N=28, RX on 10 qubits 935 us, the general kernel 872, 2^11 788, 2^12
+        // 790; N=23 36, 35.5, 34.7, 34.4; 1 qubit of a chunk of 13, N=16 2^13 20.3 us,
+        // general 19.9, 2^11 16.7); chunks below 10 qubits only beyond the memory-side
+        // cache.  complex128, whose 2^9 is as many bytes: N=28 1,638, 2^11 1,650
+        int Q = Ceff;
+        if (st->dtype == FQ_C64 && (Ceff >= 10 || st->bytes > FQ_CACHE_BYTES))
+            Q = std::min(N, std::max(targets.back() + 1, 11));
         return tile_pass(st, low_tile(Q), targets, beta, nullptr, 0, false, false, FQ_K_RX);
     }
-    const int Qmax = std::min(pass_tile_q(st->dtype), N);
-    const int per = std::max(1, Qmax - std::min(carriers_for(st->dtype), Qmax - 1));
+    const int Qfull = std::min(pass_tile_q(st->dtype), N);
+    const int per = std::max(1, Qfull - std::min(carriers_for(st->dtype), Qfull - 1));
     size_t pos = 0;
     while (pos < targets.size()) {
         std::vector<int> chunk;
         while (pos < targets.size() && (int)chunk.size() < per)
             chunk.push_back(targets[pos++]);
         std::vector<int> tile;
+        const int Qmax = std::min(Qfull, rx_width(st, (int)chunk.size()));
         for (;;) {
             // the chunk's targets plus the lowest other qubits as carriers
             tile = chunk;
