@@ -1942,19 +1942,29 @@ extern "C" int fq_multi_rx(fq_state *st, const int *targets, int gate_size, doub
 static int exchange_qubits(fq_state *st, const uint8_t *partner)
 {
     const int N = st->N;
-    SwapArgs a;
-    memset(&a, 0, sizeof(a));
     int moved = 0, least = N;   // pairs; the lowest upper qubit of one
+    SwapRuns pairs;
+    pairs.n = 0;
     for (int p = 0; p < N; ++p)
         if (partner[p] > p) {
             moved++;
             least = std::min(least, (int)partner[p]);
+            if (p > 0 && partner[p - 1] == partner[p] - 1 && partner[p - 1] > p - 1)
+                pairs.run[pairs.n - 1] += 1u << 8;
+            else
+                pairs.run[pairs.n++] = (uint32_t)p | 1u << 8 | (uint32_t)partner[p] << 16;
         }
+    // an amplitude stays where the bits of each pair are equal
+    const double bytes = 2.0 * (double)st->bytes * (1.0 - std::ldexp(1.0, -moved));
+    if (st->bytes <= FQ_SWAP_SMALL)
+        return timed(st, FQ_K_SWAP, bytes, [&] { return launch_swap_small(st->dtype, st->sv, pairs, N, st->stream); });
+    SwapArgs a;
+    memset(&a, 0, sizeof(a));
     // the tile takes qubits from the lowest up, each with its partner: 2^10
     // complex128 and 2^12 complex64 amplitudes, two of them 32 and 64 KiB
     // (complex64 N=27 13 qubits with 2^10 and 2^12: 462 and 450 us; below N=24, too
     // few units for the chip: N=20 8 qubits 7.2 and 8.5)
-    const int most = std::min(N, st->dtype == FQ_C128 || N < 24 ? 10 : 12);
+    const int most = st->dtype == FQ_C128 || N < 24 ? 10 : 12;
     bool in[FQ_MAXN] = {false};
     for (int p = 0; p < N; ++p) {
         const int n = partner[p] == p ? 1 : 2;
@@ -1992,8 +2002,6 @@ static int exchange_qubits(fq_state *st, const uint8_t *partner)
     a.npairs = (1ull << lower.size()) * ((1ull << lower.size()) + 1) / 2;
     a.rest_fast = a.nr > 0 && rest[0] < least;
     a.large = st->bytes > FQ_CACHE_BYTES;
-    // an amplitude stays where the bits of each pair are equal
-    const double bytes = 2.0 * (double)st->bytes * (1.0 - std::ldexp(1.0, -moved));
     return timed(st, FQ_K_SWAP, bytes, [&] { return launch_swap(st->dtype, st->sv, a, st->stream); });
 }
 

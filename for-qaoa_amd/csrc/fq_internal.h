@@ -249,6 +249,12 @@ size_t phase_table_entries(const TileArgs &a, int a_log);
 hipError_t launch_phase_tables(const TableJobs &m, int njobs, size_t entries, double2 *tab, double *cut,
                                hipStream_t stream);
 hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t stream);
+// Runs of pairs: the lower position, their number, the upper position (bits 0, 8, 16).
+// States up to 1 MiB: a call that waits takes 12.2 to 14.2 us instead of 13.4 to 14.5 (N=4
+// to 16 complex128, the lower half with the upper one); at 2 MiB 15.2 instead of 14.5, at
+// 16 MiB 27 instead of 18, since one side of a pair is read in single amplitudes.
+#define FQ_SWAP_SMALL ((size_t)1 << 20)
+hipError_t launch_swap_small(int dtype, void *sv, const SwapRuns &pairs, int N, hipStream_t stream);
 // one: the sums of a state that is one tile come from the first launch alone.  (More
 // tiles take a second launch of one work-group: the last of them adding up instead, by a
 // fence and an atomic of each, took N=16 18.4 us instead of 18.5, N=20 22.9 instead of

@@ -699,7 +699,7 @@ __device__ __forceinline__ void swap_unit(const SwapArgs &a, uint64_t u, uint64_
     pb = base | deposit(Y, a.lower) | deposit(X, a.upper);
 }
 
-// Tiles of 2^TB amplitudes (TB = 8: or of fewer).  Persistent; the next unit's
+// Tiles of 2^TB amplitudes.  Persistent; the next unit's
 // loads are issued once the current one is in LDS (DEEP: before that, into registers of
 // their own), and the unit after that is found behind them.
 // (register arrays of the clang vector type stay in VGPRs across the loop;
@@ -712,7 +712,6 @@ __global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const Sw
     T *__restrict__ sv = reinterpret_cast<T *>(sv0);
     extern __shared__ __align__(16) unsigned char fq_smem[];
     const int tid = threadIdx.x;
-    const bool mine = TB > 8 || tid < 1 << a.tb;
     // slot of element i: i + (i >> PAD)
     T *la = reinterpret_cast<T *>(fq_smem);
     T *lb = la + (1 << TB) + (1 << (TB - PAD));
@@ -740,20 +739,17 @@ __global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const Sw
     auto load = [&](T (&x)[E], uint64_t base) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (mine)
-                x[e] = sv[base + off_r[e] + off_t];
+            x[e] = sv[base + off_r[e] + off_t];
     };
     auto put = [&](const T (&x)[E], T *l) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (mine)
-                l[to + 256 * e + ((256 * e) >> PAD)] = x[e];
+            l[to + 256 * e + ((256 * e) >> PAD)] = x[e];
     };
     auto store = [&](uint64_t base, const T *l) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (mine)
-                sv[base + off_r[e] + off_t] = l[from_t + from_r[e]];
+            sv[base + off_r[e] + off_t] = l[from_t + from_r[e]];
     };
     const uint64_t G = gridDim.x;
     uint64_t pa = 0, pb = 0, na = 0, nb = 0;
@@ -801,6 +797,25 @@ __global__ void __launch_bounds__(256) k_exchange(T0 *__restrict__ sv0, const Sw
         }
         pa = ca;
         pb = cb;
+    }
+}
+
+// The same for small states, a thread per amplitude: nothing but a launch's latency counts
+// there, and tiles through LDS took 1 us more (FQ_SWAP_SMALL).
+template <typename T>
+__global__ void __launch_bounds__(256) k_exchange_small(T *__restrict__ sv, const SwapRuns pairs, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    uint32_t j = i;
+    for (int k = 0; k < pairs.n; ++k) {
+        const uint32_t d = pairs.run[k], p = d & 0xff, q = d >> 16;
+        const uint32_t x = ((i >> p) ^ (i >> q)) & ((1u << ((d >> 8) & 0xff)) - 1u);
+        j ^= x << p | x << q;
+    }
+    if (i < j && j < n) {
+        const T a = sv[i], b = sv[j];
+        sv[i] = b;
+        sv[j] = a;
     }
 }
 
@@ -1286,8 +1301,7 @@ template <typename T, int TB> static hipError_t launch_swap_k(void *sv, const Sw
 
 template <typename T> static hipError_t launch_swap_t(void *sv, const SwapArgs &a, hipStream_t stream)
 {
-    switch (std::max(8, a.tb)) {
-        case 8: return launch_swap_k<T, 8>(sv, a, stream);
+    switch (a.tb) {
         case 9: return launch_swap_k<T, 9>(sv, a, stream);
         case 10: return launch_swap_k<T, 10>(sv, a, stream);
     }
@@ -1298,6 +1312,18 @@ template <typename T> static hipError_t launch_swap_t(void *sv, const SwapArgs &
         }
     }
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_swap_small(int dtype, void *sv, const SwapRuns &pairs, int N, hipStream_t stream)
+{
+    const dim3 grid(((1u << N) + 255u) / 256u);
+    if (dtype == 0)
+        hipLaunchKernelGGL(k_exchange_small<double2>, grid, dim3(256), 0, stream, reinterpret_cast<double2 *>(sv), pairs,
+                           1u << N);
+    else
+        hipLaunchKernelGGL(k_exchange_small<float2>, grid, dim3(256), 0, stream, reinterpret_cast<float2 *>(sv), pairs,
+                           1u << N);
+    return hipGetLastError();
 }
 
 hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t stream)

@@ -309,6 +309,7 @@ hipError_t launch_pair(int, int, bool, bool, bool, void *, void *, const TileArg
     return hipSuccess;
 }
 hipError_t launch_finalize(const double *, uint64_t, double *, hipStream_t) { return hipSuccess; }
+hipError_t launch_swap_small(int, void *, const SwapRuns &, int, hipStream_t) { return hipSuccess; }
 hipError_t launch_swap(int, void *, const SwapArgs &, hipStream_t) { return hipSuccess; }
 hipError_t launch_topk(int, const void *, int, int, double *, uint64_t *, hipStream_t) { return hipSuccess; }
 hipError_t launch_gather(int, const void *, const uint64_t *, size_t, double *, hipStream_t) { return hipSuccess; }
