@@ -280,6 +280,7 @@ struct PlanEntry {
 struct PlanBlock {
     char *dmem = nullptr, *staging = nullptr;
     size_t used = 0, size = 0;
+    bool captured = false;   // holds a plan that a captured graph uploads and reads
 };
 
 // Plans cached per graph; beyond this the least recently used plan's buffers
@@ -318,19 +319,24 @@ struct PlanHold {
     }
 };
 
-// Drops all plans of a graph; the caller has synchronized the device (hipFree
-// waits for the whole device anyway).
-static void plans_free(fq_graph *G)
+// Drops all cached plans of a graph (all: also the memory of captured graphs' plans);
+// the caller has synchronized the device (hipFree waits for the whole device anyway).
+static void plans_free(fq_graph *G, bool all)
 {
     for (auto &kv : G->plans)
         if (kv.second.ready)
             hipEventDestroy(kv.second.ready);
     G->plans.clear();
+    std::vector<PlanBlock> kept;
     for (PlanBlock &b : G->blocks) {
+        if (b.captured && !all) {
+            kept.push_back(b);
+            continue;
+        }
         hipFree(b.dmem);
         hipHostFree(b.staging);
     }
-    G->blocks.clear();
+    G->blocks.swap(kept);
 }
 
 // cap bytes of both memories for a plan, from the last block or a new one.
@@ -825,6 +831,7 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
             hipGetLastError();
             return set_err(FQ_ERR_OOM, "no memory for a new plan under capture: the same call before it makes it");
         }
+        G->blocks.back().captured = true;
         memcpy(pe.staging, pb.bytes.data(), total);
         FQ_HIP(hipMemcpyAsync(pe.dmem, pe.staging, total, hipMemcpyHostToDevice, stream));
         *out = place_plan(pb, pe.dmem);
@@ -848,7 +855,7 @@ static int get_plan(fq_graph *G, const Geom &g, PlanDev *out, hipStream_t stream
             // every cached plan is smaller than this one: drop them all (rare;
             // hipFree waits for the device in any case)
             FQ_HIP(hipDeviceSynchronize());
-            plans_free(G);
+            plans_free(G, false);
             G->plan_epoch++;
         } else if (victim != G->plans.end()) {
             pe = victim->second;
@@ -1113,7 +1120,7 @@ extern "C" int fq_graph_destroy(fq_graph *g)
         return FQ_OK;
     if (!g->blocks.empty()) {
         hipDeviceSynchronize();
-        plans_free(g);
+        plans_free(g, true);
     }
     delete g;
     return FQ_OK;
@@ -3784,7 +3791,7 @@ static int slab_again(fq_slab *sb, const SlotHost &h, fq_state *v, const std::ve
     g.W = W;
     const int rc = tile_pass(v, lp.ps[e].tile, lp.ps[e].gates, beta, &g, gamma, true, false, FQ_K_FUSED, mode, &pre, false);
     const hipError_t done = hipStreamSynchronize(sb->stream);
-    plans_free(&g);
+    plans_free(&g, true);
     return rc == FQ_OK && done != hipSuccess ? set_err(FQ_ERR_DEVICE, "slab: %s", hipGetErrorString(done)) : rc;
 }
 

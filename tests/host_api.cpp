@@ -12,6 +12,7 @@
 //           the layer's phase and before the next one's, on passes that have an instance.
 //   newplan a captured run whose plans are not there yet: eager runs before and between
 //           the replays make their own.
+//   dropped the same, after a call that drops all cached plans (64 smaller than its own).
 //   nomem   a run where no device memory for all its phase tables is left.
 //   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
@@ -571,6 +572,42 @@ static int newplan(int N, int dtype, int sched, int P)
     return 0;
 }
 
+// dropped N dtype P: <C> plans alone are cached when the run is captured
+static int dropped(int N, int dtype, int P)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_state *st = nullptr;
+    ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+    const std::vector<double> gm(P, 0.3), bt(P, 0.2);
+    auto run = [&] { ok(fq_run(st, g, P, gm.data(), bt.data(), FQ_SCHED_FUSED)); };
+    double e;
+    ok(fq_expect_cut(st, g, &e, nullptr));
+    ok(reserve_phases(st, (size_t)1 << 20));   // (room for the tables)
+    g_capturing = true;
+    run();
+    g_capturing = false;
+    const std::vector<double> W = g->W;
+    const auto nodes = g_nodes;
+    for (int i = 1; i < FQ_PLAN_CACHE; ++i) {
+        ok(fq_graph_add_edge(g, 0, 1, 3.0 + i));
+        ok(fq_expect_cut(st, g, &e, nullptr));
+    }
+    const uint64_t epoch = g->plan_epoch;
+    ok(fq_graph_add_edge(g, 0, 1, 2.0));
+    run();
+    printf("drops %d\n", (int)(g->plan_epoch - epoch));
+    const std::vector<double> W2 = g->W;
+    g->W = W;
+    for (auto &f : nodes)
+        f();
+    g->W = W2;
+    ok(fq_state_destroy(st));
+    ok(fq_graph_destroy(g));
+    printf("nodes %zu\n", nodes.size());
+    return 0;
+}
+
 // nomem N dtype schedule P KiB: the largest allocation that succeeds once the state is made
 static int nomem(int N, int dtype, int sched, int P, int kib)
 {
@@ -661,6 +698,8 @@ int main(int argc, char **argv)
         rc = capture(num(2), num(3), num(4), num(5), num(6), num(7));
     if (what == "newplan" && argc == 6)
         rc = newplan(num(2), num(3), num(4), num(5));
+    if (what == "dropped" && argc == 5)
+        rc = dropped(num(2), num(3), num(4));
     if (what == "nomem" && argc == 7)
         rc = nomem(num(2), num(3), num(4), num(5), num(6));
     if (what == "deep" && argc == 6)

@@ -113,3 +113,11 @@ def test_plans_first_made_under_capture(host_api, N, dtype, schedule):
     """Their upload happens on each replay, so only the captured run may count on them."""
     r = host_api("newplan", N, dtype, schedule, 3)
     assert r["checked"] > 0 and r["nodes"] > 0 and r["wrong"] == 0
+
+
+@pytest.mark.parametrize("N,dtype,P", [(22, 0, 2), (24, 0, 1)])
+def test_captured_plans_outlive_a_drop_of_the_cache(host_api, N, dtype, P):
+    """A call whose plans are larger than all 64 cached ones drops those, but not the memory
+    that a captured run's graph uploads its plans to and reads them from on each replay."""
+    r = host_api("dropped", N, dtype, P)
+    assert r["drops"] > 0 and r["nodes"] > 0 and r["wrong"] == 0
