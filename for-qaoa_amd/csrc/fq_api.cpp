@@ -1306,22 +1306,35 @@ struct PassFactor {
     bool apply = false;
 };
 
-static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const double *pre_beta, bool cost, bool defer)
+// (*re, *im) times sigma^n of RX(beta) on amplitudes of st; *t as in rx_tform.
+static void absorb_rx(const fq_state *st, double beta, size_t n, double *t, double *re, double *im)
+{
+    double gr, gi;
+    rx_tform(beta, st->dtype, st->in_run, t, &gr, &gi);
+    for (size_t k = 0; k < n; ++k) {
+        const double nr = *re * gr - *im * gi;
+        *im = *re * gi + *im * gr;
+        *re = nr;
+    }
+}
+
+// later: RX(beta) on that many qubits follows this cost pass in plain passes whose factor
+// goes into it (FACTOR_TAKEN, of a plain pass: it has gone into the cost pass before it).
+// The last layer of a run is done so: a factor rounded to FP32 and multiplied in before the
+// last stores is the same for all amplitudes, and took the norm and <C> of complex64 states
+// off by up to 1.2e-7; in the cost phase every thread rounds another product.
+#define FACTOR_TAKEN ((size_t)-1)
+static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const double *pre_beta, bool cost, bool defer,
+                              size_t later = 0)
 {
     PassFactor f;
     double sr = st->pending_re, si = st->pending_im;
-    auto absorb = [&](double b, double *t) {
-        double gr, gi;
-        rx_tform(b, st->dtype, st->in_run, t, &gr, &gi);
-        for (size_t k = 0; k < ngates; ++k) {
-            const double nr = sr * gr - si * gi;
-            si = sr * gi + si * gr;
-            sr = nr;
-        }
-    };
-    absorb(beta, &f.t);
+    const bool taken = later == FACTOR_TAKEN;
+    absorb_rx(st, beta, taken ? 0 : ngates + later, &f.t, &sr, &si);
     if (pre_beta)
-        absorb(*pre_beta, &f.pre_t);
+        absorb_rx(st, *pre_beta, ngates, &f.pre_t, &sr, &si);
+    if (taken)
+        return f;
     const bool keep = !cost && defer;
     if (!keep) {
         f.re = sr;
@@ -1439,10 +1452,10 @@ static int pass_shape(int N, const std::vector<int> &tile, const std::vector<int
 
 // The factors of a prepared pass and its angle: what differs between the layers.
 static void mix_factors(fq_state *st, size_t ngates, double beta, double gamma, const double *pre_beta, bool defer,
-                        MixPass &mp)
+                        MixPass &mp, size_t later = 0)
 {
     MixArgs &a = mp.a;
-    const PassFactor f = pass_factor(st, ngates, beta, pre_beta, mp.cost, defer);
+    const PassFactor f = pass_factor(st, ngates, beta, pre_beta, mp.cost, defer, later);
     a.t = f.t;
     a.pre_t = f.pre_t;
     a.tf = (float)f.t;   // exact for complex64 (rx_tform rounds t to FP32)
@@ -2366,8 +2379,9 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
             const int L = bd ? s.layer + 1 : s.layer;
             const double gamma = cost(s) ? gammas[L] : 0.0;
             const double *pre = bd ? &betas[s.layer] : nullptr;
-            // plain passes leave their RX factor to the next cost pass, except
-            // the run's very last pass, which leaves the state exact
+            // plain passes leave their RX factor to the next cost pass; those of the last
+            // layer have none after them: theirs is in its cost pass (in the plans of tuning
+            // knobs without such passes the run's very last pass multiplies it in)
             if (!mix) {
                 if (int rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST,
                                        FQ_K_FUSED, mode, pre, !last))
@@ -2383,7 +2397,8 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
                     return rc;
             }
             mps.push_back(made[i].mp);
-            mix_factors(st, fp.gates.size(), betas[L], gamma, pre, !last, mps.back());
+            const size_t later = L + 1 < P ? 0 : cost(s) ? st->N - fp.gates.size() : FACTOR_TAKEN;
+            mix_factors(st, fp.gates.size(), betas[L], gamma, pre, !last, mps.back(), later);
         }
         bool tables = false;
         if (int rc = mix_tables(st, mps, &tables))
@@ -4041,8 +4056,9 @@ static int slab_step_packed(fq_slab *sb)
                 v->pending_im = 0.0;
             }
             const int open = kind == BOUNDARY ? L + 1 : L;
-            const PassFactor f = pass_factor(v, sb->slot_plan.ps[pass].gates.size(), s.betas[open],
-                                             kind == BOUNDARY ? &s.betas[L] : nullptr, kind != PLAIN, false);
+            const size_t ng = sb->slot_plan.ps[pass].gates.size();
+            const PassFactor f = pass_factor(v, ng, s.betas[open], kind == BOUNDARY ? &s.betas[L] : nullptr, kind != PLAIN,
+                                             false, open + 1 < s.P ? 0 : kind == PLAIN ? FACTOR_TAKEN : sb->N - ng);
             MixSlot &m = h[n++];
             m.t = f.t;
             m.pre_t = f.pre_t;
@@ -4267,6 +4283,15 @@ static int slab_close_layer(fq_slab *sb, int slot, void *tmp)
     for (int q = 0; q < FQ_MAXN; ++q)
         v.qmap[q] = q;
     v.init_amp = sb->init_amp;
+    const FusedPass &open = sb->slot_plan.ps[slab_ended_on(sb, h)];
+    if (h.layer + 1 == h.P && mix_a_log(sb->dtype, (int)open.tile.size()) > 0) {
+        // (the last layer's cost pass took the factor of its plain passes: off again)
+        double t, re = 1.0, im = 0.0;
+        absorb_rx(&v, h.betas[h.layer], sb->N - open.gates.size(), &t, &re, &im);
+        const double m = re * re + im * im;
+        v.pending_re = re / m;
+        v.pending_im = -im / m;
+    }
     const int rc = slab_again(sb, h, &v, h.W, -h.betas[h.layer], -h.gammas[h.layer], 0.0);
     free_phases(&v);
     v.sv = nullptr;

@@ -16,6 +16,7 @@
 //   nomem   a run where no device memory for all its phase tables is left.
 //   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
+//   factors the factors that a run's or a slab's passes multiply in.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
 #include <hip/hip_runtime.h>
@@ -273,11 +274,24 @@ hipError_t launch_cut_mul(int, int, const void *, void *, const TileArgs &a, dou
 }
 static int g_boundaries = 0;   // boundary passes on single states
 static int g_passes = 0;       // tile passes
+static double g_factor[2] = {1.0, 0.0};   // product of the factors in the cost phases
+static int g_common = 0;       // factors common to all amplitudes, multiplied in before the stores
 hipError_t launch_mix(int, int, bool, int kind, int, void *, const MixArgs &a, const double2 *tab, hipStream_t)
 {
     note(tab);
     ++g_passes;
     g_boundaries += kind == MIX_BOUNDARY && !a.slots;
+    const int ns = a.slots ? a.nslots : 1;
+    for (int i = 0; i < ns && a.tile0 == 0; ++i) {
+        if (kind == MIX_PLAIN) {
+            g_common += a.apply_scale != 0;
+            continue;
+        }
+        const double x = a.slots ? a.slots[i].scale_re : a.scale_re, y = a.slots ? a.slots[i].scale_im : a.scale_im;
+        const double re = g_factor[0] * x - g_factor[1] * y;
+        g_factor[1] = g_factor[0] * y + g_factor[1] * x;
+        g_factor[0] = re;
+    }
     return hipSuccess;
 }
 hipError_t launch_tile(int, int, bool, bool, bool, void *, const TileArgs &, const double2 *, hipStream_t)
@@ -670,6 +684,39 @@ static int cover(int N0, int N1)
     return 0;
 }
 
+// factors <call> N dtype P: the product of all factors is that of RX(beta_p) on N qubits each
+static int factors(const std::string &call, int N, int dtype, int P)
+{
+    fq_graph *g = dense_graph(N);
+    std::vector<double> gm(P, 0.3), bt(P);
+    for (int p = 0; p < P; ++p)
+        bt[p] = 0.3 + 0.7 * p;   // (both branches of the butterfly)
+    if (call == "slab" || call == "slab_z2") {
+        fq_slab *sb = nullptr;
+        ok(fq_slab_create_sched(N, 1, dtype, call == "slab" ? FQ_SCHED_FUSED : FQ_SCHED_Z2, &sb));
+        ok(fq_slab_assign(sb, 0, g, P, gm.data(), bt.data()));
+        for (int p = 0; p < P; ++p)
+            ok(fq_slab_step(sb, nullptr));
+    } else {
+        fq_state *st = nullptr;
+        ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
+        ok(fq_run(st, g, P, gm.data(), bt.data(),
+                  call == "z2" ? FQ_SCHED_Z2 : call == "reference" ? FQ_SCHED_REFERENCE : FQ_SCHED_FUSED));
+    }
+    double t, re = 1.0, im = 0.0;
+    for (int p = 0; p < P; ++p) {
+        double sr, si;
+        rx_tform(bt[p], dtype, true, &t, &sr, &si);
+        for (int q = 0; q < N; ++q) {
+            const double x = re * sr - im * si;
+            im = re * si + im * sr;
+            re = x;
+        }
+    }
+    printf("common %d off %d\n", g_common, (int)!(std::hypot(g_factor[0] - re, g_factor[1] - im) <= 1e-12 * std::hypot(re, im)));
+    return 0;
+}
+
 // passes N dtype schedule P
 static int passes(int N, int dtype, int sched, int P)
 {
@@ -706,6 +753,8 @@ int main(int argc, char **argv)
         rc = deep(argv[2], num(3), num(4), num(5));
     if (what == "cover" && argc == 4)
         rc = cover(num(2), num(3));
+    if (what == "factors" && argc == 6)
+        rc = factors(argv[2], num(3), num(4), num(5));
     if (what == "passes" && argc == 6)
         rc = passes(num(2), num(3), num(4), num(5));
     if (what == "reopen" && argc == 5)
