@@ -18,6 +18,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace fq {
 
 // Phase tables of every active slot (layout of k_phase_table per slot, at
@@ -371,8 +373,10 @@ hipError_t launch_slab_phase_table(const TileArgs &local, int a_log, const SlotP
 hipError_t launch_slab_tables(const SlabGeos &g, const SlabJob *jobs, int njobs, size_t entries, const SlotPlans *plans,
                               double2 *tabs, hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_slab_tables, dim3((unsigned)((entries + 255) / 256), (unsigned)njobs), dim3(256), 0, stream, g,
-                       jobs, plans, tabs);
+    // (a grid is at most 65,536 wide in y: slabs of as many slots have two tables for each)
+    for (int j = 0; j < njobs; j += 32768)
+        hipLaunchKernelGGL(k_slab_tables, dim3((unsigned)((entries + 255) / 256), (unsigned)std::min(njobs - j, 32768)),
+                           dim3(256), 0, stream, g, jobs + j, plans, tabs);
     return hipGetLastError();
 }
 
