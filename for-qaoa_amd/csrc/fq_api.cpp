@@ -385,6 +385,7 @@ struct fq_state {
     // inside fq_run: every RX applies one angle to all qubits of an
     // X^(x)N-symmetric state, so rx_tform may drop its X (see rx_tform)
     bool in_run = false;
+    bool slot = false;         // a slab's slot (pass_factor)
     double *d_part = nullptr;  // expect partials
     size_t part_cap = 0;
     double *d_cand_p = nullptr;
@@ -1320,9 +1321,11 @@ static void absorb_rx(const fq_state *st, double beta, size_t n, double *t, doub
 
 // later: RX(beta) on that many qubits follows this cost pass in plain passes whose factor
 // goes into it (FACTOR_TAKEN, of a plain pass: it has gone into the cost pass before it).
-// The last layer of a run is done so: a factor rounded to FP32 and multiplied in before the
-// last stores is the same for all amplitudes, and took the norm and <C> of complex64 states
-// off by up to 1.2e-7; in the cost phase every thread rounds another product.
+// A slab's slots do the last layer so: a factor rounded to FP32 and multiplied in before the
+// last stores is the same for all amplitudes, and took <C> of complex64 slots off by up to
+// 1.2e-7 (rms of 400 requests, N=12 and 17: 8e-8 and 6e-8; the general kernel, whose RX has
+// no such factor, 5.3e-8 and 4.7e-8; now 4.9e-8 and 3.6e-8); in the cost phase every thread
+// rounds another product.
 #define FACTOR_TAKEN ((size_t)-1)
 static PassFactor pass_factor(fq_state *st, size_t ngates, double beta, const double *pre_beta, bool cost, bool defer,
                               size_t later = 0)
@@ -2379,9 +2382,9 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
             const int L = bd ? s.layer + 1 : s.layer;
             const double gamma = cost(s) ? gammas[L] : 0.0;
             const double *pre = bd ? &betas[s.layer] : nullptr;
-            // plain passes leave their RX factor to the next cost pass; those of the last
-            // layer have none after them: theirs is in its cost pass (in the plans of tuning
-            // knobs without such passes the run's very last pass multiplies it in)
+            // plain passes leave their RX factor to the next cost pass, except
+            // the run's very last pass, which leaves the state exact (a slot's: in its
+            // last layer's cost pass)
             if (!mix) {
                 if (int rc = tile_pass(st, fp.tile, fp.gates, betas[L], g, gamma, cost(s), s.kind == STEP_FIRST,
                                        FQ_K_FUSED, mode, pre, !last))
@@ -2397,7 +2400,7 @@ static int run_layers(fq_state *st, fq_graph *g, const LayerPlan &lp, int p0, in
                     return rc;
             }
             mps.push_back(made[i].mp);
-            const size_t later = L + 1 < P ? 0 : cost(s) ? st->N - fp.gates.size() : FACTOR_TAKEN;
+            const size_t later = !st->slot || L + 1 < P ? 0 : cost(s) ? st->N - fp.gates.size() : FACTOR_TAKEN;
             mix_factors(st, fp.gates.size(), betas[L], gamma, pre, !last, mps.back(), later);
         }
         bool tables = false;
@@ -3748,6 +3751,7 @@ static int slab_make_views(fq_slab *sb)
             v->qmap[q] = q;
         v->init_amp = sb->init_amp;
         v->in_run = true;   // a slot runs fq_run's layers on a QAOA state
+        v->slot = true;
         sb->views.push_back(v);
         if (need && hipMalloc(&v->d_phase, need) != hipSuccess) {
             hipGetLastError();

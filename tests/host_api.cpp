@@ -16,7 +16,7 @@
 //   nomem   a run where no device memory for all its phase tables is left.
 //   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
-//   factors the factors that a run's or a slab's passes multiply in.
+//   factors the factors that the passes of a slab's request multiply in.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
 #include <hip/hip_runtime.h>
@@ -691,18 +691,12 @@ static int factors(const std::string &call, int N, int dtype, int P)
     std::vector<double> gm(P, 0.3), bt(P);
     for (int p = 0; p < P; ++p)
         bt[p] = 0.3 + 0.7 * p;   // (both branches of the butterfly)
-    if (call == "slab" || call == "slab_z2") {
-        fq_slab *sb = nullptr;
-        ok(fq_slab_create_sched(N, 1, dtype, call == "slab" ? FQ_SCHED_FUSED : FQ_SCHED_Z2, &sb));
-        ok(fq_slab_assign(sb, 0, g, P, gm.data(), bt.data()));
-        for (int p = 0; p < P; ++p)
-            ok(fq_slab_step(sb, nullptr));
-    } else {
-        fq_state *st = nullptr;
-        ok(fq_state_create(N, 0, 0, std::min(N, 10), dtype, &st));
-        ok(fq_run(st, g, P, gm.data(), bt.data(),
-                  call == "z2" ? FQ_SCHED_Z2 : call == "reference" ? FQ_SCHED_REFERENCE : FQ_SCHED_FUSED));
-    }
+    fq_slab *sb = nullptr;
+    ok(fq_slab_create_sched(N, 1, dtype, call == "slab" ? FQ_SCHED_FUSED : FQ_SCHED_Z2, &sb));
+    ok(fq_slab_assign(sb, 0, g, P, gm.data(), bt.data()));
+    for (int p = 0; p < P; ++p)
+        ok(fq_slab_step(sb, nullptr));
+    ok(fq_slab_destroy(sb));
     double t, re = 1.0, im = 0.0;
     for (int p = 0; p < P; ++p) {
         double sr, si;
