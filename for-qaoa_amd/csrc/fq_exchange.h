@@ -19,8 +19,11 @@ namespace fq {
 // W: the LDS slot of tile element e is the sum of W[i] over its set bits i, so
 // the thread's and the register's parts add and the latter is an address
 // constant.  W[i] is 2^i plus paddings that keep the map injective and put
-// the lanes of every layout on distinct banks (32 distinct 8-byte slots per
-// half wave in FP64, 64 distinct 4-byte slots per wave in FP32).
+// the lanes of a layout on distinct banks (32 distinct 8-byte slots per
+// half wave in FP64, 64 distinct 4-byte slots per wave in FP32).  So it is in
+// every layout but four of the narrowest tiles: 20 of 32 slots in layout 2 of
+// (double, 9, 3, 2), 36 of 64 in layout 2 of (float, 11, 4, 2), 32 and 33 of 64 in
+// layouts 1 and 2 of (float, 10, 4, 2).
 // P: tile bit of each thread bit, per layout.
 template <typename R, int Q, int A, int K> struct MixGeo;
 
