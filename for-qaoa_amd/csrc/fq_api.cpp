@@ -4101,6 +4101,20 @@ static int slab_step_packed(fq_slab *sb)
     return FQ_OK;
 }
 
+// The plans of slots [k0, k1) to the device.  Slots that enter together go in one copy,
+// with what lies between them (a copy takes 4 us, a slot's plans are 1.7 KB): 4 requests
+// on a slab of N=3 complex64 slots 149 us with a copy for each.
+static int slab_upload_plans(fq_slab *sb, int k0, int k1)
+{
+    if (k0 == k1)
+        return FQ_OK;
+    FQ_HIP(hipMemcpyAsync(sb->d_plans + k0, sb->h_plans + k0, sizeof(SlotPlans) * (size_t)(k1 - k0), hipMemcpyHostToDevice,
+                          sb->stream));
+    for (int k = k0; k < k1; ++k)
+        sb->slots[k].fresh = false;
+    return FQ_OK;
+}
+
 // Advance every active slot by one layer: one packed launch per tile pass.
 // Slots that complete their last layer also get <C> reduced; their results
 // are read with fq_slab_collect once fq_slab_poll reports the step done.
@@ -4146,6 +4160,7 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
     SlotParams *params = (SlotParams *)sb->h_step;
     int *fin = (int *)(sb->h_step + step_fin(K));
     int nact = 0, nfin = 0;
+    int fresh0 = 0, fresh1 = 0;   // slots with new plans, not uploaded yet
     for (int k = 0; k < K; ++k) {
         SlotHost &h = sb->slots[k];
         SlotParams &sp = params[k];
@@ -4154,8 +4169,12 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
             continue;
         if (h.fresh) {
             sb->h_plans[k] = h.plans;
-            FQ_HIP(hipMemcpyAsync(sb->d_plans + k, sb->h_plans + k, sizeof(SlotPlans), hipMemcpyHostToDevice, sb->stream));
-            h.fresh = false;
+            if (fresh1 == 0 || k - fresh1 > 8) {
+                if (int rc = slab_upload_plans(sb, fresh0, fresh1))
+                    return rc;
+                fresh0 = k;
+            }
+            fresh1 = k + 1;
         }
         nl[k] = sb->per_slot ? std::min(sb->layers_per_step, h.P - h.layer) : 1;
         const int L = h.layer;
@@ -4172,6 +4191,8 @@ extern "C" int fq_slab_step(fq_slab *sb, int *nfinishing)
         if (L + nl[k] == h.P)
             fin[nfin++] = k;
     }
+    if (int rc = slab_upload_plans(sb, fresh0, fresh1))
+        return rc;
     if (nfinishing)
         *nfinishing = nfin;
     if (nact == 0)

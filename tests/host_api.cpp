@@ -16,6 +16,7 @@
 //   nomem   a run where no device memory for all its phase tables is left.
 //   deep    host memory that a run or a gradient of many layers takes.
 //   passes  the launches of a slab's request, and what fq_slab_passes says.
+//   copies  the copies to the device in a step that slots enter.
 //   factors the factors that the passes of a slab's request multiply in.
 //
 // Each run prints "checked <n> wrong <m>"; tests/test_host_api.py has the programs.
@@ -92,8 +93,10 @@ hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c)
     return hipSuccess;
 }
 hipError_t hipHostFree(void *p) { return give(p); }
+static int g_copies = 0;
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
+    ++g_copies;
     now([=] { memcpy(d, s, n); });
     return hipSuccess;
 }
@@ -684,6 +687,31 @@ static int cover(int N0, int N1)
     return 0;
 }
 
+// copies N dtype K: slots 0, 3, 6 .. of K enter, then the others; every slot's result
+// comes from its own graph's plans
+static int copies(int N, int dtype, int K)
+{
+    fq_graph *g = dense_graph(N);
+    all_geoms(N, dtype);
+    fq_slab *sb = nullptr;
+    ok(fq_slab_create_sched(N, K, dtype, FQ_SCHED_Z2, &sb));
+    const std::vector<double> gm(3, 0.3), bt(3, 0.2);
+    int most = 0;
+    for (int rest = 0; rest < 2; ++rest) {
+        for (int k = 0; k < K; ++k)
+            if ((k % 3 != 0) == (rest != 0))
+                ok(fq_slab_assign(sb, k, g, 3, gm.data(), bt.data()));
+        g_copies = 0;
+        ok(fq_slab_step(sb, nullptr));
+        most = std::max(most, g_copies);
+    }
+    for (int p = 0; p < 3; ++p)
+        ok(fq_slab_step(sb, nullptr));
+    ok(fq_slab_destroy(sb));
+    printf("copies %d\n", most);
+    return 0;
+}
+
 // factors <call> N dtype P: the product of all factors is that of RX(beta_p) on N qubits each
 static int factors(const std::string &call, int N, int dtype, int P)
 {
@@ -747,6 +775,8 @@ int main(int argc, char **argv)
         rc = deep(argv[2], num(3), num(4), num(5));
     if (what == "cover" && argc == 4)
         rc = cover(num(2), num(3));
+    if (what == "copies" && argc == 5)
+        rc = copies(num(2), num(3), num(4));
     if (what == "factors" && argc == 6)
         rc = factors(argv[2], num(3), num(4), num(5));
     if (what == "passes" && argc == 6)

@@ -134,3 +134,10 @@ def test_factors_of_slots_go_into_the_cost_phases(host_api, call, N, dtype, P):
     norm), and their product is that of the layers' RX: 1e-12, some N P roundings in FP64."""
     r = host_api("factors", call, N, dtype, P)
     assert r["common"] == 0 and r["off"] == 0
+
+
+@pytest.mark.parametrize("N,dtype,K", [(8, 1, 16), (16, 1, 32), (12, 0, 4)])
+def test_plans_of_slots_that_enter_together_go_in_one_copy(host_api, N, dtype, K):
+    """And the step's parameters in another."""
+    r = host_api("copies", N, dtype, K)
+    assert r["copies"] == 2 and r["checked"] > K and r["wrong"] == 0
