@@ -255,13 +255,12 @@ hipError_t launch_swap(int dtype, void *sv, const SwapArgs &a, hipStream_t strea
 // 16 MiB 27 instead of 18, since one side of a pair is read in single amplitudes.
 #define FQ_SWAP_SMALL ((size_t)1 << 20)
 hipError_t launch_swap_small(int dtype, void *sv, const SwapRuns &pairs, int N, hipStream_t stream);
-// one: the sums of a state that is one tile come from the first launch alone.  (More
-// tiles take a second launch of one work-group: the last of them adding up instead, by a
-// fence and an atomic of each, took N=16 18.4 us instead of 18.5, N=20 22.9 instead of
-// 19.4, N=22 46 instead of 28.5, and N=3, whose work-group is one thread, 135 instead
-// of 15.)
+// partials == out2: the sums of each tile, without the second launch of one work-group that
+// adds them up.  (The last work-group adding up instead, by a fence and an atomic of each,
+// took N=16 18.4 us instead of 18.5, N=20 22.9 instead of 19.4, N=22 46 instead of 28.5, and
+// N=3, whose work-group is one thread, 135 instead of 15.)
 hipError_t launch_expect(int dtype, int a_log, const void *sv, const TileArgs &a, double *partials,
-                         double *out2, bool one, hipStream_t stream);
+                         double *out2, hipStream_t stream);
 hipError_t launch_topk(int dtype, const void *sv, int N, int nblocks, double *cand_p,
                        uint64_t *cand_i, hipStream_t stream);
 hipError_t launch_gather(int dtype, const void *sv, const uint64_t *idx, size_t n, double *out,

@@ -1352,10 +1352,8 @@ hipError_t launch_finalize(const double *partials, uint64_t n, double *out2, hip
 }
 
 hipError_t launch_expect(int dtype, int a_log, const void *sv, const TileArgs &a, double *partials,
-                         double *out2, bool one, hipStream_t stream)
+                         double *out2, hipStream_t stream)
 {
-    if (one && run_tiles(a) == 1)
-        partials = out2;
 #define FQ_EXP(R)                                                              \
     switch (a_log) {                                                           \
         case 1: return launch_expect_t<R, 1>(sv, a, partials, out2, stream);   \

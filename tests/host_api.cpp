@@ -265,7 +265,7 @@ hipError_t launch_slab_expect(int, int a_log, const void *, const TileArgs &a, c
     (void)slot_shift;
     return hipSuccess;
 }
-hipError_t launch_expect(int, int, const void *, const TileArgs &a, double *, double *, bool, hipStream_t)
+hipError_t launch_expect(int, int, const void *, const TileArgs &a, double *, double *, hipStream_t)
 {
     check(a.plan, a.Q, a.nthr, a.nh);
     return hipSuccess;
